@@ -37,6 +37,7 @@
 #include "records.hh"
 #include "ell.hh"
 #include "eigen.hh"
+#include "pack.hh"
 #include <cmath>
 #include <algorithm>
 
@@ -52,6 +53,7 @@ inline int nblocks(int64_t n, int bs = kBlock) { return int(std::max<int64_t>(1,
 struct DSub {
   double enterP[3], enterN[3], exitP[3], exitN[3];
   int reflect;
+  int periodicSecond;
   double R[9];
 };
 
@@ -61,6 +63,7 @@ DSub toDevice(const SubBoundary& b) {
     d.enterP[k] = b.enterP[k]; d.enterN[k] = b.enterN[k]; d.exitP[k] = b.exitP[k]; d.exitN[k] = b.exitN[k];
   }
   d.reflect = b.reflect;
+  d.periodicSecond = b.periodicSecond;
   for (int k = 0; k < 9; ++k) d.R[k] = b.R[k];
   return d;
 }
@@ -295,67 +298,114 @@ __global__ void k_gen_advance(GenDev* g, int b, const int32_t* __restrict__ tota
 }
 
 struct FieldPtrs {
-  double *pos, *H, *vel, *mass, *rho, *eps, *P, *cs, *omega, *fCl, *fCq, *fsh;
+  double *pos, *H, *vel, *mass, *rho, *eps, *P, *cs, *omega, *fCl, *fCq, *fsh, *seg;
 };
 
-// Ghost rows [g0, g1) of one sub-boundary from their controls.
-template <int D>
-__global__ void k_ghost_fields(FieldPtrs f, int64_t g0, int64_t g1, int64_t nInt, const int32_t* __restrict__ control,
-                               DSub b, int geometry) {
+// Where a ghost's values come from: its control may be a ghost of an earlier
+// plane (edges and corners of a box), so a ghost is reached from an internal
+// node by `depth` plane maps.  Every kernel below gives one lane to a ghost of
+// any plane and applies those maps in order from the internal node, the same
+// operations on the same values as filling plane after plane from the stored
+// ghosts, so one launch serves all planes: a 2-D box step went from 12 + 4
+// launches of 4.3 us (ghost fields, densities) to 4.
+struct GhostMap {
+  const int32_t* control;
+  const int32_t* subOf;
+  const DSub* subs;
+  int64_t nInt;
+};
+// The internal node a ghost descends from, and the number of maps.
+__device__ __forceinline__ int64_t ghostRoot(const GhostMap& m, int64_t g, int& depth) {
+  depth = 0;
+  while (g >= m.nInt) {
+    g = m.control[g - m.nInt];
+    ++depth;
+  }
+  return g;
+}
+// The plane of the map `step` controls below ghost g (step 0: g's own).
+__device__ __forceinline__ const DSub& ghostPlane(const GhostMap& m, int64_t g, int step) {
+  for (int q = 0; q < step; ++q) g = m.control[g - m.nInt];
+  return m.subs[m.subOf[g - m.nInt]];
+}
+
+// All ghost rows [nInt, nTot) from their internal nodes.  REC >= 0: also their
+// slots' records (pack sec bits, isotropic layout) from the values just stored.
+template <int D, int REC>
+__global__ void k_ghost_fields(FieldPtrs f, GhostMap m, int64_t nTot, int geometry, const int32_t* __restrict__ iperm,
+                               PackIn pin, PackOut pout) {
   constexpr int NS = NSym<D>::value;
-  const int64_t g = g0 + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (g >= g1) return;
-  const int64_t c = control[g - nInt];
+  const int64_t g = m.nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (g >= nTot) return;
+  int depth;
+  const int64_t r = ghostRoot(m, g, depth);
+  V<D> x, v = loadV<D>(f.vel, r);
+  double h[NS];
   if (geometry) {
-    const V<D> xg = ghostPosition<D>(b, loadV<D>(f.pos, c));
-    for (int k = 0; k < D; ++k) f.pos[g * D + k] = xg.c[k];
+    x = loadV<D>(f.pos, r);
+    for (int k = 0; k < NS; ++k) h[k] = f.H[r * NS + k];
+  }
+  for (int step = depth - 1; step >= 0; --step) {
+    const DSub& b = ghostPlane(m, g, step);
+    if (geometry) x = ghostPosition<D>(b, x);
     if (b.reflect) {
-      double hg[NS];
-      reflectH<D>(b.R, f.H + c * NS, hg);
-      for (int k = 0; k < NS; ++k) f.H[g * NS + k] = hg[k];
-    } else {
-      for (int k = 0; k < NS; ++k) f.H[g * NS + k] = f.H[c * NS + k];
+      v = reflectV<D>(b.R, v);
+      if (geometry) {
+        double hg[NS];
+        reflectH<D>(b.R, h, hg);
+        for (int k = 0; k < NS; ++k) h[k] = hg[k];
+      }
     }
   }
-  const V<D> v = loadV<D>(f.vel, c);
-  const V<D> vg = b.reflect ? reflectV<D>(b.R, v) : v;
-  for (int k = 0; k < D; ++k) f.vel[g * D + k] = vg.c[k];
-  f.mass[g] = f.mass[c];
-  f.rho[g] = f.rho[c];
-  f.eps[g] = f.eps[c];
-  f.P[g] = f.P[c];
-  f.cs[g] = f.cs[c];
-  f.omega[g] = f.omega[c];
-  if (f.fCl) { f.fCl[g] = f.fCl[c]; f.fCq[g] = f.fCq[c]; f.fsh[g] = f.fsh[c]; }
+  if (geometry) {
+    for (int k = 0; k < D; ++k) f.pos[g * D + k] = x.c[k];
+    for (int k = 0; k < NS; ++k) f.H[g * NS + k] = h[k];
+  }
+  for (int k = 0; k < D; ++k) f.vel[g * D + k] = v.c[k];
+  f.mass[g] = f.mass[r];
+  f.rho[g] = f.rho[r];
+  f.eps[g] = f.eps[r];
+  f.P[g] = f.P[r];
+  f.cs[g] = f.cs[r];
+  f.omega[g] = f.omega[r];
+  if (f.fCl) { f.fCl[g] = f.fCl[r]; f.fCq[g] = f.fCq[r]; f.fsh[g] = f.fsh[r]; }
+  if (f.seg) f.seg[g] = f.seg[r];
+  if constexpr (REC >= 0) packSlot<D, true, REC>(iperm[g], pin, pout);
 }
 
-__global__ void k_ghost_scalar(double* __restrict__ a, int64_t g0, int64_t g1, int64_t nInt,
-                               const int32_t* __restrict__ control) {
-  const int64_t g = g0 + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (g < g1) a[g] = a[control[g - nInt]];
+__global__ void k_ghost_scalar(double* __restrict__ a, GhostMap m, int64_t nTot) {
+  const int64_t g = m.nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  int depth;
+  if (g < nTot) a[g] = a[ghostRoot(m, g, depth)];
 }
 
-// A Vector field on ghost rows [g0, g1): R.a of the control for a reflecting
-// plane, a copy for a periodic one (ReflectingBoundary.cc:106-125).
+// A Vector field on the ghost rows: R.a for every reflecting map, a copy for a
+// periodic one (ReflectingBoundary.cc:106-125).
 template <int D>
-__global__ void k_ghost_vector(double* __restrict__ a, int64_t g0, int64_t g1, int64_t nInt,
-                               const int32_t* __restrict__ control, DSub b) {
-  const int64_t g = g0 + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (g >= g1) return;
-  const V<D> v = loadV<D>(a, control[g - nInt]);
-  const V<D> o = b.reflect ? reflectV<D>(b.R, v) : v;
-  for (int k = 0; k < D; ++k) a[g * D + k] = o.c[k];
+__global__ void k_ghost_vector(double* __restrict__ a, GhostMap m, int64_t nTot) {
+  const int64_t g = m.nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (g >= nTot) return;
+  int depth;
+  V<D> v = loadV<D>(a, ghostRoot(m, g, depth));
+  for (int step = depth - 1; step >= 0; --step) {
+    const DSub& b = ghostPlane(m, g, step);
+    if (b.reflect) v = reflectV<D>(b.R, v);
+  }
+  for (int k = 0; k < D; ++k) a[g * D + k] = v.c[k];
 }
 
-// Ghost records after sum density: the same expressions as the internal update.
+// Ghost densities and records after sum density: the density of the internal
+// node, and the same expressions as the internal update.
 template <bool ISO>
-__global__ void k_ghost_records(double* __restrict__ rec, const int32_t* __restrict__ iperm,
-                                const double* __restrict__ rho, int64_t nInt, int64_t nTot) {
+__global__ void k_ghost_records(double* __restrict__ rec, const int32_t* __restrict__ iperm, double* __restrict__ rho,
+                                GhostMap map, int64_t nTot) {
   using R = RL<ISO>;
-  const int64_t g = nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  const int64_t g = map.nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (g >= nTot) return;
+  int depth;
+  const double acc = rho[ghostRoot(map, g, depth)];
+  rho[g] = acc;
   double* r = rec + int64_t(iperm[g]) * R::STRIDE;
-  const double acc = rho[g];
   const double som = r[R::SOM], p = r[R::P], m = r[R::M];
   r[R::RHO] = acc;
   r[R::PRHO] = som * p / (acc * acc);
@@ -374,17 +424,14 @@ template <int D> __device__ __forceinline__ bool behind(const double* P, const d
 // nodes, with ReflectingBoundary::enforceBoundary of v and H
 // ((R*H)*R).Symmetric(), src/Boundary/ReflectingBoundary.cc:240-282).
 template <int D>
-__global__ void k_enforce(double* __restrict__ pos, double* __restrict__ vel, double* __restrict__ H, int64_t nInt,
-                          DSub b) {
+__device__ __forceinline__ bool enforcePlane(const DSub& b, V<D>& x, double* __restrict__ vel, double* __restrict__ H,
+                                             int64_t i) {
   constexpr int NS = NSym<D>::value;
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (i >= nInt) return;
-  const V<D> x = loadV<D>(pos, i);
-  if (!behind<D>(b.enterP, b.enterN, x)) return;
+  if (!behind<D>(b.enterP, b.enterN, x)) return false;
   // mapPosition(x, enterPlane, exitPlane)
   const V<D> p0 = closestPoint<D>(b.exitP, b.exitN, x);
   const double sd = signedDist<D>(b.enterP, b.enterN, x);
-  for (int k = 0; k < D; ++k) pos[i * D + k] = p0.c[k] - b.exitN[k] * sd;
+  for (int k = 0; k < D; ++k) x.c[k] = p0.c[k] - b.exitN[k] * sd;
   if (b.reflect) {
     const V<D> v = reflectV<D>(b.R, loadV<D>(vel, i));
     for (int k = 0; k < D; ++k) vel[i * D + k] = v.c[k];
@@ -408,22 +455,38 @@ __global__ void k_enforce(double* __restrict__ pos, double* __restrict__ vel, do
     for (int a = 0; a < D; ++a)
       for (int q = a; q < D; ++q, ++c) H[i * NS + c] = (a == q) ? t2[a * D + a] : 0.5 * (t2[a * D + q] + t2[q * D + a]);
   }
+  return true;
 }
 
 // PeriodicBoundary::updateViolationNodes: nodes still outside either plane
 // are wrapped by the fmod rule (src/Boundary/PeriodicBoundary.cc:176-207).
-template <int D>
-__global__ void k_periodic_wrap(double* __restrict__ pos, int64_t nInt, DSub b) {
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (i >= nInt) return;
-  const V<D> x = loadV<D>(pos, i);
-  // plane1 = enter, plane2 = exit of the first half of the pair
-  if (!(behind<D>(b.enterP, b.enterN, x) || behind<D>(b.exitP, b.exitN, x))) return;
+// b: the first half of the pair (plane1 = enter, plane2 = exit).
+template <int D> __device__ __forceinline__ bool wrapPair(const DSub& b, V<D>& x) {
+  if (!(behind<D>(b.enterP, b.enterN, x) || behind<D>(b.exitP, b.exitN, x))) return false;
   const V<D> p2 = arr<D>(b.exitP);
   const double L = dabs(signedDist<D>(b.enterP, b.enterN, p2));
   const double s = vdot(vsub(arr<D>(b.enterP), x), arr<D>(b.enterN));
   const double f = dmax(-1.0, dmin(1.0, fmod(signedDist<D>(b.enterP, b.enterN, x) / L, 1.0)));
-  for (int k = 0; k < D; ++k) pos[i * D + k] = (x.c[k] + b.enterN[k] * s) + b.enterN[k] * (f * L);
+  for (int k = 0; k < D; ++k) x.c[k] = (x.c[k] + b.enterN[k] * s) + b.enterN[k] * (f * L);
+  return true;
+}
+
+// Every plane in order on one node per lane (a node's enforcement reads no
+// other node): one launch instead of one per plane and periodic pair.
+template <int D>
+__global__ void k_enforce(double* __restrict__ pos, double* __restrict__ vel, double* __restrict__ H, int64_t nInt,
+                          const DSub* __restrict__ subs, int nSubs) {
+  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (i >= nInt) return;
+  V<D> x = loadV<D>(pos, i);
+  bool moved = false;
+  for (int q = 0; q < nSubs; ++q) {
+    moved |= enforcePlane<D>(subs[q], x, vel, H, i);
+    // the second half of a periodic pair closes it: wrap what is still outside
+    if (subs[q].periodicSecond) moved |= wrapPair<D>(subs[q - 1], x);
+  }
+  if (moved)
+    for (int k = 0; k < D; ++k) pos[i * D + k] = x.c[k];
 }
 
 // ---- culling ---------------------------------------------------------------
@@ -444,48 +507,34 @@ __global__ void k_keep_controls(int32_t* __restrict__ keep, int64_t nInt, int64_
   if (c >= nInt) keep[c] = 1;
 }
 
-// Compact the ghost rows [i0, n) of one caller-order field of `comps`
-// doubles per row (internal rows keep their place).
-__global__ void k_compact_rows(const double* __restrict__ src, double* __restrict__ dst, int comps,
-                               const int32_t* __restrict__ keep, const int32_t* __restrict__ scan, int64_t i0,
-                               int64_t n) {
-  const int64_t i = i0 + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (i >= n || !keep[i]) return;
-  const int64_t o = scan[i];
-  for (int c = 0; c < comps; ++c) dst[o * comps + c] = src[i * comps + c];
-}
-
-__global__ void k_compact_ghosts(const int32_t* __restrict__ control, const int32_t* __restrict__ subOf,
-                                 int32_t* __restrict__ newControl, int32_t* __restrict__ newSubOf,
-                                 const int32_t* __restrict__ keep, const int32_t* __restrict__ scan,
-                                 int64_t nInt, int64_t nTot) {
-  const int64_t g = nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (g >= nTot || !keep[g]) return;
-  const int64_t o = scan[g] - nInt;
-  newControl[o] = scan[control[g - nInt]];
-  newSubOf[o] = subOf[g - nInt];
-}
-
-// Slots keep their place; their caller index is renumbered, culled ones die.
-// The records (when current) take the new caller index; nothing else in a
-// record depends on the numbering, so they stay valid.
-__global__ void k_perm_remap(int32_t* __restrict__ perm, const int32_t* __restrict__ keep,
-                             const int32_t* __restrict__ scan, int64_t nSlots, double* __restrict__ rec, int stride,
-                             int origOff) {
-  const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (k >= nSlots) return;
-  const int32_t c = perm[k];
-  if (c < 0) return;
-  const int32_t nc = keep[c] ? scan[c] : -1;
-  perm[k] = nc;
-  const double o = nc >= 0 ? double(nc) : 2147483648.0;
-  if (rec) rec[k * stride + origOff] = o;
-}
-
-__global__ void k_iperm_remap(const int32_t* __restrict__ iperm, const int32_t* __restrict__ keep,
-                              const int32_t* __restrict__ scan, int64_t n, int32_t* __restrict__ out) {
-  const int64_t c = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (c < n && keep[c]) out[scan[c]] = iperm[c];
+// Renumbering after the cull, one lane per caller row and slot: the kept
+// ghosts' controls and planes, the caller -> slot map, and the slots' caller
+// index (slots keep their place, culled ones die).  The records (when current)
+// take the new caller index; nothing else in a record depends on the
+// numbering, so they stay valid.  The ghosts' state rows are not moved but
+// filled again at their new place: two launches in place of two per field and
+// three more (22 in 2-D).
+__global__ void k_cull(const int32_t* __restrict__ control, const int32_t* __restrict__ subOf,
+                       int32_t* __restrict__ newControl, int32_t* __restrict__ newSubOf,
+                       const int32_t* __restrict__ iperm, int32_t* __restrict__ newIperm, int32_t* __restrict__ perm,
+                       const int32_t* __restrict__ keep, const int32_t* __restrict__ scan, int64_t nInt, int64_t nTot,
+                       int64_t nSlots, double* __restrict__ rec, int stride, int origOff) {
+  const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (t < nTot && keep[t]) {
+    const int64_t o = scan[t];
+    newIperm[o] = iperm[t];
+    if (t >= nInt) {
+      newControl[o - nInt] = scan[control[t - nInt]];
+      newSubOf[o - nInt] = subOf[t - nInt];
+    }
+  }
+  if (t < nSlots) {
+    const int32_t c = perm[t];
+    if (c < 0) return;
+    const int32_t nc = keep[c] ? scan[c] : -1;
+    perm[t] = nc;
+    if (rec) rec[t * stride + origOff] = nc >= 0 ? double(nc) : 2147483648.0;
+  }
 }
 
 std::vector<DBuf*> stateBufs(Sim& s) {
@@ -521,18 +570,43 @@ FieldPtrs fieldPtrs(Sim& s) {
   f.fCl = s.hasMultipliers ? s.fCl.as<double>() : nullptr;
   f.fCq = s.hasMultipliers ? s.fCq.as<double>() : nullptr;
   f.fsh = s.hasMultipliers ? s.fshear.as<double>() : nullptr;
+  f.seg = s.ensemble || s.nLists > 1 ? s.seg.as<double>() : nullptr;
   return f;
 }
 
-template <int D> void applyFieldsD(Sim& s, bool geometry) {
+GhostMap ghostMap(const Sim& s) {
+  return GhostMap{s.ghostControl.as<int32_t>(), s.ghostSub.as<int32_t>(), s.subDev.as<DSub>(), s.nInt};
+}
+
+template <int D> void applyFieldsD(Sim& s, bool geometry, int rec) {
+  const int64_t ng = s.nTot - s.nInt;
+  if (ng <= 0) {
+    if (rec >= 0) (void)packOutputs(s, rec);
+    return;
+  }
   const FieldPtrs f = fieldPtrs(s);
-  for (size_t b = 0; b < s.subs.size(); ++b) {
-    const int64_t g0 = s.nInt + s.subStart[b], g1 = s.nInt + s.subStart[b + 1];
-    if (g1 <= g0) continue;
-    hipLaunchKernelGGL(k_ghost_fields<D>, dim3(nblocks(g1 - g0)), dim3(kBlock), 0, s.stream, f, g0, g1, s.nInt,
-                       s.ghostControl.as<int32_t>(), toDevice(s.subs[b]), geometry ? 1 : 0);
+  const GhostMap m = ghostMap(s);
+  const PackIn pin = rec >= 0 ? packInputs(s) : PackIn{};
+  const PackOut pout = rec >= 0 ? packOutputs(s, rec) : PackOut{};
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblocks(ng)), dim3(kBlock), 0, s.stream, f, m, s.nTot, geometry ? 1 : 0,
+                       s.iperm.as<int32_t>(), pin, pout);
+  };
+  switch (rec) {
+    case -1: go(k_ghost_fields<D, -1>); break;
+    case 0: go(k_ghost_fields<D, 0>); break;
+    case 1: go(k_ghost_fields<D, 1>); break;
+    case 2: go(k_ghost_fields<D, 2>); break;
+    case 4: go(k_ghost_fields<D, 4>); break;
+    case 8: go(k_ghost_fields<D, 8>); break;
+    default: SG_REQUIRE(false, SPHGPU_ERR_STATE, "unsupported record kinds for the ghost rows");
   }
   SG_CHECK_HIP(hipGetLastError());
+}
+void applyFields(Sim& s, bool geometry, int rec) {
+  if (s.dim == 1) applyFieldsD<1>(s, geometry, rec);
+  else if (s.dim == 2) applyFieldsD<2>(s, geometry, rec);
+  else applyFieldsD<3>(s, geometry, rec);
 }
 
 // Every plane's ghosts with the running row count kept on the device: the
@@ -647,7 +721,7 @@ template <int D> void generateD(Sim& s, double ext) {
   }
   s.subStart[s.subs.size()] = s.nTot - s.nInt;
   s.ghostsGenerated = s.nTot - s.nInt;
-  applyFieldsD<D>(s, false);
+  applyFieldsD<D>(s, false, -1);
 }
 
 }  // namespace
@@ -716,44 +790,28 @@ void cull(Sim& s) {
   if (nNew == n) return;
   const int32_t* scan = s.keepScan.as<int32_t>();
 
-  // caller-order fields: kept ghost rows compacted through the spare and
-  // copied back (internal rows stay where they are)
-  auto bufs = stateBufs(s);
-  for (int w = 0; w < int(bufs.size()); ++w) {
-    if (!stateUsed(s, w)) continue;
-    const int comps = stateComps(s, w);
-    DBuf& spare = s.spare[w];
-    spare.ensure(bufs[size_t(w)]->bytes);
-    hipLaunchKernelGGL(k_compact_rows, dim3(nblocks(n - nInt)), dim3(kBlock), 0, st, bufs[size_t(w)]->as<double>(),
-                       spare.as<double>(), comps, keep, scan, nInt, n);
-    if (nNew > nInt)
-      SG_CHECK_HIP(hipMemcpyAsync(bufs[size_t(w)]->as<double>() + nInt * comps, spare.as<double>() + nInt * comps,
-                                  sizeof(double) * size_t(nNew - nInt) * comps, hipMemcpyDeviceToDevice, st));
-  }
-  // ghost controls (control and sub-boundary arrays share the spare pair)
   s.ghostControlSpare.ensure(s.ghostControl.bytes);
   s.ghostSubSpare.ensure(s.ghostSub.bytes);
-  hipLaunchKernelGGL(k_compact_ghosts, dim3(nblocks(n - nInt)), dim3(kBlock), 0, st, s.ghostControl.as<int32_t>(),
-                     s.ghostSub.as<int32_t>(), s.ghostControlSpare.as<int32_t>(), s.ghostSubSpare.as<int32_t>(), keep,
-                     scan, nInt, n);
-  s.ghostControl.swap(s.ghostControlSpare);
-  s.ghostSub.swap(s.ghostSubSpare);
-  // slot <-> caller maps
+  s.ipermSpare.ensure(s.iperm.bytes);
   const bool recs = s.recValid;
   // The density records keep the pre-cull caller index of their ghosts: the
   // density sum compares a neighbour's index only with an internal node's
   // (to place the self term), and culling keeps every internal index and
   // every ghost's index above them, so no comparison changes.
-  hipLaunchKernelGGL(k_perm_remap, dim3(nblocks(s.nSlots)), dim3(kBlock), 0, st, s.perm.as<int32_t>(), keep, scan,
+  hipLaunchKernelGGL(k_cull, dim3(nblocks(std::max(n, s.nSlots))), dim3(kBlock), 0, st, s.ghostControl.as<int32_t>(),
+                     s.ghostSub.as<int32_t>(), s.ghostControlSpare.as<int32_t>(), s.ghostSubSpare.as<int32_t>(),
+                     s.iperm.as<int32_t>(), s.ipermSpare.as<int32_t>(), s.perm.as<int32_t>(), keep, scan, nInt, n,
                      s.nSlots, recs ? s.rec.as<double>() : nullptr, s.isotropic ? RL<true>::STRIDE : RL<false>::STRIDE,
                      s.isotropic ? RL<true>::ORIG : RL<false>::ORIG);
-  s.ipermSpare.ensure(s.iperm.bytes);
-  hipLaunchKernelGGL(k_iperm_remap, dim3(nblocks(n)), dim3(kBlock), 0, st, s.iperm.as<int32_t>(), keep, scan, n,
-                     s.ipermSpare.as<int32_t>());
-  s.iperm.swap(s.ipermSpare);
   SG_CHECK_HIP(hipGetLastError());
+  s.ghostControl.swap(s.ghostControlSpare);
+  s.ghostSub.swap(s.ghostSubSpare);
+  s.iperm.swap(s.ipermSpare);
   for (size_t b = 0; b < s.subStart.size(); ++b) s.subStart[b] = int64_t(starts[b]) - nInt;
   s.nTot = nNew;
+  // the kept ghost rows at their new places, filled again from the internal
+  // nodes (the same maps of the same values)
+  applyFields(s, true, -1);
   s.recValid = recs;
   // with several NodeLists the density sum also looks up a neighbour's
   // NodeList by that index: the density records are packed again
@@ -807,6 +865,13 @@ void setBoundaries(Sim& s, int n, const sphgpu_boundary* b) {
       subs.push_back(d);
     }
   }
+  std::vector<DSub> dev;
+  for (const SubBoundary& b2 : subs) dev.push_back(toDevice(b2));
+  if (s.subDev.p) SG_CHECK_HIP(hipStreamSynchronize(s.stream));   // earlier launches may still read the old planes
+  s.subDev.ensure(sizeof(DSub) * std::max<size_t>(dev.size(), 1));
+  if (!dev.empty())
+    SG_CHECK_HIP(hipMemcpyAsync(s.subDev.p, dev.data(), sizeof(DSub) * dev.size(), hipMemcpyHostToDevice, s.stream));
+  SG_CHECK_HIP(hipStreamSynchronize(s.stream));   // `dev` dies on return
   s.subs = subs;
   s.subStart.clear();
 }
@@ -842,38 +907,27 @@ void setGhostNodes(Sim& s, double ext, bool doCull) {
 
 void applyGhostBoundaries(Sim& s) {
   if (!s.deviceGhosts || s.nTot == s.nInt) return;
-  if (s.dim == 1) applyFieldsD<1>(s, true);
-  else if (s.dim == 2) applyFieldsD<2>(s, true);
-  else applyFieldsD<3>(s, true);
+  applyFields(s, true, -1);
   s.recValid = false;
+  s.derivsValid = false;
+}
+
+void applyGhostBoundariesAndRecords(Sim& s, int rec) {
+  SG_REQUIRE(s.deviceGhosts || s.nTot == s.nInt, SPHGPU_ERR_STATE, "the ghost rows were not made by the boundaries");
+  applyFields(s, true, rec);
+  s.recValid = true;
   s.derivsValid = false;
 }
 
 void enforceBoundaries(Sim& s) {
   if (s.subs.empty() || s.nInt == 0) return;
-  hipStream_t st = s.stream;
-  for (size_t b = 0; b < s.subs.size(); ++b) {
-    const DSub d = toDevice(s.subs[b]);
-    if (s.dim == 1)
-      hipLaunchKernelGGL(k_enforce<1>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.pos.as<double>(), s.vel.as<double>(),
-                         s.H.as<double>(), s.nInt, d);
-    else if (s.dim == 2)
-      hipLaunchKernelGGL(k_enforce<2>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.pos.as<double>(), s.vel.as<double>(),
-                         s.H.as<double>(), s.nInt, d);
-    else
-      hipLaunchKernelGGL(k_enforce<3>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.pos.as<double>(), s.vel.as<double>(),
-                         s.H.as<double>(), s.nInt, d);
-    // the second half of a periodic pair closes it: wrap what is still outside
-    if (s.subs[b].periodicSecond) {
-      const DSub first = toDevice(s.subs[b - 1]);
-      if (s.dim == 1)
-        hipLaunchKernelGGL(k_periodic_wrap<1>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.pos.as<double>(), s.nInt, first);
-      else if (s.dim == 2)
-        hipLaunchKernelGGL(k_periodic_wrap<2>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.pos.as<double>(), s.nInt, first);
-      else
-        hipLaunchKernelGGL(k_periodic_wrap<3>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.pos.as<double>(), s.nInt, first);
-    }
-  }
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, s.pos.as<double>(), s.vel.as<double>(),
+                       s.H.as<double>(), s.nInt, s.subDev.as<DSub>(), int(s.subs.size()));
+  };
+  if (s.dim == 1) go(k_enforce<1>);
+  else if (s.dim == 2) go(k_enforce<2>);
+  else go(k_enforce<3>);
   SG_CHECK_HIP(hipGetLastError());
   s.recValid = false;
   s.derivsValid = false;
@@ -881,12 +935,8 @@ void enforceBoundaries(Sim& s) {
 
 void applyGhostScalar(Sim& s, DBuf& field) {
   if (!s.deviceGhosts || s.nTot == s.nInt) return;
-  for (size_t b = 0; b < s.subs.size(); ++b) {
-    const int64_t g0 = s.nInt + s.subStart[b], g1 = s.nInt + s.subStart[b + 1];
-    if (g1 <= g0) continue;
-    hipLaunchKernelGGL(k_ghost_scalar, dim3(nblocks(g1 - g0)), dim3(kBlock), 0, s.stream, field.as<double>(), g0, g1,
-                       s.nInt, s.ghostControl.as<int32_t>());
-  }
+  hipLaunchKernelGGL(k_ghost_scalar, dim3(nblocks(s.nTot - s.nInt)), dim3(kBlock), 0, s.stream, field.as<double>(),
+                     ghostMap(s), s.nTot);
   SG_CHECK_HIP(hipGetLastError());
 }
 
@@ -943,40 +993,24 @@ int stateFieldComps(const Sim& s, int which) { return stateComps(s, which); }
 
 void applyGhostVector(Sim& s, DBuf& field) {
   if (!s.deviceGhosts || s.nTot == s.nInt) return;
-  for (size_t b = 0; b < s.subs.size(); ++b) {
-    const int64_t g0 = s.nInt + s.subStart[b], g1 = s.nInt + s.subStart[b + 1];
-    if (g1 <= g0) continue;
-    const DSub d = toDevice(s.subs[b]);
-    const int32_t* ctl = s.ghostControl.as<int32_t>();
-    if (s.dim == 1)
-      hipLaunchKernelGGL(k_ghost_vector<1>, dim3(nblocks(g1 - g0)), dim3(kBlock), 0, s.stream, field.as<double>(), g0,
-                         g1, s.nInt, ctl, d);
-    else if (s.dim == 2)
-      hipLaunchKernelGGL(k_ghost_vector<2>, dim3(nblocks(g1 - g0)), dim3(kBlock), 0, s.stream, field.as<double>(), g0,
-                         g1, s.nInt, ctl, d);
-    else
-      hipLaunchKernelGGL(k_ghost_vector<3>, dim3(nblocks(g1 - g0)), dim3(kBlock), 0, s.stream, field.as<double>(), g0,
-                         g1, s.nInt, ctl, d);
-  }
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblocks(s.nTot - s.nInt)), dim3(kBlock), 0, s.stream, field.as<double>(), ghostMap(s),
+                       s.nTot);
+  };
+  if (s.dim == 1) go(k_ghost_vector<1>);
+  else if (s.dim == 2) go(k_ghost_vector<2>);
+  else go(k_ghost_vector<3>);
   SG_CHECK_HIP(hipGetLastError());
 }
 
 void applyGhostDensity(Sim& s) {
   if (!s.deviceGhosts || s.nTot == s.nInt) return;
-  hipStream_t st = s.stream;
-  for (size_t b = 0; b < s.subs.size(); ++b) {
-    const int64_t g0 = s.nInt + s.subStart[b], g1 = s.nInt + s.subStart[b + 1];
-    if (g1 <= g0) continue;
-    hipLaunchKernelGGL(k_ghost_scalar, dim3(nblocks(g1 - g0)), dim3(kBlock), 0, st, s.rho.as<double>(), g0, g1,
-                       s.nInt, s.ghostControl.as<int32_t>());
-  }
-  const int64_t ng = s.nTot - s.nInt;
-  if (s.isotropic)
-    hipLaunchKernelGGL(k_ghost_records<true>, dim3(nblocks(ng)), dim3(kBlock), 0, st, s.rec.as<double>(),
-                       s.iperm.as<int32_t>(), s.rho.as<double>(), s.nInt, s.nTot);
-  else
-    hipLaunchKernelGGL(k_ghost_records<false>, dim3(nblocks(ng)), dim3(kBlock), 0, st, s.rec.as<double>(),
-                       s.iperm.as<int32_t>(), s.rho.as<double>(), s.nInt, s.nTot);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblocks(s.nTot - s.nInt)), dim3(kBlock), 0, s.stream, s.rec.as<double>(),
+                       s.iperm.as<int32_t>(), s.rho.as<double>(), ghostMap(s), s.nTot);
+  };
+  if (s.isotropic) go(k_ghost_records<true>);
+  else go(k_ghost_records<false>);
   SG_CHECK_HIP(hipGetLastError());
 }
 

@@ -1226,14 +1226,6 @@ void packD(Sim& s, int sec = 0) {
   else launchPack<D>(s, sec, nullptr, s.nSlots);
 }
 
-void packGhostRecords(Sim& s, int sec) {
-  if (s.nTot == s.nInt) { (void)packOutputs(s, sec); return; }
-  const int32_t* slots = s.iperm.as<int32_t>() + s.nInt;
-  if (s.dim == 1) launchPack<1>(s, sec, slots, s.nTot - s.nInt);
-  else if (s.dim == 2) launchPack<2>(s, sec, slots, s.nTot - s.nInt);
-  else launchPack<3>(s, sec, slots, s.nTot - s.nInt);
-}
-
 int pairRecordSec(const Sim& s, const sphgpu_hydro_params& hp) {
   const bool tensile = hp.epsTensile != 0.0;
   const bool compat = hp.compatibleEnergyEvolution != 0;

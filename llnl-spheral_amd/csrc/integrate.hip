@@ -516,11 +516,8 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
   const int recMid = recs ? pairRecordSec(s, hp) : -1;
   const int recEnd = recs ? densityRecordSec(s) : -1;
   auto ghostsAndRecords = [&](int rec) {
-    applyGhostBoundaries(s);
-    if (rec >= 0) {
-      packGhostRecords(s, rec);
-      s.recValid = true;
-    }
+    if (rec >= 0) applyGhostBoundariesAndRecords(s, rec);
+    else applyGhostBoundaries(s);
   };
   // trial advance to the midpoint
   if (compat) compatD<D>(s, b0.vel, hdt, half);
@@ -605,7 +602,7 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
                         &s.recS, &s.recSM, &s.pairDv, &s.compDe, &s.compAcc, &s.compDe0, &s.compRec, &s.out,
                         &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
                         &s.work, &s.workFlag, &s.workScan, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
-                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.pick, &s.listGamma})
+                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.pick, &s.listGamma, &s.subDev})
     keyBuf(k, *b);
   for (const DBuf& b : s.state0) keyBuf(k, b);
   return k;

@@ -186,13 +186,14 @@ struct Sim {
 
   // planar ghost boundaries generated on the device
   std::vector<SubBoundary> subs;
+  DBuf subDev;                   // the same planes on the device (DSub, ghosts.hip)
   bool deviceGhosts = false;     // ghost rows nInt..nTot-1 were made by setGhostNodes
   DBuf ghostControl, ghostSub;   // per ghost: control node (caller index), sub-boundary
   std::vector<int64_t> subStart; // first ghost (offset from nInt) of each sub-boundary, +1 entry
   int64_t ghostsGenerated = 0;   // before culling
   DBuf keep, keepScan, slotKeep, ghostControlSpare, ghostSubSpare, ipermSpare, hmaxOf;
   DBuf genDev;                   // device-held counts of a ghost generation
-  DBuf spare[13];                // one per caller-order state field (culling compacts into it)
+  DBuf spare[13];                // one per caller-order state field (member removal gathers into it)
   bool markGhostUse = false;     // the next build marks the ghost slots rows hold (for culling)
   bool rowsMapOrder = false;     // several NodeLists, reference order: rows in ConnectivityMap order
                                  // (iterateIdealH) instead of the owner loop's delivery order
@@ -308,6 +309,9 @@ double gatherProbe(Sim& s, int loads, int repeats);
 void setBoundaries(Sim& s, int n, const sphgpu_boundary* b);
 void setGhostNodes(Sim& s, double kernelExtent, bool cull);
 void applyGhostBoundaries(Sim& s);
+// The same refresh, and the ghost slots' records (pack sec bits; isotropic H):
+// the records are then current.
+void applyGhostBoundariesAndRecords(Sim& s, int rec);
 void applyGhostDensity(Sim& s);   // after sum density: ghost rho and their records
 void applyGhostScalar(Sim& s, DBuf& field);   // ghost rows of one scalar field from their controls
 void applyGhostVector(Sim& s, DBuf& field);   // ghost rows of one Vector field (R.a or a copy)

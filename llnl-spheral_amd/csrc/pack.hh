@@ -181,7 +181,5 @@ PackOut packOutputs(Sim& s, int sec);
 // 1/u for the 3-D mixed record's positions (a power of two; from the last
 // neighbour build's largest search radius)
 double quantInv(const Sim& s);
-// The records of the ghost slots only (after the ghost rows' fields changed).
-void packGhostRecords(Sim& s, int sec);
 
 }  // namespace sphgpu
