@@ -128,13 +128,6 @@ int sphgpu_create(int dim, int device, sphgpu_sim** out) {
     sphgpu_destroy(s);
     return e.code;
   }
-  void* pinned = nullptr;
-  if (hipHostMalloc(&pinned, sizeof(unsigned long long), hipHostMallocDefault) != hipSuccess) {
-    sphgpu_destroy(s);
-    return SPHGPU_ERR_HIP;
-  }
-  s->ncalcHost = static_cast<unsigned long long*>(pinned);
-  *s->ncalcHost = 0;
   *out = s;
   return SPHGPU_OK;
 }
@@ -150,7 +143,6 @@ void sphgpu_destroy(sphgpu_sim* s) {
   for (DBuf* b : bufs) b->release();
   for (auto& e : s->ev) if (e) (void)hipEventDestroy(e);
   for (auto& g : s->stepGraphs) if (g.exec) (void)hipGraphExecDestroy(g.exec);
-  if (s->ncalcHost) (void)hipHostFree(s->ncalcHost);
   if (s->pinnedOut) (void)hipHostFree(s->pinnedOut);
   if (s->pinnedIn) (void)hipHostFree(s->pinnedIn);
   if (s->pinnedInDone) (void)hipEventDestroy(s->pinnedInDone);
@@ -462,8 +454,13 @@ int sphgpu_pair_count(sphgpu_sim* s, int64_t* n) {
   return guarded(s, [&] {
     SG_REQUIRE(n, SPHGPU_ERR_ARG, "null output");
     SG_REQUIRE(s->pairsValid, SPHGPU_ERR_STATE, "no derivative pass on the current neighbour rows");
+    std::vector<uint32_t> c(static_cast<size_t>(s->pairWaves));
+    if (!c.empty())
+      SG_CHECK_HIP(hipMemcpyAsync(c.data(), s->pairCounts.p, sizeof(uint32_t) * c.size(), hipMemcpyDeviceToHost, s->stream));
     SG_CHECK_HIP(hipStreamSynchronize(s->stream));
-    *n = int64_t(*s->ncalcHost);
+    int64_t total = 0;
+    for (uint32_t v : c) total += v;
+    *n = total;
   });
 }
 

@@ -471,6 +471,14 @@ __device__ __forceinline__ void epilogue(int64_t k, int len, const Self<D>& me, 
   }
 }
 
+// The pairs a wavefront evaluated, one entry per wavefront of the work list
+// (tw: this lane's place in it): nothing to clear before the pass, no atomics,
+// and no read-back unless the caller asks for the count.
+__device__ __forceinline__ void storePairCount(unsigned pairs, int64_t tw, int64_t nInt, uint32_t* __restrict__ counts) {
+  for (int sh = 32; sh > 0; sh >>= 1) pairs += __shfl_xor(pairs, sh);
+  if ((threadIdx.x & 63) == 0 && tw < nInt) counts[tw >> 6] = pairs;
+}
+
 template <int D, bool ISO, bool TENSILE>
 __device__ __forceinline__ unsigned derivsNodeFP64(int64_t k, const double* __restrict__ rec,
                                                    const int32_t* __restrict__ rowCount, const int32_t* __restrict__ nbr,
@@ -594,14 +602,13 @@ template <int D, bool ISO, bool TENSILE, bool LDS>
 __global__ void __launch_bounds__(kBlock) k_derivs_fp64(const double* __restrict__ rec, const int32_t* __restrict__ rowCount,
                                                         const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
                                                         const int32_t* __restrict__ work, TabArgs t, PassArgs p,
-                                                        OutArgs o, unsigned long long* __restrict__ ncalc) {
+                                                        OutArgs o, uint32_t* __restrict__ pairCounts) {
   extern __shared__ double lds[];
   const double* tab = stageTable<LDS>(lds, t);
   const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
   unsigned pairs = 0;
   if (tw < nInt) pairs = derivsNodeFP64<D, ISO, TENSILE>(work[tw], rec, rowCount, nbr, n, tab, t, p, o);
-  for (int sh = 32; sh > 0; sh >>= 1) pairs += __shfl_xor(pairs, sh);
-  if ((threadIdx.x & 63) == 0 && pairs) atomicAdd(ncalc, (unsigned long long)pairs);
+  storePairCount(pairs, tw, nInt, pairCounts);
 }
 
 // ---------------------------------------------------------------------------
@@ -918,7 +925,7 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
                                                        const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
                                                        const int32_t* __restrict__ work, TabArgs t,
                                                        typename IsoTab<Real>::T tt, PassArgs p, OutArgs o,
-                                                       unsigned long long* __restrict__ ncalc) {
+                                                       uint32_t* __restrict__ pairCounts) {
   using R = RL<true>;
   using E = typename IsoTab<Real>::Elem;
   extern __shared__ double ldsIso[];
@@ -1126,8 +1133,7 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
     me.Hdet = ri_[R::HDET]; me.m = ri_[R::M]; me.rho = ri_[R::RHO]; me.mor = ri_[R::MOR];
     epilogue<D>(k, len, me, a, t, p, o);
   }
-  for (int sh = 32; sh > 0; sh >>= 1) pairs += __shfl_xor(pairs, sh);
-  if ((threadIdx.x & 63) == 0 && pairs) atomicAdd(ncalc, (unsigned long long)pairs);
+  storePairCount(pairs, tw, nInt, pairCounts);
 }
 
 TabArgs tabArgs(const Sim& s) {
@@ -1345,7 +1351,7 @@ template <> Tab32 isoTable<float>(const Sim& s) { return tab32(s); }
 template <> Tab64 isoTable<double>(const Sim& s) { return tab64(s); }
 template <typename Real, int D, bool PF, int BS>
 void isoLaunch(Sim& s, bool inLds, hipStream_t st, int64_t n, const TabArgs& t, const PassArgs& p, const OutArgs& o,
-               unsigned long long* dncalc) {
+               uint32_t* counts) {
   using Rec = typename IsoTab<Real>::Rec;
   const Rec* recN = reinterpret_cast<const Rec*>(std::is_same<Real, float>::value ? s.recM.p : s.recD.p);
   const size_t lb = inLds ? sizeof(typename IsoTab<Real>::Elem) * IsoTab<Real>::PER * size_t(s.table.n) : 0;
@@ -1353,25 +1359,25 @@ void isoLaunch(Sim& s, bool inLds, hipStream_t st, int64_t n, const TabArgs& t, 
   if (inLds)
     hipLaunchKernelGGL((k_derivs_iso<Real, D, true, PF, BS>), g, b, lb, st, s.rec.as<double>(), recN,
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
-                       isoTable<Real>(s), p, o, dncalc);
+                       isoTable<Real>(s), p, o, counts);
   else
     hipLaunchKernelGGL((k_derivs_iso<Real, D, false, PF, BS>), g, b, 0, st, s.rec.as<double>(), recN,
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
-                       isoTable<Real>(s), p, o, dncalc);
+                       isoTable<Real>(s), p, o, counts);
 }
 template <typename Real, int D, bool PF>
 void isoVariant(Sim& s, int v, bool fits, hipStream_t st, int64_t n, const TabArgs& t, const PassArgs& p,
-                const OutArgs& o, unsigned long long* dncalc) {
+                const OutArgs& o, uint32_t* counts) {
   const int bsLog = fits ? v >> 1 : v;
   const bool inLds = fits && (v & 1);
   if constexpr (D == 3) {
-    isoLaunch<Real, D, PF, 256>(s, inLds, st, n, t, p, o, dncalc);
+    isoLaunch<Real, D, PF, 256>(s, inLds, st, n, t, p, o, counts);
   } else {
     switch (bsLog) {
-      case 0: isoLaunch<Real, D, PF, 64>(s, inLds, st, n, t, p, o, dncalc); break;
-      case 1: isoLaunch<Real, D, PF, 128>(s, inLds, st, n, t, p, o, dncalc); break;
-      case 2: isoLaunch<Real, D, PF, 256>(s, inLds, st, n, t, p, o, dncalc); break;
-      default: isoLaunch<Real, D, PF, 512>(s, inLds, st, n, t, p, o, dncalc); break;
+      case 0: isoLaunch<Real, D, PF, 64>(s, inLds, st, n, t, p, o, counts); break;
+      case 1: isoLaunch<Real, D, PF, 128>(s, inLds, st, n, t, p, o, counts); break;
+      case 2: isoLaunch<Real, D, PF, 256>(s, inLds, st, n, t, p, o, counts); break;
+      default: isoLaunch<Real, D, PF, 512>(s, inLds, st, n, t, p, o, counts); break;
     }
   }
   SG_CHECK_HIP(hipGetLastError());
@@ -1384,8 +1390,9 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly) {
   const int total = derivTotalDoubles(s.dim);
   s.out.ensure(sizeof(double) * size_t(n) * total);
   s.outStride = n;
-  s.reduceTmp.ensure(sizeof(double) * 16);
-  unsigned long long* dncalc = reinterpret_cast<unsigned long long*>(s.reduceTmp.as<double>() + 8);
+  s.pairWaves = (s.nInt + 63) / 64;
+  s.pairCounts.ensure(sizeof(uint32_t) * size_t(std::max<int64_t>(s.pairWaves, 1)));
+  uint32_t* counts = s.pairCounts.as<uint32_t>();
 
   // the pair kernel decides the record it reads
   const bool tensile = hp.epsTensile != 0.0;
@@ -1405,12 +1412,6 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly) {
     packMixed<D>(s);
   } else if (sec == 2 && s.pairRec != 2) {
     packFast64<D>(s);
-  }
-  {
-    // a kernel, not a memset node, when the step is captured as a graph
-    ZeroSet z{};
-    z.add(reinterpret_cast<int32_t*>(dncalc), 2);
-    zeroMany(z, st);
   }
   if (!s.capturing) SG_CHECK_HIP(hipEventRecord(s.ev[5], st));
 
@@ -1450,28 +1451,21 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly) {
     const bool fits = s.table.n <= kLdsTablePoints;
     const int nv = fits ? 8 : 4;
     auto run = [&](int v) {
-      if (mixed) isoVariant<float, D, false>(s, v, fits, st, n, t, p, o, dncalc);
-      else isoVariant<double, D, true>(s, v, fits, st, n, t, p, o, dncalc);
+      if (mixed) isoVariant<float, D, false>(s, v, fits, st, n, t, p, o, counts);
+      else isoVariant<double, D, true>(s, v, fits, st, n, t, p, o, counts);
     };
     const int def = fits ? (4 + (lds ? 1 : 0)) : 2;      // 256 threads, the row-length rule for the table
     int v = def;
     if (D < 3) {
-      bool timed = false;
       const double perNode = s.nInt > 0 ? double(s.nEntries) / double(s.nInt) : 0.0;
-      v = tunedVariant(s, tuneKey(kTunePairIso, D, mixed ? 1 : 0, perNode, s.nInt), nv, def, run, &timed);
-      if (timed) {
-        // the trials added to the pair count
-        ZeroSet z{};
-        z.add(reinterpret_cast<int32_t*>(dncalc), 2);
-        zeroMany(z, st);
-      }
+      v = tunedVariant(s, tuneKey(kTunePairIso, D, mixed ? 1 : 0, perNode, s.nInt), nv, def, run);
     }
     run(v);
   } else {
     auto launch = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), ldsBytes, st, s.rec.as<double>(),
                          s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t, p, o,
-                         dncalc);
+                         counts);
     };
     if (lds) {
       if (s.isotropic) { if (tensile) launch(k_derivs_fp64<D, true, true, true>); else launch(k_derivs_fp64<D, true, false, true>); }
@@ -1483,7 +1477,6 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly) {
   }
   SG_CHECK_HIP(hipGetLastError());
   if (!s.capturing) SG_CHECK_HIP(hipEventRecord(s.ev[6], st));
-  SG_CHECK_HIP(hipMemcpyAsync(s.ncalcHost, dncalc, sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
 }
 
 }  // namespace

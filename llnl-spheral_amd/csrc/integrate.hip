@@ -61,62 +61,85 @@ struct Fields {
   double *pos, *vel, *eps, *rho, *H, *P, *cs;
 };
 struct Base {
-  const double *pos, *vel, *eps, *rho;
+  double *pos, *vel, *eps, *rho;
 };
 struct DerivIn {
   const double* base;  // field-major blocks of the last evaluation, slot rows
   int64_t n;
-  int oDx, oDv, oDeps, oDrho, oHid;
+  int oDx, oDv, oDeps, oDrho, oHid, oVP, oDvDx;
   const double* compDe;  // compatible energy: DepsDt of the policy per slot, else null
 };
 struct Bounds {
   double rhoMin, rhoMax, hmaxInv, hminInv;
 };
 // Ensemble members: the update's multiplier (dt or dt/2) and gamma per member.
+struct SelectArgs {
+  double cfl, dtMin, dtMax, dtGrowth;
+};
+// Integrator::selectDt of one member from its vote (src/Integrator/Integrator.cc:167-212):
+// a handful of operations on uniform values, so every kernel that needs dt
+// forms it again from the vote rather than waiting for a launch that does.
+__device__ __forceinline__ double selectDt(const SegState& g, const SelectArgs& a) {
+  const double dtMin = dmin(a.dtMin, g.tEnd - g.t), dtMax = dmin(a.dtMax, g.tEnd - g.t);
+  const double vote = a.cfl * __longlong_as_double((long long)g.voteBits);
+  double dt = dtMax;
+  if (vote > 0.0 && vote < dt) dt = vote;
+  dt = dmin(dt, a.dtGrowth * g.lastDt);
+  return dmin(dtMax, dmax(dtMin, dt));
+}
 struct SegArgs {
   const double* seg;        // member of each row; null: one simulation
-  SegState* st;             // null: the scalar multiplier and EOS apply to every row
+  SegState* st;
   int half;                 // 1: multiply by dt/2
+  SelectArgs sel;
   const double* listOf = nullptr;      // several NodeLists with their own gamma-law EOS:
   const double* listGamma = nullptr;   //   each row's NodeList, and the NodeLists' gammas
 };
+// The update's multiplier and the EOS of row i.
 __device__ __forceinline__ void rowMultEos(const SegArgs& sa, int64_t i, double& mult, Eos& e) {
   if (sa.listGamma) {
     const double g = sa.listGamma[int(sa.listOf[i])];
     e.gamma = g;
     e.gamma1 = g - 1.0;
   }
-  if (!sa.st) return;
-  if (!sa.seg) {            // one simulation whose dt was chosen on the device
-    mult = sa.half ? sa.st->hdt : sa.st->dt;
-    return;
-  }
-  const SegState& g = sa.st[int(sa.seg[i])];
-  mult = sa.half ? g.hdt : g.dt;
+  const SegState& g = sa.st[sa.seg ? int(sa.seg[i]) : 0];
+  const double dt = selectDt(g, sa.sel);
+  mult = sa.half ? 0.5 * dt : dt;
+  if (!sa.seg) return;
   e.gamma = g.gamma;
   e.gamma1 = g.gamma - 1.0;
 }
 
 // REC >= 0: also write the slot's records (pack sec bits REC, isotropic
 // layout) from the values just stored, as the record pack would.
-template <int D, int REC>
+// TRIAL: the update to t + dt/2 starts from the state itself and saves it as
+// state0 (b) on the way, in place of copies of the whole state before it (at
+// 128^3 five copies of 235 MB in all, of which H was never read back).  The
+// final update starts from b and leaves the dt vote's inputs of the next step
+// (maxViscousPressure, tr DvDx, DvDt by caller index) in dtIn.
+template <int D, int REC, bool TRIAL>
 __global__ void k_update(const int32_t* __restrict__ work, const int32_t* __restrict__ perm, int64_t nInt, Fields f,
-                         Base b, DerivIn d, double mult, Bounds bd, Eos e, SegArgs sa, PackIn pin,
-                         PackOut pout) {
+                         Base b, DerivIn d, Bounds bd, Eos e, SegArgs sa, PackIn pin, PackOut pout,
+                         double* __restrict__ dtIn) {
   constexpr int NS = NSym<D>::value;
   const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (t >= nInt) return;
   const int64_t k = work[t];
   const int64_t i = perm[k];
+  double mult;
   rowMultEos(sa, i, mult, e);
   const double* dx = d.base + int64_t(d.oDx) * d.n + k * D;
   const double* dv = d.base + int64_t(d.oDv) * d.n + k * D;
   for (int c = 0; c < D; ++c) {
-    f.pos[i * D + c] = b.pos[i * D + c] + mult * dx[c];
-    f.vel[i * D + c] = b.vel[i * D + c] + mult * dv[c];
+    const double x0 = (TRIAL ? f.pos : b.pos)[i * D + c], v0 = (TRIAL ? f.vel : b.vel)[i * D + c];
+    if (TRIAL) { b.pos[i * D + c] = x0; b.vel[i * D + c] = v0; }
+    f.pos[i * D + c] = x0 + mult * dx[c];
+    f.vel[i * D + c] = v0 + mult * dv[c];
   }
-  const double eps = d.compDe ? b.eps[i] + d.compDe[k] * mult : b.eps[i] + mult * d.base[int64_t(d.oDeps) * d.n + k];
-  const double rho = dmin(bd.rhoMax, dmax(bd.rhoMin, b.rho[i] + mult * d.base[int64_t(d.oDrho) * d.n + k]));
+  const double eps0 = (TRIAL ? f.eps : b.eps)[i], rho0 = (TRIAL ? f.rho : b.rho)[i];
+  if (TRIAL) { b.eps[i] = eps0; b.rho[i] = rho0; }
+  const double eps = d.compDe ? eps0 + d.compDe[k] * mult : eps0 + mult * d.base[int64_t(d.oDeps) * d.n + k];
+  const double rho = dmin(bd.rhoMax, dmax(bd.rhoMin, rho0 + mult * d.base[int64_t(d.oDrho) * d.n + k]));
   f.eps[i] = eps;
   f.rho[i] = rho;
   const double* hid = d.base + int64_t(d.oHid) * d.n + k * NS;
@@ -127,32 +150,23 @@ __global__ void k_update(const int32_t* __restrict__ work, const int32_t* __rest
   f.P[i] = P;
   f.cs[i] = cs;
   if constexpr (REC >= 0) packSlot<D, true, REC>(k, pin, pout);
+  if constexpr (!TRIAL) {
+    constexpr int W = 2 + D;
+    dtIn[i * W] = d.base[int64_t(d.oVP) * d.n + k];
+    const double* g = d.base + int64_t(d.oDvDx) * d.n + k * D * D;
+    double tr = g[0];
+    for (int a = 1; a < D; ++a) tr = tr + g[a * D + a];
+    dtIn[i * W + 1] = tr;
+    for (int c2 = 0; c2 < D; ++c2) dtIn[i * W + 2 + c2] = dv[c2];
+  }
   // an ensemble member whose state turns non-finite fails alone (the step's
   // final update; NaN at the midpoint reaches it)
-  if (sa.seg && !sa.half) {
+  if (!TRIAL && sa.seg) {
     bool ok = isfinite(eps) && isfinite(rho) && isfinite(P) && isfinite(cs);
     for (int c = 0; c < D; ++c) ok = ok && isfinite(f.pos[i * D + c]) && isfinite(f.vel[i * D + c]);
     for (int c = 0; c < NS; ++c) ok = ok && isfinite(f.H[i * NS + c]);
     if (!ok) atomicOr(&sa.st[int(sa.seg[i])].fail, unsigned(SPHGPU_MEMBER_NONFINITE));
   }
-}
-
-// maxViscousPressure, tr DvDx and DvDt of the last evaluation, by caller index.
-template <int D>
-__global__ void k_dt_inputs(const int32_t* __restrict__ work, const int32_t* __restrict__ perm, int64_t nInt,
-                            const double* __restrict__ out, int64_t n, int oVP, int oDvDx, int oDvDt,
-                            double* __restrict__ dtIn) {
-  const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (t >= nInt) return;
-  const int64_t k = work[t];
-  const int64_t i = perm[k];
-  constexpr int W = 2 + D;
-  dtIn[i * W] = out[int64_t(oVP) * n + k];
-  const double* g = out + int64_t(oDvDx) * n + k * D * D;
-  double tr = g[0];
-  for (int a = 1; a < D; ++a) tr = tr + g[a * D + a];
-  dtIn[i * W + 1] = tr;
-  for (int c = 0; c < D; ++c) dtIn[i * W + 2 + c] = out[int64_t(oDvDt) * n + k * D + c];
 }
 
 template <int D> __device__ __forceinline__ double vmagArr(const double* a) {
@@ -239,13 +253,14 @@ __global__ void k_compat_scatter(const int32_t* __restrict__ work, const int32_t
 template <int D>
 __global__ void k_compat_rec(const int32_t* __restrict__ perm, int64_t nSlots, const double* __restrict__ vel0,
                              const double* __restrict__ acc, const double* __restrict__ de0,
-                             const double* __restrict__ mass, double mult, SegArgs sa, double* __restrict__ crec) {
+                             const double* __restrict__ mass, SegArgs sa, double* __restrict__ crec) {
   const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (k >= nSlots) return;
   const int64_t i = perm[k];
   double r[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   if (i >= 0) {
     Eos unused{};
+    double mult;
     rowMultEos(sa, i, mult, unused);
     const double hdt = 0.5 * mult;
     for (int c = 0; c < D; ++c) r[c] = vel0[i * D + c] + acc[i * D + c] * hdt;
@@ -311,8 +326,8 @@ __global__ void k_compat(const int32_t* __restrict__ work, const int32_t* __rest
 Eos makeEos(double gamma, double Pmin, double Pmax, int floor) { return Eos{gamma, gamma - 1.0, Pmin, Pmax, floor}; }
 
 // SpecificThermalEnergyPolicy::update's DepsDt into s.compDe (slot rows) for
-// an update by `mult`, with vel0 the velocities the state holds before it.
-template <int D> void compatD(Sim& s, const double* vel0, double mult, const SegArgs& sa) {
+// the update of `sa`, with vel0 the step-start velocities (every row).
+template <int D> void compatD(Sim& s, const double* vel0, const SegArgs& sa) {
   hipStream_t st = s.stream;
   const size_t nt = size_t(std::max<int64_t>(s.nTot, 1)), ns = size_t(std::max<int64_t>(s.nSlots, 1));
   s.compAcc.ensure(sizeof(double) * D * nt);
@@ -326,7 +341,7 @@ template <int D> void compatD(Sim& s, const double* vel0, double mult, const Seg
   applyGhostVector(s, s.compAcc);
   applyGhostScalar(s, s.compDe0);
   hipLaunchKernelGGL(k_compat_rec<D>, dim3(nblocks(s.nSlots)), dim3(kBlock), 0, st, s.perm.as<int32_t>(), s.nSlots,
-                     vel0, s.compAcc.as<double>(), s.compDe0.as<double>(), s.mass.as<double>(), mult, sa,
+                     vel0, s.compAcc.as<double>(), s.compDe0.as<double>(), s.mass.as<double>(), sa,
                      s.compRec.as<double>());
   hipLaunchKernelGGL(k_compat<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
                      s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots, s.nInt, s.compRec.as<double>(),
@@ -337,41 +352,44 @@ template <int D> void compatD(Sim& s, const double* vel0, double mult, const Seg
 // rec >= 0: the update also writes the internal slots' records (pack sec bits;
 // isotropic H only) and the caller packs the ghost slots' records after the
 // ghost rows are refreshed.
-template <int D> void updateD(Sim& s, const Base& b, double mult, const Bounds& bd, const Eos& e,
-                              const double* compDe, const SegArgs& sa, int rec = -1) {
+template <int D, bool TRIAL> void updateD(Sim& s, const Base& b, const Bounds& bd, const Eos& e,
+                                          const double* compDe, const SegArgs& sa, int rec = -1) {
   Fields f{s.pos.as<double>(), s.vel.as<double>(), s.eps.as<double>(), s.rho.as<double>(), s.H.as<double>(),
            s.P.as<double>(), s.cs.as<double>()};
   DerivIn d{s.out.as<double>(), s.outStride, derivOffsetDoubles(D, SPHGPU_D_DXDT), derivOffsetDoubles(D, SPHGPU_D_DVDT),
             derivOffsetDoubles(D, SPHGPU_D_DEPSDT), derivOffsetDoubles(D, SPHGPU_D_DRHODT),
-            derivOffsetDoubles(D, SPHGPU_D_HIDEAL), compDe};
+            derivOffsetDoubles(D, SPHGPU_D_HIDEAL), derivOffsetDoubles(D, SPHGPU_D_MAX_VISCOUS_PRESSURE),
+            derivOffsetDoubles(D, SPHGPU_D_DVDX), compDe};
+  if (!TRIAL) {
+    s.dtIn.ensure(sizeof(double) * size_t(2 + D) * size_t(std::max<int64_t>(s.nInt, 1)));
+    s.haveDtIn = true;
+  }
   SG_REQUIRE(rec < 0 || s.isotropic, SPHGPU_ERR_STATE, "records from the update need H = h I");
   const PackIn pin = rec >= 0 ? packInputs(s) : PackIn{};
   const PackOut pout = rec >= 0 ? packOutputs(s, rec) : PackOut{};
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, s.work.as<int32_t>(),
-                       s.perm.as<int32_t>(), s.nInt, f, b, d, mult, bd, e, sa, pin, pout);
+                       s.perm.as<int32_t>(), s.nInt, f, b, d, bd, e, sa, pin, pout, s.dtIn.as<double>());
   };
-  switch (rec) {
-    case -1: go(k_update<D, -1>); break;
-    case 0: go(k_update<D, 0>); break;
-    case 1: go(k_update<D, 1>); break;
-    case 2: go(k_update<D, 2>); break;
-    case 4: go(k_update<D, 4>); break;
-    case 8: go(k_update<D, 8>); break;
-    default: SG_REQUIRE(false, SPHGPU_ERR_STATE, "unsupported record kinds for the update");
+  // the trial update writes the pair kernel's records, the final one the density sum's
+  if constexpr (TRIAL) {
+    switch (rec) {
+      case -1: go(k_update<D, -1, true>); break;
+      case 0: go(k_update<D, 0, true>); break;
+      case 1: go(k_update<D, 1, true>); break;
+      case 2: go(k_update<D, 2, true>); break;
+      default: SG_REQUIRE(false, SPHGPU_ERR_STATE, "unsupported record kinds for the trial update");
+    }
+  } else {
+    switch (rec) {
+      case -1: go(k_update<D, -1, false>); break;
+      case 4: go(k_update<D, 4, false>); break;
+      case 8: go(k_update<D, 8, false>); break;
+      default: SG_REQUIRE(false, SPHGPU_ERR_STATE, "unsupported record kinds for the final update");
+    }
   }
   SG_CHECK_HIP(hipGetLastError());
   s.recValid = false;
-}
-
-template <int D> void dtInputsD(Sim& s) {
-  s.dtIn.ensure(sizeof(double) * size_t(2 + D) * size_t(std::max<int64_t>(s.nInt, 1)));
-  hipLaunchKernelGGL(k_dt_inputs<D>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, s.work.as<int32_t>(),
-                     s.perm.as<int32_t>(), s.nInt, s.out.as<double>(), s.outStride,
-                     derivOffsetDoubles(D, SPHGPU_D_MAX_VISCOUS_PRESSURE), derivOffsetDoubles(D, SPHGPU_D_DVDX),
-                     derivOffsetDoubles(D, SPHGPU_D_DVDT), s.dtIn.as<double>());
-  SG_CHECK_HIP(hipGetLastError());
-  s.haveDtIn = true;
 }
 
 template <int D> double hydroDtD(Sim& s, double nPerh, double cfl, int useVelMag) {
@@ -403,45 +421,23 @@ __global__ void k_seg_vote_init(SegState* __restrict__ st, int n, unsigned long 
     st[i].fail = 0u;
   }
 }
-// dtThreshold > 0: a member whose vote falls below it (a collapsing step) is
-// flagged; its step still runs and it is evicted afterwards.
-__global__ void k_seg_select_dt(SegState* __restrict__ st, int n, double cfl, double dtMinIn, double dtMaxIn,
-                                double dtGrowth, double dtThreshold) {
+// The end of a step: the clock, and the states to pinned host memory (one
+// launch in place of a selection, an advance and a copy).  dtThreshold > 0: a
+// member whose vote falls below it (a collapsing step) is flagged; its step
+// has run and it is evicted afterwards.
+__global__ void k_seg_advance(SegState* __restrict__ st, int n, SelectArgs sel, double dtThreshold,
+                              SegState* __restrict__ host) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  SegState& g = st[i];
-  const double dtMin = dmin(dtMinIn, g.tEnd - g.t), dtMax = dmin(dtMaxIn, g.tEnd - g.t);
-  const double vote = cfl * __longlong_as_double((long long)g.voteBits);
+  SegState g = st[i];
+  const double vote = sel.cfl * __longlong_as_double((long long)g.voteBits);
   if (dtThreshold > 0.0 && !(vote >= dtThreshold)) g.fail |= unsigned(SPHGPU_MEMBER_DT_COLLAPSE);
-  double dt = dtMax;
-  if (vote > 0.0 && vote < dt) dt = vote;
-  dt = dmin(dt, dtGrowth * g.lastDt);
-  dt = dmin(dtMax, dmax(dtMin, dt));
-  g.dt = dt;
-  g.hdt = 0.5 * dt;
-}
-__global__ void k_seg_advance(SegState* __restrict__ st, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  SegState& g = st[i];
+  g.dt = selectDt(g, sel);
   g.t = g.t + g.dt;
   g.lastDt = g.dt;
   g.cycle = g.cycle + 1.0;
-}
-
-// Several device copies in one dispatch (the step's saved state of a small
-// node set: five launches cost more than the bytes).
-struct CopySet {
-  double* d[5];
-  const double* s[5];
-  int64_t n[5];
-  int m;
-};
-constexpr size_t kCopyManyMaxBytes = size_t(32) << 20;
-__global__ void k_copy_many(CopySet c) {
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int q = 0; q < c.m; ++q)
-    for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < c.n[q]; i += stride) c.d[q][i] = c.s[q][i];
+  st[i] = g;
+  host[i] = g;
 }
 
 // Integrator::preStepInitialize: ghosts and connectivity.  The build's record
@@ -462,11 +458,9 @@ void preStep(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_para
 // The two derivative passes and updates of SynchronousRK2::step, then
 // SPHHydroBase::finalize and Integrator::enforceBoundaries.  Multipliers are
 // dt/2, dt (plain simulation) or per member (half, full).
-template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip, double dt,
+template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip,
                                const SegArgs& half, const SegArgs& full) {
-  constexpr int NS = NSym<D>::value;
   hipStream_t st = s.stream;
-  const double hdt = 0.5 * dt;
   const bool compat = hp.compatibleEnergyEvolution != 0;
   SG_REQUIRE(!compat || s.deviceGhosts || s.nTot == s.nInt, SPHGPU_ERR_UNSUPPORTED,
              "compatible energy with caller-supplied ghost rows: the ghost derivatives need the device boundaries");
@@ -480,29 +474,12 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
   evalDerivs(s, hp, true);
   // state0 (the policy reads every row's step-start velocity, ghosts included)
   const size_t n = size_t(s.nInt), nv = compat ? size_t(s.nTot) : n;
-  const size_t bytes[5] = {sizeof(double) * n * D, sizeof(double) * nv * D, sizeof(double) * n, sizeof(double) * n,
-                           sizeof(double) * n * NS};
-  DBuf* src[5] = {&s.pos, &s.vel, &s.eps, &s.rho, &s.H};
-  CopySet cs{};
-  size_t total = 0;
-  for (int q = 0; q < 5; ++q) {
-    s.state0[q].ensure(std::max<size_t>(bytes[q], 8));
-    cs.d[q] = s.state0[q].as<double>();
-    cs.s[q] = src[q]->as<double>();
-    cs.n[q] = int64_t(bytes[q] / sizeof(double));
-    total += bytes[q];
-  }
-  cs.m = 5;
-  if (total <= kCopyManyMaxBytes) {
-    // one dispatch for the five copies of a small node set
-    hipLaunchKernelGGL(k_copy_many, dim3(nblocks(std::max<int64_t>(1, int64_t(total / sizeof(double) / 5)))),
-                       dim3(kBlock), 0, st, cs);
-    SG_CHECK_HIP(hipGetLastError());
-  } else {
-    for (int q = 0; q < 5; ++q)
-      if (bytes[q]) SG_CHECK_HIP(hipMemcpyAsync(s.state0[q].p, src[q]->p, bytes[q], hipMemcpyDeviceToDevice, st));
-  }
+  const size_t rows[4] = {n * D, nv * D, n, n};
+  for (int q = 0; q < 4; ++q) s.state0[q].ensure(std::max<size_t>(sizeof(double) * rows[q], 8));
   const Base b0{s.state0[0].as<double>(), s.state0[1].as<double>(), s.state0[2].as<double>(), s.state0[3].as<double>()};
+  if (nv > n)
+    SG_CHECK_HIP(hipMemcpyAsync(b0.vel + n * D, s.vel.as<double>() + n * D, sizeof(double) * (nv - n) * D,
+                                hipMemcpyDeviceToDevice, st));
   // omega has no update policy (SPHHydroBase::registerState enrolls it bare):
   // state.assign(state0) gives the final update the step-start value again
   const size_t omegaBytes = sizeof(double) * size_t(s.nTot);
@@ -520,8 +497,8 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
     else applyGhostBoundaries(s);
   };
   // trial advance to the midpoint
-  if (compat) compatD<D>(s, b0.vel, hdt, half);
-  updateD<D>(s, b0, hdt, bd, e, compat ? s.compDe.as<double>() : nullptr, half, recMid);
+  if (compat) compatD<D>(s, s.vel.as<double>(), half);
+  updateD<D, true>(s, b0, bd, e, compat ? s.compDe.as<double>() : nullptr, half, recMid);
   ghostsAndRecords(recMid);
   // derivatives at t + dt/2 with the step's neighbour rows
   if (ip.gradhCorrection) omegaGradh(s);
@@ -529,10 +506,9 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
   if (ip.gradhCorrection && omegaBytes)
     SG_CHECK_HIP(hipMemcpyAsync(s.omega.p, s.omega0.p, omegaBytes, hipMemcpyDeviceToDevice, st));
   // advance from state0 with the midpoint derivatives
-  if (compat) compatD<D>(s, b0.vel, dt, full);
-  updateD<D>(s, b0, dt, bd, e, compat ? s.compDe.as<double>() : nullptr, full, recEnd);
+  if (compat) compatD<D>(s, b0.vel, full);
+  updateD<D, false>(s, b0, bd, e, compat ? s.compDe.as<double>() : nullptr, full, recEnd);
   ghostsAndRecords(recEnd);
-  dtInputsD<D>(s);
   // SPHHydroBase::finalize: sum density
   sumDensity(s);
   // Integrator::enforceBoundaries
@@ -549,7 +525,6 @@ __global__ void k_plain_seg_init(SegState* __restrict__ g, double t, double last
   g->tEnd = tEnd;
   g->gamma = gamma;
   g->dt = 0.0;
-  g->hdt = 0.0;
   g->voteBits = vote;
   g->cycle = 0.0;
   g->fail = 0u;
@@ -595,14 +570,14 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
   keyBytes(k, hp);
   keyBytes(k, ip);
   keyBytes(k, s.dtThreshold);
-  k.push_back(reinterpret_cast<uint64_t>(s.ncalcHost));
+  k.push_back(reinterpret_cast<uint64_t>(s.pinnedOut));
   for (const DBuf* b : {&s.pos, &s.vel, &s.mass, &s.rho, &s.eps, &s.P, &s.cs, &s.H, &s.omega, &s.fCl, &s.fCq,
                         &s.fshear, &s.cellOf, &s.cellCount, &s.cellStart, &s.cellFill, &s.perm, &s.iperm, &s.xs,
                         &s.Hs, &s.rowCount, &s.nbr, &s.scanTmp, &s.reduceTmp, &s.flags, &s.rec, &s.recM, &s.recD,
                         &s.recS, &s.recSM, &s.pairDv, &s.compDe, &s.compAcc, &s.compDe0, &s.compRec, &s.out,
                         &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
                         &s.work, &s.workFlag, &s.workScan, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
-                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.pick, &s.listGamma, &s.subDev})
+                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.pick, &s.listGamma, &s.subDev, &s.pairCounts})
     keyBuf(k, *b);
   for (const DBuf& b : s.state0) keyBuf(k, b);
   return k;
@@ -610,7 +585,7 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
 
 Sim::StepFlags stepFlagsOf(const Sim& s) {
   return Sim::StepFlags{s.recValid, s.recSValid, s.recSMValid, s.derivsValid, s.pairsValid, s.haveDtIn,
-                        s.pairRec, s.outStride, s.timingPending};
+                        s.pairRec, s.outStride, s.timingPending, s.pairWaves};
 }
 void restoreStepFlags(Sim& s, const Sim::StepFlags& f) {
   s.recValid = f.recValid;
@@ -622,6 +597,7 @@ void restoreStepFlags(Sim& s, const Sim::StepFlags& f) {
   s.pairRec = f.pairRec;
   s.outStride = f.outStride;
   s.timingPending = f.timingPending;
+  s.pairWaves = f.pairWaves;
 }
 
 // A few graphs and recent keys are kept: culling swaps the state fields with
@@ -691,27 +667,25 @@ template <int D> double rk2D(Sim& s, const sphgpu_hydro_params& hp, const sphgpu
   std::memcpy(&ib, &init, sizeof(ib));
   hipLaunchKernelGGL(k_plain_seg_init, dim3(1), dim3(1), 0, st, sd, s.time, s.lastDt, maxTime, ip.gamma, ib);
   if (!s.haveDtIn) s.dtIn.ensure(sizeof(double) * 8);
+  const SelectArgs sel{ip.cfl, ip.dtMin, ip.dtMax, ip.dtGrowth};
+  SegState* hs = static_cast<SegState*>(hostStaging(s, 0, sizeof(SegState)));
   runStep(s, hp, ip, [&] {
     hipLaunchKernelGGL(k_dt<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
                        s.perm.as<int32_t>(), s.nInt, s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots,
                        s.H.as<double>(), s.cs.as<double>(), s.rho.as<double>(), s.vel.as<double>(),
                        s.dtIn.as<double>(), s.haveDtIn ? 1 : 0, hp.nPerh, ip.useVelocityMagnitudeForDt, nullptr,
                        &sd->voteBits, int64_t(0));
-    hipLaunchKernelGGL(k_seg_select_dt, dim3(1), dim3(kBlock), 0, st, sd, 1, ip.cfl, ip.dtMin, ip.dtMax, ip.dtGrowth,
-                       0.0);
     SG_CHECK_HIP(hipGetLastError());
     const bool perList = s.nLists > 1 && !s.listGammaHost.empty();
     const double* lo = perList ? s.seg.as<double>() : nullptr;
     const double* lg = perList ? s.listGamma.as<double>() : nullptr;
-    const SegArgs half{nullptr, sd, 1, lo, lg}, full{nullptr, sd, 0, lo, lg};
-    stepBody<D>(s, hp, ip, 0.0, half, full);
-    hipLaunchKernelGGL(k_seg_advance, dim3(1), dim3(kBlock), 0, st, sd, 1);
+    const SegArgs half{nullptr, sd, 1, sel, lo, lg}, full{nullptr, sd, 0, sel, lo, lg};
+    stepBody<D>(s, hp, ip, half, full);
+    hipLaunchKernelGGL(k_seg_advance, dim3(1), dim3(kBlock), 0, st, sd, 1, sel, 0.0, hs);
     SG_CHECK_HIP(hipGetLastError());
   });
-  SegState* hp2 = static_cast<SegState*>(hostStaging(s, 0, sizeof(SegState)));
-  SG_CHECK_HIP(hipMemcpyAsync(hp2, sd, sizeof(SegState), hipMemcpyDeviceToHost, st));
   SG_CHECK_HIP(hipStreamSynchronize(st));
-  const SegState h = *hp2;
+  const SegState h = *hs;
   s.time = h.t;
   s.lastDt = h.lastDt;
   s.cycle += 1;
@@ -730,6 +704,8 @@ template <int D> void ensembleRk2D(Sim& s, const sphgpu_hydro_params& hp, const 
   unsigned long long ib;
   std::memcpy(&ib, &init, sizeof(ib));
   if (!s.haveDtIn) s.dtIn.ensure(sizeof(double) * 8);
+  const SelectArgs sel{ip.cfl, ip.dtMin, ip.dtMax, ip.dtGrowth};
+  SegState* hs = static_cast<SegState*>(hostStaging(s, 0, sizeof(SegState) * size_t(ns)));
   runStep(s, hp, ip, [&] {
     hipLaunchKernelGGL(k_seg_vote_init, dim3(nblocks(ns)), dim3(kBlock), 0, st, sd, ns, ib);
     hipLaunchKernelGGL(k_dt<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
@@ -737,16 +713,12 @@ template <int D> void ensembleRk2D(Sim& s, const sphgpu_hydro_params& hp, const 
                        s.H.as<double>(), s.cs.as<double>(), s.rho.as<double>(), s.vel.as<double>(),
                        s.dtIn.as<double>(), s.haveDtIn ? 1 : 0, hp.nPerh, ip.useVelocityMagnitudeForDt,
                        s.seg.as<double>(), &sd->voteBits, int64_t(sizeof(SegState) / sizeof(unsigned long long)));
-    hipLaunchKernelGGL(k_seg_select_dt, dim3(nblocks(ns)), dim3(kBlock), 0, st, sd, ns, ip.cfl, ip.dtMin, ip.dtMax,
-                       ip.dtGrowth, s.dtThreshold);
     SG_CHECK_HIP(hipGetLastError());
-    const SegArgs half{s.seg.as<double>(), sd, 1}, full{s.seg.as<double>(), sd, 0};
-    stepBody<D>(s, hp, ip, 0.0, half, full);
-    hipLaunchKernelGGL(k_seg_advance, dim3(nblocks(ns)), dim3(kBlock), 0, st, sd, ns);
+    const SegArgs half{s.seg.as<double>(), sd, 1, sel}, full{s.seg.as<double>(), sd, 0, sel};
+    stepBody<D>(s, hp, ip, half, full);
+    hipLaunchKernelGGL(k_seg_advance, dim3(nblocks(ns)), dim3(kBlock), 0, st, sd, ns, sel, s.dtThreshold, hs);
     SG_CHECK_HIP(hipGetLastError());
   });
-  SegState* hs = static_cast<SegState*>(hostStaging(s, 0, sizeof(SegState) * size_t(ns)));
-  SG_CHECK_HIP(hipMemcpyAsync(hs, sd, sizeof(SegState) * size_t(ns), hipMemcpyDeviceToHost, st));
   SG_CHECK_HIP(hipStreamSynchronize(st));
   s.segHost.assign(hs, hs + ns);
   s.derivsValid = false;

@@ -112,7 +112,7 @@ struct SegState {
   double lastDt;            // Integrator::mLastDt
   double tEnd;              // the member runs to this time
   double gamma;             // GammaLawGas gamma
-  double dt, hdt;           // this step's dt and dt/2
+  double dt;                // the last step's dt
   unsigned long long voteBits;   // GenericHydro::dt minimum (bits of a positive double)
   double cycle;
   unsigned int fail;        // SPHGPU_MEMBER_* of this step (0: healthy)
@@ -182,7 +182,8 @@ struct Sim {
   DBuf out;                 // all derivative fields, field-major, sorted order
   int64_t outStride = 0;
   bool derivsValid = false;
-  int64_t ncalc = 0;        // unordered pairs evaluated by the last pass
+  DBuf pairCounts;          // unordered pairs of each wavefront of the last pass
+  int64_t pairWaves = 0;    // its wavefronts
 
   // planar ghost boundaries generated on the device
   std::vector<SubBoundary> subs;
@@ -208,7 +209,7 @@ struct Sim {
   double time = 0.0;
   double lastDt = 1.0e-5;        // Integrator::mLastDt default
   int64_t cycle = 0;
-  DBuf state0[5];                // pos, vel, eps, rho, H of the internal rows at the step start
+  DBuf state0[4];                // pos, vel, eps, rho of the internal rows at the step start
   DBuf omega0;                   // grad-h: every row's step-start omega (state.assign restores it)
   DBuf dtIn;                     // per internal node: maxViscousPressure, tr DvDx, DvDt (caller order)
   bool haveDtIn = false;
@@ -260,6 +261,7 @@ struct Sim {
     int pairRec;
     int64_t outStride;
     unsigned timingPending;
+    int64_t pairWaves;
   };
   struct StepGraph {
     std::vector<uint64_t> key;
@@ -271,10 +273,9 @@ struct Sim {
   int64_t graphCaptures = 0, graphReplays = 0;
   hipEvent_t ev[14] = {};          // 0-11 stage timings, 12-13 the copy probe
   Timing timing;
-  // Stage timings and the pair count are read back lazily (no host wait
-  // inside a step): bit 0 neighbours, 1 density, 2 derivatives, 3 ghosts.
+  // Stage timings are read back lazily (no host wait inside a step): bit 0
+  // neighbours, 1 density, 2 derivatives, 3 ghosts.
   unsigned timingPending = 0;
-  unsigned long long* ncalcHost = nullptr;   // pinned; written by the stream after each pass
   // Pinned host staging: small readbacks (copies into pageable memory would
   // each wait for the stream) and uploads the stream reads after the call
   // returns (the grid lists of a neighbour build).  Grown only after a sync.
@@ -387,8 +388,7 @@ bool operator<(const TuneKey& a, const TuneKey& b);
 enum { kTunePairIso = 0 };
 TuneKey tuneKey(int kernel, int dim, int precision, double rowLength, int64_t nodes);
 void tuneEnable(bool on);
-int tunedVariant(Sim& s, const TuneKey& key, int nVariants, int fallback, const std::function<void(int)>& launch,
-                 bool* timed = nullptr);
+int tunedVariant(Sim& s, const TuneKey& key, int nVariants, int fallback, const std::function<void(int)>& launch);
 std::string tuneExport();
 int tuneImport(const std::string& text);
 

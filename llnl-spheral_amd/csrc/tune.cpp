@@ -46,9 +46,7 @@ void tuneEnable(bool on) {
   gEnabled = on;
 }
 
-int tunedVariant(Sim& s, const TuneKey& key, int nVariants, int fallback, const std::function<void(int)>& launch,
-                 bool* timed) {
-  if (timed) *timed = false;
+int tunedVariant(Sim& s, const TuneKey& key, int nVariants, int fallback, const std::function<void(int)>& launch) {
   {
     std::lock_guard<std::mutex> lock(gMu);
     auto it = gTable.find(key);
@@ -68,7 +66,6 @@ int tunedVariant(Sim& s, const TuneKey& key, int nVariants, int fallback, const 
     }
   }
   c.variant = int(std::min_element(c.ms.begin(), c.ms.end()) - c.ms.begin());
-  if (timed) *timed = true;
   std::lock_guard<std::mutex> lock(gMu);
   gTable[key] = c;
   return c.variant;
