@@ -118,8 +118,10 @@ int sphgpu_create(int dim, int device, sphgpu_sim** out) {
     delete s;
     return SPHGPU_ERR_HIP;
   }
+  // timing events only: nothing waits on one to read what the stream wrote, so
+  // they need no system-scope fence (a cache write-back at every record)
   for (auto& e : s->ev) {
-    if (hipEventCreate(&e) != hipSuccess) { sphgpu_destroy(s); return SPHGPU_ERR_HIP; }
+    if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) { sphgpu_destroy(s); return SPHGPU_ERR_HIP; }
   }
   // the allocation-free entry point's scratch array on this device (once)
   try {
