@@ -140,7 +140,7 @@ void sphgpu_destroy(sphgpu_sim* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   DBuf* bufs[] = {&s->dTable, &s->dNperh, &s->dWsum, &s->pos, &s->vel, &s->mass, &s->rho, &s->eps, &s->P, &s->cs,
                   &s->H, &s->omega, &s->fCl, &s->fCq, &s->fshear, &s->cellOf, &s->cellCount, &s->cellStart,
-                  &s->cellFill, &s->perm, &s->iperm, &s->xs, &s->Hs, &s->rowCount, &s->nbr,
+                  &s->cellRank, &s->cellMembers, &s->perm, &s->iperm, &s->xs, &s->rowCount, &s->nbr,
                   &s->scanTmp, &s->reduceTmp, &s->flags, &s->rec, &s->out};
   for (DBuf* b : bufs) b->release();
   for (auto& e : s->ev) if (e) (void)hipEventDestroy(e);
@@ -148,7 +148,6 @@ void sphgpu_destroy(sphgpu_sim* s) {
   if (s->pinnedOut) (void)hipHostFree(s->pinnedOut);
   if (s->pinnedIn) (void)hipHostFree(s->pinnedIn);
   if (s->pinnedInDone) (void)hipEventDestroy(s->pinnedInDone);
-  s->pick.release();
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }

@@ -38,12 +38,11 @@
 #include "ell.hh"
 #include "eigen.hh"
 #include "pack.hh"
+#include "scan.hh"
 #include <cmath>
 #include <algorithm>
 
 namespace sphgpu {
-
-void exclusiveScanI32(const int32_t* in, int32_t* out, int64_t n, Sim& s);
 
 namespace {
 
@@ -144,158 +143,141 @@ template <int D> __device__ __forceinline__ void reflectH(const double* R, const
     for (int j = i; j < D; ++j, ++c) out[c] = (i == j) ? t2[i * D + i] : 0.5 * (t2[i * D + j] + t2[j * D + i]);
 }
 
-// 1/lambda_min(H) of the internal nodes (a ghost's is computed when it is made).
-template <int D>
-__global__ void k_hinv_min(const double* __restrict__ H, int64_t n, double* __restrict__ hmaxOf) {
-  constexpr int NS = NSym<D>::value;
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (i < n) hmaxOf[i] = 1.0 / minEigen<D>(H + i * NS);
+// Ghost generation, device-held counts: gen[0] is set when a ghost fell beyond
+// the capacity, gen[1 + b] holds the rows before plane b's ghosts (gen[1] =
+// nInt), gen[1 + nSubs] all rows.
+//
+// A plane's hmax is the maximum of h = 1/lambda_min(H) over the rows near it:
+// the internal nodes of a member or NodeList are entered for all planes by one
+// launch, and each ghost enters itself for the planes after its own when it is
+// made, so a plane needs no pass of its own for it.
+struct HmaxBits {
+  unsigned long long* bits;   // [plane][group], zero before the generation
+  int groups;
+};
+// A non-negative double's bits order as the double: the maximum is an atomic
+// max of the bits, skipped where the slot already holds as much (a plain read
+// may be stale, then the atomic decides).
+__device__ __forceinline__ void enterBits(unsigned long long* p, double h) {
+  const unsigned long long v = (unsigned long long)__double_as_longlong(h);
+  if (v > *static_cast<volatile unsigned long long*>(p)) atomicMax(p, v);
+}
+template <int D> __device__ __forceinline__ bool nearPlane(const DSub& b, const V<D>& x, double h, double ext) {
+  const double d = dmin(dabs(signedDist<D>(b.exitP, b.exitN, x)), dabs(signedDist<D>(b.enterP, b.enterN, x)));
+  return h > 0.0 && d < ext * h;
 }
 
-// hmax of the nodes near either plane, one value: grid-stride loop, a block
-// maximum and one 64-bit atomic max per block.
-// Row counts of the ghost kernels: `n` rows, or, with nDev, the count the
-// device holds (n is then the capacity the grid covers).
-__device__ __forceinline__ int64_t liveRows(int64_t n, const int64_t* nDev) { return nDev ? *nDev : n; }
-
+// h and hmax of the internal rows, the first counts, and the next generation's
+// hmax table cleared.  A wavefront walks `rows64` consecutive groups of 64 rows
+// once per plane (its rows stay in L1) and enters one maximum per plane, or,
+// when its rows span members, one per lane: with an entry per row, 2.1 M rows
+// took 534 us, all of it contention for the six words.
 template <int D>
-__global__ void k_ghost_hmax_one(const double* __restrict__ pos, const double* __restrict__ hmaxOf, int64_t n, DSub b,
-                                 double ext, unsigned long long* __restrict__ hmaxBits, const int64_t* __restrict__ nDev) {
-  __shared__ double wmax[kBlock / 64];
-  double v = 0.0;
-  const int64_t nn = liveRows(n, nDev);
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < nn; i += int64_t(gridDim.x) * blockDim.x) {
-    const V<D> x = loadV<D>(pos, i);
-    const double hmaxi = hmaxOf[i];
-    const double d = dmin(dabs(signedDist<D>(b.exitP, b.exitN, x)), dabs(signedDist<D>(b.enterP, b.enterN, x)));
-    if (hmaxi > 0.0 && d < ext * hmaxi) v = dmax(v, hmaxi);
+__global__ void k_gen_start(const double* __restrict__ pos, const double* __restrict__ H,
+                            const double* __restrict__ seg, int64_t nInt, const DSub* __restrict__ subs, int nSubs,
+                            double ext, HmaxBits hb, double* hmaxOf, int64_t* __restrict__ gen,
+                            unsigned long long* __restrict__ clear, int rows64) {
+  const int64_t tid = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (tid == 0) {
+    gen[0] = 0;
+    gen[1] = nInt;
   }
-  for (int sh = 32; sh > 0; sh >>= 1) v = dmax(v, __shfl_xor(v, sh));
-  if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < kBlock / 64; ++w) v = dmax(v, wmax[w]);
-    if (v > 0.0) atomicMax(hmaxBits, (unsigned long long)__double_as_longlong(v));
-  }
-}
-
-// hmax of the nodes near either plane per ensemble member (hmaxBits[member]).
-template <int D>
-__global__ void k_ghost_hmax(const double* __restrict__ pos, const double* __restrict__ hmaxOf,
-                             const double* __restrict__ seg, int64_t n, DSub b, double ext,
-                             unsigned long long* __restrict__ hmaxBits, const int64_t* __restrict__ nDev) {
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  double v = 0.0;
-  int m = 0;
-  if (i < liveRows(n, nDev)) {
-    const V<D> x = loadV<D>(pos, i);
-    const double hmaxi = hmaxOf[i];
-    const double d = dmin(dabs(signedDist<D>(b.exitP, b.exitN, x)), dabs(signedDist<D>(b.enterP, b.enterN, x)));
-    if (hmaxi > 0.0 && d < ext * hmaxi) v = hmaxi;
-    if (seg) m = int(seg[i]);
-  }
-  const int m0 = __shfl(m, 0);
-  if (__all(m == m0)) {
-    for (int sh = 32; sh > 0; sh >>= 1) v = dmax(v, __shfl_xor(v, sh));
-    if ((threadIdx.x & 63) == 0 && v > 0.0) atomicMax(hmaxBits + m0, (unsigned long long)__double_as_longlong(v));
-  } else if (v > 0.0) {
-    atomicMax(hmaxBits + m, (unsigned long long)__double_as_longlong(v));
-  }
-}
-
-template <int D>
-// blockCount (optional): each workgroup's count of flags, for k_ghost_make<BLK>.
-__global__ void k_ghost_flag(const double* __restrict__ pos, const double* __restrict__ seg, int64_t n, DSub b,
-                             double ext, const unsigned long long* __restrict__ hmaxBits, int32_t* __restrict__ flags,
-                             const int64_t* __restrict__ nDev, int32_t* __restrict__ blockCount) {
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  int32_t f = 0;
-  if (i < liveRows(n, nDev)) {                    // capacity rows beyond the live count take no flag
-    const double hmax = __longlong_as_double((long long)hmaxBits[seg ? int(seg[i]) : 0]);
-    if (hmax > 0.0) {
-      const double disti = signedDist<D>(b.exitP, b.exitN, loadV<D>(pos, i)) / hmax;
-      f = (disti >= 0.0 && disti <= ext) ? 1 : 0;
+  for (int64_t q = tid; q < int64_t(nSubs) * hb.groups; q += int64_t(gridDim.x) * blockDim.x) clear[q] = 0ull;
+  const int lane = threadIdx.x & 63;
+  const int64_t base = (tid >> 6) * int64_t(64 * rows64) + lane;
+  if (base - lane >= nInt) return;                 // uniform over the wavefront
+  int group = 0;
+  bool one = true;                                 // every row of the walk in one group
+  for (int it = 0; it < rows64; ++it) {
+    const int64_t i = base + int64_t(it) * 64;
+    if (i < nInt) hmaxOf[i] = 1.0 / minEigen<D>(H + i * NSym<D>::value);
+    if (seg) {
+      const int g = i < nInt ? int(seg[i]) : -1, g0 = __shfl(g, 0);
+      if (it == 0) group = g0;
+      one = one && __all(g == group || g < 0) != 0;
     }
   }
-  if (i < n) flags[i] = f;
-  if (blockCount) {
-    const int c = __syncthreads_count(f);        // every thread of the block reaches it
-    if (threadIdx.x == 0) blockCount[blockIdx.x] = c;
+  for (int b = 0; b < nSubs; ++b) {
+    double v = 0.0;
+    for (int it = 0; it < rows64; ++it) {
+      const int64_t i = base + int64_t(it) * 64;
+      if (i >= nInt) break;
+      const double h = hmaxOf[i];
+      if (!nearPlane<D>(subs[b], loadV<D>(pos, i), h, ext)) continue;
+      if (one) v = dmax(v, h);
+      else enterBits(hb.bits + int64_t(b) * hb.groups + int(seg[i]), h);
+    }
+    if (!one || __ballot(v > 0.0) == 0) continue;
+    for (int sh = 32; sh > 0; sh >>= 1) v = dmax(v, __shfl_xor(v, sh));
+    if (lane == 0) enterBits(hb.bits + int64_t(b) * hb.groups + group, v);
   }
 }
 
-// BLK: offs holds the exclusive scan of the flag kernel's per-workgroup counts
-// (same grid and workgroup size), and a row's offset is its workgroup's plus
-// its rank among the workgroup's flags: the global exclusive scan of flags.
-// Otherwise offs is that scan itself.
-template <int D, bool BLK>
-__global__ void __launch_bounds__(kBlock) k_ghost_make(double* __restrict__ pos, double* __restrict__ H, double* __restrict__ seg, int64_t n,
-                             int64_t nInt, const int32_t* __restrict__ flags, const int32_t* __restrict__ offs, DSub b,
-                             int subIdx, int32_t* __restrict__ control, int32_t* __restrict__ subOf,
-                             double* __restrict__ hmaxOf, const int64_t* __restrict__ nDev, int64_t cap,
-                             int64_t* __restrict__ overflow) {
-  constexpr int NS = NSym<D>::value;
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  const int64_t nn = liveRows(n, nDev);
-  int64_t off;
-  if constexpr (BLK) {
-    const bool f = i < nn && flags[i] != 0;
-    const unsigned long long m = __ballot(f);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    __shared__ int waveCount[kBlock / 64];
-    if (lane == 0) waveCount[wave] = __popcll(m);
-    __syncthreads();
-    if (!f) return;
-    int before = 0;
-    for (int w = 0; w < wave; ++w) before += waveCount[w];
-    off = int64_t(offs[blockIdx.x]) + before + __popcll(m & ((1ull << lane) - 1ull));
-  } else {
-    if (i >= nn || !flags[i]) return;
-    off = offs[i];
+// One plane's ghosts (scan.hh): the rows that are its controls, in index order,
+// each appended after the rows that were there.  Flag, scan, compaction and the
+// new row count in one launch (two for large node sets), where they were five.
+template <int D> struct GhostPlane {
+  static constexpr bool kCompact = true;
+  double *pos, *H, *seg;
+  int64_t cap, nInt;
+  const DSub* subs;
+  int plane, nSubs;
+  double ext;
+  HmaxBits hb;
+  double* hmaxOf;
+  int32_t *control, *subOf, *isControl;
+  int64_t* gen;
+  __device__ __forceinline__ int64_t live() const { return gen[1 + plane]; }
+  __device__ int32_t value(int64_t i) const {
+    if (i >= live()) return 0;
+    const int group = seg ? int(seg[i]) : 0;
+    const double hmax = __longlong_as_double((long long)hb.bits[int64_t(plane) * hb.groups + group]);
+    if (!(hmax > 0.0)) return 0;
+    const DSub& b = subs[plane];
+    const double d = signedDist<D>(b.exitP, b.exitN, loadV<D>(pos, i)) / hmax;
+    return d >= 0.0 && d <= ext ? 1 : 0;
   }
-  const int64_t g = nn + off;
-  if (nDev && g >= cap) { *overflow = 1; return; }   // the capacity guess was short: the build redoes it exactly
-  const V<D> xg = ghostPosition<D>(b, loadV<D>(pos, i));
-  for (int k = 0; k < D; ++k) pos[g * D + k] = xg.c[k];
-  if (b.reflect) {
-    double hg[NS];
-    reflectH<D>(b.R, H + i * NS, hg);
-    for (int k = 0; k < NS; ++k) H[g * NS + k] = hg[k];
-    hmaxOf[g] = 1.0 / minEigen<D>(hg);
-  } else {
-    for (int k = 0; k < NS; ++k) H[g * NS + k] = H[i * NS + k];
-    hmaxOf[g] = hmaxOf[i];
+  __device__ void emit(int64_t i, int32_t prefix, int32_t) const {
+    constexpr int NS = NSym<D>::value;
+    const DSub& b = subs[plane];
+    const int64_t g = live() + prefix;
+    if (g >= cap) { gen[0] = 1; return; }          // the capacity was short: the caller generates again
+    const V<D> xc = loadV<D>(pos, i), x = ghostPosition<D>(b, xc);
+    for (int k = 0; k < D; ++k) pos[g * D + k] = x.c[k];
+    // the control's h, unless the reflection changed H (an h I stays itself
+    // under an axis plane): the eigenvalue is a function of these values alone
+    const double hc = hmaxOf[i];
+    double h = hc;
+    if (b.reflect) {
+      double hg[NS];
+      bool same = true;
+      reflectH<D>(b.R, H + i * NS, hg);
+      for (int k = 0; k < NS; ++k) {
+        same = same && hg[k] == H[i * NS + k];
+        H[g * NS + k] = hg[k];
+      }
+      if (!same) h = 1.0 / minEigen<D>(hg);
+    } else {
+      for (int k = 0; k < NS; ++k) H[g * NS + k] = H[i * NS + k];
+    }
+    hmaxOf[g] = h;
+    control[g - nInt] = int32_t(i);
+    subOf[g - nInt] = plane;
+    isControl[g - nInt] = 0;
+    if (i >= nInt) isControl[i - nInt] = 1;
+    if (seg) seg[g] = seg[i];
+    const int group = seg ? int(seg[i]) : 0;
+    // nothing to enter where the control, near the plane itself, has entered as much
+    for (int q = plane + 1; q < nSubs; ++q)
+      if (nearPlane<D>(subs[q], x, h, ext) && !(hc >= h && nearPlane<D>(subs[q], xc, hc, ext)))
+        enterBits(hb.bits + int64_t(q) * hb.groups + group, h);
   }
-  control[g - nInt] = int32_t(i);
-  subOf[g - nInt] = subIdx;
-  if (seg) seg[g] = seg[i];
-}
-
-// After a plane with device-held counts: the plane's first ghost, then the new
-// live count (the count of flags is the scan's total over the capacity).
-struct GenDev {
-  int64_t n;            // live rows
-  int64_t overflow;     // set when a ghost fell beyond the capacity
-  int64_t start[16];    // first ghost (offset from nInt) of each sub-boundary
+  __device__ void total(int32_t t) const {
+    const int64_t next = live() + t;
+    if (next > cap) gen[0] = 1;
+    gen[2 + plane] = next > cap ? cap : next;
+  }
 };
-// Both also clear the hmax words of the next plane.
-__global__ void k_gen_init(GenDev* g, int64_t nInt, unsigned long long* __restrict__ hbits, int nh) {
-  for (int q = threadIdx.x; q < nh; q += blockDim.x) hbits[q] = 0ull;
-  if (threadIdx.x == 0) {
-    g->n = nInt;
-    g->overflow = 0;
-  }
-}
-__global__ void k_gen_advance(GenDev* g, int b, const int32_t* __restrict__ total, int64_t nInt, int64_t cap,
-                              unsigned long long* __restrict__ hbits, int nh) {
-  for (int q = threadIdx.x; q < nh; q += blockDim.x) hbits[q] = 0ull;
-  if (threadIdx.x == 0) {
-    g->start[b] = g->n - nInt;
-    const int64_t next = g->n + int64_t(*total);
-    if (next > cap) g->overflow = 1;
-    g->n = next > cap ? cap : next;
-  }
-}
 
 struct FieldPtrs {
   double *pos, *H, *vel, *mass, *rho, *eps, *P, *cs, *omega, *fCl, *fCq, *fsh, *seg;
@@ -332,9 +314,10 @@ __device__ __forceinline__ const DSub& ghostPlane(const GhostMap& m, int64_t g, 
 // All ghost rows [nInt, nTot) from their internal nodes.  REC >= 0: also their
 // slots' records (pack sec bits, isotropic layout) from the values just stored.
 template <int D, int REC>
-__global__ void k_ghost_fields(FieldPtrs f, GhostMap m, int64_t nTot, int geometry, const int32_t* __restrict__ iperm,
-                               PackIn pin, PackOut pout) {
+__global__ void k_ghost_fields(FieldPtrs f, GhostMap m, int64_t nTot, const int64_t* __restrict__ nDev, int geometry,
+                               const int32_t* __restrict__ iperm, PackIn pin, PackOut pout) {
   constexpr int NS = NSym<D>::value;
+  if (nDev) nTot = *nDev;                          // a generation's count, still on the device
   const int64_t g = m.nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (g >= nTot) return;
   int depth;
@@ -490,22 +473,33 @@ __global__ void k_enforce(double* __restrict__ pos, double* __restrict__ vel, do
 }
 
 // ---- culling ---------------------------------------------------------------
-// keep[c]: internal nodes, ghosts some row holds (marked by the search in slot
-// space), then every ghost that controls another ghost.
-__global__ void k_keep_gather(int32_t* __restrict__ keep, const int32_t* __restrict__ iperm,
-                              const int32_t* __restrict__ slotKeep, int64_t nInt, int64_t nTot) {
-  const int64_t c = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (c < nInt) keep[c] = 1;
-  else if (c < nTot) keep[c] = slotKeep[iperm[c]];
-}
-
-__global__ void k_keep_controls(int32_t* __restrict__ keep, int64_t nInt, int64_t nTot,
-                                const int32_t* __restrict__ control) {
-  const int64_t g = nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (g >= nTot) return;
-  const int32_t c = control[g - nInt];
-  if (c >= nInt) keep[c] = 1;
-}
+// Which ghosts stay (scan.hh, over the ghosts): those some row holds (marked by
+// the search in slot space) and those that control another ghost (marked when
+// that one was made).  keep and scan are by ghost; the new first ghost of every
+// plane, the new ghost count and the search's flags go to pinned memory.
+struct KeepScan {
+  static constexpr bool kCompact = false;
+  const int32_t *slotKeep, *iperm, *isControl;
+  int32_t *keep, *scan;
+  int64_t nInt, ng;
+  const int64_t* gen;       // gen[1 + b]: the rows before plane b's ghosts
+  int nSubs;
+  const int32_t* flags;
+  int32_t *flagsOut, *starts;
+  __device__ int32_t value(int64_t g) const { return slotKeep[iperm[nInt + g]] != 0 || isControl[g] != 0 ? 1 : 0; }
+  __device__ void emit(int64_t g, int32_t prefix, int32_t v) const {
+    keep[g] = v;
+    scan[g] = prefix;
+    for (int b = 0; b < nSubs; ++b)
+      if (gen[1 + b] - nInt == g) starts[b] = prefix;
+  }
+  __device__ void total(int32_t t) const {
+    for (int b = 0; b < nSubs; ++b)
+      if (gen[1 + b] - nInt >= ng) starts[b] = t;
+    starts[nSubs] = t;
+    for (int q = 0; q < 8; ++q) flagsOut[q] = flags[q];
+  }
+};
 
 // Renumbering after the cull, one lane per caller row and slot: the kept
 // ghosts' controls and planes, the caller -> slot map, and the slots' caller
@@ -520,18 +514,19 @@ __global__ void k_cull(const int32_t* __restrict__ control, const int32_t* __res
                        const int32_t* __restrict__ keep, const int32_t* __restrict__ scan, int64_t nInt, int64_t nTot,
                        int64_t nSlots, double* __restrict__ rec, int stride, int origOff) {
   const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (t < nTot && keep[t]) {
-    const int64_t o = scan[t];
-    newIperm[o] = iperm[t];
-    if (t >= nInt) {
-      newControl[o - nInt] = scan[control[t - nInt]];
-      newSubOf[o - nInt] = subOf[t - nInt];
-    }
+  if (t < nInt) {
+    newIperm[t] = iperm[t];
+  } else if (t < nTot && keep[t - nInt]) {
+    const int64_t o = scan[t - nInt];
+    const int32_t c = control[t - nInt];
+    newIperm[nInt + o] = iperm[t];
+    newControl[o] = c < nInt ? c : int32_t(nInt) + scan[c - nInt];
+    newSubOf[o] = subOf[t - nInt];
   }
   if (t < nSlots) {
     const int32_t c = perm[t];
-    if (c < 0) return;
-    const int32_t nc = keep[c] ? scan[c] : -1;
+    if (c < nInt) return;
+    const int32_t nc = keep[c - nInt] ? int32_t(nInt) + scan[c - nInt] : -1;
     perm[t] = nc;
     if (rec) rec[t * stride + origOff] = nc >= 0 ? double(nc) : 2147483648.0;
   }
@@ -578,8 +573,10 @@ GhostMap ghostMap(const Sim& s) {
   return GhostMap{s.ghostControl.as<int32_t>(), s.ghostSub.as<int32_t>(), s.subDev.as<DSub>(), s.nInt};
 }
 
+// Rows [nInt, nTot), or those of a generation whose count is on the device.
 template <int D> void applyFieldsD(Sim& s, bool geometry, int rec) {
-  const int64_t ng = s.nTot - s.nInt;
+  const int64_t rows = s.genPending ? s.genCap : s.nTot, ng = rows - s.nInt;
+  const int64_t* nDev = s.genPending ? s.genDev.as<int64_t>() + s.subs.size() + 1 : nullptr;
   if (ng <= 0) {
     if (rec >= 0) (void)packOutputs(s, rec);
     return;
@@ -589,7 +586,7 @@ template <int D> void applyFieldsD(Sim& s, bool geometry, int rec) {
   const PackIn pin = rec >= 0 ? packInputs(s) : PackIn{};
   const PackOut pout = rec >= 0 ? packOutputs(s, rec) : PackOut{};
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(nblocks(ng)), dim3(kBlock), 0, s.stream, f, m, s.nTot, geometry ? 1 : 0,
+    hipLaunchKernelGGL(kern, dim3(nblocks(ng)), dim3(kBlock), 0, s.stream, f, m, rows, nDev, geometry ? 1 : 0,
                        s.iperm.as<int32_t>(), pin, pout);
   };
   switch (rec) {
@@ -609,145 +606,72 @@ void applyFields(Sim& s, bool geometry, int rec) {
   else applyFieldsD<3>(s, geometry, rec);
 }
 
-// Every plane's ghosts with the running row count kept on the device: the
-// grids cover a capacity guessed from the previous generation, and one
-// readback at the end returns the count and each sub-boundary's first ghost.
-// Returns false when a plane's ghosts would pass the capacity (the caller then
-// generates again plane by plane; generation reads only internal rows).
-template <int D> bool generateFastD(Sim& s, double ext, unsigned long long* hbits, int nh) {
+// Every plane's ghosts, with the running row count kept on the device: the
+// launches cover a capacity of `est` ghosts, and the neighbour build reads the
+// counts back with its bounds (finishGeneration), one wait for both.  Generation
+// reads only internal rows, so a short capacity costs a second one.
+template <int D> void generateD(Sim& s, double ext, int64_t est) {
   hipStream_t st = s.stream;
-  const int64_t nInt = s.nInt;
-  const int64_t est = s.ghostsGenerated + s.ghostsGenerated / 4 + 1024;
-  const int64_t cap = nInt + est;
+  const int64_t nInt = s.nInt, cap = nInt + est;
   SG_REQUIRE(cap < (int64_t(1) << 31) - 1, SPHGPU_ERR_CAPACITY, "too many ghost nodes");
+  const int nSubs = int(s.subs.size()), groups = std::max(1, groupCount(s));
   ensureRows(s, cap);
-  s.hmaxOf.grow(sizeof(double) * size_t(cap), sizeof(double) * size_t(nInt), st);
-  s.ghostControl.grow(sizeof(int32_t) * size_t(est), 0, st);
-  s.ghostSub.grow(sizeof(int32_t) * size_t(est), 0, st);
-  s.keep.ensure(sizeof(int32_t) * size_t(cap + 1));
-  // per-workgroup flag counts (at nb + 1) and their exclusive scan (at 0)
-  const int64_t nb = nblocks(cap);
-  s.keepScan.ensure(sizeof(int32_t) * size_t(std::max<int64_t>(cap + 1, 2 * (nb + 1))));
-  int32_t* blkScan = s.keepScan.as<int32_t>();
-  int32_t* blkCount = blkScan + (nb + 1);
-  s.genDev.ensure(sizeof(GenDev));
-  GenDev* g = s.genDev.as<GenDev>();
-  const int64_t* nDev = &g->n;
-  hipLaunchKernelGGL(k_gen_init, dim3(1), dim3(kBlock), 0, st, g, nInt, hbits, nh);
-  const double* segp = groupCount(s) > 0 ? s.seg.as<double>() : nullptr;
-  for (size_t b = 0; b < s.subs.size(); ++b) {
-    const DSub d = toDevice(s.subs[b]);
-    if (segp)
-      hipLaunchKernelGGL(k_ghost_hmax<D>, dim3(nblocks(cap)), dim3(kBlock), 0, st, s.pos.as<double>(),
-                         s.hmaxOf.as<double>(), segp, cap, d, ext, hbits, nDev);
-    else
-      hipLaunchKernelGGL(k_ghost_hmax_one<D>, dim3(std::min(nblocks(cap), 1024)), dim3(kBlock), 0, st,
-                         s.pos.as<double>(), s.hmaxOf.as<double>(), cap, d, ext, hbits, nDev);
-    hipLaunchKernelGGL(k_ghost_flag<D>, dim3(nb), dim3(kBlock), 0, st, s.pos.as<double>(), segp, cap, d, ext, hbits,
-                       s.keep.as<int32_t>(), nDev, blkCount);
-    exclusiveScanI32(blkCount, blkScan, nb, s);
-    hipLaunchKernelGGL((k_ghost_make<D, true>), dim3(nb), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(),
-                       groupCount(s) > 0 ? s.seg.as<double>() : nullptr, cap, nInt, s.keep.as<int32_t>(), blkScan, d, int(b),
-                       s.ghostControl.as<int32_t>(), s.ghostSub.as<int32_t>(), s.hmaxOf.as<double>(), nDev, cap,
-                       &g->overflow);
-    hipLaunchKernelGGL(k_gen_advance, dim3(1), dim3(kBlock), 0, st, g, int(b), blkScan + nb, nInt, cap, hbits, nh);
-    SG_CHECK_HIP(hipGetLastError());
+  s.hmaxOf.ensure(sizeof(double) * size_t(cap));
+  for (DBuf* b : {&s.ghostControl, &s.ghostSub, &s.ghostIsControl}) b->ensure(sizeof(int32_t) * size_t(est));
+  s.genDev.ensure(sizeof(int64_t) * size_t(nSubs + 2));
+  unsigned long long* next = nullptr;
+  const HmaxBits hb{s.hmaxBits.take(size_t(nSubs) * size_t(groups), st, next), groups};
+  double* seg = groupCount(s) > 0 ? s.seg.as<double>() : nullptr;
+  // one group of 64 rows a wavefront until every SIMD has one
+  const int rows64 = int(std::min<int64_t>(16, std::max<int64_t>(1, nInt / (64 * 1024))));
+  hipLaunchKernelGGL(k_gen_start<D>, dim3(nblocks((nInt + rows64 - 1) / rows64)), dim3(kBlock), 0, st,
+                     s.pos.as<double>(), s.H.as<double>(), seg, nInt, s.subDev.as<DSub>(), nSubs, ext, hb,
+                     s.hmaxOf.as<double>(), s.genDev.as<int64_t>(), next, rows64);
+  SG_CHECK_HIP(hipGetLastError());
+  for (int b = 0; b < nSubs; ++b) {
+    // rows before plane b: all of the capacity but for the first plane
+    const GhostPlane<D> op{s.pos.as<double>(), s.H.as<double>(), seg, cap, nInt, s.subDev.as<DSub>(), b, nSubs, ext, hb,
+                           s.hmaxOf.as<double>(), s.ghostControl.as<int32_t>(), s.ghostSub.as<int32_t>(),
+                           s.ghostIsControl.as<int32_t>(), s.genDev.as<int64_t>()};
+    scanItems(op, b == 0 ? nInt : cap, s.scanTmp, st);
   }
-  GenDev* h = static_cast<GenDev*>(hostStaging(s, 0, sizeof(GenDev)));
-  SG_CHECK_HIP(hipMemcpyAsync(h, g, sizeof(GenDev), hipMemcpyDeviceToHost, st));
-  SG_CHECK_HIP(hipStreamSynchronize(st));
-  if (h->overflow) return false;
-  s.nTot = h->n;
-  for (size_t b = 0; b < s.subs.size(); ++b) s.subStart[b] = h->start[b];
-  return true;
+  s.genCap = cap;
+  s.genPending = true;
+  applyFieldsD<D>(s, false, -1);
 }
 
-template <int D> void generateD(Sim& s, double ext) {
-  hipStream_t st = s.stream;
-  constexpr int NS = NSym<D>::value;
-  (void)NS;
-  s.subStart.assign(s.subs.size() + 1, 0);
-  s.flags.ensure(sizeof(int32_t) * 8 + sizeof(unsigned long long) * 2);
-  unsigned long long* hbits = reinterpret_cast<unsigned long long*>(s.flags.as<int32_t>() + 4);
-  const int nh = std::max(1, groupCount(s));
-  if (groupCount(s) > 0) {
-    s.segHmaxBits.ensure(sizeof(unsigned long long) * size_t(nh));
-    hbits = s.segHmaxBits.as<unsigned long long>();
-  }
-  s.hmaxOf.ensure(sizeof(double) * size_t(std::max<int64_t>(s.nInt, 1)));
-  if (s.nInt > 0)
-    hipLaunchKernelGGL(k_hinv_min<D>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, st, s.H.as<double>(), s.nInt,
-                       s.hmaxOf.as<double>());
-  // after a first generation, one readback for all planes
-  bool done = false;
-  if (s.ghostsGenerated > 0 && !s.subs.empty() && s.subs.size() < 16) {
-    done = generateFastD<D>(s, ext, hbits, nh);
-    if (!done) s.nTot = s.nInt;
-  }
-  for (size_t b = 0; !done && b < s.subs.size(); ++b) {
-    const int64_t n = s.nTot;
-    s.subStart[b] = n - s.nInt;
-    const DSub d = toDevice(s.subs[b]);
-    s.keep.ensure(sizeof(int32_t) * size_t(n + 1));
-    s.keepScan.ensure(sizeof(int32_t) * size_t(n + 1));
-    const double* segp = groupCount(s) > 0 ? s.seg.as<double>() : nullptr;
-    SG_CHECK_HIP(hipMemsetAsync(hbits, 0, sizeof(unsigned long long) * size_t(nh), st));
-    if (segp)
-      hipLaunchKernelGGL(k_ghost_hmax<D>, dim3(nblocks(n)), dim3(kBlock), 0, st, s.pos.as<double>(),
-                         s.hmaxOf.as<double>(), segp, n, d, ext, hbits, nullptr);
-    else
-      hipLaunchKernelGGL(k_ghost_hmax_one<D>, dim3(std::min(nblocks(n), 1024)), dim3(kBlock), 0, st,
-                         s.pos.as<double>(), s.hmaxOf.as<double>(), n, d, ext, hbits, nullptr);
-    hipLaunchKernelGGL(k_ghost_flag<D>, dim3(nblocks(n)), dim3(kBlock), 0, st, s.pos.as<double>(), segp, n, d, ext,
-                       hbits, s.keep.as<int32_t>(), nullptr, nullptr);
-    exclusiveScanI32(s.keep.as<int32_t>(), s.keepScan.as<int32_t>(), n, s);
-    int32_t* hc = static_cast<int32_t*>(hostStaging(s, 0, sizeof(int32_t)));
-    SG_CHECK_HIP(hipMemcpyAsync(hc, s.keepScan.as<int32_t>() + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    SG_CHECK_HIP(hipStreamSynchronize(st));
-    const int32_t count = *hc;
-    SG_REQUIRE(n + int64_t(count) < (int64_t(1) << 31) - 1, SPHGPU_ERR_CAPACITY, "too many ghost nodes");
-    if (count == 0) continue;
-    ensureRows(s, n + count);
-    s.hmaxOf.grow(sizeof(double) * size_t(n + count + (n + count) / 4), sizeof(double) * size_t(n), st);
-    const int64_t ng = n + count - s.nInt;
-    s.ghostControl.grow(sizeof(int32_t) * size_t(ng + ng / 2), sizeof(int32_t) * size_t(n - s.nInt), st);
-    s.ghostSub.grow(sizeof(int32_t) * size_t(ng + ng / 2), sizeof(int32_t) * size_t(n - s.nInt), st);
-    hipLaunchKernelGGL((k_ghost_make<D, false>), dim3(nblocks(n)), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(),
-                       groupCount(s) > 0 ? s.seg.as<double>() : nullptr, n, s.nInt, s.keep.as<int32_t>(), s.keepScan.as<int32_t>(), d, int(b),
-                       s.ghostControl.as<int32_t>(), s.ghostSub.as<int32_t>(), s.hmaxOf.as<double>(), nullptr,
-                       int64_t(0), nullptr);
-    SG_CHECK_HIP(hipGetLastError());
-    s.nTot = n + count;
-  }
-  s.subStart[s.subs.size()] = s.nTot - s.nInt;
-  s.ghostsGenerated = s.nTot - s.nInt;
-  applyFieldsD<D>(s, false, -1);
+// Ghosts expected of a first generation: four layers of nodes at every plane.
+int64_t ghostGuess(const Sim& s) {
+  if (s.ghostsGenerated > 0) return s.ghostsGenerated + s.ghostsGenerated / 4 + 1024;
+  const double groups = double(std::max(1, groupCount(s))), per = double(s.nInt) / groups;
+  const double face = std::pow(std::max(per, 1.0), double(s.dim - 1) / s.dim);
+  return int64_t(6.0 * face * groups * double(s.subs.size())) + 4096;
 }
 
 }  // namespace
 
-// Integrator::cullGhostNodes, first half: keep flags (ghosts some internal row
-// uses, and the controls they chain through), their scan, and the new total
-// and first ghost of every sub-boundary copied to pinned `hostOut` (nsub + 1
-// values, read after the caller's next wait).  The neighbour build issues it
-// before its row readback so that one wait serves both.
-void cullLaunch(Sim& s, int32_t* hostOut) {
-  hipStream_t st = s.stream;
-  const int64_t n = s.nTot, nInt = s.nInt;
-  const size_t nsub = s.subStart.size();
-  SG_REQUIRE(n > nInt && nsub < 16, SPHGPU_ERR_STATE, "cullLaunch needs ghosts of at most 15 sub-boundaries");
-  s.keep.ensure(sizeof(int32_t) * size_t(n + 1));
-  s.keepScan.ensure(sizeof(int32_t) * size_t(n + 1));
-  int32_t* keep = s.keep.as<int32_t>();
-  hipLaunchKernelGGL(k_keep_gather, dim3(nblocks(n)), dim3(kBlock), 0, st, keep, s.iperm.as<int32_t>(),
-                     s.slotKeep.as<int32_t>(), nInt, n);
-  hipLaunchKernelGGL(k_keep_controls, dim3(nblocks(n - nInt)), dim3(kBlock), 0, st, keep, nInt, n,
-                     s.ghostControl.as<int32_t>());
-  exclusiveScanI32(keep, s.keepScan.as<int32_t>(), n, s);
-  int64_t at[16];
-  for (size_t b = 0; b < nsub; ++b) at[b] = nInt + s.subStart[b];
-  at[nsub] = n;
-  pickInts(s, s.keepScan.as<int32_t>(), at, int(nsub + 1), hostOut);
+void finishGeneration(Sim& s, const int64_t* gen) {
+  const size_t nSubs = s.subs.size();
+  if (gen[0]) throw GhostCapacity{};
+  s.nTot = gen[1 + nSubs];
+  s.subStart.resize(nSubs + 1);
+  for (size_t b = 0; b <= nSubs; ++b) s.subStart[b] = gen[1 + b] - s.nInt;
+  s.ghostsGenerated = s.nTot - s.nInt;
+}
+
+// Integrator::cullGhostNodes, first half: which ghosts stay and their new
+// places; the new first ghost of every plane and the ghost count (nsub + 1
+// values) and the search flags copied to pinned memory, read after the
+// caller's next wait.  The neighbour build issues it before its row readback so
+// that one wait serves both.
+void cullLaunch(Sim& s, int32_t* flagsOut, int32_t* starts) {
+  const int64_t ng = s.nTot - s.nInt;
+  s.keep.ensure(sizeof(int32_t) * size_t(ng));
+  s.keepScan.ensure(sizeof(int32_t) * size_t(ng));
+  scanItems(KeepScan{s.slotKeep.as<int32_t>(), s.iperm.as<int32_t>(), s.ghostIsControl.as<int32_t>(),
+                     s.keep.as<int32_t>(), s.keepScan.as<int32_t>(), s.nInt, ng, s.genDev.as<int64_t>(),
+                     int(s.subs.size()), s.flags.as<int32_t>(), flagsOut, starts},
+            ng, s.scanTmp, s.stream);
 }
 
 namespace {
@@ -756,37 +680,11 @@ void cull(Sim& s) {
   hipStream_t st = s.stream;
   const int64_t n = s.nTot, nInt = s.nInt;
   if (n == nInt) return;
-  const size_t nsub = s.subStart.size();
-  std::vector<int32_t> starts(nsub + 1);
-  if (s.cullStartsReady) {
-    // launched and read with the neighbour build's row readback
-    SG_REQUIRE(s.cullStarts.size() == nsub + 1, SPHGPU_ERR_STATE, "stale cull starts");
-    starts = s.cullStarts;
-    s.cullStartsReady = false;
-  } else if (nsub < 16) {
-    int32_t* h = static_cast<int32_t*>(hostStaging(s, 0, sizeof(int32_t) * 16));
-    cullLaunch(s, h);
-    SG_CHECK_HIP(hipStreamSynchronize(st));
-    std::copy(h, h + nsub + 1, starts.begin());
-  } else {
-    s.keep.ensure(sizeof(int32_t) * size_t(n + 1));
-    s.keepScan.ensure(sizeof(int32_t) * size_t(n + 1));
-    int32_t* keep = s.keep.as<int32_t>();
-    hipLaunchKernelGGL(k_keep_gather, dim3(nblocks(n)), dim3(kBlock), 0, st, keep, s.iperm.as<int32_t>(),
-                       s.slotKeep.as<int32_t>(), nInt, n);
-    hipLaunchKernelGGL(k_keep_controls, dim3(nblocks(n - nInt)), dim3(kBlock), 0, st, keep, nInt, n,
-                       s.ghostControl.as<int32_t>());
-    exclusiveScanI32(keep, s.keepScan.as<int32_t>(), n, s);
-    int32_t* h = static_cast<int32_t*>(hostStaging(s, 0, sizeof(int32_t) * (nsub + 1)));
-    for (size_t b = 0; b < nsub; ++b)
-      SG_CHECK_HIP(hipMemcpyAsync(h + b, s.keepScan.as<int32_t>() + nInt + s.subStart[b], sizeof(int32_t),
-                                  hipMemcpyDeviceToHost, st));
-    SG_CHECK_HIP(hipMemcpyAsync(h + nsub, s.keepScan.as<int32_t>() + n, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    SG_CHECK_HIP(hipStreamSynchronize(st));
-    std::copy(h, h + nsub + 1, starts.begin());
-  }
+  SG_REQUIRE(s.cullStartsReady && s.cullStarts.size() == s.subStart.size(), SPHGPU_ERR_STATE, "stale cull starts");
+  s.cullStartsReady = false;
+  const std::vector<int32_t>& starts = s.cullStarts;   // launched and read with the neighbour build's rows
   int32_t* keep = s.keep.as<int32_t>();
-  const int64_t nNew = starts.back();
+  const int64_t nNew = nInt + starts.back();
   if (nNew == n) return;
   const int32_t* scan = s.keepScan.as<int32_t>();
 
@@ -807,7 +705,7 @@ void cull(Sim& s) {
   s.ghostControl.swap(s.ghostControlSpare);
   s.ghostSub.swap(s.ghostSubSpare);
   s.iperm.swap(s.ipermSpare);
-  for (size_t b = 0; b < s.subStart.size(); ++b) s.subStart[b] = int64_t(starts[b]) - nInt;
+  for (size_t b = 0; b < s.subStart.size(); ++b) s.subStart[b] = starts[b];
   s.nTot = nNew;
   // the kept ghost rows at their new places, filled again from the internal
   // nodes (the same maps of the same values)
@@ -882,21 +780,30 @@ void setGhostNodes(Sim& s, double ext, bool doCull) {
              "sphgpu_set_ghost_nodes needs n_total = n_internal (ghosts are made on the device)");
   hipStream_t st = s.stream;
   SG_CHECK_HIP(hipEventRecord(s.ev[8], st));
-  s.nTot = s.nInt;                       // drop the previous ghosts
   s.neighborsValid = false;
   s.recValid = false;
   s.derivsValid = false;
-  if (s.dim == 1) generateD<1>(s, ext);
-  else if (s.dim == 2) generateD<2>(s, ext);
-  else generateD<3>(s, ext);
-  s.deviceGhosts = true;
-  SG_CHECK_HIP(hipEventRecord(s.ev[9], st));
-  s.markGhostUse = doCull;
-  try {
-    buildNeighbors(s, ext);
-  } catch (...) {
-    s.markGhostUse = false;
-    throw;
+  for (int64_t est = ghostGuess(s);; est *= 4) {
+    s.nTot = s.nInt;                     // drop the previous ghosts
+    s.subStart.assign(s.subs.size() + 1, 0);
+    if (!s.subs.empty()) {
+      if (s.dim == 1) generateD<1>(s, ext, est);
+      else if (s.dim == 2) generateD<2>(s, ext, est);
+      else generateD<3>(s, ext, est);
+    }
+    s.deviceGhosts = true;
+    SG_CHECK_HIP(hipEventRecord(s.ev[9], st));
+    s.markGhostUse = doCull;
+    try {
+      buildNeighbors(s, ext);
+      break;
+    } catch (const GhostCapacity&) {
+      s.markGhostUse = false;
+    } catch (...) {
+      s.markGhostUse = false;
+      s.genPending = false;
+      throw;
+    }
   }
   s.markGhostUse = false;
   SG_CHECK_HIP(hipEventRecord(s.ev[10], st));

@@ -572,12 +572,12 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
   keyBytes(k, s.dtThreshold);
   k.push_back(reinterpret_cast<uint64_t>(s.pinnedOut));
   for (const DBuf* b : {&s.pos, &s.vel, &s.mass, &s.rho, &s.eps, &s.P, &s.cs, &s.H, &s.omega, &s.fCl, &s.fCq,
-                        &s.fshear, &s.cellOf, &s.cellCount, &s.cellStart, &s.cellFill, &s.perm, &s.iperm, &s.xs,
-                        &s.Hs, &s.rowCount, &s.nbr, &s.scanTmp, &s.reduceTmp, &s.flags, &s.rec, &s.recM, &s.recD,
+                        &s.fshear, &s.cellOf, &s.cellCount, &s.cellStart, &s.cellRank, &s.cellMembers, &s.perm, &s.iperm, &s.xs,
+                        &s.rowCount, &s.nbr, &s.scanTmp, &s.reduceTmp, &s.flags, &s.rec, &s.recM, &s.recD,
                         &s.recS, &s.recSM, &s.pairDv, &s.compDe, &s.compAcc, &s.compDe0, &s.compRec, &s.out,
                         &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
-                        &s.work, &s.workFlag, &s.workScan, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
-                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.pick, &s.listGamma, &s.subDev, &s.pairCounts})
+                        &s.work, &s.ghostIsControl, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
+                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts})
     keyBuf(k, *b);
   for (const DBuf& b : s.state0) keyBuf(k, b);
   return k;

@@ -71,6 +71,39 @@ struct DBuf {
   template <class T> T* as() const { return static_cast<T*>(p); }
 };
 
+struct ZeroSet {
+  int32_t* p[4];
+  int64_t n[4];
+  int m;
+  void add(int32_t* ptr, int64_t count) {
+    if (m < 4 && count > 0) { p[m] = ptr; n[m] = count; ++m; }
+  }
+};
+// Up to four int32 buffers zeroed by one kernel (a graph-safe memset that
+// also saves dispatches).
+void zeroMany(const ZeroSet& z, hipStream_t st);
+
+// A table that is zero at the start of each use without a launch to clear it:
+// two halves in turn, the kernel that fills one clears the other (`next`).
+struct ClearedTable {
+  DBuf buf;
+  size_t words = 0;
+  int half = 0;
+  unsigned long long* take(size_t n, hipStream_t st, unsigned long long*& next) {
+    if (n != words) {
+      buf.ensure(2 * n * sizeof(unsigned long long));
+      ZeroSet z{};
+      z.add(buf.as<int32_t>(), int64_t(4 * n));
+      zeroMany(z, st);
+      words = n;
+    }
+    half ^= 1;
+    unsigned long long* b = buf.as<unsigned long long>();
+    next = b + (half ? 0 : n);
+    return b + (half ? n : 0);
+  }
+};
+
 // Tabulated kernel as held on the host: per table point i1 the parabola
 // coefficients of W and dW/deta, plus the nperh <-> Wsum tables.
 struct TableHost {
@@ -152,10 +185,10 @@ struct Sim {
   int rowOrder = SPHGPU_ROW_ORDER_REFERENCE;
   bool neighborsValid = false;
   bool isotropic = false;   // every H is h*I (off-diagonals exactly zero)
-  DBuf cellOf, cellCount, cellStart, cellFill;
+  DBuf cellOf, cellCount, cellStart, cellRank, cellMembers;
   DBuf perm;                // sorted slot -> caller index
   DBuf iperm;               // caller index -> sorted slot
-  DBuf xs, Hs;              // positions / H in sorted order
+  DBuf xs;                  // x of the cells' members (staged search)
   DBuf rowCount, nbr;
   int ellCap = 0;           // capacity of the blocked-transposed ELL (multiple of 4)
   int64_t nEntries = 0;
@@ -193,7 +226,11 @@ struct Sim {
   std::vector<int64_t> subStart; // first ghost (offset from nInt) of each sub-boundary, +1 entry
   int64_t ghostsGenerated = 0;   // before culling
   DBuf keep, keepScan, slotKeep, ghostControlSpare, ghostSubSpare, ipermSpare, hmaxOf;
-  DBuf genDev;                   // device-held counts of a ghost generation
+  DBuf ghostIsControl;           // per ghost made: 1 when it controls another ghost
+  DBuf genDev;                   // device-held counts of a ghost generation (ghosts.hip)
+  int64_t genCap = 0;            // rows the generation's launches covered
+  bool genPending = false;       // its counts are still on the device only
+  ClearedTable hmaxBits;         // ghost selection: hmax bits per plane and group
   DBuf spare[13];                // one per caller-order state field (member removal gathers into it)
   bool markGhostUse = false;     // the next build marks the ghost slots rows hold (for culling)
   bool rowsMapOrder = false;     // several NodeLists, reference order: rows in ConnectivityMap order
@@ -203,7 +240,7 @@ struct Sim {
   // keeps the slot space: culled ghosts become dead slots (perm = -1) that no
   // row holds, so rows and their order are untouched.
   int64_t nSlots = 0;
-  DBuf work, workFlag, workScan; // internal slots in slot order (n_internal entries)
+  DBuf work;                     // internal slots in slot order (n_internal entries)
 
   // time integration (SynchronousRK2)
   double time = 0.0;
@@ -238,8 +275,7 @@ struct Sim {
   void* gridList = nullptr;      //   the grids (DGrid, neighbors.hip),
   int64_t* gridCellBase = nullptr;  // their first global cells (+1 entry),
   int32_t* gridFirst = nullptr;  //   the first grid of each member (+1 entry)
-  DBuf segBoundsBits;            // per member: 9 ordered-bit bounds of the neighbour build
-  DBuf segHmaxBits;              // per member: ghost-selection hmax bits
+  ClearedTable segBoundsBits;    // per member: ordered-bit bounds of the neighbour build
   DBuf segState;                 // SegState per member
   DBuf plainSeg;                 // SegState of a plain simulation's step (device-side dt)
   std::vector<SegState> segHost;
@@ -284,7 +320,6 @@ struct Sim {
   void* pinnedIn = nullptr;
   size_t pinnedInBytes = 0;
   hipEvent_t pinnedInDone = nullptr;   // recorded after the copies that read pinnedIn
-  DBuf pick;                     // device side of gathered readback values
   std::vector<int32_t> cullStarts;  // new ghost starts read with the last build's row readback
   bool cullStartsReady = false;
   bool pairsValid = false;                   // a pass ran on the current neighbour rows
@@ -350,32 +385,16 @@ int ensembleStep(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_
 // ensemble update / dt (integrate.hip)
 void ensembleRk2(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip);
 void eosRows(Sim& s, int64_t first, int64_t rows, double gamma, double Pmin, double Pmax, int floorType);
-// scans (neighbors.hip)
-// Up to four int32 buffers zeroed by one kernel (a graph-safe memset that
-// also saves dispatches).
+// neighbors.hip
 // Pinned staging of at least `bytes`: which = 0 readbacks, 1 uploads.
 void* hostStaging(Sim& s, int which, size_t bytes);
-// Gathers up to 16 int32 values of a device array into s.pick and copies them
-// to pinned host memory, one round trip: returns the host copy.
-const int32_t* readInts(Sim& s, const int32_t* src, const int64_t* at, int m);
-// The same gather with the copy to pinned `hostOut` left in flight.
-void pickInts(Sim& s, const int32_t* src, const int64_t* at, int m, int32_t* hostOut);
-// First half of the ghost cull (keep flags, scan, new ghost starts to pinned
-// hostOut); the cull takes the starts from s.cullStarts when the neighbour
-// build has read them.
-void cullLaunch(Sim& s, int32_t* hostOut);
-
-struct ZeroSet {
-  int32_t* p[4];
-  int64_t n[4];
-  int m;
-  void add(int32_t* ptr, int64_t count) {
-    if (m < 4 && count > 0) { p[m] = ptr; n[m] = count; ++m; }
-  }
-};
-void zeroMany(const ZeroSet& z, hipStream_t st);
-void exclusiveScanI32toI64(const int32_t* in, int64_t* out, int64_t n, Sim& s);
-void exclusiveScanI32(const int32_t* in, int32_t* out, int64_t n, Sim& s);
+// First half of the ghost cull: keep flags and scan, the planes' new first
+// ghosts and the search flags to pinned memory.
+void cullLaunch(Sim& s, int32_t* flagsOut, int32_t* starts);
+// Counts of a ghost generation, read back with the neighbour build's bounds;
+// throws GhostCapacity when its capacity was short.
+struct GhostCapacity {};
+void finishGeneration(Sim& s, const int64_t* gen);
 
 // tune.cpp: launch-shape autotuner.  A workload class of one kernel family;
 // tunedVariant returns the variant to launch, timing every variant once (on

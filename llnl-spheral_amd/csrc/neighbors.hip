@@ -11,7 +11,7 @@
 //  1. bounds: min/max position, the smallest Gershgorin lower bound of
 //     lambda_min(H) over all nodes, and whether every H is h I.  |H r| <= ext
 //     implies |r| <= R = ext/min(lambda) (plus a 1e-6 relative margin).
-//  2. counting sort of nodes by cell.  Cells are numbered brick by brick
+//  2. counting sort of nodes by cell (rank by comparison inside a cell).  Cells are numbered brick by brick
 //     (4^nu cells per brick, Z-order inside) so a brick's nodes are contiguous;
 //     each cell is then ordered by node index (the order depends only on
 //     positions and indices).  Records of all nodes are packed in this order.
@@ -37,6 +37,8 @@
 #include "dgeom.hh"
 #include "records.hh"
 #include "ell.hh"
+#include "pack.hh"
+#include "scan.hh"
 #include <cstring>
 
 namespace sphgpu {
@@ -92,8 +94,11 @@ template <int D> __device__ double maxDiag(const double* h) {
   return m;
 }
 
+// n rows, or with nDev the rows the ghost generation has left on the device.
 template <int D>
-__global__ void k_bounds(const double* __restrict__ pos, const double* __restrict__ H, int64_t n, double* partials) {
+__global__ void k_bounds(const double* __restrict__ pos, const double* __restrict__ H, int64_t n,
+                         const int64_t* __restrict__ nDev, double* partials) {
+  if (nDev) n = *nDev;
   __shared__ double sh[kNB][kBlock];
   double r[kNB] = SG_BOUNDS_IDENT;
   for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
@@ -119,7 +124,10 @@ __global__ void k_bounds(const double* __restrict__ pos, const double* __restric
   if (threadIdx.x < kNB) partials[blockIdx.x * kNB + threadIdx.x] = sh[threadIdx.x][0];
 }
 
-__global__ void k_bounds_final(const double* partials, int nb, double* out) {
+// The bounds, and the ghost generation's counts, straight to pinned memory.
+__global__ void k_bounds_final(const double* partials, int nb, double* __restrict__ out, const int64_t* __restrict__ gen,
+                               int nGen, int64_t* __restrict__ genOut) {
+  for (int q = threadIdx.x; q < nGen; q += blockDim.x) genOut[q] = gen[q];
   __shared__ double sh[kNB][kBlock];
   double r[kNB] = SG_BOUNDS_IDENT;
   for (int b = threadIdx.x; b < nb; b += blockDim.x)
@@ -177,30 +185,35 @@ inline double fromOrderedBits(unsigned long long o) {
   return x;
 }
 
-__global__ void k_seg_bounds_init(unsigned long long* __restrict__ bits, int nSeg) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nSeg * kNB) bits[i] = isMaxSlot(i % kNB) ? 0ull : ~0ull;
-}
-
-// The bounds of k_bounds per member.  A wavefront walks kSegGroups consecutive
-// groups of 64 rows (members are contiguous runs of rows) and keeps a running
-// reduction in registers while its groups stay in one member, with one atomic
-// per value when the member changes or the walk ends; a group that spans
-// members makes its atomics per lane.  Min and max are order-free, so the
-// result does not depend on the grouping.
+// The bounds of k_bounds per member, as ordered bits: a max slot keeps its
+// bits, a min slot their complement, so that every slot is an atomic maximum
+// that starts at zero.  A wavefront walks `groups` consecutive groups of 64 rows
+// (members are contiguous runs of internal rows) and keeps a running reduction
+// in registers while its groups stay in one member; a group that spans members
+// (ghost rows, whose planes mix them) goes per lane.  Either way a slot that
+// already holds as much is left alone: 10 contended atomics a lane were 105 us
+// of a 30 k row batch (a plain read may be stale, then the atomic decides).
+// Max is order-free, so the result does not depend on the grouping.  `clear`
+// is the next build's table.
 constexpr int kSegGroups = 16;
 template <int D>
 __global__ void k_seg_bounds(const double* __restrict__ pos, const double* __restrict__ H,
-                             const double* __restrict__ seg, int64_t n, unsigned long long* __restrict__ bits) {
+                             const double* __restrict__ seg, int64_t n, const int64_t* __restrict__ nDev, int groups,
+                             unsigned long long* __restrict__ bits, unsigned long long* __restrict__ clear,
+                             int words) {
+  if (nDev) n = *nDev;
+  const int64_t tid = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  for (int64_t q = tid; q < words; q += int64_t(gridDim.x) * blockDim.x) clear[q] = 0ull;
   const int lane = threadIdx.x & 63;
-  const int64_t base = ((blockIdx.x * int64_t(blockDim.x) + threadIdx.x) >> 6) * int64_t(64 * kSegGroups);
+  const int64_t base = (tid >> 6) * int64_t(64 * groups);
   const double ident[kNB] = SG_BOUNDS_IDENT;
   double acc[kNB];
   for (int k = 0; k < kNB; ++k) acc[k] = ident[k];
   int mAcc = -1;                           // member of the running reduction (wave-uniform)
   auto atomicOne = [&](int m, int k, double v) {
-    if (isMaxSlot(k)) atomicMax(bits + int64_t(m) * kNB + k, orderedBits(v));
-    else atomicMin(bits + int64_t(m) * kNB + k, orderedBits(v));
+    unsigned long long* p = bits + int64_t(m) * kNB + k;
+    const unsigned long long o = isMaxSlot(k) ? orderedBits(v) : ~orderedBits(v);
+    if (o > *static_cast<volatile unsigned long long*>(p)) atomicMax(p, o);
   };
   auto flush = [&]() {                     // called by the whole wavefront
     for (int k = 0; k < kNB; ++k) {
@@ -213,7 +226,7 @@ __global__ void k_seg_bounds(const double* __restrict__ pos, const double* __res
       acc[k] = ident[k];
     }
   };
-  for (int it = 0; it < kSegGroups; ++it) {
+  for (int it = 0; it < groups; ++it) {
     const int64_t i = base + int64_t(it) * 64 + lane;
     double r[kNB];
     for (int k = 0; k < kNB; ++k) r[k] = ident[k];
@@ -246,6 +259,14 @@ __global__ void k_seg_bounds(const double* __restrict__ pos, const double* __res
   if (mAcc >= 0) flush();
 }
 
+// Member bounds and generation counts to pinned memory.
+__global__ void k_report(const unsigned long long* __restrict__ bits, int words, unsigned long long* __restrict__ out,
+                         const int64_t* __restrict__ gen, int nGen, int64_t* __restrict__ genOut) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < words) out[t] = bits[t];
+  if (t < nGen) genOut[t] = gen[t];
+}
+
 template <int D> __device__ __forceinline__ void cellCoords(const DGrid& g, const double* x, int* c) {
   c[0] = c[1] = c[2] = 0;
   for (int k = 0; k < D; ++k) {
@@ -274,7 +295,8 @@ template <int D> __device__ __forceinline__ int64_t cellId(const DGrid& g, int c
 
 template <int D>
 __global__ void k_cell_count(const double* __restrict__ pos, const double* __restrict__ H, int64_t n, DGrid g,
-                             SegGrids sg, int32_t* __restrict__ cellOf, int32_t* __restrict__ cellCount) {
+                             SegGrids sg, int32_t* __restrict__ cellOf, int32_t* __restrict__ cellCount,
+                             int32_t* __restrict__ cellRank) {
   const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (i >= n) return;
   int64_t base = 0;
@@ -293,85 +315,75 @@ __global__ void k_cell_count(const double* __restrict__ pos, const double* __res
   cellCoords<D>(g, pos + i * D, c);
   const int32_t id = int32_t(base + cellId<D>(g, c[0], c[1], c[2]));
   cellOf[i] = id;
-  atomicAdd(&cellCount[id], 1);
+  cellRank[i] = atomicAdd(&cellCount[id], 1);
 }
 
+// cellStart from cellCount (scan.hh)
+struct CellScan {
+  static constexpr bool kCompact = false;
+  const int32_t* count;
+  int32_t* start;
+  int64_t n;
+  __device__ int32_t value(int64_t i) const { return count[i]; }
+  __device__ void emit(int64_t i, int32_t prefix, int32_t) const { start[i] = prefix; }
+  __device__ void total(int32_t t) const { start[n] = t; }
+};
+
+// Each cell's members together, in the order the count met them; with `keys`
+// also their x (pos[i * stride]), which the ordering then reads contiguously.
 __global__ void k_cell_scatter(const int32_t* __restrict__ cellOf, const int32_t* __restrict__ cellStart,
-                               int32_t* __restrict__ cellFill, int32_t* __restrict__ perm, int64_t n) {
+                               const int32_t* __restrict__ cellRank, int32_t* __restrict__ members, int64_t n,
+                               const double* __restrict__ pos, int stride, double* __restrict__ keys) {
+  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (i >= n) return;
+  const int32_t q = cellStart[cellOf[i]] + cellRank[i];
+  members[q] = int32_t(i);
+  if (keys) keys[q] = pos[i * stride];
+}
+
+// The slot of every row: its rank in its cell by node index, or, XKEY, by x and
+// then node index, so that the members of a row of cells are in x order; then
+// the maps both ways and the row's records.  One lane per row compares it with
+// the members of its cell: independent reads of lines the neighbouring lanes
+// share, where one lane per cell sorting by insertion ran a dependent chain
+// over global memory (40 us in a batch of blasts, whose cells hold ~9 nodes,
+// against 9 us for this kernel with the pack in it).  Rows are walked in
+// caller order, so the fields are read contiguously and each record is written
+// whole.
+template <int D, bool ISO, int SEC, bool XKEY>
+__global__ void __launch_bounds__(kBlock) k_cell_order(const int32_t* __restrict__ cellOf,
+                                                       const int32_t* __restrict__ cellStart,
+                                                       const int32_t* __restrict__ members,
+                                                       const double* __restrict__ keys, int64_t n,
+                                                       int32_t* __restrict__ perm,
+                                                       int32_t* __restrict__ iperm, PackIn in, PackOut o) {
   const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (i >= n) return;
   const int32_t c = cellOf[i];
-  const int32_t slot = cellStart[c] + atomicAdd(&cellFill[c], 1);
-  perm[slot] = int32_t(i);
-}
-
-// Order each cell's members by node index, or, with `xkey` (x of node i at
-// xkey[i * stride]), by x and then node index, so that the members of a row
-// of cells are in x order (insertion sort; cells hold a few to tens of nodes).
-__global__ void k_cell_sort(const int32_t* __restrict__ cellStart, int32_t* __restrict__ perm, int64_t ncells,
-                            const double* __restrict__ xkey, int stride) {
-  const int64_t c = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (c >= ncells) return;
   const int32_t b = cellStart[c], e = cellStart[c + 1];
-  if (!xkey) {
-    for (int32_t a = b + 1; a < e; ++a) {
-      const int32_t v = perm[a];
-      int32_t q = a - 1;
-      while (q >= b && perm[q] > v) { perm[q + 1] = perm[q]; --q; }
-      perm[q + 1] = v;
+  int32_t rank = 0;
+  const double x = XKEY ? in.pos[i * D] : 0.0;
+  // four members at a time: their reads are in flight together
+  for (int32_t q0 = b; q0 < e; q0 += 4) {
+    int32_t u[4];
+    double xu[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int32_t at = q0 + q < e ? q0 + q : e - 1;
+      u[q] = members[at];
+      if constexpr (XKEY) xu[q] = keys[at];
     }
-    return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      bool before = u[q] < int32_t(i);
+      if constexpr (XKEY) before = xu[q] < x || (xu[q] == x && before);
+      rank += (before && q0 + q < e) ? 1 : 0;
+    }
   }
-  constexpr int kSmall = 8;
-  if (e - b <= kSmall) {
-    // all keys loaded at once (independent loads), then an odd-even
-    // transposition network in registers; padding sorts last
-    int32_t id[kSmall];
-    double xv[kSmall];
-#pragma unroll
-    for (int q = 0; q < kSmall; ++q) {
-      id[q] = INT32_MAX;
-      xv[q] = HUGE_VAL;
-      if (b + q < e) {
-        id[q] = perm[b + q];
-        xv[q] = xkey[int64_t(id[q]) * stride];
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < kSmall; ++r) {
-#pragma unroll
-      for (int q = r & 1; q + 1 < kSmall; q += 2) {
-        const bool swap = xv[q] > xv[q + 1] || (xv[q] == xv[q + 1] && id[q] > id[q + 1]);
-        const double x0 = xv[q], x1 = xv[q + 1];
-        const int32_t i0 = id[q], i1 = id[q + 1];
-        xv[q] = swap ? x1 : x0;
-        xv[q + 1] = swap ? x0 : x1;
-        id[q] = swap ? i1 : i0;
-        id[q + 1] = swap ? i0 : i1;
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kSmall; ++q)
-      if (b + q < e) perm[b + q] = id[q];
-    return;
-  }
-  for (int32_t a = b + 1; a < e; ++a) {
-    const int32_t v = perm[a];
-    const double xv = xkey[int64_t(v) * stride];
-    int32_t q = a - 1;
-    for (; q >= b; --q) {
-      const int32_t u = perm[q];
-      const double xu = xkey[int64_t(u) * stride];
-      if (xu < xv || (xu == xv && u < v)) break;
-      perm[q + 1] = u;
-    }
-    perm[q + 1] = v;
-  }
-}
-
-__global__ void k_iperm(const int32_t* __restrict__ perm, int32_t* __restrict__ iperm, int64_t n) {
-  const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (k < n) iperm[perm[k]] = int32_t(k);
+  const int32_t k = b + rank;
+  perm[k] = int32_t(i);
+  iperm[i] = k;
+  packRow<D, ISO, SEC>(k, i, loadPackRow<D, ISO>(i, in), o);
 }
 
 // Row writer: keeps four entries in registers and stores them as one int4.
@@ -419,6 +431,42 @@ struct RowWriter {
     const int4 o = r == 1 ? make_int4(buf.w, 0, 0, 0)
                           : (r == 2 ? make_int4(buf.z, buf.w, 0, 0) : make_int4(buf.y, buf.z, buf.w, 0));
     *at = o;
+  }
+};
+
+// Entries and the longest row of a search: summed in the workgroup, one pair
+// of atomics each (flags: [0] longest row, [4..5] entries).
+struct RowStats {
+  uint32_t sum = 0;
+  int32_t most = 0;
+  __device__ __forceinline__ void add(int32_t c) {
+    sum += uint32_t(c);
+    most = c > most ? c : most;
+  }
+  // called by every thread of the workgroup
+  __device__ __forceinline__ void store(int32_t* __restrict__ flags) {
+    __shared__ uint32_t ws[kBlock / 64];
+    __shared__ int32_t wm[kBlock / 64];
+    for (int sh = 32; sh > 0; sh >>= 1) {
+      sum += __shfl_xor(sum, sh);
+      const int32_t m = __shfl_xor(most, sh);
+      most = m > most ? m : most;
+    }
+    if ((threadIdx.x & 63) == 0) {
+      ws[threadIdx.x >> 6] = sum;
+      wm[threadIdx.x >> 6] = most;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < kBlock / 64; ++w) {
+        sum += ws[w];
+        most = wm[w] > most ? wm[w] : most;
+      }
+      if (sum) {
+        atomicAdd(reinterpret_cast<unsigned long long*>(flags + 4), (unsigned long long)sum);
+        if (most > *static_cast<volatile int32_t*>(flags)) atomicMax(flags, most);
+      }
+    }
   }
 };
 
@@ -472,6 +520,7 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
   const int bx = b % g.nb[0], by = (b / g.nb[0]) % g.nb[1], bz = b / (g.nb[0] * g.nb[1]);
   const int64_t h0 = cellStart[int64_t(b) * 64], h1 = cellStart[int64_t(b) * 64 + 64];
   if (h0 == h1) return;                           // uniform over the block
+  RowStats stats;
   const int cx0 = bx * 4 - 2, cy0 = by * 4 - 2, cz0 = bz * 4 - 2;
   const double ox = g.lo[0] + (bx * 4) * g.cell, oy = g.lo[1] + (by * 4) * g.cell, oz = g.lo[2] + (bz * 4) * g.cell;
   // staged cell table (x fastest)
@@ -709,21 +758,22 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
     }
     row.finish();
     rowCount[k] = row.cnt;
+    stats.add(row.cnt);
   }
+  stats.store(flags);
 }
 
 // ---------------------------------------------------------------------------
 // Global search: any dimension, any H (cell edge = R, 3^nu stencil).
 // ---------------------------------------------------------------------------
 template <int D, bool ISO>
-__global__ void k_search_global(const double* __restrict__ rec, const int32_t* __restrict__ cellStart, SearchArgs a,
-                                SegGrids sg, int32_t* __restrict__ rowCount, int4* __restrict__ nbr) {
+__device__ __forceinline__ int32_t searchRow(int64_t k, const double* __restrict__ rec,
+                                             const int32_t* __restrict__ cellStart, const SearchArgs& a,
+                                             const SegGrids& sg, int4* __restrict__ nbr) {
   using R = RL<ISO>;
-  const int64_t k = xcdBlock((a.n + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
-  if (k >= a.n) return;
   const double* ri_ = rec + k * R::STRIDE;
   const int64_t oi = int64_t(ri_[R::ORIG]);
-  if (oi >= a.nInt) { rowCount[k] = 0; return; }
+  if (oi >= a.nInt) return 0;
   int ga = 0, gb = 1;
   if (sg.g) {
     const int m = sg.seg ? int(sg.seg[oi]) : 0;
@@ -796,47 +846,37 @@ __global__ void k_search_global(const double* __restrict__ rec, const int32_t* _
   }
   }
   row.finish();
-  rowCount[k] = row.cnt;
+  return row.cnt;
+}
+template <int D, bool ISO>
+__global__ void __launch_bounds__(kBlock) k_search_global(const double* __restrict__ rec,
+                                                          const int32_t* __restrict__ cellStart, SearchArgs a,
+                                                          SegGrids sg, int32_t* __restrict__ rowCount,
+                                                          int4* __restrict__ nbr, int32_t* __restrict__ flags) {
+  const int64_t k = xcdBlock((a.n + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+  RowStats stats;
+  if (k < a.n) {
+    const int32_t c = searchRow<D, ISO>(k, rec, cellStart, a, sg, nbr);
+    rowCount[k] = c;
+    stats.add(c);
+  }
+  stats.store(flags);
 }
 
-// Internal slots in slot order: the work list of the density and pair passes.
-__global__ void k_work_flag(const int32_t* __restrict__ perm, int64_t n, int64_t nInt, int32_t* __restrict__ flag) {
-  const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (k < n) flag[k] = (perm[k] >= 0 && perm[k] < nInt) ? 1 : 0;
-}
-__global__ void k_work_scatter(const int32_t* __restrict__ flag, const int32_t* __restrict__ scan, int64_t n,
-                               int32_t* __restrict__ work) {
-  const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (k < n && flag[k]) work[scan[k]] = int32_t(k);
-}
-
-// Total entries and longest row.
-__global__ void k_row_stats(const int32_t* __restrict__ rowCount, int64_t n, unsigned long long* __restrict__ total,
-                            int32_t* __restrict__ maxRow) {
-  __shared__ unsigned long long st[kBlock];
-  __shared__ int32_t sm[kBlock];
-  unsigned long long s = 0;
-  int32_t m = 0;
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
-    const int32_t c = rowCount[i];
-    s += unsigned(c);
-    m = c > m ? c : m;
+// Internal slots in slot order: the work list of the density and pair passes
+// (scan.hh).
+struct WorkScan {
+  static constexpr bool kCompact = true;
+  const int32_t* perm;
+  int32_t* work;
+  int64_t nInt;
+  __device__ int32_t value(int64_t k) const {
+    const int32_t i = perm[k];
+    return i >= 0 && i < nInt ? 1 : 0;
   }
-  st[threadIdx.x] = s;
-  sm[threadIdx.x] = m;
-  __syncthreads();
-  for (int w = kBlock / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) {
-      st[threadIdx.x] += st[threadIdx.x + w];
-      sm[threadIdx.x] = sm[threadIdx.x] > sm[threadIdx.x + w] ? sm[threadIdx.x] : sm[threadIdx.x + w];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    atomicAdd(total, st[0]);
-    atomicMax(maxRow, sm[0]);
-  }
-}
+  __device__ void emit(int64_t k, int32_t prefix, int32_t) const { work[prefix] = int32_t(k); }
+  __device__ void total(int32_t) const {}
+};
 
 // ---------------------------------------------------------------------------
 // Reference row order: sort each row by caller index.  One wavefront per row,
@@ -979,142 +1019,11 @@ __global__ void __launch_bounds__(kBlock) k_row_sort(const int32_t* __restrict__
   }
 }
 
-// ---- gathering a few int32 values for one readback -------------------------
-struct Pick32 {
-  int64_t at[16];
-  int m;
-};
-__global__ void k_pick_i32(const int32_t* __restrict__ src, Pick32 p, int32_t* __restrict__ out) {
-  const int q = threadIdx.x;
-  if (q < p.m) out[q] = src[p.at[q]];
-}
-
 // ---- zeroing several int32 buffers in one dispatch ------------------------
 __global__ void k_zero_many(ZeroSet z) {
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   for (int q = 0; q < z.m; ++q)
     for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < z.n[q]; i += stride) z.p[q][i] = 0;
-}
-
-// ---- exclusive scans -------------------------------------------------------
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kBlock * kScanItems;
-
-template <class TI, class TO>
-__global__ void k_scan_tiles(const TI* __restrict__ in, TO* __restrict__ out, TO* __restrict__ tileSums, int64_t n) {
-  __shared__ TO sh[kBlock];
-  const int64_t base = blockIdx.x * int64_t(kScanTile) + threadIdx.x * kScanItems;
-  TO v[kScanItems];
-  TO local = 0;
-  for (int q = 0; q < kScanItems; ++q) {
-    const int64_t i = base + q;
-    v[q] = (i < n) ? TO(in[i]) : TO(0);
-    local += v[q];
-  }
-  sh[threadIdx.x] = local;
-  __syncthreads();
-  for (int s = 1; s < kBlock; s <<= 1) {
-    TO t = (threadIdx.x >= s) ? sh[threadIdx.x - s] : TO(0);
-    __syncthreads();
-    sh[threadIdx.x] += t;
-    __syncthreads();
-  }
-  TO run = sh[threadIdx.x] - local;
-  for (int q = 0; q < kScanItems; ++q) {
-    const int64_t i = base + q;
-    if (i < n) out[i] = run;
-    run += v[q];
-  }
-  if (threadIdx.x == kBlock - 1) tileSums[blockIdx.x] = sh[kBlock - 1];
-}
-
-template <class TO>
-__global__ void k_scan_sums(TO* __restrict__ sums, int64_t m, TO* __restrict__ total) {
-  __shared__ TO sh[kBlock];
-  TO carry = 0;
-  for (int64_t base = 0; base < m; base += kBlock) {
-    const int64_t i = base + threadIdx.x;
-    const TO v = (i < m) ? sums[i] : TO(0);
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = 1; s < kBlock; s <<= 1) {
-      TO t = (threadIdx.x >= s) ? sh[threadIdx.x - s] : TO(0);
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    if (i < m) sums[i] = carry + sh[threadIdx.x] - v;
-    const TO blockTotal = sh[kBlock - 1];
-    __syncthreads();
-    carry += blockTotal;
-  }
-  if (threadIdx.x == 0) *total = carry;
-}
-
-template <class TO>
-__global__ void k_scan_add(TO* __restrict__ out, const TO* __restrict__ sums, int64_t n, const TO* __restrict__ total) {
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (i < n) out[i] += sums[i / kScanTile];
-  if (i == n) out[n] = *total;
-}
-
-// Small scans in one workgroup: tiles of kScanOneTile items in sequence with a
-// running carry (one dispatch instead of three; small simulations run several
-// scans per step and are bound by dispatch latency).
-constexpr int kScanOneBlock = 1024;
-constexpr int kScanOneTile = kScanOneBlock * kScanItems;
-constexpr int64_t kScanOneMax = 4 * int64_t(kScanOneTile);
-
-template <class TI, class TO>
-__global__ void __launch_bounds__(kScanOneBlock) k_scan_one(const TI* __restrict__ in, TO* __restrict__ out,
-                                                            int64_t n) {
-  __shared__ TO sh[kScanOneBlock];
-  TO carry = 0;
-  for (int64_t tile = 0; tile < n; tile += kScanOneTile) {
-    const int64_t base = tile + int64_t(threadIdx.x) * kScanItems;
-    TO v[kScanItems];
-    TO local = 0;
-    for (int q = 0; q < kScanItems; ++q) {
-      const int64_t i = base + q;
-      v[q] = (i < n) ? TO(in[i]) : TO(0);
-      local += v[q];
-    }
-    sh[threadIdx.x] = local;
-    __syncthreads();
-    for (int s = 1; s < kScanOneBlock; s <<= 1) {
-      const TO t = (threadIdx.x >= s) ? sh[threadIdx.x - s] : TO(0);
-      __syncthreads();
-      sh[threadIdx.x] += t;
-      __syncthreads();
-    }
-    TO run = carry + sh[threadIdx.x] - local;
-    for (int q = 0; q < kScanItems; ++q) {
-      const int64_t i = base + q;
-      if (i < n) out[i] = run;
-      run += v[q];
-    }
-    carry += sh[kScanOneBlock - 1];
-    __syncthreads();                               // sh is rewritten by the next tile
-  }
-  if (threadIdx.x == 0) out[n] = carry;
-}
-
-template <class TI, class TO>
-void exclusiveScan(const TI* in, TO* out, int64_t n, Sim& s) {
-  // out has n+1 entries; out[n] = total.
-  if (n <= kScanOneMax) {
-    hipLaunchKernelGGL((k_scan_one<TI, TO>), dim3(1), dim3(kScanOneBlock), 0, s.stream, in, out, n);
-    SG_CHECK_HIP(hipGetLastError());
-    return;
-  }
-  const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  s.scanTmp.ensure(sizeof(TO) * size_t(tiles + 2));
-  TO* sums = s.scanTmp.as<TO>();
-  TO* total = sums + tiles + 1;
-  if (n > 0) hipLaunchKernelGGL((k_scan_tiles<TI, TO>), dim3(tiles), dim3(kBlock), 0, s.stream, in, out, sums, n);
-  hipLaunchKernelGGL((k_scan_sums<TO>), dim3(1), dim3(kBlock), 0, s.stream, sums, tiles, total);
-  hipLaunchKernelGGL((k_scan_add<TO>), dim3(nblocks(n + 1)), dim3(kBlock), 0, s.stream, out, sums, n, total);
-  SG_CHECK_HIP(hipGetLastError());
 }
 
 // A grid of cell edge `cell` over the bounds hb: cells per axis, bricks, cell count.
@@ -1222,11 +1131,46 @@ int64_t uploadGrids(Sim& s, const std::vector<DGrid>& grids, const std::vector<i
   return base.back();
 }
 
+template <int D, bool XKEY>
+void cellOrder(Sim& s, int64_t n) {
+  // the records the next kernel reads, written with the FP64 record: the
+  // caller's hint, else the density sum's
+  const int sec = s.isotropic ? (s.buildRecHint >= 0 ? s.buildRecHint : densityRecordSec(s)) : 0;
+  const PackOut o = packOutputs(s, sec);
+  const PackIn in = packInputs(s);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nblocks(n)), dim3(kBlock), 0, s.stream, s.cellOf.as<int32_t>(),
+                       s.cellStart.as<int32_t>(), s.cellMembers.as<int32_t>(), s.xs.as<double>(), n,
+                       s.perm.as<int32_t>(), s.iperm.as<int32_t>(), in, o);
+  };
+  if (!s.isotropic) {
+    go(k_cell_order<D, false, 0, XKEY>);
+  } else {
+    switch (sec) {
+      case 0: go(k_cell_order<D, true, 0, XKEY>); break;
+      case 1: go(k_cell_order<D, true, 1, XKEY>); break;
+      case 2: go(k_cell_order<D, true, 2, XKEY>); break;
+      case 4: go(k_cell_order<D, true, 4, XKEY>); break;
+      case 8: go(k_cell_order<D, true, 8, XKEY>); break;
+      default: SG_REQUIRE(false, SPHGPU_ERR_STATE, "unsupported record kinds for the neighbour build");
+    }
+  }
+  SG_CHECK_HIP(hipGetLastError());
+  s.recValid = true;
+}
+
 template <int D>
 void buildNeighborsD(Sim& s, double ext) {
-  const int64_t n = s.nTot;
   hipStream_t st = s.stream;
   SG_CHECK_HIP(hipEventRecord(s.ev[0], st));
+  // rows: those the caller set, or a ghost generation's whose count is still
+  // on the device (read back with the bounds)
+  const bool pending = s.genPending;
+  s.genPending = false;
+  const int64_t rows = pending ? s.genCap : s.nTot;
+  const int nGen = pending ? int(s.subs.size()) + 2 : 0;
+  const int64_t* gen = pending ? s.genDev.as<int64_t>() : nullptr;
+  const int64_t* nDev = pending ? gen + nGen - 1 : nullptr;
 
   // 1. bounds
   Grid& G = s.grid;
@@ -1237,16 +1181,25 @@ void buildNeighborsD(Sim& s, double ext) {
   SegGrids sgr{nullptr, nullptr, nullptr, nullptr, ext};
   if (s.nSeg > 0) {
     const int ns = s.nSeg;
-    s.segBoundsBits.ensure(sizeof(unsigned long long) * size_t(ns) * kNB);
-    unsigned long long* bits = s.segBoundsBits.as<unsigned long long>();
-    hipLaunchKernelGGL(k_seg_bounds_init, dim3(nblocks(int64_t(ns) * kNB)), dim3(kBlock), 0, st, bits, ns);
-    hipLaunchKernelGGL((k_seg_bounds<D>), dim3(nblocks((n + kSegGroups - 1) / kSegGroups)), dim3(kBlock), 0, st,
-                       s.pos.as<double>(), s.H.as<double>(), s.seg.as<double>(), n, bits);
-    SG_CHECK_HIP(hipGetLastError());
     const size_t nbits = size_t(ns) * kNB;
-    unsigned long long* hbits = static_cast<unsigned long long*>(hostStaging(s, 0, nbits * sizeof(unsigned long long)));
-    SG_CHECK_HIP(hipMemcpyAsync(hbits, bits, nbits * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+    unsigned long long* next = nullptr;
+    unsigned long long* bits = s.segBoundsBits.take(nbits, st, next);
+    // one group a wavefront until every SIMD has one
+    const int groups = int(std::min<int64_t>(kSegGroups, std::max<int64_t>(1, rows / (64 * 1024))));
+    hipLaunchKernelGGL((k_seg_bounds<D>), dim3(nblocks((rows + groups - 1) / groups)), dim3(kBlock), 0, st,
+                       s.pos.as<double>(), s.H.as<double>(), s.seg.as<double>(), rows, nDev, groups, bits, next,
+                       int(nbits));
+    unsigned long long* hbits = static_cast<unsigned long long*>(
+        hostStaging(s, 0, (nbits + size_t(nGen)) * sizeof(unsigned long long)));
+    int64_t* hgen = reinterpret_cast<int64_t*>(hbits + nbits);
+    hipLaunchKernelGGL(k_report, dim3(nblocks(std::max<int64_t>(int64_t(nbits), nGen))), dim3(kBlock), 0, st, bits,
+                       int(nbits), hbits, gen, nGen, hgen);
+    SG_CHECK_HIP(hipGetLastError());
     SG_CHECK_HIP(hipStreamSynchronize(st));
+    if (pending) finishGeneration(s, hgen);
+    // back to min slots as such
+    for (size_t q = 0; q < nbits; ++q)
+      if (!isMaxSlot(int(q % kNB))) hbits[q] = ~hbits[q];
     std::vector<DGrid> grids;
     std::vector<int64_t> cells;
     std::vector<int32_t> first(size_t(ns) + 1, 0);
@@ -1281,16 +1234,17 @@ void buildNeighborsD(Sim& s, double ext) {
     G.ncells = uploadGrids(s, grids, cells, first);
     sgr = SegGrids{s.seg.as<double>(), static_cast<const DGrid*>(s.gridList), s.gridCellBase, s.gridFirst, ext};
   } else {
-    const int nbB = int(std::min<int64_t>(1024, nblocks(n)));
+    const int nbB = int(std::min<int64_t>(1024, nblocks(rows)));
     s.reduceTmp.ensure(sizeof(double) * (size_t(nbB) * kNB + 16));
     double* partials = s.reduceTmp.as<double>();
-    double* bounds = partials + size_t(nbB) * kNB;
-    hipLaunchKernelGGL((k_bounds<D>), dim3(nbB), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(), n, partials);
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, st, partials, nbB, bounds);
+    double* hbp = static_cast<double*>(hostStaging(s, 0, sizeof(hb) + sizeof(int64_t) * size_t(nGen)));
+    int64_t* hgen = reinterpret_cast<int64_t*>(hbp + kNB);
+    hipLaunchKernelGGL((k_bounds<D>), dim3(nbB), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(), rows, nDev,
+                       partials);
+    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, st, partials, nbB, hbp, gen, nGen, hgen);
     SG_CHECK_HIP(hipGetLastError());
-    double* hbp = static_cast<double*>(hostStaging(s, 0, sizeof(hb)));
-    SG_CHECK_HIP(hipMemcpyAsync(hbp, bounds, sizeof(hb), hipMemcpyDeviceToHost, st));
     SG_CHECK_HIP(hipStreamSynchronize(st));
+    if (pending) finishGeneration(s, hgen);
     std::memcpy(hb, hbp, sizeof(hb));
     requireUsableBounds(hb);
     s.isotropic = hb[7] > 0.5 && !s.hasMultipliers;
@@ -1311,40 +1265,42 @@ void buildNeighborsD(Sim& s, double ext) {
     }
   }
 
+  const int64_t n = s.nTot;
   // 2. counting sort by cell, then by node index (staged search: by x) inside a cell
   s.cellOf.ensure(sizeof(int32_t) * size_t(n));
   s.cellCount.ensure(sizeof(int32_t) * size_t(G.ncells + 1));
-  s.cellFill.ensure(sizeof(int32_t) * size_t(G.ncells + 1));
+  s.cellRank.ensure(sizeof(int32_t) * size_t(n));
+  s.cellMembers.ensure(sizeof(int32_t) * size_t(n));
+  if (stagedPath) s.xs.ensure(sizeof(double) * size_t(n));
   s.cellStart.ensure(sizeof(int32_t) * size_t(G.ncells + 2));
   s.perm.ensure(sizeof(int32_t) * size_t(n));
   s.iperm.ensure(sizeof(int32_t) * size_t(n));
   // zero the cell counters, the search flags and the ghost-use marks in one dispatch
   const bool markUse = s.markGhostUse && s.nTot > s.nInt;
   if (markUse) s.slotKeep.ensure(sizeof(int32_t) * size_t(n + 1));
-  s.flags.ensure(sizeof(int32_t) * 8 + sizeof(unsigned long long) * 2);
+  s.flags.ensure(sizeof(int32_t) * 8);
   {
     ZeroSet z{};
     z.add(s.cellCount.as<int32_t>(), G.ncells + 1);
-    z.add(s.cellFill.as<int32_t>(), G.ncells + 1);
-    z.add(s.flags.as<int32_t>(), int64_t(s.flags.bytes / sizeof(int32_t)));
+    z.add(s.flags.as<int32_t>(), 8);
     if (markUse) z.add(s.slotKeep.as<int32_t>(), n);
     zeroMany(z, s.stream);
   }
   hipLaunchKernelGGL((k_cell_count<D>), dim3(nblocks(n)), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(),
-                     n, dg, sgr,
-                     s.cellOf.as<int32_t>(), s.cellCount.as<int32_t>());
-  exclusiveScan<int32_t, int32_t>(s.cellCount.as<int32_t>(), s.cellStart.as<int32_t>(), G.ncells, s);
+                     n, dg, sgr, s.cellOf.as<int32_t>(), s.cellCount.as<int32_t>(), s.cellRank.as<int32_t>());
+  scanItems(CellScan{s.cellCount.as<int32_t>(), s.cellStart.as<int32_t>(), G.ncells}, G.ncells, s.scanTmp, st);
   hipLaunchKernelGGL(k_cell_scatter, dim3(nblocks(n)), dim3(kBlock), 0, st, s.cellOf.as<int32_t>(),
-                     s.cellStart.as<int32_t>(), s.cellFill.as<int32_t>(), s.perm.as<int32_t>(), n);
-  // the staged search cuts each row of cells to the chord of its sphere by x
-  hipLaunchKernelGGL(k_cell_sort, dim3(nblocks(G.ncells)), dim3(kBlock), 0, st, s.cellStart.as<int32_t>(),
-                     s.perm.as<int32_t>(), G.ncells, stagedPath ? s.pos.as<double>() : nullptr, D);
-  hipLaunchKernelGGL(k_iperm, dim3(nblocks(n)), dim3(kBlock), 0, st, s.perm.as<int32_t>(), s.iperm.as<int32_t>(), n);
+                     s.cellStart.as<int32_t>(), s.cellRank.as<int32_t>(), s.cellMembers.as<int32_t>(), n,
+                     s.pos.as<double>(), D, stagedPath ? s.xs.as<double>() : nullptr);
   SG_CHECK_HIP(hipGetLastError());
   s.nSlots = n;
-  // the records the next kernel reads, written with the FP64 record: the
-  // caller's hint, else the density sum's
-  packRecords(s, s.isotropic ? (s.buildRecHint >= 0 ? s.buildRecHint : densityRecordSec(s)) : 0);
+  // the staged search cuts each row of cells to the chord of its sphere by x
+  if constexpr (D == 3) {
+    if (stagedPath) cellOrder<D, true>(s, n);
+    else cellOrder<D, false>(s, n);
+  } else {
+    cellOrder<D, false>(s, n);
+  }
 
   // 3. rows
   SearchArgs sa{};
@@ -1372,7 +1328,6 @@ void buildNeighborsD(Sim& s, double ext) {
   if (markUse) sa.keepSlot = s.slotKeep.as<int32_t>();
   if (s.ellCap <= 0) s.ellCap = D == 3 ? 160 : (D == 2 ? 48 : 16);
   s.rowCount.ensure(sizeof(int32_t) * size_t(n));
-  unsigned long long* dTotal = reinterpret_cast<unsigned long long*>(s.flags.as<int32_t>() + 4);
   for (int attempt = 0; attempt < 2; ++attempt) {
     sa.cap = s.ellCap;
     s.nbr.ensure(ellBytes(n, s.ellCap));
@@ -1380,7 +1335,7 @@ void buildNeighborsD(Sim& s, double ext) {
       // the first attempt's flags were zeroed with the cell counters; ghost
       // marks of the first attempt are a subset of the second's
       ZeroSet z{};
-      z.add(s.flags.as<int32_t>(), int64_t(s.flags.bytes / sizeof(int32_t)));
+      z.add(s.flags.as<int32_t>(), 8);
       zeroMany(z, s.stream);
     }
     if (stagedPath) {
@@ -1389,26 +1344,26 @@ void buildNeighborsD(Sim& s, double ext) {
                          s.flags.as<int32_t>());
     } else if (s.isotropic) {
       hipLaunchKernelGGL((k_search_global<D, true>), dim3(int(xcdGrid(nblocks(n)))), dim3(kBlock), 0, st, s.rec.as<double>(),
-                         s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>());
+                         s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
+                         s.flags.as<int32_t>());
     } else {
       hipLaunchKernelGGL((k_search_global<D, false>), dim3(int(xcdGrid(nblocks(n)))), dim3(kBlock), 0, st, s.rec.as<double>(),
-                         s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>());
+                         s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
+                         s.flags.as<int32_t>());
     }
-    hipLaunchKernelGGL(k_row_stats, dim3(int(std::min<int64_t>(1024, nblocks(n)))), dim3(kBlock), 0, st,
-                       s.rowCount.as<int32_t>(), n, dTotal, s.flags.as<int32_t>());
     SG_CHECK_HIP(hipGetLastError());
-    struct Flags { int32_t f[4]; unsigned long long total; };
-    char* hp = static_cast<char*>(hostStaging(s, 0, 256 + sizeof(int32_t) * 16));
-    // the ghost cull's first half rides on the same wait
-    const bool cullHere = markUse && s.subStart.size() < 16;
-    if (cullHere) cullLaunch(s, reinterpret_cast<int32_t*>(hp + 256));
-    Flags* hfp = reinterpret_cast<Flags*>(hp);
-    SG_CHECK_HIP(hipMemcpyAsync(hfp, s.flags.p, sizeof(Flags), hipMemcpyDeviceToHost, st));
+    struct Flags { int32_t f[4]; unsigned long long total, pad; };
+    static_assert(sizeof(Flags) == sizeof(int32_t) * 8, "the flags buffer");
+    char* hp = static_cast<char*>(hostStaging(s, 0, sizeof(Flags) + sizeof(int32_t) * (s.subs.size() + 1)));
+    const Flags* hfp = reinterpret_cast<const Flags*>(hp);
+    int32_t* hcull = reinterpret_cast<int32_t*>(hp + sizeof(Flags));
+    // the ghost cull's first half rides on the same wait and brings the flags along
+    if (markUse) cullLaunch(s, reinterpret_cast<int32_t*>(hp), hcull);
+    else SG_CHECK_HIP(hipMemcpyAsync(hp, s.flags.p, sizeof(Flags), hipMemcpyDeviceToHost, st));
     SG_CHECK_HIP(hipStreamSynchronize(st));
     const Flags hf = *hfp;
-    if (cullHere) {
-      const int32_t* cs = reinterpret_cast<const int32_t*>(hp + 256);
-      s.cullStarts.assign(cs, cs + s.subStart.size() + 1);
+    if (markUse) {
+      s.cullStarts.assign(hcull, hcull + s.subs.size() + 1);
       s.cullStartsReady = true;
     }
     s.maxRow = hf.f[0];
@@ -1424,22 +1379,14 @@ void buildNeighborsD(Sim& s, double ext) {
                        s.nbr.as<int32_t>(), n, s.perm.as<int32_t>(), s.iperm.as<int32_t>(),
                        s.nLists > 1 ? s.seg.as<double>() : nullptr, s.nInt, s.rowsMapOrder ? 1 : 0);
   // 5. work list of internal slots
-  s.workFlag.ensure(sizeof(int32_t) * size_t(n + 1));
-  s.workScan.ensure(sizeof(int32_t) * size_t(n + 1));
   s.work.ensure(sizeof(int32_t) * size_t(std::max<int64_t>(s.nInt, 1)));
-  hipLaunchKernelGGL(k_work_flag, dim3(nblocks(n)), dim3(kBlock), 0, st, s.perm.as<int32_t>(), n, s.nInt,
-                     s.workFlag.as<int32_t>());
-  exclusiveScan<int32_t, int32_t>(s.workFlag.as<int32_t>(), s.workScan.as<int32_t>(), n, s);
-  hipLaunchKernelGGL(k_work_scatter, dim3(nblocks(n)), dim3(kBlock), 0, st, s.workFlag.as<int32_t>(),
-                     s.workScan.as<int32_t>(), n, s.work.as<int32_t>());
+  scanItems(WorkScan{s.perm.as<int32_t>(), s.work.as<int32_t>(), s.nInt}, n, s.scanTmp, st);
   SG_CHECK_HIP(hipGetLastError());
   SG_CHECK_HIP(hipEventRecord(s.ev[1], st));
 }
 
 }  // namespace
 
-void exclusiveScanI32toI64(const int32_t* in, int64_t* out, int64_t n, Sim& s) { exclusiveScan<int32_t, int64_t>(in, out, n, s); }
-void exclusiveScanI32(const int32_t* in, int32_t* out, int64_t n, Sim& s) { exclusiveScan<int32_t, int32_t>(in, out, n, s); }
 void* hostStaging(Sim& s, int which, size_t bytes) {
   void*& p = which ? s.pinnedIn : s.pinnedOut;
   size_t& cap = which ? s.pinnedInBytes : s.pinnedOutBytes;
@@ -1455,24 +1402,6 @@ void* hostStaging(Sim& s, int which, size_t bytes) {
     cap = want;
   }
   return p;
-}
-
-void pickInts(Sim& s, const int32_t* src, const int64_t* at, int m, int32_t* hostOut) {
-  SG_REQUIRE(m >= 1 && m <= 16, SPHGPU_ERR_ARG, "pickInts takes 1 to 16 values");
-  Pick32 pk{};
-  for (int q = 0; q < m; ++q) pk.at[q] = at[q];
-  pk.m = m;
-  s.pick.ensure(sizeof(int32_t) * 16);
-  hipLaunchKernelGGL(k_pick_i32, dim3(1), dim3(64), 0, s.stream, src, pk, s.pick.as<int32_t>());
-  SG_CHECK_HIP(hipGetLastError());
-  SG_CHECK_HIP(hipMemcpyAsync(hostOut, s.pick.p, sizeof(int32_t) * size_t(m), hipMemcpyDeviceToHost, s.stream));
-}
-
-const int32_t* readInts(Sim& s, const int32_t* src, const int64_t* at, int m) {
-  int32_t* h = static_cast<int32_t*>(hostStaging(s, 0, sizeof(int32_t) * 16));
-  pickInts(s, src, at, m, h);
-  SG_CHECK_HIP(hipStreamSynchronize(s.stream));
-  return h;
 }
 
 void zeroMany(const ZeroSet& z, hipStream_t st) {

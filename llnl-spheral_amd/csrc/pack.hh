@@ -117,53 +117,29 @@ struct PackOut {
   double qInv;     // 1/u of the 3-D mixed record's positions
 };
 
-// The records of slot k.  SEC (bits): also write, from the values in
-// registers, the mixed pair kernel's record (1), the FP64 isotropic pair
-// kernel's record (2), the FP64 density sum's record (4) and the mixed density
-// sum's record (8).
+// A row's fields, as the records take them.
+template <int D> struct PackRow {
+  V<D> x, v;
+  S<D> h;
+  double rho, m, P, cs, omega, fcl, fcq, fsh;
+};
+template <int D, bool ISO>
+__device__ __forceinline__ PackRow<D> loadPackRow(int64_t i, const PackIn& in) {
+  PackRow<D> w;
+  for (int c = 0; c < D; ++c) { w.x.c[c] = in.pos[i * D + c]; w.v.c[c] = in.vel[i * D + c]; }
+  for (int c = 0; c < NSym<D>::value; ++c) w.h.c[c] = in.H[i * NSym<D>::value + c];
+  w.rho = in.rho[i]; w.m = in.mass[i]; w.P = in.P[i]; w.cs = in.cs[i]; w.omega = in.omega[i];
+  w.fcl = w.fcq = w.fsh = 1.0;
+  if constexpr (!ISO) {
+    if (in.fCl) { w.fcl = in.fCl[i]; w.fcq = in.fCq[i]; w.fsh = in.fsh[i]; }
+  }
+  return w;
+}
+
 template <int D, bool ISO, int SEC>
-__device__ __forceinline__ void packSlot(int64_t k, const PackIn& in, const PackOut& o) {
+__device__ __forceinline__ void storeRecords(int64_t k, const double* r, const PackOut& o) {
   static_assert(SEC == 0 || ISO, "the pair kernels' records are isotropic");
   using R = RL<ISO>;
-  constexpr int NS = NSym<D>::value;
-  const int64_t i = in.perm[k];
-  double r[R::STRIDE];
-#pragma unroll
-  for (int c = 0; c < R::STRIDE; ++c) r[c] = 0.0;
-  if (i < 0) {                      // dead slot (culled ghost): no row holds it
-    r[R::ORIG] = 2147483648.0;
-    double2* dst = reinterpret_cast<double2*>(o.rec + k * R::STRIDE);
-#pragma unroll
-    for (int c = 0; c < R::STRIDE / 2; ++c) dst[c] = make_double2(r[2 * c], r[2 * c + 1]);
-    if constexpr ((SEC & 1) != 0) writeMixedRec<D>(r, o.nInt, o.qInv, static_cast<float4*>(o.sec) + k * MixedRec<D>::F4);
-    if constexpr ((SEC & 2) != 0)
-      writeFast64Rec<D>(r, o.nInt, static_cast<double2*>(o.sec) + k * 4, static_cast<double2*>(o.sec) + 4 * o.n + k * 2);
-    if constexpr ((SEC & 4) != 0) writeDensRec<D>(r, static_cast<double2*>(o.sec2) + k * 3);
-    if constexpr ((SEC & 8) != 0) writeDensRecMixed<D>(r, static_cast<float4*>(o.sec3) + k * DensMixedRec<D>::F4);
-    return;
-  }
-  for (int c = 0; c < D; ++c) { r[R::X + c] = in.pos[i * D + c]; r[R::V + c] = in.vel[i * D + c]; }
-  S<D> h;
-  for (int c = 0; c < NS; ++c) h.c[c] = in.H[i * NS + c];
-  const double rh = in.rho[i], m = in.mass[i], p = in.P[i];
-  const double som = safeInv(in.omega[i], 1.0e-30);
-  if constexpr (ISO) {
-    r[RL<true>::HINV] = h.c[0];
-  } else {
-    for (int c = 0; c < NS; ++c) r[RL<false>::H + c] = h.c[c];
-    r[RL<false>::FCL] = in.fCl ? in.fCl[i] : 1.0;
-    r[RL<false>::FCQ] = in.fCq ? in.fCq[i] : 1.0;
-    r[RL<false>::FSH] = in.fsh ? in.fsh[i] : 1.0;
-  }
-  r[R::HDET] = sdet(h);
-  r[R::M] = m;
-  r[R::ORIG] = double(i);
-  r[R::RHO] = rh;
-  r[R::CS] = in.cs[i];
-  r[R::P] = p;
-  r[R::SOM] = som;
-  r[R::PRHO] = som * p / (rh * rh);
-  r[R::MOR] = m / rh;
   double2* dst = reinterpret_cast<double2*>(o.rec + k * R::STRIDE);
 #pragma unroll
   for (int c = 0; c < R::STRIDE / 2; ++c) dst[c] = make_double2(r[2 * c], r[2 * c + 1]);
@@ -172,6 +148,56 @@ __device__ __forceinline__ void packSlot(int64_t k, const PackIn& in, const Pack
     writeFast64Rec<D>(r, o.nInt, static_cast<double2*>(o.sec) + k * 4, static_cast<double2*>(o.sec) + 4 * o.n + k * 2);
   if constexpr ((SEC & 4) != 0) writeDensRec<D>(r, static_cast<double2*>(o.sec2) + k * 3);
   if constexpr ((SEC & 8) != 0) writeDensRecMixed<D>(r, static_cast<float4*>(o.sec3) + k * DensMixedRec<D>::F4);
+}
+
+// The records of slot k, which holds caller row i with the fields `w` (from
+// memory, or still in the registers of the kernel that wrote them: reading a
+// row back right after storing it waits for the stores).  SEC (bits): besides
+// the FP64 record also the mixed pair kernel's record (1), the FP64 isotropic
+// pair kernel's (2), the FP64 density sum's (4) and the mixed density sum's (8).
+template <int D, bool ISO, int SEC>
+__device__ __forceinline__ void packRow(int64_t k, int64_t i, const PackRow<D>& w, const PackOut& o) {
+  using R = RL<ISO>;
+  double r[R::STRIDE];
+#pragma unroll
+  for (int c = 0; c < R::STRIDE; ++c) r[c] = 0.0;
+  for (int c = 0; c < D; ++c) { r[R::X + c] = w.x.c[c]; r[R::V + c] = w.v.c[c]; }
+  const double som = safeInv(w.omega, 1.0e-30);
+  if constexpr (ISO) {
+    r[RL<true>::HINV] = w.h.c[0];
+  } else {
+    for (int c = 0; c < NSym<D>::value; ++c) r[RL<false>::H + c] = w.h.c[c];
+    r[RL<false>::FCL] = w.fcl;
+    r[RL<false>::FCQ] = w.fcq;
+    r[RL<false>::FSH] = w.fsh;
+  }
+  r[R::HDET] = sdet(w.h);
+  r[R::M] = w.m;
+  r[R::ORIG] = double(i);
+  r[R::RHO] = w.rho;
+  r[R::CS] = w.cs;
+  r[R::P] = w.P;
+  r[R::SOM] = som;
+  r[R::PRHO] = som * w.P / (w.rho * w.rho);
+  r[R::MOR] = w.m / w.rho;
+  storeRecords<D, ISO, SEC>(k, r, o);
+}
+
+// The same from the fields in memory; a dead slot (culled ghost, in no row)
+// gets an empty record.
+template <int D, bool ISO, int SEC>
+__device__ __forceinline__ void packSlot(int64_t k, const PackIn& in, const PackOut& o) {
+  using R = RL<ISO>;
+  const int64_t i = in.perm[k];
+  if (i < 0) {
+    double r[R::STRIDE];
+#pragma unroll
+    for (int c = 0; c < R::STRIDE; ++c) r[c] = 0.0;
+    r[R::ORIG] = 2147483648.0;
+    storeRecords<D, ISO, SEC>(k, r, o);
+    return;
+  }
+  packRow<D, ISO, SEC>(k, i, loadPackRow<D, ISO>(i, in), o);
 }
 
 struct Sim;
