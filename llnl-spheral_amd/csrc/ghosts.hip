@@ -315,15 +315,15 @@ __device__ __forceinline__ const DSub& ghostPlane(const GhostMap& m, int64_t g, 
 // slots' records (pack sec bits, isotropic layout) from the values just stored.
 template <int D, int REC>
 __global__ void k_ghost_fields(FieldPtrs f, GhostMap m, int64_t nTot, const int64_t* __restrict__ nDev, int geometry,
-                               const int32_t* __restrict__ iperm, PackIn pin, PackOut pout) {
+                               const int32_t* __restrict__ iperm, PackOut pout) {
   constexpr int NS = NSym<D>::value;
   if (nDev) nTot = *nDev;                          // a generation's count, still on the device
   const int64_t g = m.nInt + blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   if (g >= nTot) return;
   int depth;
   const int64_t r = ghostRoot(m, g, depth);
-  V<D> x, v = loadV<D>(f.vel, r);
-  double h[NS];
+  V<D> x = vzero<D>(), v = loadV<D>(f.vel, r);
+  double h[NS] = {};
   if (geometry) {
     x = loadV<D>(f.pos, r);
     for (int k = 0; k < NS; ++k) h[k] = f.H[r * NS + k];
@@ -345,15 +345,22 @@ __global__ void k_ghost_fields(FieldPtrs f, GhostMap m, int64_t nTot, const int6
     for (int k = 0; k < NS; ++k) f.H[g * NS + k] = h[k];
   }
   for (int k = 0; k < D; ++k) f.vel[g * D + k] = v.c[k];
-  f.mass[g] = f.mass[r];
-  f.rho[g] = f.rho[r];
+  PackRow<D> w;
+  w.m = f.mass[r]; w.rho = f.rho[r]; w.P = f.P[r]; w.cs = f.cs[r]; w.omega = f.omega[r];
   f.eps[g] = f.eps[r];
-  f.P[g] = f.P[r];
-  f.cs[g] = f.cs[r];
-  f.omega[g] = f.omega[r];
+  f.mass[g] = w.m;
+  f.rho[g] = w.rho;
+  f.P[g] = w.P;
+  f.cs[g] = w.cs;
+  f.omega[g] = w.omega;
   if (f.fCl) { f.fCl[g] = f.fCl[r]; f.fCq[g] = f.fCq[r]; f.fsh[g] = f.fsh[r]; }
   if (f.seg) f.seg[g] = f.seg[r];
-  if constexpr (REC >= 0) packSlot<D, true, REC>(iperm[g], pin, pout);
+  if constexpr (REC >= 0) {                        // always with the geometry
+    w.x = x;
+    w.v = v;
+    for (int k = 0; k < NS; ++k) w.h.c[k] = h[k];
+    packRow<D, true, REC>(iperm[g], g, w, pout);
+  }
 }
 
 __global__ void k_ghost_scalar(double* __restrict__ a, GhostMap m, int64_t nTot) {
@@ -583,11 +590,11 @@ template <int D> void applyFieldsD(Sim& s, bool geometry, int rec) {
   }
   const FieldPtrs f = fieldPtrs(s);
   const GhostMap m = ghostMap(s);
-  const PackIn pin = rec >= 0 ? packInputs(s) : PackIn{};
+  SG_REQUIRE(rec < 0 || geometry, SPHGPU_ERR_STATE, "ghost records take the refreshed geometry");
   const PackOut pout = rec >= 0 ? packOutputs(s, rec) : PackOut{};
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(nblocks(ng)), dim3(kBlock), 0, s.stream, f, m, rows, nDev, geometry ? 1 : 0,
-                       s.iperm.as<int32_t>(), pin, pout);
+                       s.iperm.as<int32_t>(), pout);
   };
   switch (rec) {
     case -1: go(k_ghost_fields<D, -1>); break;

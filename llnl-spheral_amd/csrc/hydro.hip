@@ -471,12 +471,16 @@ __device__ __forceinline__ void epilogue(int64_t k, int len, const Self<D>& me, 
   }
 }
 
-// The pairs a wavefront evaluated, one entry per wavefront of the work list
-// (tw: this lane's place in it): nothing to clear before the pass, no atomics,
-// and no read-back unless the caller asks for the count.
-__device__ __forceinline__ void storePairCount(unsigned pairs, int64_t tw, int64_t nInt, uint32_t* __restrict__ counts) {
+// The pairs a wavefront evaluated, one entry per wavefront of the work list:
+// nothing to clear before the pass, no atomics, and no read-back unless the
+// caller asks for the count.  The entry's index is formed again here from
+// scalars: a lane's work index kept through the pair loop cost two VGPRs, which
+// took the mixed 3-D kernel from 167 to 169 and from three waves per SIMD to two.
+template <int BS>
+__device__ __forceinline__ void storePairCount(unsigned pairs, int64_t nInt, uint32_t* __restrict__ counts) {
   for (int sh = 32; sh > 0; sh >>= 1) pairs += __shfl_xor(pairs, sh);
-  if ((threadIdx.x & 63) == 0 && tw < nInt) counts[tw >> 6] = pairs;
+  const int64_t wave = xcdBlock((nInt + BS - 1) / BS) * (BS / 64) + (__builtin_amdgcn_readfirstlane(threadIdx.x) >> 6);
+  if (__lane_id() == 0 && wave * 64 < nInt) counts[wave] = pairs;
 }
 
 template <int D, bool ISO, bool TENSILE>
@@ -608,7 +612,7 @@ __global__ void __launch_bounds__(kBlock) k_derivs_fp64(const double* __restrict
   const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
   unsigned pairs = 0;
   if (tw < nInt) pairs = derivsNodeFP64<D, ISO, TENSILE>(work[tw], rec, rowCount, nbr, n, tab, t, p, o);
-  storePairCount(pairs, tw, nInt, pairCounts);
+  storePairCount<kBlock>(pairs, nInt, pairCounts);
 }
 
 // ---------------------------------------------------------------------------
@@ -1133,7 +1137,7 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
     me.Hdet = ri_[R::HDET]; me.m = ri_[R::M]; me.rho = ri_[R::RHO]; me.mor = ri_[R::MOR];
     epilogue<D>(k, len, me, a, t, p, o);
   }
-  storePairCount(pairs, tw, nInt, pairCounts);
+  storePairCount<BS>(pairs, nInt, pairCounts);
 }
 
 TabArgs tabArgs(const Sim& s) {

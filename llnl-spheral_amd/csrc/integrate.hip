@@ -19,8 +19,8 @@
 // (src/Hydro/SpecificThermalEnergyPolicy.cc:64-189): eps += m*DepsDt with
 // DepsDt rebuilt from the pair accelerations of the pass and the step-start
 // velocities.
-// The derivative fields are read in slot order (one lane per internal slot of
-// the work list) and the state is written at the caller index of the slot.
+// The state is walked in caller order and the derivative fields gathered from
+// each row's slot.
 #include "internal.hh"
 #include "dgeom.hh"
 #include "eigen.hh"
@@ -117,24 +117,31 @@ __device__ __forceinline__ void rowMultEos(const SegArgs& sa, int64_t i, double&
 // 128^3 five copies of 235 MB in all, of which H was never read back).  The
 // final update starts from b and leaves the dt vote's inputs of the next step
 // (maxViscousPressure, tr DvDx, DvDt by caller index) in dtIn.
+// One lane per caller row: its eleven state arrays are then read and written
+// contiguously, and only the five derivatives are gathered from its slot (an
+// internal row's slot is iperm[i]).  By slot it was the other way round.
 template <int D, int REC, bool TRIAL>
-__global__ void k_update(const int32_t* __restrict__ work, const int32_t* __restrict__ perm, int64_t nInt, Fields f,
-                         Base b, DerivIn d, Bounds bd, Eos e, SegArgs sa, PackIn pin, PackOut pout,
-                         double* __restrict__ dtIn) {
+__global__ void __launch_bounds__(kBlock) k_update(const int32_t* __restrict__ iperm, int64_t nInt, Fields f, Base b,
+                                                   DerivIn d, Bounds bd, Eos e, SegArgs sa, PackIn pin, PackOut pout,
+                                                   double* __restrict__ dtIn) {
   constexpr int NS = NSym<D>::value;
-  const int64_t t = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (t >= nInt) return;
-  const int64_t k = work[t];
-  const int64_t i = perm[k];
+  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  if (i >= nInt) return;
+  const int64_t k = iperm[i];
   double mult;
   rowMultEos(sa, i, mult, e);
   const double* dx = d.base + int64_t(d.oDx) * d.n + k * D;
   const double* dv = d.base + int64_t(d.oDv) * d.n + k * D;
+  PackRow<D> w;
+  double dvc[D];
   for (int c = 0; c < D; ++c) {
     const double x0 = (TRIAL ? f.pos : b.pos)[i * D + c], v0 = (TRIAL ? f.vel : b.vel)[i * D + c];
     if (TRIAL) { b.pos[i * D + c] = x0; b.vel[i * D + c] = v0; }
-    f.pos[i * D + c] = x0 + mult * dx[c];
-    f.vel[i * D + c] = v0 + mult * dv[c];
+    dvc[c] = dv[c];
+    w.x.c[c] = x0 + mult * dx[c];
+    w.v.c[c] = v0 + mult * dvc[c];
+    f.pos[i * D + c] = w.x.c[c];
+    f.vel[i * D + c] = w.v.c[c];
   }
   const double eps0 = (TRIAL ? f.eps : b.eps)[i], rho0 = (TRIAL ? f.rho : b.rho)[i];
   if (TRIAL) { b.eps[i] = eps0; b.rho[i] = rho0; }
@@ -145,11 +152,21 @@ __global__ void k_update(const int32_t* __restrict__ work, const int32_t* __rest
   const double* hid = d.base + int64_t(d.oHid) * d.n + k * NS;
   int c = 0;
   for (int a = 0; a < D; ++a)
-    for (int q = a; q < D; ++q, ++c) f.H[i * NS + c] = (a == q) ? dmin(bd.hminInv, dmax(bd.hmaxInv, hid[c])) : hid[c];
+    for (int q = a; q < D; ++q, ++c) {
+      w.h.c[c] = (a == q) ? dmin(bd.hminInv, dmax(bd.hmaxInv, hid[c])) : hid[c];
+      f.H[i * NS + c] = w.h.c[c];
+    }
   const double P = eosP(e, rho, eps), cs = eosCs(e, eps);
   f.P[i] = P;
   f.cs[i] = cs;
-  if constexpr (REC >= 0) packSlot<D, true, REC>(k, pin, pout);
+  if constexpr (REC >= 0) {
+    w.rho = rho;
+    w.P = P;
+    w.cs = cs;
+    w.m = pin.mass[i];
+    w.omega = pin.omega[i];
+    packRow<D, true, REC>(k, i, w, pout);
+  }
   if constexpr (!TRIAL) {
     constexpr int W = 2 + D;
     dtIn[i * W] = d.base[int64_t(d.oVP) * d.n + k];
@@ -157,14 +174,14 @@ __global__ void k_update(const int32_t* __restrict__ work, const int32_t* __rest
     double tr = g[0];
     for (int a = 1; a < D; ++a) tr = tr + g[a * D + a];
     dtIn[i * W + 1] = tr;
-    for (int c2 = 0; c2 < D; ++c2) dtIn[i * W + 2 + c2] = dv[c2];
+    for (int c2 = 0; c2 < D; ++c2) dtIn[i * W + 2 + c2] = dvc[c2];
   }
   // an ensemble member whose state turns non-finite fails alone (the step's
   // final update; NaN at the midpoint reaches it)
   if (!TRIAL && sa.seg) {
     bool ok = isfinite(eps) && isfinite(rho) && isfinite(P) && isfinite(cs);
-    for (int c = 0; c < D; ++c) ok = ok && isfinite(f.pos[i * D + c]) && isfinite(f.vel[i * D + c]);
-    for (int c = 0; c < NS; ++c) ok = ok && isfinite(f.H[i * NS + c]);
+    for (int c2 = 0; c2 < D; ++c2) ok = ok && isfinite(w.x.c[c2]) && isfinite(w.v.c[c2]);
+    for (int c2 = 0; c2 < NS; ++c2) ok = ok && isfinite(w.h.c[c2]);
     if (!ok) atomicOr(&sa.st[int(sa.seg[i])].fail, unsigned(SPHGPU_MEMBER_NONFINITE));
   }
 }
@@ -368,8 +385,8 @@ template <int D, bool TRIAL> void updateD(Sim& s, const Base& b, const Bounds& b
   const PackIn pin = rec >= 0 ? packInputs(s) : PackIn{};
   const PackOut pout = rec >= 0 ? packOutputs(s, rec) : PackOut{};
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, s.work.as<int32_t>(),
-                       s.perm.as<int32_t>(), s.nInt, f, b, d, bd, e, sa, pin, pout, s.dtIn.as<double>());
+    hipLaunchKernelGGL(kern, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, s.iperm.as<int32_t>(), s.nInt, f, b, d,
+                       bd, e, sa, pin, pout, s.dtIn.as<double>());
   };
   // the trial update writes the pair kernel's records, the final one the density sum's
   if constexpr (TRIAL) {
