@@ -367,7 +367,21 @@ struct OutArgs {
   double* pairDv;    // compatible energy: the pair term of every row entry in the node's own
                      // frame, component c at pairDv[c*plane + ellIndex(w, n, k)]; null otherwise
   int64_t plane;
+  double* relV;      // dt vote: the largest |v_ij|^2 of the row per slot (1-D: |v_ij|), -1 for an
+                     // empty row; null otherwise
 };
+
+// The pair limit of GenericHydro::dt (src/Physics/GenericHydro.cc:218-283) is
+// the smallest nodeScale/|v_ij|, and rounding is monotonic, so the largest
+// |v_ij| of a row gives it to the bit.  The pass at the step start has every
+// v_ij at hand; a vote that gathered the velocities again took 1.45 ms at 128^3,
+// these terms under 0.1 ms.  A NaN is passed over, as the vote's minimum does.
+template <int D> __device__ __forceinline__ double relSpeed(const double* d) {
+  if constexpr (D == 1) return dabs(d[0]);
+  double s = d[0] * d[0];
+  for (int c = 1; c < D; ++c) s = s + d[c] * d[c];
+  return s;
+}
 
 __device__ __forceinline__ double* outRow(const OutArgs& o, int field, int64_t k, int comps) {
   return o.base + int64_t(o.off[field]) * o.n + k * comps;
@@ -500,6 +514,7 @@ __device__ __forceinline__ unsigned derivsNodeFP64(int64_t k, const double* __re
   T<D> DvDx = tzero<D>(), M = tzero<D>();
   S<D> m2nd = szero<D>();
   unsigned pairs = 0;
+  double relV = 0.0;
 
   const int len = rowCount[k];
   const int4* nb4 = reinterpret_cast<const int4*>(nbr);
@@ -514,6 +529,7 @@ __device__ __forceinline__ unsigned derivsNodeFP64(int64_t k, const double* __re
     pairs += ownerI ? 1u : 0u;
     const V<D> rij = vsub(ri, nb.x);
     const V<D> vij = vsub(vi, nb.v);
+    if (o.relV) relV = dmax(relV, relSpeed<D>(vij.c));
     const S<D>& Hj = nb.H;
     const double Hdetj = nb.hdet, mj = nb.m, rhoj = nb.rho, cj = nb.cs, morj = nb.mor;
 
@@ -592,6 +608,7 @@ __device__ __forceinline__ unsigned derivsNodeFP64(int64_t k, const double* __re
     }
   }
 
+  if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
   // per-node epilogue (SPHHydroBase.cc:834-902)
   Acc<D> a;
   a.rhoSum = rhoSum; a.norm = norm; a.DepsDt = DepsDt; a.maxVP = maxVP; a.effVP = effVP; a.viscW = viscW;
@@ -977,6 +994,7 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
     SumsF<F32 ? D : 1> af;
     if constexpr (F32) af.zero();
     Real maxVP = Real(0);
+    double relV = 0.0;
     const int len = rowCount[k];
     const int4* nb4 = reinterpret_cast<const int4*>(nbr);
     int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
@@ -992,6 +1010,9 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
         vij[c] = vi[c] - nb.v[c];
         r2 = fmaR(rij[c], rij[c], r2);
         vdotr = fmaR(vij[c], rij[c], vdotr);
+      }
+      if constexpr (!F32) {
+        if (o.relV) relV = dmax(relV, relSpeed<D>(vij));
       }
       const Real rinv = r2 > Real(1.0e-30) ? rsqR(r2) : Real(0);
       const Real rmag = r2 * rinv;
@@ -1127,6 +1148,9 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
     for (int c = 0; c < D; ++c)
       for (int b = 0; b < c; ++b) a.M.c[c * D + b] = a.M.c[b * D + c];
     a.maxVP = double(maxVP);
+    if constexpr (!F32) {
+      if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
+    }
     // the node's own state for the epilogue, read again after the loop so it
     // holds no registers during it
     Self<D> me;
@@ -1193,6 +1217,7 @@ PackOut packOutputs(Sim& s, int sec) {
     s.recSM.ensure(sizeof(float) * 8 * size_t(std::max<int64_t>(n, 1)));
     o.sec3 = s.recSM.p;
   }
+  o.vel = nullptr;
   s.recSValid = (sec & 4) != 0;
   s.recSMValid = (sec & 8) != 0;
   s.pairRec = sec & 3;
@@ -1388,7 +1413,7 @@ void isoVariant(Sim& s, int v, bool fits, hipStream_t st, int64_t n, const TabAr
 }
 
 template <int D>
-void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly) {
+void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool relV) {
   const int64_t n = s.nSlots;
   hipStream_t st = s.stream;
   const int total = derivTotalDoubles(s.dim);
@@ -1437,6 +1462,11 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly) {
   o.base = s.out.as<double>();
   o.n = n;
   o.updateOnly = updateOnly ? 1 : 0;
+  if (relV) {
+    SG_REQUIRE(!mixed, SPHGPU_ERR_STATE, "the dt vote takes FP64 velocities");
+    s.relV.ensure(sizeof(double) * size_t(std::max<int64_t>(n, 1)));
+    o.relV = s.relV.as<double>();
+  }
   for (int f = 0; f < SPHGPU_NUM_DERIV_FIELDS; ++f) o.off[f] = derivOffsetDoubles(s.dim, f);
   if (compat) {
     // pairAccelerations: the own-frame pair term of every row entry
@@ -1640,7 +1670,7 @@ void sumDensity(Sim& s) {
   s.derivsValid = false;
 }
 
-void evalDerivs(Sim& s, const sphgpu_hydro_params& p, bool updateOnly) {
+void evalDerivs(Sim& s, const sphgpu_hydro_params& p, bool updateOnly, bool relV) {
   SG_REQUIRE(s.neighborsValid, SPHGPU_ERR_STATE, "evaluateDerivatives needs a neighbour build");
   SG_REQUIRE(s.table.n > 0, SPHGPU_ERR_STATE, "no kernel table installed");
   SG_REQUIRE(!(p.compatibleEnergyEvolution && p.evolveTotalEnergy), SPHGPU_ERR_ARG,
@@ -1649,9 +1679,9 @@ void evalDerivs(Sim& s, const sphgpu_hydro_params& p, bool updateOnly) {
              "unknown precision");
   SG_REQUIRE(p.nPerh > 0.0, SPHGPU_ERR_ARG, "nPerh must be positive");
   s.derivsValid = false;
-  if (s.dim == 1) evalDerivsD<1>(s, p, updateOnly);
-  else if (s.dim == 2) evalDerivsD<2>(s, p, updateOnly);
-  else evalDerivsD<3>(s, p, updateOnly);
+  if (s.dim == 1) evalDerivsD<1>(s, p, updateOnly, relV);
+  else if (s.dim == 2) evalDerivsD<2>(s, p, updateOnly, relV);
+  else evalDerivsD<3>(s, p, updateOnly, relV);
   if (!s.capturing) s.timingPending |= 4u;
   s.derivsValid = true;
   s.pairsValid = true;

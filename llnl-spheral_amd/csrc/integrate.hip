@@ -196,52 +196,123 @@ template <int D> __device__ __forceinline__ double vmagArr(const double* a) {
 // GenericHydro::dt candidates of one internal node; the minimum over all
 // nodes is reduced with one 64-bit atomic min per wavefront on the bit
 // pattern of the (positive) candidate.
-template <int D>
-__global__ void k_dt(const int32_t* __restrict__ work, const int32_t* __restrict__ perm, int64_t nInt,
-                     const int32_t* __restrict__ rowCount, const int32_t* __restrict__ nbr, int64_t n,
-                     const double* __restrict__ H, const double* __restrict__ cs, const double* __restrict__ rho,
-                     const double* __restrict__ vel, const double* __restrict__ dtIn, int haveDtIn, double nPerh,
-                     int useVelMag, const double* __restrict__ seg, unsigned long long* __restrict__ minBits,
-                     int64_t minStride) {
+// Where the pair limit's velocities come from:
+//   kVoteRows   the caller-order velocities of the row's nodes (sphgpu_hydro_dt)
+//   kVoteSlots  velocities packed by slot with the build (a mixed step, whose pair
+//               kernel holds FP32 velocities: the vote stays FP64); four
+//               neighbours' loads in flight
+//   kVoteDone   the row maxima the FP64 pass at the step start left (relV)
+// An entry that would not lower the minimum is left out (a plain read may be
+// stale, then the atomic decides): 32 k atomics on one word were 0.3 ms of the
+// vote at 128^3.
+__device__ __forceinline__ void enterMin(unsigned long long* p, double m) {
+  const unsigned long long v = (unsigned long long)__double_as_longlong(m);
+  if (v < *static_cast<volatile unsigned long long*>(p)) atomicMin(p, v);
+}
+enum { kVoteRows, kVoteSlots, kVoteDone };
+struct VoteArgs {
+  const int32_t *list, *perm, *rowCount, *nbr;   // list: kVoteDone caller row -> slot, else the work list
+  int64_t n, nInt;
+  const double *H, *cs, *rho, *vel, *dtIn;
+  int haveDtIn;
+  double nPerh;
+  int useVelMag;
+  const double* seg;
+  const double *velS, *relV;
+};
+template <int D, int FROM>
+__global__ void __launch_bounds__(kBlock) k_dt(VoteArgs a, unsigned long long* __restrict__ minBits, int64_t minStride) {
   constexpr int NS = NSym<D>::value;
-  const int64_t t = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+  // rows in slot order where neighbours are gathered, else in caller order
+  const int64_t t = xcdBlock((a.nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
   double m = double(FLT_MAX);
   int sg = 0;
-  if (t < nInt) {
-    const int64_t k = work[t];
-    const int64_t i = perm[k];
-    if (seg) sg = int(seg[i]);
-    const double nodeScale = 1.0 / maxEigen<D>(H + i * NS) / nPerh;
-    m = dmin(m, nodeScale / (cs[i] + FLT_MIN));
+  if (t < a.nInt) {
+    int64_t k, i;
+    if constexpr (FROM == kVoteDone) {
+      i = t;
+      k = a.list[i];
+    } else {
+      k = a.list[t];
+      i = a.perm[k];
+    }
+    if (a.seg) sg = int(a.seg[i]);
+    const double nodeScale = 1.0 / maxEigen<D>(a.H + i * NS) / a.nPerh;
+    m = dmin(m, nodeScale / (a.cs[i] + FLT_MIN));
     constexpr int W = 2 + D;
     double vp = 0.0, divv = 0.0, acc[3] = {0.0, 0.0, 0.0};
-    if (haveDtIn) {
-      vp = dtIn[i * W];
-      divv = dtIn[i * W + 1];
-      for (int c = 0; c < D; ++c) acc[c] = dtIn[i * W + 2 + c];
+    if (a.haveDtIn) {
+      vp = a.dtIn[i * W];
+      divv = a.dtIn[i * W + 1];
+      for (int c = 0; c < D; ++c) acc[c] = a.dtIn[i * W + 2 + c];
     }
-    const double csq = sqrt(vp / rho[i]);
+    const double csq = sqrt(vp / a.rho[i]);
     m = dmin(m, nodeScale / (csq + FLT_MIN));
     m = dmin(m, 1.0 / (dabs(divv) + FLT_MIN));
     double vi[3];
-    for (int c = 0; c < D; ++c) vi[c] = vel[i * D + c];
-    const int len = rowCount[k];
-    for (int w = 0; w < len; ++w) {
-      const int64_t j = perm[nbr[ellIndex(w, n, k)]];
-      double d[3];
-      for (int c = 0; c < D; ++c) d[c] = vi[c] - vel[j * D + c];
-      m = dmin(m, nodeScale * (1.0 / dmax(1.0e-30, vmagArr<D>(d))));
+    for (int c = 0; c < D; ++c) vi[c] = a.vel[i * D + c];
+    if constexpr (FROM == kVoteDone) {
+      const double r = a.relV[k];
+      if (r >= 0.0) m = dmin(m, nodeScale * (1.0 / dmax(1.0e-30, D == 1 ? r : sqrt(r))));
+    } else if constexpr (FROM == kVoteSlots) {
+      // the pair term is monotonic in |v_ij|^2, to the bit: one square root a row
+      const int len = a.rowCount[k];
+      const int4* nb4 = reinterpret_cast<const int4*>(a.nbr);
+      double r = 0.0;
+      for (int w = 0; w < len; w += 4) {
+        const int4 j4 = nb4[ellChunk(w >> 2, a.n, k)];
+        const int32_t j[4] = {j4.x, j4.y, j4.z, j4.w};
+        double d[4][3];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const double* p = a.velS + int64_t(w + q < len ? j[q] : j[0]) * velStride(D);
+          if constexpr (D == 1) {
+            d[q][0] = p[0];
+          } else {
+            const double2 lo = reinterpret_cast<const double2*>(p)[0];
+            d[q][0] = lo.x;
+            d[q][1] = lo.y;
+            if constexpr (D == 3) d[q][2] = p[2];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          for (int c = 0; c < D; ++c) d[q][c] = vi[c] - d[q][c];
+          double s = D == 1 ? dabs(d[q][0]) : d[q][0] * d[q][0];
+          for (int c = 1; c < D; ++c) s = s + d[q][c] * d[q][c];
+          r = dmax(r, s);
+        }
+      }
+      if (len > 0) m = dmin(m, nodeScale * (1.0 / dmax(1.0e-30, D == 1 ? r : sqrt(r))));
+    } else {
+      const int len = a.rowCount[k];
+      for (int w = 0; w < len; ++w) {
+        const int64_t j = a.perm[a.nbr[ellIndex(w, a.n, k)]];
+        double d[3];
+        for (int c = 0; c < D; ++c) d[c] = vi[c] - a.vel[j * D + c];
+        m = dmin(m, nodeScale * (1.0 / dmax(1.0e-30, vmagArr<D>(d))));
+      }
     }
     m = dmin(m, sqrt(nodeScale / (vmagArr<D>(acc) + FLT_MIN)));
-    if (useVelMag) m = dmin(m, nodeScale / (vmagArr<D>(vi) + 1.0e-10));
+    if (a.useVelMag) m = dmin(m, nodeScale / (vmagArr<D>(vi) + 1.0e-10));
   }
   const int s0 = __shfl(sg, 0);
   if (__all(sg == s0)) {
     for (int sh = 32; sh > 0; sh >>= 1) m = dmin(m, __shfl_xor(m, sh));
-    if ((threadIdx.x & 63) == 0) atomicMin(minBits + s0 * minStride, (unsigned long long)__double_as_longlong(m));
-  } else if (t < nInt) {
-    atomicMin(minBits + sg * minStride, (unsigned long long)__double_as_longlong(m));
+    if ((threadIdx.x & 63) == 0) enterMin(minBits + s0 * minStride, m);
+  } else if (t < a.nInt) {
+    enterMin(minBits + sg * minStride, m);
   }
+}
+
+template <int D, int FROM>
+void voteD(Sim& s, double nPerh, int useVelMag, const double* seg, unsigned long long* bits, int64_t stride) {
+  VoteArgs a{FROM == kVoteDone ? s.iperm.as<int32_t>() : s.work.as<int32_t>(), s.perm.as<int32_t>(),
+             s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots, s.nInt, s.H.as<double>(), s.cs.as<double>(),
+             s.rho.as<double>(), s.vel.as<double>(), s.dtIn.as<double>(), s.haveDtIn ? 1 : 0, nPerh, useVelMag, seg,
+             s.velS.as<double>(), s.relV.as<double>()};
+  hipLaunchKernelGGL((k_dt<D, FROM>), dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, s.stream, a, bits, stride);
+  SG_CHECK_HIP(hipGetLastError());
 }
 
 __global__ void k_set_u64(unsigned long long* p, unsigned long long v) { *p = v; }
@@ -417,11 +488,7 @@ template <int D> double hydroDtD(Sim& s, double nPerh, double cfl, int useVelMag
   std::memcpy(&ib, &init, sizeof(ib));
   hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, s.stream, bits, ib);
   if (!s.haveDtIn) s.dtIn.ensure(sizeof(double) * 8);
-  hipLaunchKernelGGL(k_dt<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, s.stream, s.work.as<int32_t>(),
-                     s.perm.as<int32_t>(), s.nInt, s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots,
-                     s.H.as<double>(), s.cs.as<double>(), s.rho.as<double>(), s.vel.as<double>(), s.dtIn.as<double>(),
-                     s.haveDtIn ? 1 : 0, nPerh, useVelMag, nullptr, bits, int64_t(0));
-  SG_CHECK_HIP(hipGetLastError());
+  voteD<D, kVoteRows>(s, nPerh, useVelMag, nullptr, bits, 0);
   unsigned long long hb = 0;
   SG_CHECK_HIP(hipMemcpyAsync(&hb, bits, sizeof(hb), hipMemcpyDeviceToHost, s.stream));
   SG_CHECK_HIP(hipStreamSynchronize(s.stream));
@@ -465,18 +532,29 @@ void preStep(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_para
   const bool fast64 = s.rowOrder == SPHGPU_ROW_ORDER_SEARCH && hp.epsTensile == 0.0 && !hp.compatibleEnergyEvolution;
   struct Hint {     // the hint holds for this build only, also when it throws
     Sim& s;
-    ~Hint() { s.buildRecHint = -1; }
+    ~Hint() {
+      s.buildRecHint = -1;
+      s.buildVel = false;
+    }
   } hint{s};
+  s.buildVel = mixed;
   s.buildRecHint = ip.gradhCorrection ? 0 : (mixed ? 1 : (fast64 ? 2 : 0));
   if (!s.subs.empty()) setGhostNodes(s, ip.kernelExtent, ip.cullGhostNodes != 0);
   else buildNeighbors(s, ip.kernelExtent);
 }
 
-// The two derivative passes and updates of SynchronousRK2::step, then
+// Where the dt votes go: one word, or one per ensemble member.
+struct Vote {
+  const double* seg;
+  unsigned long long* bits;
+  int64_t stride;
+};
+
+// The dt vote, the two derivative passes and updates of SynchronousRK2::step, then
 // SPHHydroBase::finalize and Integrator::enforceBoundaries.  Multipliers are
 // dt/2, dt (plain simulation) or per member (half, full).
 template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip,
-                               const SegArgs& half, const SegArgs& full) {
+                               const Vote& vote, const SegArgs& half, const SegArgs& full) {
   hipStream_t st = s.stream;
   const bool compat = hp.compatibleEnergyEvolution != 0;
   SG_REQUIRE(!compat || s.deviceGhosts || s.nTot == s.nInt, SPHGPU_ERR_UNSUPPORTED,
@@ -487,8 +565,13 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
   // derivatives at t (SPHHydroBase::initialize first: the grad-h correction); the
   // midpoint pass below rewrites every field before anything but the trial
   // update reads one, so this pass stores only the fields the update reads
+  // (the vote needs nothing the pass writes but the rows' largest relative speeds,
+  // and the pass nothing of the vote)
+  const bool mixed = hp.precision == SPHGPU_PRECISION_MIXED;
+  if (mixed) voteD<D, kVoteSlots>(s, hp.nPerh, ip.useVelocityMagnitudeForDt, vote.seg, vote.bits, vote.stride);
   if (ip.gradhCorrection) omegaGradh(s);
-  evalDerivs(s, hp, true);
+  evalDerivs(s, hp, true, !mixed);
+  if (!mixed) voteD<D, kVoteDone>(s, hp.nPerh, ip.useVelocityMagnitudeForDt, vote.seg, vote.bits, vote.stride);
   // state0 (the policy reads every row's step-start velocity, ghosts included)
   const size_t n = size_t(s.nInt), nv = compat ? size_t(s.nTot) : n;
   const size_t rows[4] = {n * D, nv * D, n, n};
@@ -594,7 +677,7 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
                         &s.recS, &s.recSM, &s.pairDv, &s.compDe, &s.compAcc, &s.compDe0, &s.compRec, &s.out,
                         &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
                         &s.work, &s.ghostIsControl, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
-                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts})
+                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts, &s.velS, &s.relV})
     keyBuf(k, *b);
   for (const DBuf& b : s.state0) keyBuf(k, b);
   return k;
@@ -687,17 +770,12 @@ template <int D> double rk2D(Sim& s, const sphgpu_hydro_params& hp, const sphgpu
   const SelectArgs sel{ip.cfl, ip.dtMin, ip.dtMax, ip.dtGrowth};
   SegState* hs = static_cast<SegState*>(hostStaging(s, 0, sizeof(SegState)));
   runStep(s, hp, ip, [&] {
-    hipLaunchKernelGGL(k_dt<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
-                       s.perm.as<int32_t>(), s.nInt, s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots,
-                       s.H.as<double>(), s.cs.as<double>(), s.rho.as<double>(), s.vel.as<double>(),
-                       s.dtIn.as<double>(), s.haveDtIn ? 1 : 0, hp.nPerh, ip.useVelocityMagnitudeForDt, nullptr,
-                       &sd->voteBits, int64_t(0));
-    SG_CHECK_HIP(hipGetLastError());
+    const Vote vote{nullptr, &sd->voteBits, 0};
     const bool perList = s.nLists > 1 && !s.listGammaHost.empty();
     const double* lo = perList ? s.seg.as<double>() : nullptr;
     const double* lg = perList ? s.listGamma.as<double>() : nullptr;
     const SegArgs half{nullptr, sd, 1, sel, lo, lg}, full{nullptr, sd, 0, sel, lo, lg};
-    stepBody<D>(s, hp, ip, half, full);
+    stepBody<D>(s, hp, ip, vote, half, full);
     hipLaunchKernelGGL(k_seg_advance, dim3(1), dim3(kBlock), 0, st, sd, 1, sel, 0.0, hs);
     SG_CHECK_HIP(hipGetLastError());
   });
@@ -725,14 +803,10 @@ template <int D> void ensembleRk2D(Sim& s, const sphgpu_hydro_params& hp, const 
   SegState* hs = static_cast<SegState*>(hostStaging(s, 0, sizeof(SegState) * size_t(ns)));
   runStep(s, hp, ip, [&] {
     hipLaunchKernelGGL(k_seg_vote_init, dim3(nblocks(ns)), dim3(kBlock), 0, st, sd, ns, ib);
-    hipLaunchKernelGGL(k_dt<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
-                       s.perm.as<int32_t>(), s.nInt, s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots,
-                       s.H.as<double>(), s.cs.as<double>(), s.rho.as<double>(), s.vel.as<double>(),
-                       s.dtIn.as<double>(), s.haveDtIn ? 1 : 0, hp.nPerh, ip.useVelocityMagnitudeForDt,
-                       s.seg.as<double>(), &sd->voteBits, int64_t(sizeof(SegState) / sizeof(unsigned long long)));
+    const Vote vote{s.seg.as<double>(), &sd->voteBits, int64_t(sizeof(SegState) / sizeof(unsigned long long))};
     SG_CHECK_HIP(hipGetLastError());
     const SegArgs half{s.seg.as<double>(), sd, 1, sel}, full{s.seg.as<double>(), sd, 0, sel};
-    stepBody<D>(s, hp, ip, half, full);
+    stepBody<D>(s, hp, ip, vote, half, full);
     hipLaunchKernelGGL(k_seg_advance, dim3(nblocks(ns)), dim3(kBlock), 0, st, sd, ns, sel, s.dtThreshold, hs);
     SG_CHECK_HIP(hipGetLastError());
   });

@@ -205,6 +205,9 @@ struct Sim {
   int pairRec = 0;           // pair-kernel record current with rec: 1 mixed, 2 FP64 isotropic, 0 none
   int buildRecHint = -1;     // record kinds (pack sec bits, isotropic H) the neighbour build's pack also
                              // writes: -1 the density sum's, else what the caller will read first
+  bool buildVel = false;     // the build also writes velS (the dt vote of a mixed step)
+  DBuf velS;                 // velocities by slot at the last build
+  DBuf relV;                 // per slot: the largest relative speed of its row (dt vote of an FP64 step)
   bool recSValid = false;    // recS matches rec (written by the record pack; valid through a cull)
   DBuf recSM;               // mixed density-sum neighbour records (32 B per slot)
   bool recSMValid = false;   // recSM matches rec (written by the record pack; the cull keeps it)
@@ -334,7 +337,8 @@ void packRecords(Sim& s, int sec = 0);
 void sumDensity(Sim& s);
 // updateOnly: store only DxDt, DvDt, DepsDt, DrhoDt and Hideal (the fields an
 // integrator update reads); the other fields keep what they held
-void evalDerivs(Sim& s, const sphgpu_hydro_params& p, bool updateOnly = false);
+// relV: also leave the largest relative speed of every row in s.relV (FP64)
+void evalDerivs(Sim& s, const sphgpu_hydro_params& p, bool updateOnly = false, bool relV = false);
 // The pack sec bits of the records the pair kernel and the density sum read.
 int pairRecordSec(const Sim& s, const sphgpu_hydro_params& hp);
 int densityRecordSec(const Sim& s);

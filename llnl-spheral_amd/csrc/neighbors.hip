@@ -1136,7 +1136,11 @@ void cellOrder(Sim& s, int64_t n) {
   // the records the next kernel reads, written with the FP64 record: the
   // caller's hint, else the density sum's
   const int sec = s.isotropic ? (s.buildRecHint >= 0 ? s.buildRecHint : densityRecordSec(s)) : 0;
-  const PackOut o = packOutputs(s, sec);
+  PackOut o = packOutputs(s, sec);
+  if (s.buildVel) {
+    s.velS.ensure(sizeof(double) * size_t(velStride(D)) * size_t(n));
+    o.vel = s.velS.as<double>();
+  }
   const PackIn in = packInputs(s);
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(nblocks(n)), dim3(kBlock), 0, s.stream, s.cellOf.as<int32_t>(),

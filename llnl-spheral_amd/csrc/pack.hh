@@ -115,7 +115,10 @@ struct PackOut {
   int64_t n, nInt;
   void* sec3;
   double qInv;     // 1/u of the 3-D mixed record's positions
+  double* vel;     // velocities by slot for the dt vote (velStride doubles each), or null
 };
+// One or two 16-B loads a neighbour in 2-D and 3-D.
+constexpr int velStride(int D) { return D == 3 ? 4 : D; }
 
 // A row's fields, as the records take them.
 template <int D> struct PackRow {
@@ -181,6 +184,15 @@ __device__ __forceinline__ void packRow(int64_t k, int64_t i, const PackRow<D>& 
   r[R::PRHO] = som * w.P / (w.rho * w.rho);
   r[R::MOR] = w.m / w.rho;
   storeRecords<D, ISO, SEC>(k, r, o);
+  if (o.vel) {
+    double* p = o.vel + k * velStride(D);
+    if constexpr (D == 1) {
+      p[0] = w.v.c[0];
+    } else {
+      reinterpret_cast<double2*>(p)[0] = make_double2(w.v.c[0], w.v.c[1]);
+      if constexpr (D == 3) reinterpret_cast<double2*>(p)[1] = make_double2(w.v.c[2], 0.0);
+    }
+  }
 }
 
 // The same from the fields in memory; a dead slot (culled ghost, in no row)
