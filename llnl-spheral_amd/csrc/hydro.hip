@@ -29,6 +29,7 @@
 #include "pack.hh"
 #include "ell.hh"
 #include "eigen.hh"
+#include "lanes.hh"
 #include <cstring>
 #include <cmath>
 
@@ -238,7 +239,8 @@ __device__ __forceinline__ DNbr<D, true> loadDensRec(const double* __restrict__ 
 
 // Neighbours come from nrec: the density records (DensRec) for isotropic H, else
 // the full records.
-template <int D, bool ISO, bool LDS>
+// L > 1: L lanes to a node, the table through L1.
+template <int D, bool ISO, bool LDS, int L = 1>
 __global__ void __launch_bounds__(kBlock) k_sum_density(double* __restrict__ rec, const int32_t* __restrict__ rowCount,
                                                         const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
                                                         const int32_t* __restrict__ work, TabArgs t,
@@ -247,40 +249,58 @@ __global__ void __launch_bounds__(kBlock) k_sum_density(double* __restrict__ rec
   using R = RL<ISO>;
   extern __shared__ double lds[];
   const double* tab = stageTable<LDS>(lds, t);
-  const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+  const int64_t tw = (xcdBlock((nInt * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
   if (tw >= nInt) return;
   const int64_t k = work[tw];
   double* ri_ = rec + k * R::STRIDE;
   const double oi = ri_[R::ORIG];
-  if (oi >= double(nInt)) return;
   const DNbr<D, ISO> me = loadDNbr<D, ISO>(rec, int32_t(k));
   const double mi = me.m;
   const double self = mi * lookupW(tab, t, 0.0, me.hdet);
   double acc = 0.0;
   bool selfDone = false;
   const int len = rowCount[k];
-  const int4* nb4 = reinterpret_cast<const int4*>(nbr);
-  int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
-  int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
-  DNbr<D, ISO> nx;
   auto load = [&](int32_t j) {
     if constexpr (ISO) return loadDensRec<D>(nrec, j);
     else return loadDNbr<D, false>(nrec, j);
   };
-  if (len > 0) nx = load(cur.x);
-  for (int w = 0; w < len; ++w) {
-    const DNbr<D, ISO> nb = nx;
-    if (w + 1 < len) nx = load(nextIndex(nb4, n, k, len, w + 1, cur, nxt));
-    if (!selfDone && nb.orig > oi) { acc += self; selfDone = true; }
+  auto term = [&](const DNbr<D, ISO>& nb) {
     // several NodeLists: a pair across them counts with sumAll only, the node
     // taking its own mass (computeSPHSumMassDensity.cc:77-100)
     const bool same = !listOf || listOf[int64_t(nb.orig)] == listOf[int64_t(oi)];
-    if (!same && !sumAll) continue;
+    if (!same && !sumAll) return -0.0;
     const V<D> rij = vsub(me.x, nb.x);
     const double etaj = vmag(hdot<D, ISO>(nb.H, rij));
-    acc += (same ? nb.m : mi) * lookupW(tab, t, etaj, nb.hdet);
+    return (same ? nb.m : mi) * lookupW(tab, t, etaj, nb.hdet);
+  };
+  if constexpr (L > 1) {
+    alignas(16) __shared__ double buf[kBlock];
+    double* wbuf = buf + (threadIdx.x & ~63);
+    const int sub = threadIdx.x % L;
+    for (int w0 = 0; w0 < len; w0 += L) {
+      const bool live = w0 + sub < len;
+      const DNbr<D, ISO> nb = load(live ? nbr[ellIndex(w0 + sub, n, k)] : int32_t(k));
+      const int first = firstLane<L>(live && nb.orig > oi);
+      const double tm = term(nb);
+      acc = addInOrder<L>(acc, live ? tm : -0.0, wbuf, selfDone ? 64 : first, self);
+      selfDone = selfDone || first < L;
+    }
+    if (!selfDone) acc += self;
+    if (sub != 0) return;
+  } else {
+    const int4* nb4 = reinterpret_cast<const int4*>(nbr);
+    int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
+    int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
+    DNbr<D, ISO> nx;
+    if (len > 0) nx = load(cur.x);
+    for (int w = 0; w < len; ++w) {
+      const DNbr<D, ISO> nb = nx;
+      if (w + 1 < len) nx = load(nextIndex(nb4, n, k, len, w + 1, cur, nxt));
+      if (!selfDone && nb.orig > oi) { acc += self; selfDone = true; }
+      acc += term(nb);
+    }
+    if (!selfDone) acc += self;
   }
-  if (!selfDone) acc += self;
   rhoOut[int64_t(oi)] = acc;
   // keep the record consistent with the new density (the pass reads only
   // positions, H and masses of the neighbours)
@@ -301,39 +321,61 @@ __global__ void __launch_bounds__(kBlock) k_sum_density(double* __restrict__ rec
 // lower index first, then i's own pairs), and the owner of a pair is still its
 // end of lower caller index, so the self term goes to the same place.
 // ---------------------------------------------------------------------------
-template <int D, bool ISO, bool LDS>
+template <int D, bool ISO, bool LDS, int L = 1>
 __global__ void __launch_bounds__(kBlock) k_omega(const double* __restrict__ rec, const int32_t* __restrict__ rowCount,
                                                   const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
                                                   const int32_t* __restrict__ work, TabArgs t,
                                                   double* __restrict__ omegaOut) {
   extern __shared__ double lds[];
   const double* tab = stageTable<LDS>(lds, t);
-  const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+  const int64_t tw = (xcdBlock((nInt * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
   if (tw >= nInt) return;
   const int64_t k = work[tw];
   const DNbr<D, ISO> me = loadDNbr<D, ISO>(rec, int32_t(k));
   const int len = rowCount[k];
-  if (len == 0) {
-    omegaOut[int64_t(me.orig)] = 1.0;
-    return;
-  }
   const double self = lookupW(tab, t, 0.0, me.hdet);
   double om = 0.0, gs = 0.0;
   bool selfDone = false;
-  const int4* nb4 = reinterpret_cast<const int4*>(nbr);
-  int4 cur = nb4[ellChunk(0, n, k)];
-  int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
-  DNbr<D, ISO> nx = loadDNbr<D, ISO>(rec, cur.x);
-  for (int w = 0; w < len; ++w) {
-    const DNbr<D, ISO> nb = nx;
-    if (w + 1 < len) nx = loadDNbr<D, ISO>(rec, nextIndex(nb4, n, k, len, w + 1, cur, nxt));
-    if (!selfDone && nb.orig > me.orig) { om += self; selfDone = true; }
+  auto terms = [&](const DNbr<D, ISO>& nb, double& Wv, double& eg) {
     const V<D> rij = vsub(me.x, nb.x);
     const double eta = vmag(hdot<D, ISO>(me.H, rij));
-    double Wv, gW;
+    double gW;
     lookupWG(tab, t, eta, me.hdet, Wv, gW);
-    om += Wv;
-    gs += eta * gW;
+    eg = eta * gW;
+  };
+  if constexpr (L > 1) {
+    alignas(16) __shared__ double buf[kBlock];
+    double* wbuf = buf + (threadIdx.x & ~63);
+    const int sub = threadIdx.x % L;
+    for (int w0 = 0; w0 < len; w0 += L) {
+      const bool live = w0 + sub < len;
+      const DNbr<D, ISO> nb = loadDNbr<D, ISO>(rec, live ? nbr[ellIndex(w0 + sub, n, k)] : int32_t(k));
+      const int first = firstLane<L>(live && nb.orig > me.orig);
+      double Wv, eg;
+      terms(nb, Wv, eg);
+      om = addInOrder<L>(om, live ? Wv : -0.0, wbuf, selfDone ? 64 : first, self);
+      gs = addInOrder<L>(gs, live ? eg : -0.0, wbuf);
+      selfDone = selfDone || first < L;
+    }
+    if (sub != 0) return;
+  } else if (len > 0) {
+    const int4* nb4 = reinterpret_cast<const int4*>(nbr);
+    int4 cur = nb4[ellChunk(0, n, k)];
+    int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
+    DNbr<D, ISO> nx = loadDNbr<D, ISO>(rec, cur.x);
+    for (int w = 0; w < len; ++w) {
+      const DNbr<D, ISO> nb = nx;
+      if (w + 1 < len) nx = loadDNbr<D, ISO>(rec, nextIndex(nb4, n, k, len, w + 1, cur, nxt));
+      if (!selfDone && nb.orig > me.orig) { om += self; selfDone = true; }
+      double Wv, eg;
+      terms(nb, Wv, eg);
+      om += Wv;
+      gs += eg;
+    }
+  }
+  if (len == 0) {
+    omegaOut[int64_t(me.orig)] = 1.0;
+    return;
   }
   if (!selfDone) om += self;
   omegaOut[int64_t(me.orig)] = -gs / (double(D) * om);
@@ -497,126 +539,119 @@ __device__ __forceinline__ void storePairCount(unsigned pairs, int64_t nInt, uin
   if (__lane_id() == 0 && wave * 64 < nInt) counts[wave] = pairs;
 }
 
-template <int D, bool ISO, bool TENSILE>
-__device__ __forceinline__ unsigned derivsNodeFP64(int64_t k, const double* __restrict__ rec,
-                                                   const int32_t* __restrict__ rowCount, const int32_t* __restrict__ nbr,
-                                                   int64_t n, const double* __restrict__ tab, const TabArgs& t,
-                                                   const PassArgs& p, const OutArgs& o) {
-  const Nbr<D, ISO> me = loadNbr<D, ISO, true>(rec, int32_t(k));
-  const V<D> ri = me.x, vi = me.v;
-  const S<D> Hi = me.H;
-  const double oi = me.orig;
-  const double Hdeti = me.hdet, mi = me.m, rhoi = me.rho, ci = me.cs, Pi = me.p;
-  const double somi = me.som, Prhoi0 = me.prho, mori = me.mor;
+// The sums of the pair loop by number, in the order pairTerms adds to them.
+template <int D> struct Sum {
+  static constexpr int NS = NSym<D>::value;
+  static constexpr int WNS = 0, M2 = 1, RHO = M2 + NS, NORM = RHO + 1, EFFVP = NORM + 1, VISCW = EFFVP + 1,
+                       DV = VISCW + 1, DEPS = DV + D, DVDX = DEPS + 1, M = DVDX + D * D, XW = M + D * D, XDV = XW + 1,
+                       COUNT = XDV + D;
+};
+template <int D> __device__ __forceinline__ Acc<D> accOf(const double* a) {
+  using S_ = Sum<D>;
+  Acc<D> o;
+  o.wNS = a[S_::WNS]; o.rhoSum = a[S_::RHO]; o.norm = a[S_::NORM]; o.effVP = a[S_::EFFVP]; o.viscW = a[S_::VISCW];
+  o.DepsDt = a[S_::DEPS]; o.xsphW = a[S_::XW];
+  for (int c = 0; c < D; ++c) { o.DvDt.c[c] = a[S_::DV + c]; o.xsphDV.c[c] = a[S_::XDV + c]; }
+  for (int c = 0; c < D * D; ++c) { o.DvDx.c[c] = a[S_::DVDX + c]; o.M.c[c] = a[S_::M + c]; }
+  for (int c = 0; c < NSym<D>::value; ++c) o.m2nd.c[c] = a[S_::M2 + c];
+  return o;
+}
 
-  double rhoSum = 0.0, norm = 0.0, DepsDt = 0.0, maxVP = 0.0, effVP = 0.0, viscW = 0.0, xsphW = 0.0, wNS = 0.0;
-  V<D> DvDt = vzero<D>(), xsphDV = vzero<D>();
-  T<D> DvDx = tzero<D>(), M = tzero<D>();
-  S<D> m2nd = szero<D>();
-  unsigned pairs = 0;
-  double relV = 0.0;
+// One pair in node i's frame, with the reference's operations: every term goes
+// to add(sum, term), sums in ascending number.  Returns 1 for a pair i owns.
+template <int D, bool ISO, bool TENSILE, class Add>
+__device__ __forceinline__ unsigned pairTerms(const Nbr<D, ISO>& me, const Nbr<D, ISO>& nb, int w, int64_t n, int64_t k,
+                                              const double* __restrict__ tab, const TabArgs& t, const PassArgs& p,
+                                              const OutArgs& o, double& maxVP, double& relV, Add&& add) {
+  using S_ = Sum<D>;
+  const double Hdeti = me.hdet, rhoi = me.rho, ci = me.cs, mori = me.mor;
+  const bool ownerI = nb.orig > me.orig;
+  const V<D> rij = vsub(me.x, nb.x);
+  const V<D> vij = vsub(me.v, nb.v);
+  if (o.relV) relV = dmax(relV, relSpeed<D>(vij.c));
+  const S<D>& Hi = me.H;
+  const S<D>& Hj = nb.H;
+  const double Hdetj = nb.hdet, mj = nb.m, rhoj = nb.rho, cj = nb.cs, morj = nb.mor;
 
-  const int len = rowCount[k];
-  const int4* nb4 = reinterpret_cast<const int4*>(nbr);
-  int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
-  int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
-  Nbr<D, ISO> nx;
-  if (len > 0) nx = loadNbr<D, ISO, TENSILE>(rec, cur.x);
-  for (int w = 0; w < len; ++w) {
-    const Nbr<D, ISO> nb = nx;
-    if (w + 1 < len) nx = loadNbr<D, ISO, TENSILE>(rec, nextIndex(nb4, n, k, len, w + 1, cur, nxt));
-    const bool ownerI = nb.orig > oi;
-    pairs += ownerI ? 1u : 0u;
-    const V<D> rij = vsub(ri, nb.x);
-    const V<D> vij = vsub(vi, nb.v);
-    if (o.relV) relV = dmax(relV, relSpeed<D>(vij.c));
-    const S<D>& Hj = nb.H;
-    const double Hdetj = nb.hdet, mj = nb.m, rhoj = nb.rho, cj = nb.cs, morj = nb.mor;
+  const V<D> etai = hdot<D, ISO>(Hi, rij), etaj = hdot<D, ISO>(Hj, rij);
+  const double eta2i = vmag2(etai), eta2j = vmag2(etaj);
+  const double etaMagi = (D == 1) ? fabs(etai.c[0]) : __builtin_sqrt(eta2i);
+  const double etaMagj = (D == 1) ? fabs(etaj.c[0]) : __builtin_sqrt(eta2j);
+  const V<D> Hetai = hdot<D, ISO>(Hi, vunit(etai, etaMagi));
+  const V<D> Hetaj = hdot<D, ISO>(Hj, vunit(etaj, etaMagj));
+  double Wi, gWi, Wj, gWj;
+  lookupWG(tab, t, etaMagi, Hdeti, Wi, gWi);
+  lookupWG(tab, t, etaMagj, Hdetj, Wj, gWj);
+  const V<D> gradWi = vscale(Hetai, gWi);
+  const V<D> gradWj = vscale(Hetaj, gWj);
 
-    const V<D> etai = hdot<D, ISO>(Hi, rij), etaj = hdot<D, ISO>(Hj, rij);
-    const double eta2i = vmag2(etai), eta2j = vmag2(etaj);
-    const double etaMagi = (D == 1) ? fabs(etai.c[0]) : __builtin_sqrt(eta2i);
-    const double etaMagj = (D == 1) ? fabs(etaj.c[0]) : __builtin_sqrt(eta2j);
-    const V<D> Hetai = hdot<D, ISO>(Hi, vunit(etai, etaMagi));
-    const V<D> Hetaj = hdot<D, ISO>(Hj, vunit(etaj, etaMagj));
-    double Wi, gWi, Wj, gWj;
-    lookupWG(tab, t, etaMagi, Hdeti, Wi, gWi);
-    lookupWG(tab, t, etaMagj, Hdetj, Wj, gWj);
-    const V<D> gradWi = vscale(Hetai, gWi);
-    const V<D> gradWj = vscale(Hetaj, gWj);
-
-    // moments for the ideal H (SPHHydroBase.cc:737-743)
-    const double rij2 = vmag2(rij);
-    const double sinv = safeInvVar(rij2 * rij2 * rij2);
-    const double g2 = vmag2(gradWi);
-    wNS += fabs(gWi);
-    {
-      int s = 0;
-      for (int a = 0; a < D; ++a)
-        for (int b = a; b < D; ++b, ++s) m2nd.c[s] += (rij.c[a] * rij.c[b]) * sinv * g2;
-    }
-    if (!p.listOf || p.listOf[int64_t(nb.orig)] == p.listOf[int64_t(oi)]) {   // SPHHydroBase.cc:746-751
-      rhoSum += mj * Wi;
-      norm += mori * Wi;
-    }
-
-    // Monaghan-Gingold Q (MonaghanGingoldViscosity.cc:83-132)
-    double Cl = p.Cl, Cq = p.Cq;
-    if constexpr (!ISO) {
-      const double fsh = dmax(me.fsh, nb.fsh);
-      Cl *= 0.5 * (me.fcl + nb.fcl) * fsh;
-      Cq *= 0.5 * (me.fcq + nb.fcq) * fsh;
-    }
-    const double mui = vdot(vij, etai) / (eta2i + p.eps2);
-    const double muj = vdot(vij, etaj) / (eta2j + p.eps2);
-    const double QPi = muQ(mui, Cl, Cq, ci, p) / rhoi;
-    const double QPj = muQ(muj, Cl, Cq, cj, p) / rhoj;
-    V<D> Qacci, Qaccj;
-    for (int c = 0; c < D; ++c) { Qacci.c[c] = 0.5 * (QPi * gradWi.c[c]); Qaccj.c[c] = 0.5 * (QPj * gradWj.c[c]); }
-    const double workQi = vdot(vij, Qacci);
-    const double Qi = rhoi * rhoi * fabs(QPi);
-    maxVP = dmax(maxVP, Qi);
-    effVP += morj * Qi * Wi;
-    viscW += mj * workQi;
-
-    double Prhoi = Prhoi0, Prhoj = nb.prho;
-    if constexpr (TENSILE) {
-      const double Wo = ownerI ? Wi : Wj, Hdeto = ownerI ? Hdeti : Hdetj;
-      const double x = Wo / (Hdeto * p.WnPerh);
-      const double fij = p.epsTensile * (x * x * x * x);
-      const double Pj = nb.p;
-      Prhoi = somi * (Pi + fij * (Pi < 0.0 ? -Pi : 0.0)) / (rhoi * rhoi);
-      Prhoj = nb.som * (Pj + fij * (Pj < 0.0 ? -Pj : 0.0)) / (rhoj * rhoj);
-    }
-    for (int c = 0; c < D; ++c) {
-      const double qf = ownerI ? Qacci.c[c] : Qaccj.c[c];
-      const double qs = ownerI ? Qaccj.c[c] : Qacci.c[c];
-      const double dv = gradWi.c[c] * Prhoi + gradWj.c[c] * Prhoj + qf + qs;
-      DvDt.c[c] += dv * (-mj);
-      if (o.pairDv) o.pairDv[int64_t(c) * o.plane + ellIndex(w, n, k)] = dv;
-    }
-    DepsDt += mj * (Prhoi * vdot(vij, gradWi) + workQi);
+  // moments for the ideal H (SPHHydroBase.cc:737-743)
+  const double rij2 = vmag2(rij);
+  const double sinv = safeInvVar(rij2 * rij2 * rij2);
+  const double g2 = vmag2(gradWi);
+  add(S_::WNS, fabs(gWi));
+  {
+    int s = 0;
     for (int a = 0; a < D; ++a)
-      for (int b = 0; b < D; ++b) {
-        DvDx.c[a * D + b] -= (vij.c[a] * gradWi.c[b]) * mj;
-        M.c[a * D + b] -= (rij.c[a] * gradWi.c[b]) * mj;
-      }
-    if (p.XSPH) {
-      const double w2 = 0.5 * (mori * Wi + morj * Wj);
-      xsphW += w2;
-      for (int c = 0; c < D; ++c) xsphDV.c[c] -= vij.c[c] * w2;
-    }
+      for (int b = a; b < D; ++b, ++s) add(S_::M2 + s, (rij.c[a] * rij.c[b]) * sinv * g2);
   }
+  // same-NodeList pairs only (SPHHydroBase.cc:746-751); adding -0 changes no sum
+  const bool same = !p.listOf || p.listOf[int64_t(nb.orig)] == p.listOf[int64_t(me.orig)];
+  add(S_::RHO, same ? mj * Wi : -0.0);
+  add(S_::NORM, same ? mori * Wi : -0.0);
 
-  if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
-  // per-node epilogue (SPHHydroBase.cc:834-902)
-  Acc<D> a;
-  a.rhoSum = rhoSum; a.norm = norm; a.DepsDt = DepsDt; a.maxVP = maxVP; a.effVP = effVP; a.viscW = viscW;
-  a.xsphW = xsphW; a.wNS = wNS; a.DvDt = DvDt; a.xsphDV = xsphDV; a.DvDx = DvDx; a.M = M; a.m2nd = m2nd;
-  Self<D> self;
-  self.v = vi; self.H = Hi; self.Hdet = Hdeti; self.m = mi; self.rho = rhoi; self.mor = mori;
-  epilogue<D>(k, len, self, a, t, p, o);
-  return pairs;
+  // Monaghan-Gingold Q (MonaghanGingoldViscosity.cc:83-132)
+  double Cl = p.Cl, Cq = p.Cq;
+  if constexpr (!ISO) {
+    const double fsh = dmax(me.fsh, nb.fsh);
+    Cl *= 0.5 * (me.fcl + nb.fcl) * fsh;
+    Cq *= 0.5 * (me.fcq + nb.fcq) * fsh;
+  }
+  const double mui = vdot(vij, etai) / (eta2i + p.eps2);
+  const double muj = vdot(vij, etaj) / (eta2j + p.eps2);
+  const double QPi = muQ(mui, Cl, Cq, ci, p) / rhoi;
+  const double QPj = muQ(muj, Cl, Cq, cj, p) / rhoj;
+  V<D> Qacci, Qaccj;
+  for (int c = 0; c < D; ++c) { Qacci.c[c] = 0.5 * (QPi * gradWi.c[c]); Qaccj.c[c] = 0.5 * (QPj * gradWj.c[c]); }
+  const double workQi = vdot(vij, Qacci);
+  const double Qi = rhoi * rhoi * fabs(QPi);
+  maxVP = dmax(maxVP, Qi);
+  add(S_::EFFVP, morj * Qi * Wi);
+  add(S_::VISCW, mj * workQi);
+
+  double Prhoi = me.prho, Prhoj = nb.prho;
+  if constexpr (TENSILE) {
+    const double Wo = ownerI ? Wi : Wj, Hdeto = ownerI ? Hdeti : Hdetj;
+    const double x = Wo / (Hdeto * p.WnPerh);
+    const double fij = p.epsTensile * (x * x * x * x);
+    const double Pi = me.p, Pj = nb.p;
+    Prhoi = me.som * (Pi + fij * (Pi < 0.0 ? -Pi : 0.0)) / (rhoi * rhoi);
+    Prhoj = nb.som * (Pj + fij * (Pj < 0.0 ? -Pj : 0.0)) / (rhoj * rhoj);
+  }
+  for (int c = 0; c < D; ++c) {
+    const double qf = ownerI ? Qacci.c[c] : Qaccj.c[c];
+    const double qs = ownerI ? Qaccj.c[c] : Qacci.c[c];
+    const double dv = gradWi.c[c] * Prhoi + gradWj.c[c] * Prhoj + qf + qs;
+    add(S_::DV + c, dv * (-mj));
+    if (o.pairDv) o.pairDv[int64_t(c) * o.plane + ellIndex(w, n, k)] = dv;
+  }
+  add(S_::DEPS, mj * (Prhoi * vdot(vij, gradWi) + workQi));
+  // a difference is the sum with the term's negative, to the bit
+  for (int a = 0; a < D; ++a)
+    for (int b = 0; b < D; ++b) add(S_::DVDX + a * D + b, -((vij.c[a] * gradWi.c[b]) * mj));
+  for (int a = 0; a < D; ++a)
+    for (int b = 0; b < D; ++b) add(S_::M + a * D + b, -((rij.c[a] * gradWi.c[b]) * mj));
+  const double w2 = 0.5 * (mori * Wi + morj * Wj);
+  add(S_::XW, p.XSPH ? w2 : -0.0);
+  for (int c = 0; c < D; ++c) add(S_::XDV + c, p.XSPH ? -(vij.c[c] * w2) : -0.0);
+  return ownerI ? 1u : 0u;
+}
+
+template <int D, bool ISO>
+__device__ __forceinline__ Self<D> selfOf(const Nbr<D, ISO>& me) {
+  Self<D> s;
+  s.v = me.v; s.H = me.H; s.Hdet = me.hdet; s.m = me.m; s.rho = me.rho; s.mor = me.mor;
+  return s;
 }
 
 template <int D, bool ISO, bool TENSILE, bool LDS>
@@ -628,8 +663,112 @@ __global__ void __launch_bounds__(kBlock) k_derivs_fp64(const double* __restrict
   const double* tab = stageTable<LDS>(lds, t);
   const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
   unsigned pairs = 0;
-  if (tw < nInt) pairs = derivsNodeFP64<D, ISO, TENSILE>(work[tw], rec, rowCount, nbr, n, tab, t, p, o);
+  if (tw < nInt) {
+    const int64_t k = work[tw];
+    const Nbr<D, ISO> me = loadNbr<D, ISO, true>(rec, int32_t(k));
+    double sum[Sum<D>::COUNT];
+#pragma unroll
+    for (int q = 0; q < Sum<D>::COUNT; ++q) sum[q] = 0.0;
+    double maxVP = 0.0, relV = 0.0;
+    const int len = rowCount[k];
+    const int4* nb4 = reinterpret_cast<const int4*>(nbr);
+    int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
+    int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
+    Nbr<D, ISO> nx;
+    if (len > 0) nx = loadNbr<D, ISO, TENSILE>(rec, cur.x);
+    for (int w = 0; w < len; ++w) {
+      const Nbr<D, ISO> nb = nx;
+      if (w + 1 < len) nx = loadNbr<D, ISO, TENSILE>(rec, nextIndex(nb4, n, k, len, w + 1, cur, nxt));
+      pairs += pairTerms<D, ISO, TENSILE>(me, nb, w, n, k, tab, t, p, o, maxVP, relV,
+                                          [&](int q, double v) { sum[q] += v; });
+    }
+    if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
+    Acc<D> a = accOf<D>(sum);
+    a.maxVP = maxVP;
+    epilogue<D>(k, len, selfOf(me), a, t, p, o);
+  }
   storePairCount<kBlock>(pairs, nInt, pairCounts);
+}
+
+// The same pass with L lanes to a node: the terms of L sums at a time go through
+// LDS, and each lane adds up one of them, entry by entry (one read and one add
+// per sum and L entries, where sums kept by every lane would take L adds each).
+// A lane holds COUNT / L sums instead of COUNT.  LDS rows are padded to 65
+// doubles: lane q reads row q, so rows a multiple of 64 apart would all hit the
+// same banks.
+template <int D, bool ISO, bool TENSILE, int L>
+__global__ void __launch_bounds__(kBlock) k_derivs_rows(const double* __restrict__ rec,
+                                                        const int32_t* __restrict__ rowCount,
+                                                        const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
+                                                        const int32_t* __restrict__ work, TabArgs t, PassArgs p,
+                                                        OutArgs o, uint32_t* __restrict__ pairCounts) {
+  constexpr int COUNT = Sum<D>::COUNT, BATCH = (COUNT + L - 1) / L, NODES = kBlock / L, PAD = 65;
+  __shared__ double terms[kBlock / 64][L][PAD];
+  __shared__ double sums[NODES][BATCH * L + 2];
+  const int64_t block = xcdBlock((nInt * L + kBlock - 1) / kBlock);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = threadIdx.x % L;
+  const int64_t tw = block * NODES + threadIdx.x / L;
+  unsigned pairs = 0;
+  double maxVP = 0.0, relV = 0.0, acc[BATCH];
+#pragma unroll
+  for (int q = 0; q < BATCH; ++q) acc[q] = 0.0;
+  const int64_t k = tw < nInt ? work[tw] : 0;
+  const int len = tw < nInt ? rowCount[k] : 0;
+  const Nbr<D, ISO> me = loadNbr<D, ISO, true>(rec, int32_t(k));
+  for (int w0 = 0; w0 < len; w0 += L) {
+    const int w = w0 + sub;
+    const bool live = w < len;
+    // a lane past its row evaluates the node's pair with itself, unused
+    const int32_t j = live ? nbr[ellIndex(w, n, k)] : int32_t(k);
+    const Nbr<D, ISO> nb = loadNbr<D, ISO, TENSILE>(rec, j);
+    OutArgs oo = o;
+    if (!live) oo.pairDv = nullptr;
+    double vp = maxVP, rv = relV;
+    const unsigned own = pairTerms<D, ISO, TENSILE>(
+        me, nb, w, n, k, t.g, t, p, oo, vp, rv, [&](int q, double v) {
+          terms[wave][q % L][lane] = live ? v : -0.0;
+          if (q % L == L - 1 || q == COUNT - 1) {
+            waveLdsOrder();
+            double a = acc[q / L];
+#pragma unroll
+            for (int e = 0; e < L; ++e) a += terms[wave][sub][lane - sub + e];
+            acc[q / L] = a;
+            waveLdsOrder();
+          }
+        });
+    if (live) {
+      maxVP = vp;
+      relV = rv;
+      pairs += own;
+    }
+  }
+  for (int s = L / 2; s > 0; s >>= 1) {
+    maxVP = dmax(maxVP, __shfl_xor(maxVP, s));
+    relV = dmax(relV, __shfl_xor(relV, s));
+  }
+  double* mine = sums[threadIdx.x / L];
+#pragma unroll
+  for (int q = 0; q < BATCH; ++q) mine[q * L + sub] = acc[q];
+  if (sub == 0) {
+    mine[BATCH * L] = maxVP;
+    mine[BATCH * L + 1] = relV;
+  }
+  __syncthreads();
+  // the epilogue, one lane to a node again
+  const int64_t te = block * NODES + threadIdx.x;
+  if (threadIdx.x < NODES && te < nInt) {
+    const int64_t ke = work[te];
+    const int le = rowCount[ke];
+    const double* a = sums[threadIdx.x];
+    double sum[COUNT];
+#pragma unroll
+    for (int q = 0; q < COUNT; ++q) sum[q] = a[q];
+    Acc<D> ac = accOf<D>(sum);
+    ac.maxVP = a[BATCH * L];
+    if (o.relV) o.relV[ke] = le > 0 ? a[BATCH * L + 1] : -1.0;
+    epilogue<D>(ke, le, selfOf(loadNbr<D, ISO, true>(rec, int32_t(ke))), ac, t, p, o);
+  }
+  storePairCount<kBlock>(pairs, nInt * L, pairCounts);
 }
 
 // ---------------------------------------------------------------------------
@@ -816,7 +955,7 @@ __device__ __forceinline__ Real muQR(Real mu, Real Cl, Real Cq, Real cs, int lin
   return -Cl * cs * lin + Cq * quad;
 }
 
-template <int D, bool LDS>
+template <int D, bool LDS, int L = 1>
 __global__ void __launch_bounds__(kBlock) k_sum_density_mixed(double* __restrict__ rec, const float4* __restrict__ recSM,
                                                               const int32_t* __restrict__ rowCount,
                                                               const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
@@ -826,7 +965,7 @@ __global__ void __launch_bounds__(kBlock) k_sum_density_mixed(double* __restrict
   using R = RL<true>;
   extern __shared__ float lds32[];
   const float* tab = stageTable32<LDS>(lds32, t);
-  const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+  const int64_t tw = (xcdBlock((nInt * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
   if (tw >= nInt) return;
   const int64_t k = work[tw];
   double* ri_ = rec + k * R::STRIDE;
@@ -834,9 +973,6 @@ __global__ void __launch_bounds__(kBlock) k_sum_density_mixed(double* __restrict
   const double mi = ri_[R::M], hdeti = ri_[R::HDET];
   double acc = mi * (W0 * hdeti);
   const int len = rowCount[k];
-  const int4* nb4 = reinterpret_cast<const int4*>(nbr);
-  int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
-  int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
   // the mixed density record: x (FP64 bits), 1/h, m
   auto load = [&](int32_t j, float4& a, float4& b) {
     const float4* p = recSM + int64_t(j) * DensMixedRec<D>::F4;
@@ -848,19 +984,10 @@ __global__ void __launch_bounds__(kBlock) k_sum_density_mixed(double* __restrict
   // node taking its own mass (computeSPHSumMassDensity.cc:77-100)
   const int32_t lk = slotList ? slotList[k] : 0;
   const float mif = float(mi);
-  float4 na, nb2;
-  int32_t jn = cur.x;
-  if (len > 0) load(jn, na, nb2);
-  for (int w = 0; w < len; ++w) {
-    const float4 a = na, b = nb2;
-    const int32_t j = jn;
-    if (w + 1 < len) {
-      jn = nextIndex(nb4, n, k, len, w + 1, cur, nxt);
-      load(jn, na, nb2);
-    }
+  auto term = [&](const float4 a, const float4 b, int32_t j) {
     float mj = b.w;
     if (slotList && slotList[j] != lk) {
-      if (!sumAll) continue;
+      if (!sumAll) return -0.0;
       mj = mif;
     }
     const double xj[3] = {__hiloint2double(__float_as_int(a.y), __float_as_int(a.x)),
@@ -874,7 +1001,37 @@ __global__ void __launch_bounds__(kBlock) k_sum_density_mixed(double* __restrict
     const float hj = b.z;
     const float hdetj = D == 1 ? hj : (D == 2 ? hj * hj : hj * hj * hj);
     const float eta = hj * __builtin_sqrtf(r2);
-    acc += double(mj * lookupW32(tab, t32, eta, hdetj));
+    return double(mj * lookupW32(tab, t32, eta, hdetj));
+  };
+  if constexpr (L > 1) {
+    alignas(16) __shared__ double buf[kBlock];
+    double* wbuf = buf + (threadIdx.x & ~63);
+    const int sub = threadIdx.x % L;
+    for (int w0 = 0; w0 < len; w0 += L) {
+      const bool live = w0 + sub < len;
+      const int32_t j = live ? nbr[ellIndex(w0 + sub, n, k)] : int32_t(k);
+      float4 a, b;
+      load(j, a, b);
+      const double tm = term(a, b, j);
+      acc = addInOrder<L>(acc, live ? tm : -0.0, wbuf);
+    }
+    if (sub != 0) return;
+  } else {
+    const int4* nb4 = reinterpret_cast<const int4*>(nbr);
+    int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
+    int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
+    float4 na, nb2;
+    int32_t jn = cur.x;
+    if (len > 0) load(jn, na, nb2);
+    for (int w = 0; w < len; ++w) {
+      const float4 a = na, b = nb2;
+      const int32_t j = jn;
+      if (w + 1 < len) {
+        jn = nextIndex(nb4, n, k, len, w + 1, cur, nxt);
+        load(jn, na, nb2);
+      }
+      acc += term(a, b, j);
+    }
   }
   rhoOut[int64_t(ri_[R::ORIG])] = acc;
   const double som = ri_[R::SOM], p = ri_[R::P];
@@ -916,30 +1073,151 @@ template <int D> struct SumsF {
     DepsDt = viscW = effVP = rhoSum = norm = wNS = xsphW = 0.0f;
   }
   // add into the FP64 accumulators (M and m2nd as upper triangles) and restart
-  __device__ __forceinline__ void flushInto(Acc<D>& a) {
+  template <class Add> __device__ __forceinline__ void flushInto(Acc<D>& a, Add&& add) {
+    auto to = [&](double& s, float v) { s = add(s, double(v)); };
     for (int c = 0; c < D; ++c) {
-      a.DvDt.c[c] += double(DvDt[c]);
-      a.xsphDV.c[c] += double(xsphDV[c]);
+      to(a.DvDt.c[c], DvDt[c]);
+      to(a.xsphDV.c[c], xsphDV[c]);
     }
-    for (int c = 0; c < D * D; ++c) a.DvDx.c[c] += double(DvDx[c]);
+    for (int c = 0; c < D * D; ++c) to(a.DvDx.c[c], DvDx[c]);
     int s2 = 0;
     for (int c = 0; c < D; ++c)
       for (int b = c; b < D; ++b, ++s2) {
-        a.M.c[c * D + b] += double(M[s2]);
-        a.m2nd.c[s2] += double(m2nd[s2]);
+        to(a.M.c[c * D + b], M[s2]);
+        to(a.m2nd.c[s2], m2nd[s2]);
       }
-    a.DepsDt += double(DepsDt);
-    a.viscW += double(viscW);
-    a.effVP += double(effVP);
-    a.rhoSum += double(rhoSum);
-    a.norm += double(norm);
-    a.wNS += double(wNS);
-    a.xsphW += double(xsphW);
+    to(a.DepsDt, DepsDt);
+    to(a.viscW, viscW);
+    to(a.effVP, effVP);
+    to(a.rhoSum, rhoSum);
+    to(a.norm, norm);
+    to(a.wNS, wNS);
+    to(a.xsphW, xsphW);
     zero();
   }
 };
 
-template <typename Real, int D, bool LDS, bool PREFETCH, int BS = kBlock>
+// The node's own state for the epilogue, read again after the loop so that it
+// holds no registers during it.
+template <int D>
+__device__ __forceinline__ void isoEpilogue(int64_t k, int len, const double* __restrict__ ri_, Acc<D>& a,
+                                            const TabArgs& t, const PassArgs& p, const OutArgs& o) {
+  using R = RL<true>;
+  Self<D> me;
+  for (int c = 0; c < D; ++c) me.v.c[c] = ri_[R::V + c];
+  const double hinvD = ri_[RL<true>::HINV];
+  for (int c = 0; c < NSym<D>::value; ++c) me.H.c[c] = 0.0;
+  for (int c = 0; c < D; ++c) me.H.c[sdiag<D>(c)] = hinvD;
+  me.Hdet = ri_[R::HDET]; me.m = ri_[R::M]; me.rho = ri_[R::RHO]; me.mor = ri_[R::MOR];
+  epilogue<D>(k, len, me, a, t, p, o);
+}
+
+// The node's side of a pair.
+template <typename Real, int D> struct IsoNode {
+  double xi[3];
+  uint32_t qi[3];
+  Real vi[3];
+  Real hi, ci, hdeti, invRhoi, rhoi2, Prhoi, mori, Cl, Cq, eps2;
+};
+// the 3-D mixed record holds quantised positions
+template <typename Real, int D> constexpr bool kQPos = std::is_same<Real, float>::value && D == 3;
+template <typename Real, int D>
+__device__ __forceinline__ IsoNode<Real, D> loadIsoNode(const double* __restrict__ ri_, const PassArgs& p) {
+  using R = RL<true>;
+  IsoNode<Real, D> m;
+  for (int c = 0; c < 3; ++c) {
+    m.xi[c] = c < D ? ri_[R::X + c] : 0.0;
+    if constexpr (kQPos<Real, D>) m.qi[c] = quantPos(m.xi[c], p.qInv);
+    m.vi[c] = c < D ? Real(ri_[R::V + c]) : Real(0);
+  }
+  const double rho0 = ri_[R::RHO];
+  m.hi = Real(ri_[RL<true>::HINV]);
+  m.ci = Real(ri_[R::CS]);
+  // det H as a neighbour's record gives it (from the same 1/h), so that the
+  // two ends of a pair evaluate the same kernel gradient and their pair
+  // terms are exact negatives of each other (FP64: the packed det H is
+  // already that value)
+  m.hdeti = std::is_same<Real, float>::value ? (D == 1 ? m.hi : (D == 2 ? m.hi * m.hi : m.hi * m.hi * m.hi))
+                                             : Real(ri_[R::HDET]);
+  m.invRhoi = Real(1.0 / rho0);
+  m.rhoi2 = Real(rho0 * rho0);
+  m.Prhoi = Real(ri_[R::PRHO]);
+  m.mori = Real(ri_[R::MOR]);
+  m.Cl = Real(p.Cl);
+  m.Cq = Real(p.Cq);
+  m.eps2 = Real(p.eps2);
+  return m;
+}
+
+// One neighbour's factors of the sums.
+template <typename Real, int D> struct IsoPair {
+  Real rij[3], vij[3];
+  Real Wi, absG, wg, fsr, f2, mv, pi, halfQi, Qi, morQi, w2, dsc;
+};
+template <typename Real, int D>
+__device__ __forceinline__ IsoPair<Real, D> isoPair(const IsoNode<Real, D>& m, const INbr<Real>& nb,
+                                                    const typename IsoTab<Real>::Elem* __restrict__ tab,
+                                                    const typename IsoTab<Real>::T& tt, const PassArgs& p) {
+  IsoPair<Real, D> o;
+  Real r2 = Real(0), vdotr = Real(0);
+  for (int c = 0; c < D; ++c) {
+    if constexpr (kQPos<Real, D>) o.rij[c] = Real(int32_t(m.qi[c] - nb.q[c])) * p.qUnit;
+    else o.rij[c] = Real(m.xi[c] - nb.x[c]);
+    o.vij[c] = m.vi[c] - nb.v[c];
+    r2 = fmaR(o.rij[c], o.rij[c], r2);
+    vdotr = fmaR(o.vij[c], o.rij[c], vdotr);
+  }
+  const Real hi = m.hi, hj = nb.hinv;
+  const Real rinv = r2 > Real(1.0e-30) ? rsqR(r2) : Real(0);
+  const Real rmag = r2 * rinv;
+  Real Wi, gWi, Wj, gWj;
+  lookupWGR(tab, tt, hi * rmag, m.hdeti, Wi, gWi);
+  lookupWGR(tab, tt, hj * rmag, nb.hdet, Wj, gWj);
+  const Real gi = hi * gWi, gj = hj * gWj;     // grad W = r_hat * g
+  // Monaghan-Gingold Q: mu = v_ij . eta / (eta^2 + eps2), eta = h r_ij
+  // (FP64: one refined reciprocal of the product serves both ends)
+  const Real da = fmaR(hi * hi, r2, m.eps2), db = fmaR(hj * hj, r2, m.eps2);
+  Real ia, ib;
+  if constexpr (std::is_same<Real, double>::value) {
+    const Real inv = rcpR(da * db);
+    ia = db * inv;
+    ib = da * inv;
+  } else {
+    ia = rcpR(da);
+    ib = rcpR(db);
+  }
+  const Real mui = hi * vdotr * ia;
+  const Real muj = hj * vdotr * ib;
+  const Real QPi = muQR(mui, m.Cl, m.Cq, m.ci, p.linearInExpansion, p.quadraticInExpansion) * m.invRhoi;
+  const Real QPj = muQR(muj, m.Cl, m.Cq, nb.cs, p.linearInExpansion, p.quadraticInExpansion) * nb.invRho;
+  o.Qi = m.rhoi2 * absR(QPi);
+  const Real vdr = vdotr * rinv;                 // v_ij . r_hat
+  o.halfQi = Real(0.5) * QPi * gi;
+  o.pi = fmaR(gi, m.Prhoi, o.halfQi);
+  const Real pj = fmaR(gj, nb.prho, Real(0.5) * QPj * gj);
+  const Real mj = nb.m;
+  o.fsr = mj * (o.pi + pj) * rinv;              // acceleration along r_ij
+  o.wg = mj * gi * rinv;                       // grad W_i * m_j = r_ij * wg
+  // gi^2 / max(1e-30, r^6); FP64 takes 1/r^6 from 1/r
+  if constexpr (std::is_same<Real, double>::value) {
+    const Real ri2 = rinv * rinv;
+    o.f2 = r2 * r2 * r2 > Real(1.0e-30) ? gi * gi * (ri2 * ri2 * ri2) : gi * gi * Real(1.0e30);
+  } else {
+    o.f2 = gi * gi * rcpR(maxR(Real(1.0e-30), r2 * r2 * r2));
+  }
+  o.dsc = (o.pi + pj) * rinv;                   // compatible energy: the own-frame pair term along r_ij
+  o.mv = mj * vdr;
+  o.morQi = nb.mor * o.Qi;
+  o.Wi = Wi;
+  o.absG = absR(gWi);
+  o.w2 = Real(0.5) * fmaR(m.mori, Wi, nb.mor * Wj);
+  return o;
+}
+
+// L > 1 (mixed, small node sets): L lanes to a node, each taking whole blocks of
+// kSumBlock entries, and the blocks' FP32 sums enter the FP64 sums in row order:
+// the bits are those of one lane.
+template <typename Real, int D, bool LDS, bool PREFETCH, int BS = kBlock, int L = 1>
 __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ rec,
                                                        const typename IsoTab<Real>::Rec* __restrict__ recN,
                                                        const int32_t* __restrict__ rowCount,
@@ -949,219 +1227,288 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
                                                        uint32_t* __restrict__ pairCounts) {
   using R = RL<true>;
   using E = typename IsoTab<Real>::Elem;
+  constexpr bool F32 = std::is_same<Real, float>::value;
+  static_assert(L == 1 || (F32 && !LDS), "several lanes to a node: mixed, the table through L1");
   extern __shared__ double ldsIso[];
   const E* tab;
   if constexpr (LDS) {
     E* l = reinterpret_cast<E*>(ldsIso);
-    const E* g = std::is_same<Real, float>::value ? reinterpret_cast<const E*>(t.g32) : reinterpret_cast<const E*>(t.g);
+    const E* g = F32 ? reinterpret_cast<const E*>(t.g32) : reinterpret_cast<const E*>(t.g);
     for (int q = threadIdx.x; q < IsoTab<Real>::PER * t.n; q += blockDim.x) l[q] = g[q];
     __syncthreads();
     tab = l;
   } else {
-    tab = std::is_same<Real, float>::value ? reinterpret_cast<const E*>(t.g32) : reinterpret_cast<const E*>(t.g);
+    tab = F32 ? reinterpret_cast<const E*>(t.g32) : reinterpret_cast<const E*>(t.g);
   }
-  const int64_t tw = xcdBlock((nInt + BS - 1) / BS) * BS + threadIdx.x;
+  const int64_t tw = (xcdBlock((nInt * L + BS - 1) / BS) * BS + threadIdx.x) / L;
   unsigned pairs = 0;
-  // the 3-D mixed record holds quantised positions
-  constexpr bool QPOS = std::is_same<Real, float>::value && D == 3;
   if (tw < nInt) {
     const int64_t k = work[tw];
     const int32_t lk = p.slotList ? p.slotList[k] : 0;
     const double* ri_ = rec + k * R::STRIDE;
-    double xi[3];
-    uint32_t qi[3];
-    Real vi[3];
-    for (int c = 0; c < 3; ++c) {
-      xi[c] = c < D ? ri_[R::X + c] : 0.0;
-      if constexpr (QPOS) qi[c] = quantPos(xi[c], p.qInv);
-      vi[c] = c < D ? Real(ri_[R::V + c]) : Real(0);
-    }
-    const double rho0 = ri_[R::RHO];
-    const Real hi = Real(ri_[RL<true>::HINV]), ci = Real(ri_[R::CS]);
-    // det H as a neighbour's record gives it (from the same 1/h), so that the
-    // two ends of a pair evaluate the same kernel gradient and their pair
-    // terms are exact negatives of each other (FP64: the packed det H is
-    // already that value)
-    const Real hdeti = std::is_same<Real, float>::value ? (D == 1 ? hi : (D == 2 ? hi * hi : hi * hi * hi))
-                                                        : Real(ri_[R::HDET]);
-    const Real invRhoi = Real(1.0 / rho0), rhoi2 = Real(rho0 * rho0);
-    const Real Prhoi = Real(ri_[R::PRHO]), mori = Real(ri_[R::MOR]);
-    const Real Cl = Real(p.Cl), Cq = Real(p.Cq), eps2 = Real(p.eps2);
+    const IsoNode<Real, D> me = loadIsoNode<Real, D>(ri_, p);
 
     Acc<D> a;
     a.zero();
-    constexpr bool F32 = std::is_same<Real, float>::value;
     SumsF<F32 ? D : 1> af;
     if constexpr (F32) af.zero();
     Real maxVP = Real(0);
     double relV = 0.0;
     const int len = rowCount[k];
-    const int4* nb4 = reinterpret_cast<const int4*>(nbr);
-    int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
-    int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
     // One neighbour's contribution, in row order (w: its place in the row).
     auto pair = [&](const INbr<Real>& nb, int32_t j, int w) {
       pairs += (nb.ghost || j > int32_t(k)) ? 1u : 0u;
-      Real rij[3], vij[3];
-      Real r2 = Real(0), vdotr = Real(0);
-      for (int c = 0; c < D; ++c) {
-        if constexpr (QPOS) rij[c] = Real(int32_t(qi[c] - nb.q[c])) * p.qUnit;
-        else rij[c] = Real(xi[c] - nb.x[c]);
-        vij[c] = vi[c] - nb.v[c];
-        r2 = fmaR(rij[c], rij[c], r2);
-        vdotr = fmaR(vij[c], rij[c], vdotr);
-      }
+      const IsoPair<Real, D> q = isoPair<Real, D>(me, nb, tab, tt, p);
       if constexpr (!F32) {
-        if (o.relV) relV = dmax(relV, relSpeed<D>(vij));
+        if (o.relV) relV = dmax(relV, relSpeed<D>(q.vij));
       }
-      const Real rinv = r2 > Real(1.0e-30) ? rsqR(r2) : Real(0);
-      const Real rmag = r2 * rinv;
-      const Real hj = nb.hinv;
-      Real Wi, gWi, Wj, gWj;
-      lookupWGR(tab, tt, hi * rmag, hdeti, Wi, gWi);
-      lookupWGR(tab, tt, hj * rmag, nb.hdet, Wj, gWj);
-      const Real gi = hi * gWi, gj = hj * gWj;     // grad W = r_hat * g
-      // Monaghan-Gingold Q: mu = v_ij . eta / (eta^2 + eps2), eta = h r_ij
-      // (FP64: one refined reciprocal of the product serves both ends)
-      const Real da = fmaR(hi * hi, r2, eps2), db = fmaR(hj * hj, r2, eps2);
-      Real ia, ib;
-      if constexpr (std::is_same<Real, double>::value) {
-        const Real inv = rcpR(da * db);
-        ia = db * inv;
-        ib = da * inv;
-      } else {
-        ia = rcpR(da);
-        ib = rcpR(db);
-      }
-      const Real mui = hi * vdotr * ia;
-      const Real muj = hj * vdotr * ib;
-      const Real QPi = muQR(mui, Cl, Cq, ci, p.linearInExpansion, p.quadraticInExpansion) * invRhoi;
-      const Real QPj = muQR(muj, Cl, Cq, nb.cs, p.linearInExpansion, p.quadraticInExpansion) * nb.invRho;
-      const Real Qi = rhoi2 * absR(QPi);
-      maxVP = maxR(maxVP, Qi);
-      const Real vdr = vdotr * rinv;                 // v_ij . r_hat
-      const Real halfQi = Real(0.5) * QPi * gi;
-      const Real pi = fmaR(gi, Prhoi, halfQi);
-      const Real pj = fmaR(gj, nb.prho, Real(0.5) * QPj * gj);
-      const Real mj = nb.m;
-      const Real fsr = mj * (pi + pj) * rinv;        // acceleration along r_ij
-      const Real wg = mj * gi * rinv;               // grad W_i * m_j = r_ij * wg
-      // gi^2 / max(1e-30, r^6); FP64 takes 1/r^6 from 1/r
-      Real f2;
-      if constexpr (std::is_same<Real, double>::value) {
-        const Real ri2 = rinv * rinv;
-        f2 = r2 * r2 * r2 > Real(1.0e-30) ? gi * gi * (ri2 * ri2 * ri2) : gi * gi * Real(1.0e30);
-      } else {
-        f2 = gi * gi * rcpR(maxR(Real(1.0e-30), r2 * r2 * r2));
-      }
-      if (o.pairDv) {
-        // compatible energy: the own-frame pair term, DvDt_i += -m_j dv
-        const Real dsc = (pi + pj) * rinv;
-        for (int c = 0; c < D; ++c) o.pairDv[int64_t(c) * o.plane + ellIndex(w, n, k)] = double(rij[c] * dsc);
-      }
+      maxVP = maxR(maxVP, q.Qi);
+      if (o.pairDv)
+        for (int c = 0; c < D; ++c) o.pairDv[int64_t(c) * o.plane + ellIndex(w, n, k)] = double(q.rij[c] * q.dsc);
       // several NodeLists: rhoSum and the normalization take same-NodeList
       // pairs only (SPHHydroBase.cc:746-751)
       const bool sameList = !p.slotList || p.slotList[j] == lk;
-      if constexpr (F32) {
-        for (int c = 0; c < D; ++c) af.DvDt[c] = fmaR(-rij[c], fsr, af.DvDt[c]);
-        af.DepsDt = fmaR(mj * vdr, pi, af.DepsDt);
-        af.viscW = fmaR(mj * vdr, halfQi, af.viscW);
-        af.effVP = fmaR(nb.mor * Qi, Wi, af.effVP);
+      auto addTo = [&](auto& b, auto* DvDt, auto* xsphDV, auto* DvDx, auto&& M, auto* m2nd) {
+        for (int c = 0; c < D; ++c) DvDt[c] = fmaR(-q.rij[c], q.fsr, DvDt[c]);
+        b.DepsDt = fmaR(q.mv, q.pi, b.DepsDt);
+        b.viscW = fmaR(q.mv, q.halfQi, b.viscW);
+        b.effVP = fmaR(q.morQi, q.Wi, b.effVP);
         if (sameList) {
-          af.rhoSum = fmaR(mj, Wi, af.rhoSum);
-          af.norm = fmaR(mori, Wi, af.norm);
+          b.rhoSum = fmaR(nb.m, q.Wi, b.rhoSum);
+          b.norm = fmaR(me.mori, q.Wi, b.norm);
         }
-        af.wNS += absR(gWi);
+        b.wNS += q.absG;
         for (int c = 0; c < D; ++c) {
-          const Real u = vij[c] * wg;
-          for (int b = 0; b < D; ++b) af.DvDx[c * D + b] = fmaR(-u, rij[b], af.DvDx[c * D + b]);
+          const Real u = q.vij[c] * q.wg;
+          for (int e = 0; e < D; ++e) DvDx[c * D + e] = fmaR(-u, q.rij[e], DvDx[c * D + e]);
         }
         int s2 = 0;
         for (int c = 0; c < D; ++c) {
-          const Real rw = rij[c] * wg, rf = rij[c] * f2;
-          for (int b = c; b < D; ++b, ++s2) {
-            af.M[s2] = fmaR(-rw, rij[b], af.M[s2]);
-            af.m2nd[s2] = fmaR(rf, rij[b], af.m2nd[s2]);
+          const Real rw = q.rij[c] * q.wg, rf = q.rij[c] * q.f2;
+          for (int e = c; e < D; ++e, ++s2) {
+            M(c, e, s2) = fmaR(-rw, q.rij[e], M(c, e, s2));
+            m2nd[s2] = fmaR(rf, q.rij[e], m2nd[s2]);
           }
         }
         if (p.XSPH) {
-          const Real w2 = Real(0.5) * fmaR(mori, Wi, nb.mor * Wj);
-          af.xsphW += w2;
-          for (int c = 0; c < D; ++c) af.xsphDV[c] = fmaR(-vij[c], w2, af.xsphDV[c]);
+          b.xsphW += q.w2;
+          for (int c = 0; c < D; ++c) xsphDV[c] = fmaR(-q.vij[c], q.w2, xsphDV[c]);
         }
+      };
+      if constexpr (F32) {
+        addTo(af, af.DvDt, af.xsphDV, af.DvDx, [&](int, int, int s2) -> float& { return af.M[s2]; }, af.m2nd);
       } else {
         // FP64, search row order: every accumulation fused
-        for (int c = 0; c < D; ++c) a.DvDt.c[c] = fmaR(-rij[c], fsr, a.DvDt.c[c]);
-        const Real mv = mj * vdr;
-        a.DepsDt = fmaR(mv, pi, a.DepsDt);
-        a.viscW = fmaR(mv, halfQi, a.viscW);
-        a.effVP = fmaR(nb.mor * Qi, Wi, a.effVP);
-        if (sameList) {
-          a.rhoSum = fmaR(mj, Wi, a.rhoSum);
-          a.norm = fmaR(mori, Wi, a.norm);
-        }
-        a.wNS += absR(gWi);
-        for (int c = 0; c < D; ++c) {
-          const Real u = vij[c] * wg;
-          for (int b = 0; b < D; ++b) a.DvDx.c[c * D + b] = fmaR(-u, rij[b], a.DvDx.c[c * D + b]);
-        }
-        int s2 = 0;
-        for (int c = 0; c < D; ++c) {
-          const Real rw = rij[c] * wg, rf = rij[c] * f2;
-          for (int b = c; b < D; ++b, ++s2) {
-            a.M.c[c * D + b] = fmaR(-rw, rij[b], a.M.c[c * D + b]);
-            a.m2nd.c[s2] = fmaR(rf, rij[b], a.m2nd.c[s2]);
-          }
-        }
-        if (p.XSPH) {
-          const Real w2 = Real(0.5) * fmaR(mori, Wi, nb.mor * Wj);
-          a.xsphW += w2;
-          for (int c = 0; c < D; ++c) a.xsphDV.c[c] = fmaR(-vij[c], w2, a.xsphDV.c[c]);
-        }
+        addTo(a, a.DvDt.c, a.xsphDV.c, a.DvDx.c, [&](int c, int e, int) -> double& { return a.M.c[c * D + e]; },
+              a.m2nd.c);
       }
     };
-    INbr<Real> nx;
-    int32_t jn = cur.x;
-    if (PREFETCH && len > 0) loadIso<D>(recN, n, jn, nx);
-    for (int w = 0; w < len; ++w) {
-      INbr<Real> nb;
-      int32_t j;
-      if constexpr (PREFETCH) {
-        // the next record is loaded while this pair is evaluated
-        nb = nx;
-        j = jn;
-        if (w + 1 < len) {
-          jn = nextIndex(nb4, n, k, len, w + 1, cur, nxt);
-          loadIso<D>(recN, n, jn, nx);
+    if constexpr (L > 1) {
+      alignas(16) __shared__ double buf[BS];
+      double* wbuf = buf + (threadIdx.x & ~63);
+      const int sub = threadIdx.x % L;
+      for (int w0 = 0; w0 < len; w0 += L * kSumBlock) {
+        const int wb = w0 + sub * kSumBlock;
+        const int we = wb + kSumBlock < len ? wb + kSumBlock : len;
+        for (int w = wb; w < we; ++w) {
+          const int32_t j = nbr[ellIndex(w, n, k)];
+          INbr<Real> nb;
+          loadIso<D>(recN, n, j, nb);
+          pair(nb, j, w);
         }
-      } else {
-        // one record in flight per lane (fewer registers, more waves)
-        j = w == 0 ? cur.x : nextIndex(nb4, n, k, len, w, cur, nxt);
-        loadIso<D>(recN, n, j, nb);
+        af.flushInto(a, [&](double s, double v) { return addInOrder<L>(s, v, wbuf); });
       }
-      pair(nb, j, w);
-      if constexpr (F32) {
-        if ((w & (kSumBlock - 1)) == kSumBlock - 1) af.flushInto(a);
+      a.maxVP = double(maxVP);
+      for (int s = L / 2; s > 0; s >>= 1) a.maxVP = dmax(a.maxVP, __shfl_xor(a.maxVP, s));
+    } else {
+      const int4* nb4 = reinterpret_cast<const int4*>(nbr);
+      int4 cur = len > 0 ? nb4[ellChunk(0, n, k)] : make_int4(0, 0, 0, 0);
+      int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
+      INbr<Real> nx;
+      int32_t jn = cur.x;
+      if (PREFETCH && len > 0) loadIso<D>(recN, n, jn, nx);
+      for (int w = 0; w < len; ++w) {
+        INbr<Real> nb;
+        int32_t j;
+        if constexpr (PREFETCH) {
+          // the next record is loaded while this pair is evaluated
+          nb = nx;
+          j = jn;
+          if (w + 1 < len) {
+            jn = nextIndex(nb4, n, k, len, w + 1, cur, nxt);
+            loadIso<D>(recN, n, jn, nx);
+          }
+        } else {
+          // one record in flight per lane (fewer registers, more waves)
+          j = w == 0 ? cur.x : nextIndex(nb4, n, k, len, w, cur, nxt);
+          loadIso<D>(recN, n, j, nb);
+        }
+        pair(nb, j, w);
+        if constexpr (F32) {
+          if ((w & (kSumBlock - 1)) == kSumBlock - 1) af.flushInto(a, [](double s, double v) { return s + v; });
+        }
       }
+      if constexpr (F32) af.flushInto(a, [](double s, double v) { return s + v; });
+      a.maxVP = double(maxVP);
     }
-    if constexpr (F32) af.flushInto(a);
-    for (int c = 0; c < D; ++c)
-      for (int b = 0; b < c; ++b) a.M.c[c * D + b] = a.M.c[b * D + c];
-    a.maxVP = double(maxVP);
-    if constexpr (!F32) {
-      if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
+    if (L == 1 || threadIdx.x % L == 0) {
+      for (int c = 0; c < D; ++c)
+        for (int b = 0; b < c; ++b) a.M.c[c * D + b] = a.M.c[b * D + c];
+      if constexpr (!F32) {
+        if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
+      }
+      isoEpilogue<D>(k, len, ri_, a, t, p, o);
     }
-    // the node's own state for the epilogue, read again after the loop so it
-    // holds no registers during it
-    Self<D> me;
-    for (int c = 0; c < D; ++c) me.v.c[c] = ri_[R::V + c];
-    const double hinvD = ri_[RL<true>::HINV];
-    for (int c = 0; c < NSym<D>::value; ++c) me.H.c[c] = 0.0;
-    for (int c = 0; c < D; ++c) me.H.c[sdiag<D>(c)] = hinvD;
-    me.Hdet = ri_[R::HDET]; me.m = ri_[R::M]; me.rho = ri_[R::RHO]; me.mor = ri_[R::MOR];
-    epilogue<D>(k, len, me, a, t, p, o);
   }
-  storePairCount<BS>(pairs, nInt, pairCounts);
+  storePairCount<BS>(pairs, nInt * L, pairCounts);
+}
+
+// The factors of the FP64 sums, one LDS row each, and each sum as the product of
+// two of them (a fused multiply-add per entry): every sum of k_derivs_iso<double>
+// is fma(A, B, sum) for the rows named here, to the bit (a sign moves between the
+// factors exactly, and a plain addition is a factor of one).
+template <int D> struct IsoRow {
+  static constexpr int NR = 0, FSR = D, U = FSR + 1, RW = U + D, NRF = RW + D, MV = NRF + D, PI = MV + 1, HQ = PI + 1,
+                       MQ = HQ + 1, WI = MQ + 1, MJ = WI + 1, MORI = MJ + 1, AG = MORI + 1, NW2 = AG + 1, V0 = NW2 + 1,
+                       ONE = V0 + D, MONE = ONE + 1, COUNT = MONE + 1;
+  static constexpr int SUMS = Sum<D>::COUNT - D * (D - 1) / 2;   // M by its upper triangle
+  // rows of sum q, in the order of Acc's members below
+  static constexpr int pack(int a, int b) { return a | (b << 8); }
+  static __device__ __forceinline__ int rows(int q) {
+    int at = 0;
+    if (q < D) return pack(FSR, NR + q);                                   // DvDt
+    at = D;
+    if (q < at + D * D) return pack(U + (q - at) / D, NR + (q - at) % D);  // DvDx
+    at += D * D;
+    for (int c = 0; c < D; ++c)
+      for (int e = c; e < D; ++e, ++at)
+        if (q == at) return pack(RW + c, NR + e);                          // M
+    for (int c = 0; c < D; ++c)
+      for (int e = c; e < D; ++e, ++at)
+        if (q == at) return pack(NRF + c, NR + e);                         // m2nd
+    if (q < at + D) return pack(V0 + (q - at), NW2);                       // xsphDV
+    at += D;
+    switch (q - at) {
+      case 0: return pack(MV, PI);        // DepsDt
+      case 1: return pack(MV, HQ);        // viscW
+      case 2: return pack(MQ, WI);        // effVP
+      case 3: return pack(MJ, WI);        // rhoSum
+      case 4: return pack(MORI, WI);      // norm
+      case 5: return pack(AG, ONE);       // wNS
+      case 6: return pack(NW2, MONE);     // xsphW
+    }
+    return pack(0, 0);
+  }
+  static __device__ __forceinline__ Acc<D> acc(const double* s) {
+    Acc<D> a;
+    int q = 0;
+    for (int c = 0; c < D; ++c) a.DvDt.c[c] = s[q++];
+    for (int c = 0; c < D * D; ++c) a.DvDx.c[c] = s[q++];
+    for (int c = 0; c < D; ++c)
+      for (int e = c; e < D; ++e) { a.M.c[c * D + e] = a.M.c[e * D + c] = s[q++]; }
+    for (int c = 0; c < NSym<D>::value; ++c) a.m2nd.c[c] = s[q++];
+    for (int c = 0; c < D; ++c) a.xsphDV.c[c] = s[q++];
+    a.DepsDt = s[q++]; a.viscW = s[q++]; a.effVP = s[q++]; a.rhoSum = s[q++]; a.norm = s[q++]; a.wNS = s[q++];
+    a.xsphW = s[q++];
+    return a;
+  }
+};
+
+// The FP64 collapsed pass with L lanes to a node (small node sets), bitwise
+// k_derivs_iso<double>: a lane evaluates one entry of L and leaves its factors in
+// LDS, then runs SUMS / L of the sums over the L entries, in row order.  Lanes
+// past the row leave zeros (a sum that starts at +0 is never -0, so adding a
+// zero product leaves it).
+template <int D, int L>
+__global__ void __launch_bounds__(kBlock) k_derivs_iso_rows(const double* __restrict__ rec,
+                                                            const double2* __restrict__ recN,
+                                                            const int32_t* __restrict__ rowCount,
+                                                            const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
+                                                            const int32_t* __restrict__ work, TabArgs t, Tab64 tt,
+                                                            PassArgs p, OutArgs o, uint32_t* __restrict__ pairCounts) {
+  using R = RL<true>;
+  using W = IsoRow<D>;
+  constexpr int BATCH = (W::SUMS + L - 1) / L, NODES = kBlock / L, PAD = 65;
+  __shared__ double rows[kBlock / 64][W::COUNT][PAD];
+  const int64_t block = xcdBlock((nInt * L + kBlock - 1) / kBlock);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, sub = threadIdx.x % L;
+  const int64_t tw = block * NODES + threadIdx.x / L;
+  unsigned pairs = 0;
+  double maxVP = 0.0, relV = 0.0, sum[BATCH];
+  int which[BATCH];
+#pragma unroll
+  for (int q = 0; q < BATCH; ++q) {
+    sum[q] = 0.0;
+    which[q] = W::rows(q * L + sub);
+  }
+  const int64_t k = tw < nInt ? work[tw] : 0;
+  const int len = tw < nInt ? rowCount[k] : 0;
+  const IsoNode<double, D> me = loadIsoNode<double, D>(rec + k * R::STRIDE, p);
+  double(*row)[PAD] = rows[wave];
+  row[W::ONE][lane] = 1.0;
+  row[W::MONE][lane] = -1.0;
+  for (int w0 = 0; w0 < len; w0 += L) {
+    const int w = w0 + sub;
+    const bool live = w < len;
+    const int32_t j = live ? nbr[ellIndex(w, n, k)] : int32_t(k);
+    INbr<double> nb;
+    loadIso<D>(recN, n, j, nb);
+    const IsoPair<double, D> q = isoPair<double, D>(me, nb, t.g, tt, p);
+    if (live) {
+      pairs += (nb.ghost || j > int32_t(k)) ? 1u : 0u;
+      if (o.relV) relV = dmax(relV, relSpeed<D>(q.vij));
+      maxVP = maxR(maxVP, q.Qi);
+    }
+    auto put = [&](int r, double v) { row[r][lane] = live ? v : 0.0; };
+    for (int c = 0; c < D; ++c) {
+      put(W::NR + c, -q.rij[c]);
+      put(W::U + c, q.vij[c] * q.wg);
+      put(W::RW + c, q.rij[c] * q.wg);
+      put(W::NRF + c, -(q.rij[c] * q.f2));
+      put(W::V0 + c, p.XSPH ? q.vij[c] : 0.0);
+    }
+    put(W::FSR, q.fsr); put(W::MV, q.mv); put(W::PI, q.pi); put(W::HQ, q.halfQi); put(W::MQ, q.morQi);
+    put(W::WI, q.Wi); put(W::MJ, nb.m); put(W::MORI, me.mori); put(W::AG, q.absG);
+    put(W::NW2, p.XSPH ? -q.w2 : 0.0);
+    waveLdsOrder();
+#pragma unroll
+    for (int b = 0; b < BATCH; ++b) {
+      const double* ra = row[which[b] & 0xff] + (lane - sub);
+      const double* rb = row[which[b] >> 8] + (lane - sub);
+      double s = sum[b];
+#pragma unroll
+      for (int e = 0; e < L; ++e) s = __builtin_fma(ra[e], rb[e], s);
+      sum[b] = s;
+    }
+    waveLdsOrder();
+  }
+  for (int s = L / 2; s > 0; s >>= 1) {
+    maxVP = dmax(maxVP, __shfl_xor(maxVP, s));
+    relV = dmax(relV, __shfl_xor(relV, s));
+  }
+  // the epilogue, one lane to a node again: the sums through the same LDS
+  __syncthreads();
+  static_assert(sizeof(double) * NODES * (BATCH * L + 2) <= sizeof(rows), "the sums fit the rows' LDS");
+  double(*sums)[BATCH * L + 2] = reinterpret_cast<double(*)[BATCH * L + 2]>(&rows[0][0][0]);
+  double* mine = sums[threadIdx.x / L];
+#pragma unroll
+  for (int b = 0; b < BATCH; ++b) mine[b * L + sub] = sum[b];
+  if (sub == 0) {
+    mine[BATCH * L] = maxVP;
+    mine[BATCH * L + 1] = relV;
+  }
+  __syncthreads();
+  const int64_t te = block * NODES + threadIdx.x;
+  if (threadIdx.x < NODES && te < nInt) {
+    const int64_t ke = work[te];
+    const int le = rowCount[ke];
+    const double* sm = sums[threadIdx.x];
+    Acc<D> a = W::acc(sm);
+    a.maxVP = sm[BATCH * L];
+    if (o.relV) o.relV[ke] = le > 0 ? sm[BATCH * L + 1] : -1.0;
+    isoEpilogue<D>(ke, le, rec + ke * R::STRIDE, a, t, p, o);
+  }
+  storePairCount<kBlock>(pairs, nInt * L, pairCounts);
 }
 
 TabArgs tabArgs(const Sim& s) {
@@ -1338,12 +1685,17 @@ void sumDensityD(Sim& s) {
     const size_t lds32 = lds ? sizeof(float) * 8 * size_t(s.table.n) : 0;
     const double W0 = s.table.kernelValue(0.0, 1.0);
     const int32_t* lists = slotLists(s);
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), lds32, s.stream, s.rec.as<double>(),
+    auto go = [&](auto kern, int L, size_t ldsB) {
+      hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), ldsB, s.stream, s.rec.as<double>(),
                          s.recSM.as<float4>(), s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt,
                          s.work.as<int32_t>(), t, tab32(s), W0, s.rho.as<double>(), lists, s.sumAllLists ? 1 : 0);
     };
-    if (lds) go(k_sum_density_mixed<D, true>); else go(k_sum_density_mixed<D, false>);
+    withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+      constexpr int L = decltype(lanes)::value;
+      if (L > 1) go(k_sum_density_mixed<D, false, L>, L, 0);
+      else if (lds) go(k_sum_density_mixed<D, true>, 1, lds32);
+      else go(k_sum_density_mixed<D, false>, 1, 0);
+    });
     SG_CHECK_HIP(hipGetLastError());
     applyGhostDensity(s);
     if (!s.capturing) SG_CHECK_HIP(hipEventRecord(s.ev[3], s.stream));
@@ -1359,13 +1711,21 @@ void sumDensityD(Sim& s) {
   }
   const double* nrec = s.isotropic ? s.recS.as<double>() : s.rec.as<double>();
   const double* listOf = s.nLists > 1 ? s.seg.as<double>() : nullptr;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), ldsBytes, s.stream, s.rec.as<double>(),
+  auto go = [&](auto kern, int L, size_t ldsB) {
+    hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), ldsB, s.stream, s.rec.as<double>(),
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        s.rho.as<double>(), nrec, listOf, s.sumAllLists ? 1 : 0);
   };
-  if (s.isotropic) { if (lds) go(k_sum_density<D, true, true>); else go(k_sum_density<D, true, false>); }
-  else { if (lds) go(k_sum_density<D, false, true>); else go(k_sum_density<D, false, false>); }
+  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+    constexpr int L = decltype(lanes)::value;
+    auto any = [&](auto iso) {
+      constexpr bool ISO = decltype(iso)::value;
+      if (L > 1) go(k_sum_density<D, ISO, false, L>, L, 0);
+      else if (lds) go(k_sum_density<D, ISO, true>, 1, ldsBytes);
+      else go(k_sum_density<D, ISO, false>, 1, 0);
+    };
+    if (s.isotropic) any(std::true_type{}); else any(std::false_type{});
+  });
   SG_CHECK_HIP(hipGetLastError());
   // SPHHydroBase::finalize then applies the boundaries to the mass density
   applyGhostDensity(s);
@@ -1378,19 +1738,19 @@ void sumDensityD(Sim& s) {
 template <typename Real> typename IsoTab<Real>::T isoTable(const Sim& s);
 template <> Tab32 isoTable<float>(const Sim& s) { return tab32(s); }
 template <> Tab64 isoTable<double>(const Sim& s) { return tab64(s); }
-template <typename Real, int D, bool PF, int BS>
+template <typename Real, int D, bool PF, int BS, int L = 1>
 void isoLaunch(Sim& s, bool inLds, hipStream_t st, int64_t n, const TabArgs& t, const PassArgs& p, const OutArgs& o,
                uint32_t* counts) {
   using Rec = typename IsoTab<Real>::Rec;
   const Rec* recN = reinterpret_cast<const Rec*>(std::is_same<Real, float>::value ? s.recM.p : s.recD.p);
   const size_t lb = inLds ? sizeof(typename IsoTab<Real>::Elem) * IsoTab<Real>::PER * size_t(s.table.n) : 0;
-  const dim3 g(unsigned(xcdGrid(nblocks(s.nInt, BS)))), b(BS);
-  if (inLds)
-    hipLaunchKernelGGL((k_derivs_iso<Real, D, true, PF, BS>), g, b, lb, st, s.rec.as<double>(), recN,
+  const dim3 g(unsigned(xcdGrid(nblocks(s.nInt * L, BS)))), b(BS);
+  if (L == 1 && inLds)
+    hipLaunchKernelGGL((k_derivs_iso<Real, D, L == 1, PF, BS, L>), g, b, lb, st, s.rec.as<double>(), recN,
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        isoTable<Real>(s), p, o, counts);
   else
-    hipLaunchKernelGGL((k_derivs_iso<Real, D, false, PF, BS>), g, b, 0, st, s.rec.as<double>(), recN,
+    hipLaunchKernelGGL((k_derivs_iso<Real, D, false, PF, BS, L>), g, b, 0, st, s.rec.as<double>(), recN,
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        isoTable<Real>(s), p, o, counts);
 }
@@ -1419,7 +1779,9 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
   const int total = derivTotalDoubles(s.dim);
   s.out.ensure(sizeof(double) * size_t(n) * total);
   s.outStride = n;
-  s.pairWaves = (s.nInt + 63) / 64;
+  // lanes to a node: mixed blocks need rows of several blocks, so 1-D keeps one
+  const int lanes = hp.precision == SPHGPU_PRECISION_MIXED ? mixedLanes(D, s.nInt) : rowLanes(D, s.nInt);
+  s.pairWaves = (s.nInt * lanes + 63) / 64;
   s.pairCounts.ensure(sizeof(uint32_t) * size_t(std::max<int64_t>(s.pairWaves, 1)));
   uint32_t* counts = s.pairCounts.as<uint32_t>();
 
@@ -1478,7 +1840,18 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
   // wavefronts per SIMD (2.11 ms at 128^3 against 2.53 ms with the next
   // record prefetched at 179 VGPRs, two wavefronts).  FP64: the prefetch wins
   // (3.44 ms at 194 VGPRs against 3.51 ms at 168).
-  if (mixed || fast64) {
+  if (mixed && lanes > 1) {
+    if constexpr (D > 1) isoLaunch<float, D, false, kBlock, D == 3 ? 8 : 2>(s, false, st, n, t, p, o, counts);
+    SG_CHECK_HIP(hipGetLastError());
+  } else if (fast64 && lanes > 1) {
+    withLanes<D>(lanes, [&](auto ln) {
+      constexpr int L = decltype(ln)::value;
+      if constexpr (L > 1)
+        hipLaunchKernelGGL((k_derivs_iso_rows<D, L>), dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), 0, st,
+                           s.rec.as<double>(), s.recD.as<double2>(), s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n,
+                           s.nInt, s.work.as<int32_t>(), t, tab64(s), p, o, counts);
+    });
+  } else if (mixed || fast64) {
     // 1-D and 2-D (ensembles, serving): the workgroup size and the table's
     // place (LDS or read through L1) are autotuned per workload class.  3-D
     // runs 256-thread workgroups with the table in LDS when it fits.
@@ -1501,7 +1874,23 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
                          s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t, p, o,
                          counts);
     };
-    if (lds) {
+    if (lanes > 1) {
+      withLanes<D>(lanes, [&](auto ln) {
+        constexpr int L = decltype(ln)::value;
+        if constexpr (L > 1) {
+          auto any = [&](auto iso, auto tens) {
+            hipLaunchKernelGGL((k_derivs_rows<D, decltype(iso)::value, decltype(tens)::value, L>),
+                               dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), 0, st, s.rec.as<double>(),
+                               s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t, p, o,
+                               counts);
+          };
+          const std::true_type yes{};
+          const std::false_type no{};
+          if (s.isotropic) { if (tensile) any(yes, yes); else any(yes, no); }
+          else { if (tensile) any(no, yes); else any(no, no); }
+        }
+      });
+    } else if (lds) {
       if (s.isotropic) { if (tensile) launch(k_derivs_fp64<D, true, true, true>); else launch(k_derivs_fp64<D, true, false, true>); }
       else { if (tensile) launch(k_derivs_fp64<D, false, true, true>); else launch(k_derivs_fp64<D, false, false, true>); }
     } else {
@@ -1521,13 +1910,21 @@ void omegaGradhD(Sim& s) {
   TabArgs t = tabArgs(s);
   const bool lds = ldsTable(s);
   const size_t ldsBytes = lds ? sizeof(double) * 6 * size_t(s.table.n) : 0;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), ldsBytes, s.stream, s.rec.as<double>(),
+  auto go = [&](auto kern, int L, size_t ldsB) {
+    hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), ldsB, s.stream, s.rec.as<double>(),
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        s.omega.as<double>());
   };
-  if (s.isotropic) { if (lds) go(k_omega<D, true, true>); else go(k_omega<D, true, false>); }
-  else { if (lds) go(k_omega<D, false, true>); else go(k_omega<D, false, false>); }
+  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+    constexpr int L = decltype(lanes)::value;
+    auto any = [&](auto iso) {
+      constexpr bool ISO = decltype(iso)::value;
+      if (L > 1) go(k_omega<D, ISO, false, L>, L, 0);
+      else if (lds) go(k_omega<D, ISO, true>, 1, ldsBytes);
+      else go(k_omega<D, ISO, false>, 1, 0);
+    };
+    if (s.isotropic) any(std::true_type{}); else any(std::false_type{});
+  });
   SG_CHECK_HIP(hipGetLastError());
 }
 
@@ -1551,7 +1948,8 @@ void omegaGradh(Sim& s) {
 // change max|phi - 1| over the eigenvalues c/lambda(H_i) of H1^1/2 H_i^-1 H1^1/2
 // (H1 = c I).  Node i reads only its own H (neighbour positions come from
 // the records), so H is replaced in place.
-template <int D, bool ISO, bool LDS>
+// L > 1: L lanes to a node (its rows are of one length in a wavefront, nearly).
+template <int D, bool ISO, bool LDS, int L = 1>
 __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ rec, const int32_t* __restrict__ rowCount,
                                                     const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
                                                     const int32_t* __restrict__ work, const int32_t* __restrict__ perm,
@@ -1563,11 +1961,12 @@ __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ r
   constexpr int NS = NSym<D>::value;
   extern __shared__ double lds[];
   const double* tab = stageTable<LDS>(lds, t);
-  const int64_t tw = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+  const int64_t tw = (xcdBlock((nInt * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
   double d = 0.0;
   if (tw < nInt) {
     const int64_t k = work[tw];
     const int64_t i = perm[k];
+    // the lanes of a node agree: its change is written after the last of them read it
     if (deltaH[i] > tol) {
       S<D> Hi;
       for (int c = 0; c < NS; ++c) Hi.c[c] = H[i * NS + c];
@@ -1579,8 +1978,8 @@ __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ r
       const double li = listOf ? listOf[i] : 0.0, mi = ri_[R::M], rhoi = ri_[R::RHO];
       double zeroth = 0.0;
       const int len = rowCount[k];
-      for (int w = 0; w < len; ++w) {
-        const double* rj = rec + int64_t(nbr[ellIndex(w, n, k)]) * R::STRIDE;
+      auto term = [&](int32_t j) {
+        const double* rj = rec + int64_t(j) * R::STRIDE;
         V<D> xij;
         for (int c = 0; c < D; ++c) xij.c[c] = xi.c[c] - rj[R::X + c];
         const double etai = vmag(sdot(Hi, xij));
@@ -1588,16 +1987,31 @@ __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ r
         lookupWG(tab, t, etai, 1.0, Wv, gW);
         double fw = 1.0;
         if (listOf && listOf[int64_t(rj[R::ORIG])] != li) fw = rj[R::M] * rhoi / (mi * rj[R::RHO]);
-        zeroth += fw * dabs(gW);
+        return fw * dabs(gW);
+      };
+      if constexpr (L > 1) {
+        // (a node done earlier leaves its lanes out of the exchange as a group)
+        alignas(16) __shared__ double buf[kBlock];
+        double* wbuf = buf + (threadIdx.x & ~63);
+        const int sub = threadIdx.x % L;
+        for (int w0 = 0; w0 < len; w0 += L) {
+          const bool live = w0 + sub < len;
+          const double tm = term(live ? nbr[ellIndex(w0 + sub, n, k)] : int32_t(k));
+          zeroth = addInOrder<L>(zeroth, live ? tm : -0.0, wbuf);
+        }
+      } else {
+        for (int w = 0; w < len; ++w) zeroth += term(nbr[ellIndex(w, n, k)]);
       }
       zeroth = rootnu<D>(zeroth);
       const double c1 = idealHinv(t, zeroth, Hi.c[0], nPerh, hmin, hmax);
       const double phimin = c1 / maxEigen<D>(Hi.c), phimax = c1 / minEigen<D>(Hi.c);
       d = dmax(dabs(phimin - 1.0), dabs(phimax - 1.0));
-      deltaH[i] = d;
-      int q = 0;
-      for (int a = 0; a < D; ++a)
-        for (int b = a; b < D; ++b, ++q) H[i * NS + q] = (a == b) ? c1 : 0.0;
+      if (threadIdx.x % L == 0) {
+        deltaH[i] = d;
+        int q = 0;
+        for (int a = 0; a < D; ++a)
+          for (int b = a; b < D; ++b, ++q) H[i * NS + q] = (a == b) ? c1 : 0.0;
+      }
     }
   }
   for (int sh = 32; sh > 0; sh >>= 1) d = dmax(d, __shfl_xor(d, sh));
@@ -1610,14 +2024,22 @@ double idealHPassD(Sim& s, const sphgpu_hydro_params& hp, double tol, double* de
   TabArgs t = tabArgs(s);
   const bool lds = ldsTable(s);
   const size_t ldsBytes = lds ? sizeof(double) * 6 * size_t(s.table.n) : 0;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), ldsBytes, s.stream, s.rec.as<double>(),
+  auto go = [&](auto kern, int L, size_t ldsB) {
+    hipLaunchKernelGGL(kern, dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), ldsB, s.stream, s.rec.as<double>(),
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(),
                        s.perm.as<int32_t>(), t, hp.nPerh, hp.hmin, hp.hmax, tol, s.H.as<double>(), deltaH, bits,
                        s.nLists > 1 ? s.seg.as<double>() : nullptr);
   };
-  if (s.isotropic) { if (lds) go(k_ideal_h<D, true, true>); else go(k_ideal_h<D, true, false>); }
-  else { if (lds) go(k_ideal_h<D, false, true>); else go(k_ideal_h<D, false, false>); }
+  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+    constexpr int L = decltype(lanes)::value;
+    auto any = [&](auto iso) {
+      constexpr bool ISO = decltype(iso)::value;
+      if (L > 1) go(k_ideal_h<D, ISO, false, L>, L, 0);
+      else if (lds) go(k_ideal_h<D, ISO, true>, 1, ldsBytes);
+      else go(k_ideal_h<D, ISO, false>, 1, 0);
+    };
+    if (s.isotropic) any(std::true_type{}); else any(std::false_type{});
+  });
   SG_CHECK_HIP(hipGetLastError());
   unsigned long long hb = 0;
   SG_CHECK_HIP(hipMemcpyAsync(&hb, bits, sizeof(hb), hipMemcpyDeviceToHost, s.stream));

@@ -26,6 +26,7 @@
 #include "eigen.hh"
 #include "ell.hh"
 #include "pack.hh"
+#include "lanes.hh"
 #include <cfloat>
 #include <cstring>
 #include <algorithm>
@@ -370,11 +371,13 @@ __global__ void k_compat_rec(const int32_t* __restrict__ perm, int64_t nSlots, c
 // here from the receiving node with the owner's operands in the reference's
 // order.  With rows in caller-index order the sum runs in the reference's
 // order (owners j < i ascending, then the node's own pairs).
-template <int D>
-__global__ void k_compat(const int32_t* __restrict__ work, const int32_t* __restrict__ rowCount,
-                         const int32_t* __restrict__ nbr, int64_t n, int64_t nInt, const double* __restrict__ crec,
-                         const double* __restrict__ pairDv, int64_t plane, double* __restrict__ compDe) {
-  const int64_t t = xcdBlock((nInt + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+// L > 1: L lanes to a node (lanes.hh).
+template <int D, int L>
+__global__ void __launch_bounds__(kBlock) k_compat(const int32_t* __restrict__ work, const int32_t* __restrict__ rowCount,
+                                                   const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
+                                                   const double* __restrict__ crec, const double* __restrict__ pairDv,
+                                                   int64_t plane, double* __restrict__ compDe) {
+  const int64_t t = (xcdBlock((nInt * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
   if (t >= nInt) return;
   const int64_t k = work[t];
   const double2* mr = reinterpret_cast<const double2*>(crec + k * 8);
@@ -383,8 +386,7 @@ __global__ void k_compat(const int32_t* __restrict__ work, const int32_t* __rest
   const double wti = a1.y, mi = a2.x, oi = a2.y;
   double de = 0.0;
   const int len = rowCount[k];
-  for (int w = 0; w < len; ++w) {
-    const int64_t e = ellIndex(w, n, k);
+  auto term = [&](int64_t e) {
     const double2* nr = reinterpret_cast<const double2*>(crec + int64_t(nbr[e]) * 8);
     const double2 b0 = nr[0], b1 = nr[1], b2 = nr[2];
     const double vj[3] = {b0.x, b0.y, b1.x};
@@ -397,18 +399,29 @@ __global__ void k_compat(const int32_t* __restrict__ work, const int32_t* __rest
         du = (c == 0) ? tc : du + tc;
       }
       const double wi = wti / (wti + wtj);
-      de += wi * du;
-    } else {
-      for (int c = 0; c < D; ++c) {
-        const double pa = pairDv[int64_t(c) * plane + e] * mi;
-        const double tc = (vi[c] - vj[c]) * pa;
-        du = (c == 0) ? tc : du + tc;
-      }
-      const double wj = wtj / (wtj + wti);
-      de += (1.0 - wj) * du * mj / mi;
+      return wi * du;
     }
+    for (int c = 0; c < D; ++c) {
+      const double pa = pairDv[int64_t(c) * plane + e] * mi;
+      const double tc = (vi[c] - vj[c]) * pa;
+      du = (c == 0) ? tc : du + tc;
+    }
+    const double wj = wtj / (wtj + wti);
+    return (1.0 - wj) * du * mj / mi;
+  };
+  if constexpr (L > 1) {
+    alignas(16) __shared__ double buf[kBlock];
+    double* wbuf = buf + (threadIdx.x & ~63);
+    const int sub = threadIdx.x % L;
+    for (int w0 = 0; w0 < len; w0 += L) {
+      const double v = w0 + sub < len ? term(ellIndex(w0 + sub, n, k)) : -0.0;
+      de = addInOrder<L>(de, v, wbuf);
+    }
+    if (sub == 0) compDe[k] = de;
+  } else {
+    for (int w = 0; w < len; ++w) de += term(ellIndex(w, n, k));
+    compDe[k] = de;
   }
-  compDe[k] = de;
 }
 
 Eos makeEos(double gamma, double Pmin, double Pmax, int floor) { return Eos{gamma, gamma - 1.0, Pmin, Pmax, floor}; }
@@ -431,9 +444,12 @@ template <int D> void compatD(Sim& s, const double* vel0, const SegArgs& sa) {
   hipLaunchKernelGGL(k_compat_rec<D>, dim3(nblocks(s.nSlots)), dim3(kBlock), 0, st, s.perm.as<int32_t>(), s.nSlots,
                      vel0, s.compAcc.as<double>(), s.compDe0.as<double>(), s.mass.as<double>(), sa,
                      s.compRec.as<double>());
-  hipLaunchKernelGGL(k_compat<D>, dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
-                     s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots, s.nInt, s.compRec.as<double>(),
-                     s.pairDv.as<double>(), s.nSlots * int64_t(s.ellCap), s.compDe.as<double>());
+  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+    constexpr int L = decltype(lanes)::value;
+    hipLaunchKernelGGL((k_compat<D, L>), dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
+                       s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots, s.nInt, s.compRec.as<double>(),
+                       s.pairDv.as<double>(), s.nSlots * int64_t(s.ellCap), s.compDe.as<double>());
+  });
   SG_CHECK_HIP(hipGetLastError());
 }
 
