@@ -475,8 +475,14 @@ struct RowStats {
 // ---------------------------------------------------------------------------
 constexpr int kStageEdge = 8;                       // 4-cell brick + 2 cells each side
 constexpr int kStaged = kStageEdge * kStageEdge * kStageEdge;
-constexpr int kCandCap = 2048;
-constexpr int kRunRows = 9;      // one z slab: 5 runs, 3 sentinels, the read-ahead row
+// Candidates a brick stages.  A 4 R wide halo of a lattice at nPerh = 1.51 is 12
+// or 13 planes wide on each axis: 13^3 = 2197 where all three axes catch one
+// more, and such a brick must not fall back to reading every candidate from
+// global memory: a few dozen of 13 k bricks held a whole 128^3 search up (1.84 ms
+// with room for 2048 candidates, 1.58 ms with 2240).  2240 is what three
+// workgroups per CU leave room for.
+constexpr int kCandCap = 2240;
+constexpr int kRunRows = 6;      // one z slab: 5 runs and the sentinel
 
 struct SearchArgs {
   DGrid g;
@@ -506,10 +512,9 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
   __shared__ float4 sCand[kCandCap];               // x,y,z offsets from the brick origin, (1/h)^2 (FP32)
   __shared__ int32_t sSlot[kCandCap];
   // per lane: the runs of one z slab of its stencil (t0 | t1 << 16),
-  // lane-strided; up to 5 runs, three sentinels and the row the reader reads
-  // ahead of them.  Before the runs are formed the same memory holds each
-  // staged cell's first slot and the scan's partial sums (52 KB in all: three
-  // workgroups per CU)
+  // lane-strided; up to 5 runs and the sentinel the reader stays on past them.
+  // Before the runs are formed the same memory holds each staged cell's first
+  // slot and the scan's partial sums (52 KB in all: three workgroups per CU)
   __shared__ uint32_t sRun[kRunRows * kBlock];
   static_assert(kRunRows * kBlock >= kStaged + kBlock, "sStart and sc alias the run table");
   int32_t* const sStart = reinterpret_cast<int32_t*>(sRun);
@@ -655,7 +660,7 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
         //    as its longest candidate list in the slab, not its longest run in
         //    every (dz, dy) row.  Candidates are read two ahead of their test (three
         //    register sets in rotation); the reader steps through the runs with
-        //    no branch and, past the last candidate, through three sentinel runs
+        //    no branch and, past the last candidate, stays on the sentinel run
         //    (candidate 0), so every index it forms stays inside the tables.
         //    The rare paths (the exact FP64 test, ghost marks) are entered only
         //    when some lane of the wavefront needs them.
@@ -666,17 +671,19 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
         // in it, so the walk skips both checks
         auto walk = [&](auto marksOn, auto plainOn) {
           constexpr bool plain = decltype(plainOn)::value;
-          for (int q = 0; q < 3; ++q) sRun[(nr + q) * kBlock + threadIdx.x] = 0u;
+          sRun[nr * kBlock + threadIdx.x] = 0u;
           const uint32_t first = sRun[threadIdx.x];
           int32_t t = int32_t(first & 0xffffu), tEnd = int32_t(first >> 16);
           uint32_t nxt = sRun[kBlock + threadIdx.x];
-          int r = 0;
+          int at = kBlock + int(threadIdx.x);               // where nxt came from
+          const int last = nr * kBlock + int(threadIdx.x);  // the sentinel
           auto advance = [&]() {
             const bool same = t + 1 < tEnd;
-            r = same ? r : r + 1;
+            const int next = at + kBlock < last ? at + kBlock : last;
             t = same ? t + 1 : int32_t(nxt & 0xffffu);
             tEnd = same ? tEnd : int32_t(nxt >> 16);
-            nxt = sRun[(r + 1) * kBlock + threadIdx.x];
+            at = same ? at : next;
+            nxt = sRun[at];
           };
           auto read = [&](float4& c, int32_t& raw) {
             c = sCand[t];
