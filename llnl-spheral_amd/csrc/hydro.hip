@@ -827,9 +827,9 @@ __device__ __forceinline__ void loadIso(const float4* __restrict__ recM, int64_t
 // (the off-diagonal products are exact zeros), so the value is bitwise the
 // packed one; m/rho is m * (1/rho), within an ulp.
 template <int D>
-__device__ __forceinline__ void loadIso(const double2* __restrict__ recD, int64_t n, int32_t j, INbr<double>& o) {
-  const double2* a = recD + int64_t(j) * 4;
-  const double2* b = recD + 4 * n + int64_t(j) * 2;
+__device__ __forceinline__ void loadIso(const double2* __restrict__ recD, int64_t, int32_t j, INbr<double>& o) {
+  const double2* a = recD + int64_t(j) * 6;
+  const double2* b = a + 4;
   const double2 d0 = a[0], d1 = a[1], d2 = a[2], d3 = a[3], e0 = b[0], e1 = b[1];
   o.x[0] = d0.x; o.x[1] = d0.y; o.x[2] = d1.x;
   o.ghost = d1.y < 0.0;
@@ -851,7 +851,7 @@ __global__ void k_pack_mixed(const double* __restrict__ rec, int64_t n, int64_t 
 template <int D>
 __global__ void k_pack_fast64(const double* __restrict__ rec, int64_t n, int64_t nInt, double2* __restrict__ recD) {
   const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (k < n) writeFast64Rec<D>(rec + k * RL<true>::STRIDE, nInt, recD + k * 4, recD + 4 * n + k * 2);
+  if (k < n) writeFast64Rec<D>(rec + k * RL<true>::STRIDE, nInt, recD + k * 6, recD + k * 6 + 4);
 }
 
 template <int D>

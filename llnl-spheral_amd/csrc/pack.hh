@@ -148,7 +148,7 @@ __device__ __forceinline__ void storeRecords(int64_t k, const double* r, const P
   for (int c = 0; c < R::STRIDE / 2; ++c) dst[c] = make_double2(r[2 * c], r[2 * c + 1]);
   if constexpr ((SEC & 1) != 0) writeMixedRec<D>(r, o.nInt, o.qInv, static_cast<float4*>(o.sec) + k * MixedRec<D>::F4);
   if constexpr ((SEC & 2) != 0)
-    writeFast64Rec<D>(r, o.nInt, static_cast<double2*>(o.sec) + k * 4, static_cast<double2*>(o.sec) + 4 * o.n + k * 2);
+    writeFast64Rec<D>(r, o.nInt, static_cast<double2*>(o.sec) + k * 6, static_cast<double2*>(o.sec) + k * 6 + 4);
   if constexpr ((SEC & 4) != 0) writeDensRec<D>(r, static_cast<double2*>(o.sec2) + k * 3);
   if constexpr ((SEC & 8) != 0) writeDensRecMixed<D>(r, static_cast<float4*>(o.sec3) + k * DensMixedRec<D>::F4);
 }
