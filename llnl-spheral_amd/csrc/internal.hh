@@ -323,6 +323,7 @@ struct Sim {
   void* pinnedIn = nullptr;
   size_t pinnedInBytes = 0;
   hipEvent_t pinnedInDone = nullptr;   // recorded after the copies that read pinnedIn
+  DBuf unsorted;                   // a derivative field in the caller's order, on its way to the host
   std::vector<int32_t> cullStarts;  // new ghost starts read with the last build's row readback
   bool cullStartsReady = false;
   bool pairsValid = false;                   // a pass ran on the current neighbour rows
@@ -392,6 +393,13 @@ void eosRows(Sim& s, int64_t first, int64_t rows, double gamma, double Pmin, dou
 // neighbors.hip
 // Pinned staging of at least `bytes`: which = 0 readbacks, 1 uploads.
 void* hostStaging(Sim& s, int which, size_t bytes);
+// transfer.hip
+// Queue the test of `rows` device rows of H; after the stream's next wait the
+// word returned (pinned, valid until the next readback) is 1 if any is not h I.
+int32_t* queueIsotropyTest(Sim& s, const double* H, int64_t rows);
+// A derivative field's internal rows (comps doubles each, src in slot order) in
+// the caller's order: a workspace, valid until the next call.
+const double* unsortDerivative(Sim& s, const double* src, int comps);
 // First half of the ghost cull: keep flags and scan, the planes' new first
 // ghosts and the search flags to pinned memory.
 void cullLaunch(Sim& s, int32_t* flagsOut, int32_t* starts);
