@@ -787,7 +787,7 @@ __global__ void __launch_bounds__(kBlock) k_derivs_rows(const double* __restrict
 // mixed-precision bar (1e-5).
 //
 // Neighbour records (written in pack.hh): the mixed record (MixedRec, 32 / 48 /
-// 48 B in 1-D / 2-D / 3-D) and the FP64 record (96 B in two planes); both mark
+// 48 B in 1-D / 2-D / 3-D) and the FP64 record (96 B); both mark
 // ghosts by a negative 1/h, and the reader forms det H = (1/h)^D.
 // ---------------------------------------------------------------------------
 template <typename Real> struct INbr {
@@ -1690,7 +1690,7 @@ void sumDensityD(Sim& s) {
                          s.recSM.as<float4>(), s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt,
                          s.work.as<int32_t>(), t, tab32(s), W0, s.rho.as<double>(), lists, s.sumAllLists ? 1 : 0);
     };
-    withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+    withLanes<D>(rowLanes(RowPass::kDensity, D, s.nInt), [&](auto lanes) {
       constexpr int L = decltype(lanes)::value;
       if (L > 1) go(k_sum_density_mixed<D, false, L>, L, 0);
       else if (lds) go(k_sum_density_mixed<D, true>, 1, lds32);
@@ -1716,7 +1716,7 @@ void sumDensityD(Sim& s) {
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        s.rho.as<double>(), nrec, listOf, s.sumAllLists ? 1 : 0);
   };
-  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+  withLanes<D>(rowLanes(RowPass::kDensity, D, s.nInt), [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     auto any = [&](auto iso) {
       constexpr bool ISO = decltype(iso)::value;
@@ -1779,12 +1779,6 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
   const int total = derivTotalDoubles(s.dim);
   s.out.ensure(sizeof(double) * size_t(n) * total);
   s.outStride = n;
-  // lanes to a node: mixed blocks need rows of several blocks, so 1-D keeps one
-  const int lanes = hp.precision == SPHGPU_PRECISION_MIXED ? mixedLanes(D, s.nInt) : rowLanes(D, s.nInt);
-  s.pairWaves = (s.nInt * lanes + 63) / 64;
-  s.pairCounts.ensure(sizeof(uint32_t) * size_t(std::max<int64_t>(s.pairWaves, 1)));
-  uint32_t* counts = s.pairCounts.as<uint32_t>();
-
   // the pair kernel decides the record it reads
   const bool tensile = hp.epsTensile != 0.0;
   const bool compat = hp.compatibleEnergyEvolution != 0;
@@ -1794,6 +1788,12 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
                "mixed precision needs H = h I, no Q multipliers and epsTensile = 0");
   const int sec = pairRecordSec(s, hp);
   const bool fast64 = sec == 2;
+  // lanes to a node: mixed blocks need rows of several blocks, so 1-D keeps one
+  const int lanes = mixed ? mixedLanes(D, s.nInt)
+                          : rowLanes(fast64 ? RowPass::kIsoPairs : RowPass::kPairs, D, s.nInt);
+  s.pairWaves = (s.nInt * lanes + 63) / 64;
+  s.pairCounts.ensure(sizeof(uint32_t) * size_t(std::max<int64_t>(s.pairWaves, 1)));
+  uint32_t* counts = s.pairCounts.as<uint32_t>();
 
   if (!s.capturing) SG_CHECK_HIP(hipEventRecord(s.ev[4], st));
   if (!s.recValid) {
@@ -1915,7 +1915,7 @@ void omegaGradhD(Sim& s) {
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        s.omega.as<double>());
   };
-  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+  withLanes<D>(rowLanes(RowPass::kOmega, D, s.nInt), [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     auto any = [&](auto iso) {
       constexpr bool ISO = decltype(iso)::value;
@@ -1961,13 +1961,15 @@ __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ r
   constexpr int NS = NSym<D>::value;
   extern __shared__ double lds[];
   const double* tab = stageTable<LDS>(lds, t);
-  const int64_t tw = (xcdBlock((nInt * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
-  double d = 0.0;
+  const int64_t block = xcdBlock((nInt * L + kBlock - 1) / kBlock);
+  const int64_t tw = (block * kBlock + threadIdx.x) / L;
+  double zeroth = 0.0, d = 0.0;
+  bool open = false;      // the node still iterates
   if (tw < nInt) {
     const int64_t k = work[tw];
     const int64_t i = perm[k];
-    // the lanes of a node agree: its change is written after the last of them read it
-    if (deltaH[i] > tol) {
+    open = deltaH[i] > tol;
+    if (open) {
       S<D> Hi;
       for (int c = 0; c < NS; ++c) Hi.c[c] = H[i * NS + c];
       const double* ri_ = rec + k * R::STRIDE;
@@ -1976,7 +1978,6 @@ __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ r
       // several NodeLists: a neighbour of another NodeList counts with
       // m_j rho_i / (m_i rho_j) (iterateIdealH.cc:183-194)
       const double li = listOf ? listOf[i] : 0.0, mi = ri_[R::M], rhoi = ri_[R::RHO];
-      double zeroth = 0.0;
       const int len = rowCount[k];
       auto term = [&](int32_t j) {
         const double* rj = rec + int64_t(j) * R::STRIDE;
@@ -2000,19 +2001,49 @@ __global__ void __launch_bounds__(kBlock) k_ideal_h(const double* __restrict__ r
           zeroth = addInOrder<L>(zeroth, live ? tm : -0.0, wbuf);
         }
       } else {
-        for (int w = 0; w < len; ++w) zeroth += term(nbr[ellIndex(w, n, k)]);
-      }
-      zeroth = rootnu<D>(zeroth);
-      const double c1 = idealHinv(t, zeroth, Hi.c[0], nPerh, hmin, hmax);
-      const double phimin = c1 / maxEigen<D>(Hi.c), phimax = c1 / minEigen<D>(Hi.c);
-      d = dmax(dabs(phimin - 1.0), dabs(phimax - 1.0));
-      if (threadIdx.x % L == 0) {
-        deltaH[i] = d;
-        int q = 0;
-        for (int a = 0; a < D; ++a)
-          for (int b = a; b < D; ++b, ++q) H[i * NS + q] = (a == b) ? c1 : 0.0;
+        // four entries at a time: their four records are in flight together
+        // (40^3 nodes: 104 us one by one, 88 us)
+        const int4* nb4 = reinterpret_cast<const int4*>(nbr);
+        for (int w = 0; w < len; w += 4) {
+          const int4 j = nb4[ellChunk(w / 4, n, k)];
+          const int32_t self = int32_t(k);
+          const double t0 = term(j.x), t1 = term(w + 1 < len ? j.y : self);
+          const double t2 = term(w + 2 < len ? j.z : self), t3 = term(w + 3 < len ? j.w : self);
+          zeroth += t0;
+          zeroth += w + 1 < len ? t1 : -0.0;
+          zeroth += w + 2 < len ? t2 : -0.0;
+          zeroth += w + 3 < len ? t3 : -0.0;
+        }
       }
     }
+  }
+  // The root, the table's inverse and the eigenvalues take as long as a row: one
+  // lane to a node again, in as few wavefronts as hold them.
+  int64_t te = tw;
+  if constexpr (L > 1) {
+    __shared__ double sums[kBlock / L];
+    __shared__ int still[kBlock / L];
+    if (threadIdx.x % L == 0) {
+      sums[threadIdx.x / L] = zeroth;
+      still[threadIdx.x / L] = open;
+    }
+    __syncthreads();
+    open = threadIdx.x < kBlock / L && still[threadIdx.x % (kBlock / L)];
+    zeroth = sums[threadIdx.x % (kBlock / L)];
+    te = block * (kBlock / L) + threadIdx.x;
+  }
+  if (open) {
+    const int64_t i = perm[work[te]];
+    S<D> Hi;
+    for (int c = 0; c < NS; ++c) Hi.c[c] = H[i * NS + c];
+    zeroth = rootnu<D>(zeroth);
+    const double c1 = idealHinv(t, zeroth, Hi.c[0], nPerh, hmin, hmax);
+    const double phimin = c1 / maxEigen<D>(Hi.c), phimax = c1 / minEigen<D>(Hi.c);
+    d = dmax(dabs(phimin - 1.0), dabs(phimax - 1.0));
+    deltaH[i] = d;
+    int q = 0;
+    for (int a = 0; a < D; ++a)
+      for (int b = a; b < D; ++b, ++q) H[i * NS + q] = (a == b) ? c1 : 0.0;
   }
   for (int sh = 32; sh > 0; sh >>= 1) d = dmax(d, __shfl_xor(d, sh));
   if ((threadIdx.x & 63) == 0 && d > 0.0) atomicMax(maxBits, (unsigned long long)__double_as_longlong(d));
@@ -2030,7 +2061,7 @@ double idealHPassD(Sim& s, const sphgpu_hydro_params& hp, double tol, double* de
                        s.perm.as<int32_t>(), t, hp.nPerh, hp.hmin, hp.hmax, tol, s.H.as<double>(), deltaH, bits,
                        s.nLists > 1 ? s.seg.as<double>() : nullptr);
   };
-  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+  withLanes<D>(rowLanes(RowPass::kIdealH, D, s.nInt), [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     auto any = [&](auto iso) {
       constexpr bool ISO = decltype(iso)::value;

@@ -371,7 +371,9 @@ __global__ void k_compat_rec(const int32_t* __restrict__ perm, int64_t nSlots, c
 // here from the receiving node with the owner's operands in the reference's
 // order.  With rows in caller-index order the sum runs in the reference's
 // order (owners j < i ascending, then the node's own pairs).
-// L > 1: L lanes to a node (lanes.hh).
+// L > 1: L lanes to a node (lanes.hh).  One lane to a node waits for each
+// entry's record in turn; eight have theirs in flight together, and a term costs
+// far more than the exchange, so two and three dimensions take them at any size.
 template <int D, int L>
 __global__ void __launch_bounds__(kBlock) k_compat(const int32_t* __restrict__ work, const int32_t* __restrict__ rowCount,
                                                    const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
@@ -444,7 +446,7 @@ template <int D> void compatD(Sim& s, const double* vel0, const SegArgs& sa) {
   hipLaunchKernelGGL(k_compat_rec<D>, dim3(nblocks(s.nSlots)), dim3(kBlock), 0, st, s.perm.as<int32_t>(), s.nSlots,
                      vel0, s.compAcc.as<double>(), s.compDe0.as<double>(), s.mass.as<double>(), sa,
                      s.compRec.as<double>());
-  withLanes<D>(rowLanes(D, s.nInt), [&](auto lanes) {
+  withLanes<D, D == 1>(rowLanes(RowPass::kCompat, D, s.nInt), [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     hipLaunchKernelGGL((k_compat<D, L>), dim3(xcdGrid(nblocks(s.nInt * L))), dim3(kBlock), 0, st, s.work.as<int32_t>(),
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots, s.nInt, s.compRec.as<double>(),

@@ -200,7 +200,7 @@ struct Sim {
   DBuf rec;
   bool recValid = false;    // records match the caller-order state
   DBuf recM;                // mixed-precision neighbour records (32 / 48 / 48 B per slot in 1 / 2 / 3-D)
-  DBuf recD;                // FP64 records of the collapsed isotropic pair loop (96 B per slot, two planes)
+  DBuf recD;                // FP64 records of the collapsed isotropic pair loop (96 B per slot)
   DBuf recS;                // FP64 density-sum neighbour records, isotropic H (48 B per slot)
   int pairRec = 0;           // pair-kernel record current with rec: 1 mixed, 2 FP64 isotropic, 0 none
   int buildRecHint = -1;     // record kinds (pack sec bits, isotropic H) the neighbour build's pack also

@@ -55,10 +55,12 @@ __device__ __forceinline__ void writeMixedRec(const double* r, int64_t nInt, dou
     p[2] = make_float4(float(r[R::V + 2]), cs, prho, mor);
   }
 }
-// The FP64 isotropic pair kernel's record, 96 B per slot in two planes so that
-// the gathered arrays (230 MB at 2.4 M slots) fit the 256 MB Infinity Cache:
-// plane a (64 B): x y z, 1/h (negative for ghosts), m, 1/rho, c, P/rho^2/omega;
-// plane b (32 B): v, 0.  det H and m/rho are recomputed by the loader.
+// The FP64 isotropic pair kernel's record, 96 B per slot: x y z, 1/h (negative for
+// ghosts), m, 1/rho, c, P/rho^2/omega (a), v, 0 (b).  det H and m/rho are
+// recomputed by the loader.  230 MB at 2.4 M slots fit the 256 MB Infinity Cache,
+// and one plane beats two: the gather brings in 1.5 lines a record instead of 2
+// (loads of all records of the rows at 128^3: 2.15 ms, as 64 + 32 B 2.38 ms, one
+// to a 128-B line 2.55 ms).
 template <int D>
 __device__ __forceinline__ void writeFast64Rec(const double* r, int64_t nInt, double2* __restrict__ a,
                                                double2* __restrict__ b) {
