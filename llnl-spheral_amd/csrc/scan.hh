@@ -13,30 +13,36 @@
 // Up to kScanOnce items one launch does all: a workgroup sums the counts of
 // the tiles before its own by itself, at most 12 extra values a lane.  Beyond,
 // a first launch writes the tiles' sums and the second adds up those before its
-// tile (at most n / 2048).  Measured: 4.5 us for one launch of 8 k items, 9-11 us
-// for the two at 30 k, where one launch took 14-28 us (its last tile counts
-// 28 k items again) and a scan in one workgroup 11 us without the producer and
-// the consumer.
+// tile.  Measured: 4.5 us for one launch of 8 k items; at 30 k 8 us for the two,
+// where one launch took 14-28 us (its last tile counts 28 k items again) and a
+// scan in one workgroup 11 us without the producer and the consumer.
 #pragma once
 #include <cstdint>
+#include <type_traits>
 #include <hip/hip_runtime.h>
 
 namespace sphgpu {
 
 constexpr int kScanBlock = 512;
-constexpr int kScanPer = 4;
-constexpr int kScanTile = kScanBlock * kScanPer;
-constexpr int64_t kScanOnce = 4 * int64_t(kScanTile);
+constexpr int64_t kScanOnce = 8192;
+// Items a lane.  A GhostPlane's ones lie together (a face of a lattice), so a tile
+// may emit all of its items, four rounds of dependent loads at four a lane: 11.0 us
+// for the second launch at 82 k rows, 6.4 us at one a lane, where its tiles fill the
+// chip as well.  Beyond half a million items each workgroup's pass over the tile
+// sums before it costs more than that gives (2.4 M rows: 31 us at four, 38 at two,
+// 63 at one).
+constexpr int64_t kScanOnePer = 524288;
 
 // The workgroup's tile, given each thread's part of the sum before the tile.
-template <class F>
+template <int PER, class F>
 __device__ __forceinline__ void scanTile(const F& f, int64_t n, int32_t before) {
+  constexpr int kTile = kScanBlock * PER;
   __shared__ int32_t waveSum[kScanBlock / 64], waveBefore[kScanBlock / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t base = blockIdx.x * int64_t(kScanTile) + int64_t(threadIdx.x) * kScanPer;
-  int32_t v[kScanPer], local = 0;
+  const int64_t base = blockIdx.x * int64_t(kTile) + int64_t(threadIdx.x) * PER;
+  int32_t v[PER], local = 0;
 #pragma unroll
-  for (int q = 0; q < kScanPer; ++q) {
+  for (int q = 0; q < PER; ++q) {
     v[q] = base + q < n ? f.value(base + q) : 0;
     local += v[q];
   }
@@ -60,21 +66,21 @@ __device__ __forceinline__ void scanTile(const F& f, int64_t n, int32_t before) 
     run += w < wave ? waveSum[w] : 0;
   }
   if constexpr (F::kCompact) {
-    __shared__ int32_t ones[kScanTile];
+    __shared__ int32_t ones[kTile];
     int32_t at = run;
 #pragma unroll
-    for (int q = 0; q < kScanPer; ++q)
-      if (v[q]) ones[at++] = threadIdx.x * kScanPer + q;
+    for (int q = 0; q < PER; ++q)
+      if (v[q]) ones[at++] = threadIdx.x * PER + q;
     int32_t count = 0;
 #pragma unroll
     for (int w = 0; w < kScanBlock / 64; ++w) count += waveSum[w];
     __syncthreads();
     for (int32_t t = threadIdx.x; t < count; t += kScanBlock)
-      f.emit(blockIdx.x * int64_t(kScanTile) + ones[t], first + t, 1);
+      f.emit(blockIdx.x * int64_t(kTile) + ones[t], first + t, 1);
   } else {
     int32_t at = first + run;
 #pragma unroll
-    for (int q = 0; q < kScanPer; ++q) {
+    for (int q = 0; q < PER; ++q) {
       if (base + q < n) f.emit(base + q, at, v[q]);
       at += v[q];
     }
@@ -84,20 +90,20 @@ __device__ __forceinline__ void scanTile(const F& f, int64_t n, int32_t before) 
 
 template <class F>
 __global__ void __launch_bounds__(kScanBlock) k_scan_once(F f, int64_t n) {
-  const int64_t tile0 = blockIdx.x * int64_t(kScanTile);   // <= n: the grid covers n items
+  const int64_t tile0 = blockIdx.x * int64_t(kScanBlock * 4);   // <= n: the grid covers n items
   int32_t before = 0;
 #pragma unroll 4
   for (int64_t i = threadIdx.x; i < tile0; i += kScanBlock) before += f.value(i);
-  scanTile(f, n, before);
+  scanTile<4>(f, n, before);
 }
 
-template <class F>
+template <int PER, class F>
 __global__ void __launch_bounds__(kScanBlock) k_scan_sums(F f, int64_t n, int32_t* __restrict__ tileSums) {
   __shared__ int32_t waveSum[kScanBlock / 64];
-  const int64_t base = blockIdx.x * int64_t(kScanTile) + threadIdx.x;
+  const int64_t base = blockIdx.x * int64_t(kScanBlock * PER) + threadIdx.x;
   int32_t sum = 0;
 #pragma unroll
-  for (int q = 0; q < kScanPer; ++q) {
+  for (int q = 0; q < PER; ++q) {
     const int64_t i = base + int64_t(q) * kScanBlock;
     if (i < n) sum += f.value(i);
   }
@@ -110,23 +116,26 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_sums(F f, int64_t n, int32_
   }
 }
 
-template <class F>
+template <int PER, class F>
 __global__ void __launch_bounds__(kScanBlock) k_scan_emit(F f, int64_t n, const int32_t* __restrict__ tileSums) {
   int32_t before = 0;
   for (int64_t t = threadIdx.x; t < blockIdx.x; t += kScanBlock) before += tileSums[t];
-  scanTile(f, n, before);
+  scanTile<PER>(f, n, before);
 }
 
 // Runs F over n items (n = 0 still calls total(0)); `tmp` holds the tile sums.
 template <class F> void scanItems(const F& f, int64_t n, DBuf& tmp, hipStream_t st) {
-  const int64_t tiles = n > 0 ? (n + kScanTile - 1) / kScanTile : 1;
-  if (n <= kScanOnce) {
-    hipLaunchKernelGGL(k_scan_once<F>, dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n);
-  } else {
+  auto tilesOf = [n](int per) { return n > 0 ? (n + kScanBlock * per - 1) / (kScanBlock * per) : 1; };
+  auto two = [&](auto per) {
+    constexpr int PER = decltype(per)::value;
+    const int64_t tiles = tilesOf(PER);
     tmp.ensure(sizeof(int32_t) * size_t(tiles));
-    hipLaunchKernelGGL(k_scan_sums<F>, dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n, tmp.as<int32_t>());
-    hipLaunchKernelGGL(k_scan_emit<F>, dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n, tmp.as<int32_t>());
-  }
+    hipLaunchKernelGGL((k_scan_sums<PER, F>), dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n, tmp.as<int32_t>());
+    hipLaunchKernelGGL((k_scan_emit<PER, F>), dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n, tmp.as<int32_t>());
+  };
+  if (n <= kScanOnce) hipLaunchKernelGGL(k_scan_once<F>, dim3(unsigned(tilesOf(4))), dim3(kScanBlock), 0, st, f, n);
+  else if (n <= kScanOnePer) two(std::integral_constant<int, 1>{});
+  else two(std::integral_constant<int, 4>{});
   SG_CHECK_HIP(hipGetLastError());
 }
 
