@@ -410,21 +410,6 @@ struct RowWriter {
       at += n;
     }
   }
-  // push(v) when acc, with the entry shifted in by selects: only the chunk
-  // store is conditional
-  // (ROOM: the caller has shown that the row stays within its capacity)
-  template <bool ROOM = false>
-  __device__ __forceinline__ void pushIf(bool acc, int32_t v) {
-    buf.x = acc ? buf.y : buf.x;
-    buf.y = acc ? buf.z : buf.y;
-    buf.z = acc ? buf.w : buf.z;
-    buf.w = acc ? v : buf.w;
-    cnt += acc ? 1 : 0;
-    if (acc && (cnt & 3) == 0 && (ROOM || cnt <= cap)) {
-      *at = buf;
-      at += n;
-    }
-  }
   __device__ __forceinline__ void finish() {
     const int r = cnt & 3;
     if (r == 0 || cnt > cap) return;
@@ -434,9 +419,43 @@ struct RowWriter {
   }
 };
 
+// RowWriter of the staged search, in fewer instructions an entry: a marker goes
+// in below the entries of the chunk buffer, so the buffer itself tells when the
+// next entry fills it, and only whole chunks are counted.
+struct ChunkWriter {
+  int4 buf;
+  int chunks, room;
+  int64_t n;
+  int4* at;
+  __device__ __forceinline__ ChunkWriter(int4* o, int64_t n_, int64_t k_, int cap)
+      : buf{0, 0, 0, -1}, chunks(0), room(cap / 4), n(n_), at(o + ellChunk(0, n_, k_)) {}
+  // append v when acc, shifted in by selects
+  __device__ __forceinline__ void pushIf(bool acc, int32_t v) {
+    const bool full = acc && buf.x == -1;
+    buf.x = acc ? buf.y : buf.x;
+    buf.y = acc ? buf.z : buf.y;
+    buf.z = acc ? buf.w : buf.z;
+    buf.w = acc ? v : buf.w;
+    if (full) {
+      if (chunks < room) *at = buf;
+      at += n;
+      ++chunks;
+      buf.w = -1;
+    }
+  }
+  // the last chunk, and the row's length (which may pass its capacity)
+  __device__ __forceinline__ int32_t finish() {
+    const int r = buf.w == -1 ? 0 : (buf.z == -1 ? 1 : (buf.y == -1 ? 2 : 3));
+    if (r != 0 && chunks < room)
+      *at = r == 1 ? make_int4(buf.w, 0, 0, 0)
+                   : (r == 2 ? make_int4(buf.z, buf.w, 0, 0) : make_int4(buf.y, buf.z, buf.w, 0));
+    return 4 * chunks + r;
+  }
+};
+
 // Entries and the longest row of a search: summed in the workgroup, one pair
 // of atomics each (flags: [0] longest row, [4..5] entries).
-struct RowStats {
+template <int BS = kBlock> struct RowStats {
   uint32_t sum = 0;
   int32_t most = 0;
   __device__ __forceinline__ void add(int32_t c) {
@@ -445,8 +464,8 @@ struct RowStats {
   }
   // called by every thread of the workgroup
   __device__ __forceinline__ void store(int32_t* __restrict__ flags) {
-    __shared__ uint32_t ws[kBlock / 64];
-    __shared__ int32_t wm[kBlock / 64];
+    __shared__ uint32_t ws[BS / 64];
+    __shared__ int32_t wm[BS / 64];
     for (int sh = 32; sh > 0; sh >>= 1) {
       sum += __shfl_xor(sum, sh);
       const int32_t m = __shfl_xor(most, sh);
@@ -458,7 +477,7 @@ struct RowStats {
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-      for (int w = 1; w < kBlock / 64; ++w) {
+      for (int w = 1; w < BS / 64; ++w) {
         sum += ws[w];
         most = wm[w] > most ? wm[w] : most;
       }
@@ -482,12 +501,20 @@ constexpr int kStaged = kStageEdge * kStageEdge * kStageEdge;
 // with room for 2048 candidates, 1.58 ms with 2240).  2240 is what three
 // workgroups per CU leave room for.
 constexpr int kCandCap = 2240;
+// A brick's outer layers hold 7 x 7 x 6 or 7^3 nodes with the ghosts, more than
+// 256 lanes, and a second round of the walk is as long as the first.  While every
+// brick has a place on the chip at two workgroups of 512 lanes to a CU, one round
+// does (343 bricks: 170 us with 256 lanes, 96 with 512; 500 bricks: 143 and 107);
+// beyond, three workgroups of 256 hide each other's rounds (729 bricks: 190 and
+// 195 us).
+constexpr int kWideBlock = 512;
+constexpr int64_t kWideBricks = 512;
 constexpr int kRunRows = 6;      // one z slab: 5 runs and the sentinel
 
 struct SearchArgs {
   DGrid g;
   double ext, ext2;
-  float lo32, hi32;         // ext2*(1 -+ 1e-5): FP32 classification margins
+  float mid32, half32;      // ext2 and half the band around it that the exact test decides (FP32)
   float prune2, cell32, invCell32;   // staged path: (search radius (1 + 1e-4))^2, cell edge and its inverse (FP32)
   int64_t n, nInt;
   int cap;
@@ -504,7 +531,8 @@ __device__ __forceinline__ bool exactIso(double rx, double ry, double rz, double
   return (e2i <= ext2 || e2j <= ext2);
 }
 
-__global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restrict__ rec, const int32_t* __restrict__ cellStart,
+template <int BS>
+__global__ void __launch_bounds__(BS) k_search_staged(const double* __restrict__ rec, const int32_t* __restrict__ cellStart,
                                                          SearchArgs a, int32_t* __restrict__ rowCount,
                                                          int4* __restrict__ nbr, int32_t* __restrict__ flags) {
   using R = RL<true>;
@@ -515,8 +543,9 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
   // lane-strided; up to 5 runs and the sentinel the reader stays on past them.
   // Before the runs are formed the same memory holds each staged cell's first
   // slot and the scan's partial sums (52 KB in all: three workgroups per CU)
-  __shared__ uint32_t sRun[kRunRows * kBlock];
-  static_assert(kRunRows * kBlock >= kStaged + kBlock, "sStart and sc alias the run table");
+  __shared__ uint32_t sRun[kRunRows * BS];
+  __shared__ int32_t sMembers;                     // bits of the staged cells' member counts
+  static_assert(kRunRows * BS >= kStaged + BS / 64, "sStart and sc alias the run table");
   int32_t* const sStart = reinterpret_cast<int32_t*>(sRun);
   int32_t* const sc = sStart + kStaged;
   const DGrid& g = a.g;
@@ -525,11 +554,11 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
   const int bx = b % g.nb[0], by = (b / g.nb[0]) % g.nb[1], bz = b / (g.nb[0] * g.nb[1]);
   const int64_t h0 = cellStart[int64_t(b) * 64], h1 = cellStart[int64_t(b) * 64 + 64];
   if (h0 == h1) return;                           // uniform over the block
-  RowStats stats;
+  RowStats<BS> stats;
   const int cx0 = bx * 4 - 2, cy0 = by * 4 - 2, cz0 = bz * 4 - 2;
   const double ox = g.lo[0] + (bx * 4) * g.cell, oy = g.lo[1] + (by * 4) * g.cell, oz = g.lo[2] + (bz * 4) * g.cell;
   // staged cell table (x fastest)
-  for (int t = threadIdx.x; t < kStaged; t += blockDim.x) {
+  for (int t = threadIdx.x; t < kStaged; t += BS) {
     const int sx = t % kStageEdge, sy = (t / kStageEdge) % kStageEdge, sz = t / (kStageEdge * kStageEdge);
     const int cx = cx0 + sx, cy = cy0 + sy, cz = cz0 + sz;
     int32_t st = 0, cnt = 0;
@@ -541,31 +570,46 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
     sStart[t] = st;
     sOff[t + 1] = cnt;
   }
-  if (threadIdx.x == 0) sOff[0] = 0;
+  if (threadIdx.x == 0) {
+    sOff[0] = 0;
+    sMembers = 0;
+  }
   __syncthreads();
-  // inclusive scan of sOff[1..512] (two elements per thread)
+  // inclusive scan of sOff[1..512], kStaged / BS elements a thread: within the
+  // wavefront, then over the wavefronts' sums
   {
-    const int t0 = 2 * threadIdx.x + 1, t1 = t0 + 1;
-    const int32_t v0 = sOff[t0], v1 = sOff[t1];
-    const int32_t pair = v0 + v1;
-    sc[threadIdx.x] = pair;
-    __syncthreads();
-    for (int s = 1; s < kBlock; s <<= 1) {
-      const int32_t add = threadIdx.x >= s ? sc[threadIdx.x - s] : 0;
-      __syncthreads();
-      sc[threadIdx.x] += add;
-      __syncthreads();
+    constexpr int PER = kStaged / BS;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int32_t v[PER], own = 0;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      v[q] = sOff[PER * threadIdx.x + 1 + q];
+      own += v[q];
+      if (v[q]) atomicOr(&sMembers, v[q]);
     }
-    const int32_t excl = sc[threadIdx.x] - pair;
-    sOff[t0] = excl + v0;
-    sOff[t1] = excl + v0 + v1;
+    int32_t incl = own;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int32_t up = __shfl_up(incl, d);
+      if (lane >= d) incl += up;
+    }
+    if (lane == 63) sc[wave] = incl;
+    __syncthreads();
+    int32_t run = incl - own;
+#pragma unroll
+    for (int w = 0; w < BS / 64; ++w) run += w < wave ? sc[w] : 0;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+      run += v[q];
+      sOff[PER * threadIdx.x + 1 + q] = run;
+    }
   }
   __syncthreads();
   const int32_t total = sOff[kStaged];
-  const bool staged = total <= kCandCap;
+  const bool staged = total < kCandCap;           // and one more: the candidate that no node takes
   int ghosts = 0;
   if (staged) {
-    for (int t = threadIdx.x; t < kStaged; t += blockDim.x) {
+    for (int t = threadIdx.x; t < kStaged; t += BS) {
       const int32_t o = sOff[t], cnt = sOff[t + 1] - o, st = sStart[t];
       for (int q = 0; q < cnt; ++q) {
         const double4 r = *reinterpret_cast<const double4*>(rec + int64_t(st + q) * R::STRIDE);
@@ -576,6 +620,10 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
         sSlot[o + q] = int32_t(uint32_t(st + q) | (ghost ? 0x80000000u : 0u));
       }
     }
+    if (threadIdx.x == 0) {
+      sCand[total] = make_float4(1.0e30f, 0.0f, 0.0f, 1.0f);
+      sSlot[total] = 0;
+    }
   } else if (threadIdx.x == 0) {
     atomicAdd(&flags[1], 1);                      // bricks that read candidates from global memory
   }
@@ -585,128 +633,138 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
   const bool marks =
       __builtin_amdgcn_readfirstlane(__syncthreads_or(ghosts)) != 0 && a.keepSlot != nullptr;
 
+  const int steps = 32 - __builtin_clz(__builtin_amdgcn_readfirstlane(sMembers) | 1);   // bisections of a cell
   // One lane per node; the node's 25 (dz, dy) runs of up to 5 staged cells
   // are contiguous candidate ranges in LDS.  Rows leave as int4 chunks, one
   // per lane, contiguous across a wavefront's slots.  Bricks whose candidates
   // exceed the stage read them from the records in global memory.
   // the cell table's first slots are read again only by bricks that are not
   // staged, which write no runs
-  for (int64_t k = h0 + threadIdx.x; k < h1; k += blockDim.x) {
+  for (int64_t k = h0 + threadIdx.x; k < h1; k += BS) {
     const double* ri = rec + k * R::STRIDE;
     if (int64_t(ri[R::ORIG]) >= a.nInt) { rowCount[k] = 0; continue; }
     const double xi = ri[R::X], yi = ri[R::X + 1], zi = ri[R::X + 2], hi = ri[R::HINV];
     const float fx = float(xi - ox), fy = float(yi - oy), fz = float(zi - oz);
-    const float hi2 = float(hi) * float(hi);
+    const int32_t hi2 = __float_as_int(float(hi) * float(hi));
     int c[3];
     const double xv[3] = {xi, yi, zi};
     cellCoords<3>(g, xv, c);
     const int sx = c[0] - cx0, sy = c[1] - cy0, sz = c[2] - cz0;   // in [2, 5]
-    RowWriter row(nbr, a.n, k, a.cap);
+    ChunkWriter row(nbr, a.n, k, a.cap);
     if (staged) {
       for (int dz = -2; dz <= 2; ++dz) {
         // 1. the node's non-empty runs of this z slab, in dy order, into its
         //    column of the run table: the candidates of each (dz, dy) row of
         //    staged cells inside the x chord of a sphere of the search radius
-        //    (with a 1e-4 margin) around the node
-        int nr = 0, nCand = 0;
-        {
-          // distance from the node to the cell slab along z (staged cell t spans
-          // [(t - 2) c, (t - 1) c) in brick-origin offsets)
-          const float zlo = float(sz + dz - 2) * a.cell32, zhi = zlo + a.cell32;
-          const float dzm = fz < zlo ? zlo - fz : (fz > zhi ? fz - zhi : 0.f);
-          for (int dy = -2; dy <= 2; ++dy) {
-            const float ylo = float(sy + dy - 2) * a.cell32, yhi = ylo + a.cell32;
-            const float dym = fy < ylo ? ylo - fy : (fy > yhi ? fy - yhi : 0.f);
-            const float rem2 = a.prune2 - (dzm * dzm + dym * dym);
-            if (rem2 < 0.f) continue;
-            const float rem = __builtin_sqrtf(rem2);
-            int x0 = int(floorf((fx - rem) * a.invCell32)) + 2, x1 = int(floorf((fx + rem) * a.invCell32)) + 2;
-            x0 = x0 < sx - 2 ? sx - 2 : x0;
-            x1 = x1 > sx + 2 ? sx + 2 : x1;
-            if (x0 > x1) continue;
-            const int rowb = ((sz + dz) * kStageEdge + (sy + dy)) * kStageEdge;
-            // the members of a cell are in x order: the chord [fx - rem, fx + rem]
-            // starts and ends inside the end cells, found by two bisections
-            int32_t t0 = sOff[rowb + x0], t1 = sOff[rowb + x1 + 1];
-            {
-              int32_t lo = t0, up = sOff[rowb + x0 + 1];
-              const float key = fx - rem;
-              while (lo < up) {
-                const int32_t mid = (lo + up) >> 1;
-                const bool below = sCand[mid].x < key;
-                lo = below ? mid + 1 : lo;
-                up = below ? up : mid;
-              }
-              t0 = lo;
-            }
-            {
-              int32_t lo = sOff[rowb + x1], up = t1;
-              const float key = fx + rem;
-              while (lo < up) {
-                const int32_t mid = (lo + up) >> 1;
-                const bool inside = sCand[mid].x <= key;
-                lo = inside ? mid + 1 : lo;
-                up = inside ? up : mid;
-              }
-              t1 = lo;
-            }
-            if (t1 > t0) {
-              sRun[nr++ * kBlock + threadIdx.x] = uint32_t(t0) | (uint32_t(t1) << 16);
-              nCand += t1 - t0;
-            }
+        //    (with a 1e-4 margin) around the node.  The members of a cell are in
+        //    x order, so the chord's ends inside the end cells are bisections, and
+        //    the slab's ten run side by side, as many steps as the largest staged
+        //    cell needs: one after the other, each with its own loop, they took a
+        //    fifth of the kernel waiting for LDS.
+        int32_t lo[10], up[10];
+        float key[5], rem[5];
+        // distance from the node to the cell slab along z (staged cell t spans
+        // [(t - 2) c, (t - 1) c) in brick-origin offsets)
+        const float zlo = float(sz + dz - 2) * a.cell32, zhi = zlo + a.cell32;
+        const float dzm = fz < zlo ? zlo - fz : (fz > zhi ? fz - zhi : 0.f);
+#pragma unroll
+        for (int y = 0; y < 5; ++y) {
+          const int dy = y - 2;
+          const float ylo = float(sy + dy - 2) * a.cell32, yhi = ylo + a.cell32;
+          const float dym = fy < ylo ? ylo - fy : (fy > yhi ? fy - yhi : 0.f);
+          const float rem2 = a.prune2 - (dzm * dzm + dym * dym);
+          rem[y] = __builtin_sqrtf(rem2 < 0.f ? 0.f : rem2);
+          int x0 = int(floorf((fx - rem[y]) * a.invCell32)) + 2, x1 = int(floorf((fx + rem[y]) * a.invCell32)) + 2;
+          x0 = x0 < sx - 2 ? sx - 2 : x0;
+          x1 = x1 > sx + 2 ? sx + 2 : x1;
+          const bool any = rem2 >= 0.f && x0 <= x1;
+          const int rowb = ((sz + dz) * kStageEdge + (sy + dy)) * kStageEdge;
+          const int c0 = any ? rowb + x0 : 0, c1 = any ? rowb + x1 : 0;
+          lo[y] = sOff[c0];
+          up[y] = sOff[c0 + 1];
+          lo[5 + y] = sOff[c1];
+          up[5 + y] = any ? sOff[c1 + 1] : -1;     // (-1: no run)
+          key[y] = fx - rem[y];
+        }
+        for (int st = 0; st < steps; ++st) {
+          float x[10];
+          int32_t mid[10];
+#pragma unroll
+          for (int q = 0; q < 10; ++q) {
+            mid[q] = (lo[q] + up[q]) >> 1;
+            x[q] = sCand[mid[q] < 0 ? 0 : mid[q]].x;
+          }
+#pragma unroll
+          for (int q = 0; q < 10; ++q) {
+            const bool before = q < 5 ? x[q] < key[q] : x[q] <= fx + rem[q - 5];
+            const bool open = lo[q] < up[q];
+            lo[q] = open && before ? mid[q] + 1 : lo[q];
+            up[q] = open && !before ? mid[q] : up[q];
           }
         }
+        int nr = 0, nCand = 0;
+#pragma unroll
+        for (int y = 0; y < 5; ++y) {
+          const int32_t t0 = lo[y], t1 = up[5 + y] < 0 ? -1 : lo[5 + y];
+          if (t1 > t0) {
+            sRun[nr++ * BS + threadIdx.x] = uint32_t(4 * t0) | (uint32_t(4 * t1) << 16);
+            nCand += t1 - t0;
+          }
+        }
+        sRun[nr * BS + threadIdx.x] = uint32_t(4 * total);
         // 2. one walk over the slab's candidates: a wavefront iterates as often
         //    as its longest candidate list in the slab, not its longest run in
         //    every (dz, dy) row.  Candidates are read two ahead of their test (three
         //    register sets in rotation); the reader steps through the runs with
-        //    no branch and, past the last candidate, stays on the sentinel run
-        //    (candidate 0), so every index it forms stays inside the tables.
-        //    The rare paths (the exact FP64 test, ghost marks) are entered only
-        //    when some lane of the wavefront needs them.
+        //    no branch and, past the last one, stays on the sentinel run, the
+        //    candidate that no node takes: a lane that has finished its list
+        //    needs no test and no branch of its own.  (Runs hold 4 t: the byte
+        //    offsets of the slots.)  Two thirds of the kernel's time issue VALU
+        //    instructions, so the walk counts them: the row's state is one marker
+        //    in its chunk buffer.  With the bisections side by side: 1.58 -> 1.50 ms
+        //    at 128^3.  The rare paths (the exact FP64 test, ghost marks) are
+        //    entered only when some lane of the wavefront needs them.
         // one instance of the walk with ghost marks and one without, chosen by
-        // the block-uniform flag
-        // plain: no lane of the wavefront can meet itself in this slab (only
-        // the dz = 0 slab holds the node's own cell) or pass its row capacity
-        // in it, so the walk skips both checks
-        auto walk = [&](auto marksOn, auto plainOn) {
-          constexpr bool plain = decltype(plainOn)::value;
-          sRun[nr * kBlock + threadIdx.x] = 0u;
+        // the block-uniform flag; another pair for the slab that holds the node
+        auto walk = [&](auto marksOn, auto selfOn) {
           const uint32_t first = sRun[threadIdx.x];
           int32_t t = int32_t(first & 0xffffu), tEnd = int32_t(first >> 16);
-          uint32_t nxt = sRun[kBlock + threadIdx.x];
-          int at = kBlock + int(threadIdx.x);               // where nxt came from
-          const int last = nr * kBlock + int(threadIdx.x);  // the sentinel
+          const int last = nr * BS + int(threadIdx.x);      // the sentinel
+          int at = nr > 0 ? BS + int(threadIdx.x) : last;   // where nxt came from
+          uint32_t nxt = sRun[at];
           auto advance = [&]() {
-            const bool same = t + 1 < tEnd;
-            const int next = at + kBlock < last ? at + kBlock : last;
-            t = same ? t + 1 : int32_t(nxt & 0xffffu);
+            const bool same = t + 4 < tEnd;
+            const int next = at + BS < last ? at + BS : last;
+            t = same ? t + 4 : int32_t(nxt & 0xffffu);
             tEnd = same ? tEnd : int32_t(nxt >> 16);
             at = same ? at : next;
             nxt = sRun[at];
           };
           auto read = [&](float4& c, int32_t& raw) {
-            c = sCand[t];
-            raw = sSlot[t];
+            c = *static_cast<const float4*>(
+                __builtin_assume_aligned(reinterpret_cast<const char*>(sCand) + 4 * t, 16));
+            raw = *reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(sSlot) + t);
           };
           auto test = [&](const float4 cj, const int32_t raw) {
             const float rx = fx - cj.x, ry = fy - cj.y, rz = fz - cj.z;
             // FP32 estimate of min(h_i^2, h_j^2) |r|^2: fused products (any
             // rounding change stays inside the band that takes the exact test);
-            // q min(a, b) = min(q a, q b) exactly for q >= 0
+            // q min(a, b) = min(q a, q b) exactly for q >= 0, and positive floats
+            // compare as their bits
             const float q = __builtin_fmaf(rz, rz, __builtin_fmaf(ry, ry, rx * rx));
-            const float tmin = q * (cj.w < hi2 ? cj.w : hi2);
-            bool in = tmin < a.lo32;
-            const bool band = (tmin >= a.lo32) & (tmin <= a.hi32);
+            const int32_t wj = __float_as_int(cj.w);
+            const float d = q * __int_as_float(wj < hi2 ? wj : hi2) - a.mid32;
+            bool in = d < -a.half32;
+            const bool band = fabsf(d) <= a.half32;
             const int32_t sj = raw & 0x7fffffff;
-            // the exact test in the rare band (the branch is skipped when no
-            // lane of the wavefront takes it)
-            if (band) {
-              const double* rj = rec + int64_t(sj) * R::STRIDE;
-              in = exactIso(xi - rj[R::X], yi - rj[R::X + 1], zi - rj[R::X + 2], hi, rj[R::HINV], a.ext2);
+            if (__any(band)) {
+              if (band) {
+                const double* rj = rec + int64_t(sj) * R::STRIDE;
+                in = exactIso(xi - rj[R::X], yi - rj[R::X + 1], zi - rj[R::X + 2], hi, rj[R::HINV], a.ext2);
+              }
             }
-            const bool acc = in && (plain || sj != int32_t(k));
-            row.template pushIf<plain>(acc, sj);
+            const bool acc = decltype(selfOn)::value ? in && sj != int32_t(k) : in;
+            row.pushIf(acc, sj);
             if constexpr (decltype(marksOn)::value) {
               if (acc && raw < 0) a.keepSlot[sj] = 1;
             }
@@ -717,29 +775,26 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
           advance();
           read(c1, s1);
           advance();
-          for (int left = nCand;;) {
+          for (int done = 3;; done += 3) {
             read(c2, s2);
             advance();
             test(c0, s0);
-            if (--left == 0) break;
             read(c0, s0);
             advance();
             test(c1, s1);
-            if (--left == 0) break;
             read(c1, s1);
             advance();
             test(c2, s2);
-            if (--left == 0) break;
+            if (!__any(done < nCand)) break;
           }
         };
-        if (nr > 0) {
-          const bool plain = dz != 0 && __all(row.cnt + nCand <= a.cap);
+        if (__any(nr > 0)) {
           if (marks) {
-            if (plain) walk(std::true_type{}, std::true_type{});
-            else walk(std::true_type{}, std::false_type{});
+            if (dz != 0) walk(std::true_type{}, std::false_type{});
+            else walk(std::true_type{}, std::true_type{});
           } else {
-            if (plain) walk(std::false_type{}, std::true_type{});
-            else walk(std::false_type{}, std::false_type{});
+            if (dz != 0) walk(std::false_type{}, std::false_type{});
+            else walk(std::false_type{}, std::true_type{});
           }
         }
       }
@@ -755,7 +810,7 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
               if (sj == int32_t(k)) continue;
               const double* rj = rec + int64_t(sj) * R::STRIDE;
               if (exactIso(xi - rj[R::X], yi - rj[R::X + 1], zi - rj[R::X + 2], hi, rj[R::HINV], a.ext2)) {
-                row.push(sj);
+                row.pushIf(true, sj);
                 if (a.keepSlot && rj[R::ORIG] >= double(a.nInt)) a.keepSlot[sj] = 1;
               }
             }
@@ -763,9 +818,9 @@ __global__ void __launch_bounds__(kBlock) k_search_staged(const double* __restri
         }
       }
     }
-    row.finish();
-    rowCount[k] = row.cnt;
-    stats.add(row.cnt);
+    const int32_t cnt = row.finish();
+    rowCount[k] = cnt;
+    stats.add(cnt);
   }
   stats.store(flags);
 }
@@ -861,7 +916,7 @@ __global__ void __launch_bounds__(kBlock) k_search_global(const double* __restri
                                                           SegGrids sg, int32_t* __restrict__ rowCount,
                                                           int4* __restrict__ nbr, int32_t* __restrict__ flags) {
   const int64_t k = xcdBlock((a.n + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
-  RowStats stats;
+  RowStats<> stats;
   if (k < a.n) {
     const int32_t c = searchRow<D, ISO>(k, rec, cellStart, a, sg, nbr);
     rowCount[k] = c;
@@ -1325,8 +1380,8 @@ void buildNeighborsD(Sim& s, double ext) {
   // products.  The band is four times that, and never narrower than 1e-5.
   const double ratio = hb[8] / hb[6];
   const double band = std::max(1.0e-5, 4.0 * (1.44e-6 * ratio + 5.0e-7));
-  sa.lo32 = float(sa.ext2 * (1.0 - band));
-  sa.hi32 = float(sa.ext2 * (1.0 + band));
+  sa.mid32 = float(sa.ext2);
+  sa.half32 = float(sa.ext2 * band);
   {
     const double Rm = ext / hb[6] * (1.0 + 1.0e-6) * (1.0 + 1.0e-4);
     sa.prune2 = float(Rm * Rm);
@@ -1350,9 +1405,13 @@ void buildNeighborsD(Sim& s, double ext) {
       zeroMany(z, s.stream);
     }
     if (stagedPath) {
-      hipLaunchKernelGGL(k_search_staged, dim3(int(xcdGrid(bricks))), dim3(kBlock), 0, st, s.rec.as<double>(),
-                         s.cellStart.as<int32_t>(), sa, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
-                         s.flags.as<int32_t>());
+      auto staged = [&](auto kern, int bs) {
+        hipLaunchKernelGGL(kern, dim3(int(xcdGrid(bricks))), dim3(bs), 0, st, s.rec.as<double>(),
+                           s.cellStart.as<int32_t>(), sa, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
+                           s.flags.as<int32_t>());
+      };
+      if (bricks <= kWideBricks) staged(k_search_staged<kWideBlock>, kWideBlock);
+      else staged(k_search_staged<kBlock>, kBlock);
     } else if (s.isotropic) {
       hipLaunchKernelGGL((k_search_global<D, true>), dim3(int(xcdGrid(nblocks(n)))), dim3(kBlock), 0, st, s.rec.as<double>(),
                          s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
