@@ -492,7 +492,8 @@ struct KeepScan {
   const int64_t* gen;       // gen[1 + b]: the rows before plane b's ghosts
   int nSubs;
   const int32_t* flags;
-  int32_t *flagsOut, *starts;
+  SearchFlags* flagsOut;
+  int32_t* starts;
   __device__ int32_t value(int64_t g) const { return slotKeep[iperm[nInt + g]] != 0 || isControl[g] != 0 ? 1 : 0; }
   __device__ void emit(int64_t g, int32_t prefix, int32_t v) const {
     keep[g] = v;
@@ -504,7 +505,7 @@ struct KeepScan {
     for (int b = 0; b < nSubs; ++b)
       if (gen[1 + b] - nInt >= ng) starts[b] = t;
     starts[nSubs] = t;
-    for (int q = 0; q < 8; ++q) flagsOut[q] = flags[q];
+    *flagsOut = foldFlags(flags);
   }
 };
 
@@ -671,7 +672,7 @@ void finishGeneration(Sim& s, const int64_t* gen) {
 // values) and the search flags copied to pinned memory, read after the
 // caller's next wait.  The neighbour build issues it before its row readback so
 // that one wait serves both.
-void cullLaunch(Sim& s, int32_t* flagsOut, int32_t* starts) {
+void cullLaunch(Sim& s, SearchFlags* flagsOut, int32_t* starts) {
   const int64_t ng = s.nTot - s.nInt;
   s.keep.ensure(sizeof(int32_t) * size_t(ng));
   s.keepScan.ensure(sizeof(int32_t) * size_t(ng));

@@ -400,9 +400,27 @@ int32_t* queueIsotropyTest(Sim& s, const double* H, int64_t rows);
 // A derivative field's internal rows (comps doubles each, src in slot order) in
 // the caller's order: a workspace, valid until the next call.
 const double* unsortDerivative(Sim& s, const double* src, int comps);
+// The search's flags on the device: [1] bricks that read candidates from global
+// memory, then kRowBins bins a cache line apart, [0] longest row and [2..3]
+// entries.  Workgroups spread over the bins: at 33 ns an atomic, one word held
+// 62 k workgroups of a search up for 2 ms.
+constexpr int kRowBins = 32, kRowBinStride = 16, kSearchFlags = kRowBinStride * (kRowBins + 1);
+struct SearchFlags {
+  int32_t longest, fallbacks;
+  unsigned long long entries;
+};
+__host__ __device__ inline SearchFlags foldFlags(const int32_t* f) {
+  SearchFlags o{0, f[1], 0};
+  for (int b = 0; b < kRowBins; ++b) {
+    const int32_t* q = f + kRowBinStride * (b + 1);
+    o.longest = q[0] > o.longest ? q[0] : o.longest;
+    o.entries += *reinterpret_cast<const unsigned long long*>(q + 2);
+  }
+  return o;
+}
 // First half of the ghost cull: keep flags and scan, the planes' new first
 // ghosts and the search flags to pinned memory.
-void cullLaunch(Sim& s, int32_t* flagsOut, int32_t* starts);
+void cullLaunch(Sim& s, SearchFlags* flagsOut, int32_t* starts);
 // Counts of a ghost generation, read back with the neighbour build's bounds;
 // throws GhostCapacity when its capacity was short.
 struct GhostCapacity {};

@@ -386,42 +386,12 @@ __global__ void __launch_bounds__(kBlock) k_cell_order(const int32_t* __restrict
   packRow<D, ISO, SEC>(k, i, loadPackRow<D, ISO>(i, in), o);
 }
 
-// Row writer: keeps four entries in registers and stores them as one int4.
-// Each entry is shifted in at w, so after every fourth the buffer holds them
-// oldest first with no branch on the position; the last partial chunk is
-// aligned once per row.  Entries past the row length are zero.  `at` walks
-// the row's chunks (ellChunk(c, n, k) = c n + k).
-struct RowWriter {
-  int4 buf;
-  int cnt;
-  int cap;
-  int64_t n;
-  int4* at;
-  __device__ __forceinline__ RowWriter(int4* o, int64_t n_, int64_t k_, int cap_)
-      : buf{0, 0, 0, 0}, cnt(0), cap(cap_), n(n_), at(o + ellChunk(0, n_, k_)) {}
-  __device__ __forceinline__ void push(int32_t v) {
-    buf.x = buf.y;
-    buf.y = buf.z;
-    buf.z = buf.w;
-    buf.w = v;
-    ++cnt;
-    if ((cnt & 3) == 0 && cnt <= cap) {
-      *at = buf;
-      at += n;
-    }
-  }
-  __device__ __forceinline__ void finish() {
-    const int r = cnt & 3;
-    if (r == 0 || cnt > cap) return;
-    const int4 o = r == 1 ? make_int4(buf.w, 0, 0, 0)
-                          : (r == 2 ? make_int4(buf.z, buf.w, 0, 0) : make_int4(buf.y, buf.z, buf.w, 0));
-    *at = o;
-  }
-};
-
-// RowWriter of the staged search, in fewer instructions an entry: a marker goes
-// in below the entries of the chunk buffer, so the buffer itself tells when the
-// next entry fills it, and only whole chunks are counted.
+// Row writer of one lane: keeps up to four entries in registers and stores them as
+// one int4.  Each entry is shifted in at w and a marker goes in below them, so the
+// buffer itself tells when the next entry fills it, and only whole chunks are
+// counted; the last partial chunk is aligned once per row, zeros after its
+// entries.  `at` walks the row's chunks (ellChunk(c, n, k) = c n + k).  Capacities
+// are multiples of 4.
 struct ChunkWriter {
   int4 buf;
   int chunks, room;
@@ -454,7 +424,7 @@ struct ChunkWriter {
 };
 
 // Entries and the longest row of a search: summed in the workgroup, one pair
-// of atomics each (flags: [0] longest row, [4..5] entries).
+// of atomics each, in the workgroup's bin of the flags.
 template <int BS = kBlock> struct RowStats {
   uint32_t sum = 0;
   int32_t most = 0;
@@ -482,8 +452,9 @@ template <int BS = kBlock> struct RowStats {
         most = wm[w] > most ? wm[w] : most;
       }
       if (sum) {
-        atomicAdd(reinterpret_cast<unsigned long long*>(flags + 4), (unsigned long long)sum);
-        if (most > *static_cast<volatile int32_t*>(flags)) atomicMax(flags, most);
+        int32_t* bin = flags + kRowBinStride * (1 + blockIdx.x % kRowBins);
+        atomicAdd(reinterpret_cast<unsigned long long*>(bin + 2), (unsigned long long)sum);
+        if (most > *static_cast<volatile int32_t*>(bin)) atomicMax(bin, most);
       }
     }
   }
@@ -827,11 +798,32 @@ __global__ void __launch_bounds__(BS) k_search_staged(const double* __restrict__
 
 // ---------------------------------------------------------------------------
 // Global search: any dimension, any H (cell edge = R, 3^nu stencil).
+//
+// Bound by the latency of its candidates' records: one after the other, a row took
+// 50 us in 2-D and 400 us in 3-D however few rows there were.  L consecutive lanes
+// walk a node's candidates in order, L at a time: the lanes that accept theirs
+// append them at once, each at its place among them, so the row is the one that a
+// single lane writes.  One lane to a node takes four candidates of a cell at a
+// time and writes its row in chunks, which is less work where there are rows
+// enough to fill the chip.
 // ---------------------------------------------------------------------------
-template <int D, bool ISO>
-__device__ __forceinline__ int32_t searchRow(int64_t k, const double* __restrict__ rec,
+// Lanes to a node, by slots: the lines lie where the measured times cross (one by
+// one as before / 1 / 4 / 16 lanes, us).
+//   1-D 200 7.2 / 6.6 / 5.8 / 4.9, 2 k 9.4 / 8.6 / 4.3 / 3.4, 20 k 10.3 / 8.5 / 6.0 / 8.5,
+//       100 k 21 / 12 / 16 / 30, 1 M 276 / 104 / 125 / 267
+//   2-D 1 k 50 / 38 / 20 / 9, 10 k 54 / 42 / 19 / 14, 48 k 54 / 43 / 36 / 44,
+//       250 k 128 / 92 / 142 / 171
+//   3-D 1.7 k 432 / 313 / 132 / 48, 14 k 403 / 299 / 164 / 127, 33 k 405 / 303 / 279 / 219,
+//       111 k 653 / 606 / 723 / 725
+inline int searchLanes(int dim, int64_t slots) {
+  if (slots > 65536) return 1;
+  if (dim == 2) return slots <= 16384 ? 16 : 4;
+  return dim == 1 ? 4 : 16;
+}
+template <int D, bool ISO, int L>
+__device__ __forceinline__ int32_t searchRow(int64_t k, int sub, const double* __restrict__ rec,
                                              const int32_t* __restrict__ cellStart, const SearchArgs& a,
-                                             const SegGrids& sg, int4* __restrict__ nbr) {
+                                             const SegGrids& sg, int32_t* __restrict__ nbr) {
   using R = RL<ISO>;
   const double* ri_ = rec + k * R::STRIDE;
   const int64_t oi = int64_t(ri_[R::ORIG]);
@@ -843,84 +835,167 @@ __device__ __forceinline__ int32_t searchRow(int64_t k, const double* __restrict
     gb = sg.first[m + 1];
   }
   constexpr int NS = NSym<D>::value;
-  V<D> ri; S<D> Hi;
+  auto loadH = [](const double* r) {
+    S<D> H;
+    if constexpr (ISO) {
+      for (int c = 0; c < NS; ++c) H.c[c] = 0.0;
+      for (int c = 0; c < D; ++c) H.c[sdiag<D>(c)] = r[RL<true>::HINV];
+    } else {
+      for (int c = 0; c < NS; ++c) H.c[c] = r[RL<false>::H + c];
+    }
+    return H;
+  };
+  V<D> ri;
   for (int c = 0; c < D; ++c) ri.c[c] = ri_[R::X + c];
-  if constexpr (ISO) {
-    for (int c = 0; c < NS; ++c) Hi.c[c] = 0.0;
-    for (int c = 0; c < D; ++c) Hi.c[sdiag<D>(c)] = ri_[RL<true>::HINV];
-  } else {
-    for (int c = 0; c < NS; ++c) Hi.c[c] = ri_[RL<false>::H + c];
-  }
+  const S<D> Hi = loadH(ri_);
   // own search radius bound (only needed with several levels)
   double Ri = 0.0;
   if (gb - ga > 1) {
     if constexpr (ISO) Ri = a.ext / ri_[RL<true>::HINV] * (1.0 + 1.0e-6);
     else Ri = a.ext / gershgorinMin<D>(Hi.c) * (1.0 + 1.0e-6);
   }
-  RowWriter row(nbr, a.n, k, a.cap);
+  ChunkWriter row(reinterpret_cast<int4*>(nbr), a.n, k, a.cap);     // L = 1
+  int32_t cnt = 0;
+  const unsigned long long below = ((1ull << sub) - 1ull) << (threadIdx.x & 63 & ~(L - 1));
+  const unsigned long long group = ((1ull << L) - 1ull) << (threadIdx.x & 63 & ~(L - 1));
+  auto hit = [&](int32_t j) {
+    const double* rj_ = rec + int64_t(j) * R::STRIDE;
+    V<D> rij;
+    for (int c = 0; c < D; ++c) rij.c[c] = ri.c[c] - rj_[R::X + c];
+    double eta2i, eta2j;
+    if constexpr (ISO) {
+      // the products with zeros left out: the same sums for finite positions
+      const double hi = Hi.c[0], hj = rj_[RL<true>::HINV];
+      V<D> ei, ej;
+      for (int c = 0; c < D; ++c) {
+        ei.c[c] = hi * rij.c[c];
+        ej.c[c] = hj * rij.c[c];
+      }
+      eta2i = vmag2(ei);
+      eta2j = vmag2(ej);
+    } else {
+      eta2i = vmag2(sdot(Hi, rij));
+      eta2j = vmag2(sdot(loadH(rj_), rij));
+    }
+    return (eta2i <= a.ext2) | (eta2j <= a.ext2);
+  };
+  auto append = [&](bool in, int32_t j) {
+    const unsigned long long m = __ballot(in);
+    if (in) {
+      const int32_t at = cnt + __popcll(m & below);
+      if (at < a.cap) nbr[ellIndex(at, a.n, k)] = j;
+      if (a.keepSlot && rec[int64_t(j) * R::STRIDE + R::ORIG] >= double(a.nInt)) a.keepSlot[j] = 1;
+    }
+    cnt += __popcll(m & group);
+  };
   for (int q = ga; q < gb; ++q) {
-  const DGrid g = sg.g ? sg.g[q] : a.g;
-  const int64_t base = sg.g ? sg.base[q] : 0;
-  // cells that can hold a neighbour: the 3^nu stencil when the grid's cell
-  // covers both radii (nodes of a grid have radius <= its cell), else every
-  // cell within Ri
-  int c0[3] = {0, 0, 0}, c1[3] = {0, 0, 0};
-  {
-    int cc[3];
-    cellCoords<D>(g, ri.c, cc);
-    for (int d = 0; d < D; ++d) {
-      if (Ri <= g.cell) {
-        c0[d] = cc[d] - 1 < 0 ? 0 : cc[d] - 1;
-        c1[d] = cc[d] + 1 >= g.nc[d] ? g.nc[d] - 1 : cc[d] + 1;
-      } else {
-        const double t0 = floor((ri.c[d] - Ri - g.lo[d]) * g.invCell), t1 = floor((ri.c[d] + Ri - g.lo[d]) * g.invCell);
-        c0[d] = t0 < 0.0 ? 0 : (t0 > double(g.nc[d] - 1) ? g.nc[d] - 1 : int(t0));
-        c1[d] = t1 < 0.0 ? 0 : (t1 > double(g.nc[d] - 1) ? g.nc[d] - 1 : int(t1));
+    const DGrid g = sg.g ? sg.g[q] : a.g;
+    const int64_t base = sg.g ? sg.base[q] : 0;
+    // cells that can hold a neighbour: the 3^nu stencil when the grid's cell
+    // covers both radii (nodes of a grid have radius <= its cell), else every
+    // cell within Ri
+    int c0[3] = {0, 0, 0}, nc[3] = {1, 1, 1};
+    {
+      int cc[3];
+      cellCoords<D>(g, ri.c, cc);
+      for (int d = 0; d < D; ++d) {
+        int c1;
+        if (Ri <= g.cell) {
+          c0[d] = cc[d] - 1 < 0 ? 0 : cc[d] - 1;
+          c1 = cc[d] + 1 >= g.nc[d] ? g.nc[d] - 1 : cc[d] + 1;
+        } else {
+          const double t0 = floor((ri.c[d] - Ri - g.lo[d]) * g.invCell), t1 = floor((ri.c[d] + Ri - g.lo[d]) * g.invCell);
+          c0[d] = t0 < 0.0 ? 0 : (t0 > double(g.nc[d] - 1) ? g.nc[d] - 1 : int(t0));
+          c1 = t1 < 0.0 ? 0 : (t1 > double(g.nc[d] - 1) ? g.nc[d] - 1 : int(t1));
+        }
+        nc[d] = c1 - c0[d] + 1;
       }
     }
-  }
-  for (int z = c0[2]; z <= c1[2]; ++z) {
-    for (int y = c0[1]; y <= c1[1]; ++y) {
-      for (int x = c0[0]; x <= c1[0]; ++x) {
-        const int64_t id = base + cellId<D>(g, x, y, z);
-        const int32_t b = cellStart[id], e = cellStart[id + 1];
-        for (int32_t j = b; j < e; ++j) {
-          if (j == k) continue;
-          const double* rj_ = rec + int64_t(j) * R::STRIDE;
-          V<D> rij;
-          for (int c = 0; c < D; ++c) rij.c[c] = ri.c[c] - rj_[R::X + c];
-          S<D> Hj;
-          if constexpr (ISO) {
-            for (int c = 0; c < NS; ++c) Hj.c[c] = 0.0;
-            for (int c = 0; c < D; ++c) Hj.c[sdiag<D>(c)] = rj_[RL<true>::HINV];
-          } else {
-            for (int c = 0; c < NS; ++c) Hj.c[c] = rj_[RL<false>::H + c];
+    if constexpr (L == 1) {
+      // four candidates of a cell in flight together
+      for (int z = 0; z < nc[2]; ++z)
+        for (int y = 0; y < nc[1]; ++y)
+          for (int x = 0; x < (D == 1 ? 1 : nc[0]); ++x) {
+            const int64_t id = base + cellId<D>(g, c0[0] + x, c0[1] + y, c0[2] + z);
+            const int32_t b = cellStart[id], e = cellStart[id + (D == 1 ? nc[0] : 1)];
+            for (int32_t j = b; j < e; j += 4) {
+              bool in[4];
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const bool is = j + t < e && j + t != k;
+                const bool h = hit(is ? j + t : int32_t(k));
+                in[t] = is && h;
+              }
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                row.pushIf(in[t], j + t);
+                if (a.keepSlot && in[t] && rec[int64_t(j + t) * R::STRIDE + R::ORIG] >= double(a.nInt))
+                  a.keepSlot[j + t] = 1;
+              }
+            }
           }
-          const double eta2i = vmag2(sdot(Hi, rij));
-          const double eta2j = vmag2(sdot(Hj, rij));
-          if (eta2i <= a.ext2 || eta2j <= a.ext2) {
-            row.push(j);
-            if (a.keepSlot && rj_[R::ORIG] >= double(a.nInt)) a.keepSlot[j] = 1;
+      continue;
+    }
+    // 1-D cells follow each other in slot order: one range.  Else the lanes load
+    // the bounds of L cells (x fastest) and take them three at a time, the first
+    // L candidates of each in flight together.
+    const uint32_t cells = D == 1 ? 1u : uint32_t(nc[0]) * uint32_t(nc[1]) * uint32_t(nc[2]);   // below 2^31
+    for (uint32_t m0 = 0; m0 < cells; m0 += L) {
+      const uint32_t m = m0 + sub;
+      int32_t b = 0, e = 0;
+      if (m < cells) {
+        const uint32_t row = D == 1 ? 0u : m / uint32_t(nc[0]), mx = D == 1 ? 0u : m - row * uint32_t(nc[0]);
+        const uint32_t mz = D == 3 ? row / uint32_t(nc[1]) : 0u, my = row - mz * uint32_t(nc[1]);
+        const int64_t id = base + cellId<D>(g, c0[0] + int(mx), c0[1] + int(my), c0[2] + int(mz));
+        b = cellStart[id];
+        e = cellStart[id + (D == 1 ? nc[0] : 1)];
+      }
+      const int here = cells - m0 < L ? int(cells - m0) : L;
+      constexpr int T = D == 1 ? 1 : 3;
+      for (int c = 0; c < here; c += T) {
+        int32_t j[T], end[T];
+        bool in[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const bool cell = c + t < here;
+          j[t] = __shfl(b, cell ? c + t : c, L) + sub;
+          end[t] = cell ? __shfl(e, cell ? c + t : c, L) : 0;
+          const bool is = j[t] < end[t] && j[t] != k;
+          const bool h = hit(is ? j[t] : int32_t(k));
+          in[t] = is && h;
+        }
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          append(in[t], j[t]);
+          for (int32_t j0 = j[t] - sub + L; j0 < end[t]; j0 += L) {
+            const int32_t jn = j0 + sub;
+            const bool is = jn < end[t] && jn != k;
+            const bool h = hit(is ? jn : int32_t(k));
+            append(is && h, jn);
           }
         }
       }
     }
   }
-  }
-  row.finish();
-  return row.cnt;
+  if constexpr (L == 1) return row.finish();
+  // the rest of the last chunk
+  if (sub < (-cnt & 3) && cnt + sub < a.cap) nbr[ellIndex(cnt + sub, a.n, k)] = 0;
+  return cnt;
 }
-template <int D, bool ISO>
+template <int D, bool ISO, int L>
 __global__ void __launch_bounds__(kBlock) k_search_global(const double* __restrict__ rec,
                                                           const int32_t* __restrict__ cellStart, SearchArgs a,
                                                           SegGrids sg, int32_t* __restrict__ rowCount,
-                                                          int4* __restrict__ nbr, int32_t* __restrict__ flags) {
-  const int64_t k = xcdBlock((a.n + kBlock - 1) / kBlock) * kBlock + threadIdx.x;
+                                                          int32_t* __restrict__ nbr, int32_t* __restrict__ flags) {
+  const int64_t k = (xcdBlock((a.n * L + kBlock - 1) / kBlock) * kBlock + threadIdx.x) / L;
+  const int sub = threadIdx.x % L;
   RowStats<> stats;
   if (k < a.n) {
-    const int32_t c = searchRow<D, ISO>(k, rec, cellStart, a, sg, nbr);
-    rowCount[k] = c;
-    stats.add(c);
+    const int32_t c = searchRow<D, ISO, L>(k, sub, rec, cellStart, a, sg, nbr);
+    if (sub == 0) {
+      rowCount[k] = c;
+      stats.add(c);
+    }
   }
   stats.store(flags);
 }
@@ -1344,11 +1419,11 @@ void buildNeighborsD(Sim& s, double ext) {
   // zero the cell counters, the search flags and the ghost-use marks in one dispatch
   const bool markUse = s.markGhostUse && s.nTot > s.nInt;
   if (markUse) s.slotKeep.ensure(sizeof(int32_t) * size_t(n + 1));
-  s.flags.ensure(sizeof(int32_t) * 8);
+  s.flags.ensure(sizeof(int32_t) * kSearchFlags);
   {
     ZeroSet z{};
     z.add(s.cellCount.as<int32_t>(), G.ncells + 1);
-    z.add(s.flags.as<int32_t>(), 8);
+    z.add(s.flags.as<int32_t>(), kSearchFlags);
     if (markUse) z.add(s.slotKeep.as<int32_t>(), n);
     zeroMany(z, s.stream);
   }
@@ -1401,7 +1476,7 @@ void buildNeighborsD(Sim& s, double ext) {
       // the first attempt's flags were zeroed with the cell counters; ghost
       // marks of the first attempt are a subset of the second's
       ZeroSet z{};
-      z.add(s.flags.as<int32_t>(), 8);
+      z.add(s.flags.as<int32_t>(), kSearchFlags);
       zeroMany(z, s.stream);
     }
     if (stagedPath) {
@@ -1412,33 +1487,41 @@ void buildNeighborsD(Sim& s, double ext) {
       };
       if (bricks <= kWideBricks) staged(k_search_staged<kWideBlock>, kWideBlock);
       else staged(k_search_staged<kBlock>, kBlock);
-    } else if (s.isotropic) {
-      hipLaunchKernelGGL((k_search_global<D, true>), dim3(int(xcdGrid(nblocks(n)))), dim3(kBlock), 0, st, s.rec.as<double>(),
-                         s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
-                         s.flags.as<int32_t>());
     } else {
-      hipLaunchKernelGGL((k_search_global<D, false>), dim3(int(xcdGrid(nblocks(n)))), dim3(kBlock), 0, st, s.rec.as<double>(),
-                         s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int4>(),
-                         s.flags.as<int32_t>());
+      auto global = [&](auto kern, int L) {
+        hipLaunchKernelGGL(kern, dim3(int(xcdGrid(nblocks(n * L)))), dim3(kBlock), 0, st, s.rec.as<double>(),
+                           s.cellStart.as<int32_t>(), sa, sgr, s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(),
+                           s.flags.as<int32_t>());
+      };
+      auto lanes = [&](auto ln) {
+        constexpr int L = decltype(ln)::value;
+        if (s.isotropic) global(k_search_global<D, true, L>, L);
+        else global(k_search_global<D, false, L>, L);
+      };
+      const int L = searchLanes(D, n);
+      if (L == 1) lanes(std::integral_constant<int, 1>{});
+      else if (D < 3 && L == 4) lanes(std::integral_constant<int, (D < 3 ? 4 : 16)>{});
+      else lanes(std::integral_constant<int, (D > 1 ? 16 : 4)>{});
     }
     SG_CHECK_HIP(hipGetLastError());
-    struct Flags { int32_t f[4]; unsigned long long total, pad; };
-    static_assert(sizeof(Flags) == sizeof(int32_t) * 8, "the flags buffer");
-    char* hp = static_cast<char*>(hostStaging(s, 0, sizeof(Flags) + sizeof(int32_t) * (s.subs.size() + 1)));
-    const Flags* hfp = reinterpret_cast<const Flags*>(hp);
-    int32_t* hcull = reinterpret_cast<int32_t*>(hp + sizeof(Flags));
+    // pinned: the folded flags, the cull's starts; or the flags as they are
+    const size_t raw = sizeof(int32_t) * kSearchFlags;
+    char* hp = static_cast<char*>(
+        hostStaging(s, 0, std::max(raw, sizeof(SearchFlags) + sizeof(int32_t) * (s.subs.size() + 1))));
+    int32_t* hcull = reinterpret_cast<int32_t*>(hp + sizeof(SearchFlags));
     // the ghost cull's first half rides on the same wait and brings the flags along
-    if (markUse) cullLaunch(s, reinterpret_cast<int32_t*>(hp), hcull);
-    else SG_CHECK_HIP(hipMemcpyAsync(hp, s.flags.p, sizeof(Flags), hipMemcpyDeviceToHost, st));
+    if (markUse) cullLaunch(s, reinterpret_cast<SearchFlags*>(hp), hcull);
+    else SG_CHECK_HIP(hipMemcpyAsync(hp, s.flags.p, raw, hipMemcpyDeviceToHost, st));
     SG_CHECK_HIP(hipStreamSynchronize(st));
-    const Flags hf = *hfp;
+    const SearchFlags hf = markUse ? *reinterpret_cast<const SearchFlags*>(hp)
+                                   : foldFlags(reinterpret_cast<const int32_t*>(hp));
     if (markUse) {
       s.cullStarts.assign(hcull, hcull + s.subs.size() + 1);
       s.cullStartsReady = true;
     }
-    s.maxRow = hf.f[0];
-    s.stagedFallbacks = hf.f[1];
-    s.nEntries = int64_t(hf.total);
+    s.maxRow = hf.longest;
+    s.stagedFallbacks = hf.fallbacks;
+    s.nEntries = int64_t(hf.entries);
     if (s.maxRow <= s.ellCap) break;
     SG_REQUIRE(attempt == 0, SPHGPU_ERR_CAPACITY, "neighbour row capacity exceeded twice");
     s.ellCap = ((s.maxRow + 15) / 16) * 16 + 16;
