@@ -189,12 +189,14 @@ inline double fromOrderedBits(unsigned long long o) {
 // bits, a min slot their complement, so that every slot is an atomic maximum
 // that starts at zero.  A wavefront walks `groups` consecutive groups of 64 rows
 // (members are contiguous runs of internal rows) and keeps a running reduction
-// in registers while its groups stay in one member; a group that spans members
-// (ghost rows, whose planes mix them) goes per lane.  Either way a slot that
-// already holds as much is left alone: 10 contended atomics a lane were 105 us
-// of a 30 k row batch (a plain read may be stale, then the atomic decides).
-// Max is order-free, so the result does not depend on the grouping.  `clear`
-// is the next build's table.
+// in registers while its groups stay in one member; in a group that spans members
+// (ghost rows, whose planes mix them) each run of a member's rows is reduced to its
+// first lane.  Either way a slot that already holds as much is left alone: 10
+// contended atomics a lane were 105 us of a 30 k row batch (a plain read may be
+// stale, then the atomic decides).  Max is order-free, so the result does not
+// depend on the grouping.  A lane enters one slot of a uniform wavefront, where
+// lane 0 entered all eleven, a read and an atomic each: 33 -> 15 us for six 2-D
+// members (39 k rows), 18 -> 8 us for 24 tubes.  `clear` is the next build's table.
 constexpr int kSegGroups = 16;
 template <int D>
 __global__ void k_seg_bounds(const double* __restrict__ pos, const double* __restrict__ H,
@@ -210,20 +212,22 @@ __global__ void k_seg_bounds(const double* __restrict__ pos, const double* __res
   double acc[kNB];
   for (int k = 0; k < kNB; ++k) acc[k] = ident[k];
   int mAcc = -1;                           // member of the running reduction (wave-uniform)
-  auto atomicOne = [&](int m, int k, double v) {
-    unsigned long long* p = bits + int64_t(m) * kNB + k;
-    const unsigned long long o = isMaxSlot(k) ? orderedBits(v) : ~orderedBits(v);
-    if (o > *static_cast<volatile unsigned long long*>(p)) atomicMax(p, o);
-  };
+  auto entry = [&](int k, double v) { return isMaxSlot(k) ? orderedBits(v) : ~orderedBits(v); };
   auto flush = [&]() {                     // called by the whole wavefront
+    // lane k enters slot k: one read and one atomic in a row instead of kNB
+    unsigned long long mine = 0;
     for (int k = 0; k < kNB; ++k) {
       double v = acc[k];
       for (int sh = 32; sh > 0; sh >>= 1) {
         const double o = __shfl_xor(v, sh);
         v = isMaxSlot(k) ? dmax(v, o) : dmin(v, o);
       }
-      if (lane == 0) atomicOne(mAcc, k, v);
+      mine = lane == k ? entry(k, v) : mine;
       acc[k] = ident[k];
+    }
+    if (lane < kNB) {
+      unsigned long long* p = bits + int64_t(mAcc) * kNB + lane;
+      if (mine > *static_cast<volatile unsigned long long*>(p)) atomicMax(p, mine);
     }
   };
   for (int it = 0; it < groups; ++it) {
@@ -252,8 +256,28 @@ __global__ void k_seg_bounds(const double* __restrict__ pos, const double* __res
     } else {
       if (mAcc >= 0) flush();
       mAcc = -1;
-      if (m >= 0)
-        for (int k = 0; k < kNB; ++k) atomicOne(m, k, r[k]);
+      // a run of one member's rows is reduced to its first lane
+      for (int sh = 1; sh < 64; sh <<= 1) {
+        const int mo = __shfl_down(m, sh);
+        const bool same = lane + sh < 64 && mo == m;
+        for (int k = 0; k < kNB; ++k) {
+          const double o = __shfl_down(r[k], sh);
+          const double v = isMaxSlot(k) ? dmax(r[k], o) : dmin(r[k], o);
+          r[k] = same ? v : r[k];
+        }
+      }
+      const int before = __shfl_up(m, 1);
+      if (m >= 0 && (lane == 0 || before != m)) {
+        unsigned long long* p = bits + int64_t(m) * kNB;
+        unsigned long long held[kNB];      // all reads before the first wait
+#pragma unroll
+        for (int k = 0; k < kNB; ++k) held[k] = static_cast<volatile unsigned long long*>(p)[k];
+#pragma unroll
+        for (int k = 0; k < kNB; ++k) {
+          const unsigned long long o = entry(k, r[k]);
+          if (o > held[k]) atomicMax(p + k, o);
+        }
+      }
     }
   }
   if (mAcc >= 0) flush();
