@@ -409,8 +409,8 @@ struct OutArgs {
   double* pairDv;    // compatible energy: the pair term of every row entry in the node's own
                      // frame, component c at pairDv[c*plane + ellIndex(w, n, k)]; null otherwise
   int64_t plane;
-  double* relV;      // dt vote: the largest |v_ij|^2 of the row per slot (1-D: |v_ij|), -1 for an
-                     // empty row; null otherwise
+  double* relV;      // dt vote: the largest |v_ij|^2 of the row per slot (FP64 in 1-D: |v_ij|; mixed:
+                     // FP32, 3-D with one lane to a node only), -1 for an empty row; null otherwise
 };
 
 // The pair limit of GenericHydro::dt (src/Physics/GenericHydro.cc:218-283) is
@@ -1217,8 +1217,12 @@ __device__ __forceinline__ IsoPair<Real, D> isoPair(const IsoNode<Real, D>& m, c
 // L > 1 (mixed, small node sets): L lanes to a node, each taking whole blocks of
 // kSumBlock entries, and the blocks' FP32 sums enter the FP64 sums in row order:
 // the bits are those of one lane.
+// The 3-D mixed kernel is held to 168 VGPRs, three wavefronts per SIMD: one register
+// more, for the vote's maximum, and it would run at two.
+template <typename Real, int D, int L>
+constexpr int kIsoBlocks = std::is_same<Real, float>::value && D == 3 && L == 1 ? 3 : 1;
 template <typename Real, int D, bool LDS, bool PREFETCH, int BS = kBlock, int L = 1>
-__global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ rec,
+__global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, L>)) k_derivs_iso(const double* __restrict__ rec,
                                                        const typename IsoTab<Real>::Rec* __restrict__ recN,
                                                        const int32_t* __restrict__ rowCount,
                                                        const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
@@ -1252,8 +1256,7 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
     a.zero();
     SumsF<F32 ? D : 1> af;
     if constexpr (F32) af.zero();
-    Real maxVP = Real(0);
-    double relV = 0.0;
+    Real maxVP = Real(0), relV = Real(0);
     const int len = rowCount[k];
     // One neighbour's contribution, in row order (w: its place in the row).
     auto pair = [&](const INbr<Real>& nb, int32_t j, int w) {
@@ -1261,6 +1264,12 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
       const IsoPair<Real, D> q = isoPair<Real, D>(me, nb, tab, tt, p);
       if constexpr (!F32) {
         if (o.relV) relV = dmax(relV, relSpeed<D>(q.vij));
+      } else if constexpr (D == 3 && L == 1) {
+        if (o.relV) {
+          float v2 = q.vij[0] * q.vij[0];
+          for (int c = 1; c < D; ++c) v2 = fmaR(q.vij[c], q.vij[c], v2);
+          relV = maxR(relV, v2);
+        }
       }
       maxVP = maxR(maxVP, q.Qi);
       if (o.pairDv)
@@ -1354,8 +1363,8 @@ __global__ void __launch_bounds__(BS) k_derivs_iso(const double* __restrict__ re
     if (L == 1 || threadIdx.x % L == 0) {
       for (int c = 0; c < D; ++c)
         for (int b = 0; b < c; ++b) a.M.c[c * D + b] = a.M.c[b * D + c];
-      if constexpr (!F32) {
-        if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
+      if constexpr (!F32 || (D == 3 && L == 1)) {
+        if (o.relV) o.relV[k] = len > 0 ? double(relV) : -1.0;
       }
       isoEpilogue<D>(k, len, ri_, a, t, p, o);
     }
@@ -1825,7 +1834,7 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
   o.n = n;
   o.updateOnly = updateOnly ? 1 : 0;
   if (relV) {
-    SG_REQUIRE(!mixed, SPHGPU_ERR_STATE, "the dt vote takes FP64 velocities");
+    SG_REQUIRE(!mixed || (D == 3 && lanes == 1), SPHGPU_ERR_STATE, "mixed row maxima: 3-D, one lane to a node");
     s.relV.ensure(sizeof(double) * size_t(std::max<int64_t>(n, 1)));
     o.relV = s.relV.as<double>();
   }

@@ -203,6 +203,12 @@ template <int D> __device__ __forceinline__ double vmagArr(const double* a) {
 //               kernel holds FP32 velocities: the vote stays FP64); four
 //               neighbours' loads in flight
 //   kVoteDone   the row maxima the FP64 pass at the step start left (relV)
+//   kVoteBounds the FP32 row maxima a large mixed step's pass left: bounds of the
+//               FP64 maximum.  The upper end of each pair limit enters the vote, the
+//               lower goes to `low`, and k_dt_exact gathers the FP64 velocities of
+//               the rows whose lower end lies under the vote: the row that decides is
+//               among them, so the result is the gather's, to the bit.  100^3: 0.42 ms
+//               for the gather of all rows, 0.10 for the two and 0.04 more in each pass
 // An entry that would not lower the minimum is left out (a plain read may be
 // stale, then the atomic decides): 32 k atomics on one word were 0.3 ms of the
 // vote at 128^3.
@@ -210,9 +216,9 @@ __device__ __forceinline__ void enterMin(unsigned long long* p, double m) {
   const unsigned long long v = (unsigned long long)__double_as_longlong(m);
   if (v < *static_cast<volatile unsigned long long*>(p)) atomicMin(p, v);
 }
-enum { kVoteRows, kVoteSlots, kVoteDone };
+enum { kVoteRows, kVoteSlots, kVoteDone, kVoteBounds };
 struct VoteArgs {
-  const int32_t *list, *perm, *rowCount, *nbr;   // list: kVoteDone caller row -> slot, else the work list
+  const int32_t *list, *perm, *rowCount, *nbr;   // list: kVoteDone, kVoteBounds caller row -> slot, else the work list
   int64_t n, nInt;
   const double *H, *cs, *rho, *vel, *dtIn;
   int haveDtIn;
@@ -220,7 +226,43 @@ struct VoteArgs {
   int useVelMag;
   const double* seg;
   const double *velS, *relV;
+  double* low;
 };
+// The largest |v_ij|^2 (1-D: |v_ij|) of slot k's row from the velocities packed by
+// slot, four neighbours' loads in flight.
+template <int D>
+__device__ __forceinline__ double rowRelSpeed(const VoteArgs& a, int64_t k, int len, const double* vi) {
+  const int4* nb4 = reinterpret_cast<const int4*>(a.nbr);
+  double r = 0.0;
+  for (int w = 0; w < len; w += 4) {
+    const int4 j4 = nb4[ellChunk(w >> 2, a.n, k)];
+    const int32_t j[4] = {j4.x, j4.y, j4.z, j4.w};
+    double d[4][3];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const double* p = a.velS + int64_t(w + q < len ? j[q] : j[0]) * velStride(D);
+      if constexpr (D == 1) {
+        d[q][0] = p[0];
+      } else {
+        const double2 lo = reinterpret_cast<const double2*>(p)[0];
+        d[q][0] = lo.x;
+        d[q][1] = lo.y;
+        if constexpr (D == 3) d[q][2] = p[2];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      for (int c = 0; c < D; ++c) d[q][c] = vi[c] - d[q][c];
+      double s = D == 1 ? dabs(d[q][0]) : d[q][0] * d[q][0];
+      for (int c = 1; c < D; ++c) s = s + d[q][c] * d[q][c];
+      r = dmax(r, s);
+    }
+  }
+  return r;
+}
+template <int D> __device__ __forceinline__ double pairLimit(double nodeScale, double speed) {
+  return nodeScale * (1.0 / dmax(1.0e-30, speed));
+}
 template <int D, int FROM>
 __global__ void __launch_bounds__(kBlock) k_dt(VoteArgs a, unsigned long long* __restrict__ minBits, int64_t minStride) {
   constexpr int NS = NSym<D>::value;
@@ -230,7 +272,7 @@ __global__ void __launch_bounds__(kBlock) k_dt(VoteArgs a, unsigned long long* _
   int sg = 0;
   if (t < a.nInt) {
     int64_t k, i;
-    if constexpr (FROM == kVoteDone) {
+    if constexpr (FROM == kVoteDone || FROM == kVoteBounds) {
       i = t;
       k = a.list[i];
     } else {
@@ -254,37 +296,25 @@ __global__ void __launch_bounds__(kBlock) k_dt(VoteArgs a, unsigned long long* _
     for (int c = 0; c < D; ++c) vi[c] = a.vel[i * D + c];
     if constexpr (FROM == kVoteDone) {
       const double r = a.relV[k];
-      if (r >= 0.0) m = dmin(m, nodeScale * (1.0 / dmax(1.0e-30, D == 1 ? r : sqrt(r))));
+      if (r >= 0.0) m = dmin(m, pairLimit<D>(nodeScale, D == 1 ? r : sqrt(r)));
+    } else if constexpr (FROM == kVoteBounds) {
+      const double r = a.relV[k];
+      double low = double(FLT_MAX);
+      if (r >= 0.0) {
+        // FP32 velocities are within u |v| of theirs (u = 2^-24), so the maximum is
+        // within u (2 |v_i| + 4 M) of M; three times that, and room for products
+        // that underflow.  Speeds near the end of the FP32 range give no bounds.
+        const double M = sqrt(r), vm = vmagArr<D>(vi), err = 4.0e-7 * vm + 6.0e-7 * M + 1.0e-18;
+        const bool safe = r < 1.0e36 && vm < 1.0e18;
+        low = safe ? pairLimit<D>(nodeScale, M + err) : 0.0;
+        if (safe) m = dmin(m, pairLimit<D>(nodeScale, M - err));
+      }
+      a.low[i] = low;
     } else if constexpr (FROM == kVoteSlots) {
       // the pair term is monotonic in |v_ij|^2, to the bit: one square root a row
       const int len = a.rowCount[k];
-      const int4* nb4 = reinterpret_cast<const int4*>(a.nbr);
-      double r = 0.0;
-      for (int w = 0; w < len; w += 4) {
-        const int4 j4 = nb4[ellChunk(w >> 2, a.n, k)];
-        const int32_t j[4] = {j4.x, j4.y, j4.z, j4.w};
-        double d[4][3];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const double* p = a.velS + int64_t(w + q < len ? j[q] : j[0]) * velStride(D);
-          if constexpr (D == 1) {
-            d[q][0] = p[0];
-          } else {
-            const double2 lo = reinterpret_cast<const double2*>(p)[0];
-            d[q][0] = lo.x;
-            d[q][1] = lo.y;
-            if constexpr (D == 3) d[q][2] = p[2];
-          }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          for (int c = 0; c < D; ++c) d[q][c] = vi[c] - d[q][c];
-          double s = D == 1 ? dabs(d[q][0]) : d[q][0] * d[q][0];
-          for (int c = 1; c < D; ++c) s = s + d[q][c] * d[q][c];
-          r = dmax(r, s);
-        }
-      }
-      if (len > 0) m = dmin(m, nodeScale * (1.0 / dmax(1.0e-30, D == 1 ? r : sqrt(r))));
+      const double r = rowRelSpeed<D>(a, k, len, vi);
+      if (len > 0) m = dmin(m, pairLimit<D>(nodeScale, D == 1 ? r : sqrt(r)));
     } else {
       const int len = a.rowCount[k];
       for (int w = 0; w < len; ++w) {
@@ -306,13 +336,34 @@ __global__ void __launch_bounds__(kBlock) k_dt(VoteArgs a, unsigned long long* _
   }
 }
 
+// The rows that k_dt<D, kVoteBounds> left open, one lane to a caller row.
+template <int D>
+__global__ void __launch_bounds__(kBlock) k_dt_exact(VoteArgs a, unsigned long long* __restrict__ minBits,
+                                                     int64_t minStride) {
+  const int64_t i = blockIdx.x * int64_t(kBlock) + threadIdx.x;
+  if (i >= a.nInt) return;
+  unsigned long long* word = minBits + (a.seg ? int64_t(a.seg[i]) * minStride : 0);
+  if (!(a.low[i] <= __longlong_as_double((long long)*static_cast<volatile unsigned long long*>(word)))) return;
+  const int64_t k = a.list[i];
+  const int len = a.rowCount[k];
+  if (len == 0) return;
+  double vi[3];
+  for (int c = 0; c < D; ++c) vi[c] = a.vel[i * D + c];
+  const double r = rowRelSpeed<D>(a, k, len, vi);
+  const double nodeScale = 1.0 / maxEigen<D>(a.H + i * NSym<D>::value) / a.nPerh;
+  enterMin(word, dmin(double(FLT_MAX), pairLimit<D>(nodeScale, D == 1 ? r : sqrt(r))));
+}
+
 template <int D, int FROM>
 void voteD(Sim& s, double nPerh, int useVelMag, const double* seg, unsigned long long* bits, int64_t stride) {
-  VoteArgs a{FROM == kVoteDone ? s.iperm.as<int32_t>() : s.work.as<int32_t>(), s.perm.as<int32_t>(),
+  if (FROM == kVoteBounds) s.voteLow.ensure(sizeof(double) * size_t(std::max<int64_t>(s.nInt, 1)));
+  VoteArgs a{FROM == kVoteDone || FROM == kVoteBounds ? s.iperm.as<int32_t>() : s.work.as<int32_t>(), s.perm.as<int32_t>(),
              s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), s.nSlots, s.nInt, s.H.as<double>(), s.cs.as<double>(),
              s.rho.as<double>(), s.vel.as<double>(), s.dtIn.as<double>(), s.haveDtIn ? 1 : 0, nPerh, useVelMag, seg,
-             s.velS.as<double>(), s.relV.as<double>()};
+             s.velS.as<double>(), s.relV.as<double>(), s.voteLow.as<double>()};
   hipLaunchKernelGGL((k_dt<D, FROM>), dim3(xcdGrid(nblocks(s.nInt))), dim3(kBlock), 0, s.stream, a, bits, stride);
+  if constexpr (FROM == kVoteBounds)
+    hipLaunchKernelGGL(k_dt_exact<D>, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, a, bits, stride);
   SG_CHECK_HIP(hipGetLastError());
 }
 
@@ -586,10 +637,20 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
   // (the vote needs nothing the pass writes but the rows' largest relative speeds,
   // and the pass nothing of the vote)
   const bool mixed = hp.precision == SPHGPU_PRECISION_MIXED;
-  if (mixed) voteD<D, kVoteSlots>(s, hp.nPerh, ip.useVelocityMagnitudeForDt, vote.seg, vote.bits, vote.stride);
+  auto cast = [&](auto from) {
+    voteD<D, decltype(from)::value>(s, hp.nPerh, ip.useVelocityMagnitudeForDt, vote.seg, vote.bits, vote.stride);
+  };
+  // In 2-D a row has 28 neighbours and the gather is no slower than the two launches
+  // (250 k nodes: 20 and 18 + 5 us); a small 3-D set has several lanes to a node in
+  // the pair pass, which keep no maxima.
+  const bool bounds = mixed && D == 3 && s.nInt > 131072;
+  if (mixed && !bounds) cast(std::integral_constant<int, kVoteSlots>{});
   if (ip.gradhCorrection) omegaGradh(s);
-  evalDerivs(s, hp, true, !mixed);
-  if (!mixed) voteD<D, kVoteDone>(s, hp.nPerh, ip.useVelocityMagnitudeForDt, vote.seg, vote.bits, vote.stride);
+  evalDerivs(s, hp, true, !mixed || bounds);
+  if (!mixed) cast(std::integral_constant<int, kVoteDone>{});
+  else if constexpr (D == 3) {
+    if (bounds) cast(std::integral_constant<int, kVoteBounds>{});
+  }
   // state0 (the policy reads every row's step-start velocity, ghosts included)
   const size_t n = size_t(s.nInt), nv = compat ? size_t(s.nTot) : n;
   const size_t rows[4] = {n * D, nv * D, n, n};
@@ -695,7 +756,8 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
                         &s.recS, &s.recSM, &s.pairDv, &s.compDe, &s.compAcc, &s.compDe0, &s.compRec, &s.out,
                         &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
                         &s.work, &s.ghostIsControl, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
-                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts, &s.velS, &s.relV})
+                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts, &s.velS, &s.relV,
+                        &s.voteLow})
     keyBuf(k, *b);
   for (const DBuf& b : s.state0) keyBuf(k, b);
   return k;

@@ -207,7 +207,8 @@ struct Sim {
                              // writes: -1 the density sum's, else what the caller will read first
   bool buildVel = false;     // the build also writes velS (the dt vote of a mixed step)
   DBuf velS;                 // velocities by slot at the last build
-  DBuf relV;                 // per slot: the largest relative speed of its row (dt vote of an FP64 step)
+  DBuf relV;                 // per slot: the largest relative speed of its row (dt vote)
+  DBuf voteLow;              // per caller row: the least its pair limit can be (dt vote of a large mixed step)
   bool recSValid = false;    // recS matches rec (written by the record pack; valid through a cull)
   DBuf recSM;               // mixed density-sum neighbour records (32 B per slot)
   bool recSMValid = false;   // recSM matches rec (written by the record pack; the cull keeps it)
@@ -338,7 +339,8 @@ void packRecords(Sim& s, int sec = 0);
 void sumDensity(Sim& s);
 // updateOnly: store only DxDt, DvDt, DepsDt, DrhoDt and Hideal (the fields an
 // integrator update reads); the other fields keep what they held
-// relV: also leave the largest relative speed of every row in s.relV (FP64)
+// relV: also leave the largest relative speed of every row in s.relV (FP64; mixed,
+// to FP32, in 3-D where one lane goes to a node)
 void evalDerivs(Sim& s, const sphgpu_hydro_params& p, bool updateOnly = false, bool relV = false);
 // The pack sec bits of the records the pair kernel and the density sum read.
 int pairRecordSec(const Sim& s, const sphgpu_hydro_params& hp);
