@@ -148,6 +148,8 @@ void sphgpu_destroy(sphgpu_sim* s) {
   if (s->pinnedOut) (void)hipHostFree(s->pinnedOut);
   if (s->pinnedIn) (void)hipHostFree(s->pinnedIn);
   if (s->pinnedInDone) (void)hipEventDestroy(s->pinnedInDone);
+  if (s->ring) (void)hipHostFree(s->ring);
+  for (auto& e : s->ringDone) (void)hipEventDestroy(e);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -286,8 +288,7 @@ int sphgpu_download(sphgpu_sim* s, int field, double* host, int64_t nRows) {
       std::fill(host, host + nRows, 1.0);
       return;
     }
-    if (bytes) SG_CHECK_HIP(hipMemcpyAsync(host, b.p, bytes, hipMemcpyDeviceToHost, s->stream));
-    SG_CHECK_HIP(hipStreamSynchronize(s->stream));
+    copyToHost(*s, host, b.p, bytes);
   });
 }
 
@@ -449,8 +450,7 @@ int sphgpu_download_derivative(sphgpu_sim* s, int field, double* host, int64_t n
     // put in order on the device: with the host's own pass over each of 19 fields,
     // and the slots read back for it, a pass at 125 k nodes took 29.3 ms; now 10.7
     src = unsortDerivative(*s, src, comps);
-    SG_CHECK_HIP(hipMemcpyAsync(host, src, sizeof(double) * size_t(nRows) * comps, hipMemcpyDeviceToHost, s->stream));
-    SG_CHECK_HIP(hipStreamSynchronize(s->stream));
+    copyToHost(*s, host, src, sizeof(double) * size_t(nRows) * comps);
   });
 }
 

@@ -324,6 +324,8 @@ struct Sim {
   void* pinnedIn = nullptr;
   size_t pinnedInBytes = 0;
   hipEvent_t pinnedInDone = nullptr;   // recorded after the copies that read pinnedIn
+  void* ring = nullptr;            // pinned slots that large downloads pass through
+  std::vector<hipEvent_t> ringDone;
   DBuf unsorted;                   // a derivative field in the caller's order, on its way to the host
   std::vector<int32_t> cullStarts;  // new ghost starts read with the last build's row readback
   bool cullStartsReady = false;
@@ -420,6 +422,8 @@ __host__ __device__ inline SearchFlags foldFlags(const int32_t* f) {
   }
   return o;
 }
+// Device memory to the caller's, complete on return.
+void copyToHost(Sim& s, void* host, const void* dev, size_t bytes);
 // First half of the ghost cull: keep flags and scan, the planes' new first
 // ghosts and the search flags to pinned memory.
 void cullLaunch(Sim& s, SearchFlags* flagsOut, int32_t* starts);
