@@ -1845,9 +1845,10 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
     s.pairDv.ensure(sizeof(double) * size_t(D) * size_t(std::max<int64_t>(o.plane, 1)));
     o.pairDv = s.pairDv.as<double>();
   }
-  // Mixed: one record in flight per lane keeps the kernel at 167 VGPRs, three
+  // Mixed: one record in flight per lane keeps the kernel at 168 VGPRs, three
   // wavefronts per SIMD (2.11 ms at 128^3 against 2.53 ms with the next
-  // record prefetched at 179 VGPRs, two wavefronts).  FP64: the prefetch wins
+  // record prefetched at 179 VGPRs, two wavefronts; 2.20 ms since it can leave the
+  // row maxima of the vote).  FP64: the prefetch wins
   // (3.44 ms at 194 VGPRs against 3.51 ms at 168).
   if (mixed && lanes > 1) {
     if constexpr (D > 1) isoLaunch<float, D, false, kBlock, D == 3 ? 8 : 2>(s, false, st, n, t, p, o, counts);
