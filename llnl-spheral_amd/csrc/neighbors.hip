@@ -94,11 +94,19 @@ template <int D> __device__ double maxDiag(const double* h) {
   return m;
 }
 
-// n rows, or with nDev the rows the ghost generation has left on the device.
+// n rows, or with nDev the rows the ghost generation has left on the device.  The
+// workgroups' bounds of up to kBoundsHost of them go to pinned memory, with the
+// generation's counts (genOut), and the host, which waits for them anyway, takes the
+// last step: 22 KB at most in 3 us, where a launch of one workgroup took 5 us and
+// 4 us of the host.  Beyond, k_bounds_final reduces them.
+constexpr int kBoundsHost = 256;
 template <int D>
 __global__ void k_bounds(const double* __restrict__ pos, const double* __restrict__ H, int64_t n,
-                         const int64_t* __restrict__ nDev, double* partials) {
+                         const int64_t* __restrict__ nDev, double* partials, const int64_t* __restrict__ gen, int nGen,
+                         int64_t* __restrict__ genOut) {
   if (nDev) n = *nDev;
+  if (genOut && blockIdx.x == 0)
+    for (int q = threadIdx.x; q < nGen; q += blockDim.x) genOut[q] = gen[q];
   __shared__ double sh[kNB][kBlock];
   double r[kNB] = SG_BOUNDS_IDENT;
   for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
@@ -1440,16 +1448,25 @@ void buildNeighborsD(Sim& s, double ext) {
   } else {
     const int nbB = int(std::min<int64_t>(1024, nblocks(rows)));
     s.reduceTmp.ensure(sizeof(double) * (size_t(nbB) * kNB + 16));
-    double* partials = s.reduceTmp.as<double>();
-    double* hbp = static_cast<double*>(hostStaging(s, 0, sizeof(hb) + sizeof(int64_t) * size_t(nGen)));
-    int64_t* hgen = reinterpret_cast<int64_t*>(hbp + kNB);
+    const bool onHost = nbB <= kBoundsHost;
+    const int parts = onHost ? std::max(nbB, 1) : 1;
+    double* hbp = static_cast<double*>(
+        hostStaging(s, 0, sizeof(double) * kNB * size_t(parts) + sizeof(int64_t) * size_t(nGen)));
+    int64_t* hgen = reinterpret_cast<int64_t*>(hbp + kNB * parts);
+    double* partials = onHost ? hbp : s.reduceTmp.as<double>();
     hipLaunchKernelGGL((k_bounds<D>), dim3(nbB), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(), rows, nDev,
-                       partials);
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, st, partials, nbB, hbp, gen, nGen, hgen);
+                       partials, gen, nGen, onHost ? hgen : nullptr);
+    if (!onHost)
+      hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(kBlock), 0, st, partials, nbB, hbp, gen, nGen, hgen);
     SG_CHECK_HIP(hipGetLastError());
     SG_CHECK_HIP(hipStreamSynchronize(st));
     if (pending) finishGeneration(s, hgen);
     std::memcpy(hb, hbp, sizeof(hb));
+    for (int b = 1; b < parts; ++b)
+      for (int k = 0; k < kNB; ++k) {
+        const double v = hbp[b * kNB + k];
+        hb[k] = isMaxSlot(k) ? std::max(hb[k], v) : std::min(hb[k], v);
+      }
     requireUsableBounds(hb);
     s.isotropic = hb[7] > 0.5 && !s.hasMultipliers;
     s.rMax = ext / hb[6];
