@@ -147,7 +147,6 @@ void sphgpu_destroy(sphgpu_sim* s) {
   for (auto& g : s->stepGraphs) if (g.exec) (void)hipGraphExecDestroy(g.exec);
   if (s->pinnedOut) (void)hipHostFree(s->pinnedOut);
   if (s->pinnedIn) (void)hipHostFree(s->pinnedIn);
-  if (s->pinnedInDone) (void)hipEventDestroy(s->pinnedInDone);
   if (s->ring) (void)hipHostFree(s->ring);
   for (auto& e : s->ringDone) (void)hipEventDestroy(e);
   if (s->stream) (void)hipStreamDestroy(s->stream);

@@ -75,12 +75,15 @@ struct ZeroSet {
   int32_t* p[4];
   int64_t n[4];
   int m;
+  const uint32_t* from;     // a pinned host list copied along, read by the kernel itself
+  uint32_t* to;
+  int64_t words;
   void add(int32_t* ptr, int64_t count) {
     if (m < 4 && count > 0) { p[m] = ptr; n[m] = count; ++m; }
   }
 };
 // Up to four int32 buffers zeroed by one kernel (a graph-safe memset that
-// also saves dispatches).
+// also saves dispatches), and a short list from pinned memory copied.
 void zeroMany(const ZeroSet& z, hipStream_t st);
 
 // A table that is zero at the start of each use without a launch to clear it:
@@ -323,7 +326,7 @@ struct Sim {
   size_t pinnedOutBytes = 0;
   void* pinnedIn = nullptr;
   size_t pinnedInBytes = 0;
-  hipEvent_t pinnedInDone = nullptr;   // recorded after the copies that read pinnedIn
+  bool pinnedInBusy = false;           // a kernel that reads pinnedIn may not have run
   void* ring = nullptr;            // pinned slots that large downloads pass through
   std::vector<hipEvent_t> ringDone;
   DBuf unsorted;                   // a derivative field in the caller's order, on its way to the host

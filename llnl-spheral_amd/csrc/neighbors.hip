@@ -1232,6 +1232,8 @@ __global__ void k_zero_many(ZeroSet z) {
   const int64_t stride = int64_t(gridDim.x) * blockDim.x;
   for (int q = 0; q < z.m; ++q)
     for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < z.n[q]; i += stride) z.p[q][i] = 0;
+  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < z.words; i += stride)
+    z.to[i] = __hip_atomic_load(z.from + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);   // host memory, written anew
 }
 
 // A grid of cell edge `cell` over the bounds hb: cells per axis, bricks, cell count.
@@ -1311,31 +1313,34 @@ void levelGrids(const double* hb, double ext, std::vector<DGrid>& out, std::vect
   }
 }
 
-// Grid lists to the device; returns the total cell count.
+// Grid lists to the device, with the kernel that runs z; returns the total cell
+// count.
 int64_t uploadGrids(Sim& s, const std::vector<DGrid>& grids, const std::vector<int64_t>& cells,
-                    const std::vector<int32_t>& first) {
-  hipStream_t st = s.stream;
+                    const std::vector<int32_t>& first, ZeroSet& z) {
   const size_t ng = grids.size();
   std::vector<int64_t> base(ng + 1, 0);
   for (size_t q = 0; q < ng; ++q) base[q + 1] = base[q] + cells[q];
   SG_REQUIRE(base.back() < (int64_t(1) << 31) - 2, SPHGPU_ERR_CAPACITY, "neighbour grid too large");
   // the grids, their first global cells and each member's first grid in one
-  // buffer, staged in pinned memory at the same offsets and sent in one copy;
-  // the next use of the staging waits for pinnedInDone, so no wait here
+  // buffer, staged in pinned memory at the same offsets and read from there by the
+  // zeroing kernel: a copy of a few KB and the event behind it were 15 us of a step
+  // that takes 200.  The build's own wait frees the staging.
   const size_t bG = sizeof(DGrid) * ng, bB = sizeof(int64_t) * (ng + 1), bF = sizeof(int32_t) * first.size();
   const size_t oB = (bG + 63) / 64 * 64, oF = oB + (bB + 63) / 64 * 64;
-  s.segGrid.ensure(oF + bF);
+  const size_t bytes = (oF + bF + 3) / 4 * 4;
+  s.segGrid.ensure(bytes);
   char* d = static_cast<char*>(s.segGrid.p);
   s.gridList = d;
   s.gridCellBase = reinterpret_cast<int64_t*>(d + oB);
   s.gridFirst = reinterpret_cast<int32_t*>(d + oF);
-  char* h = static_cast<char*>(hostStaging(s, 1, oF + bF));
+  char* h = static_cast<char*>(hostStaging(s, 1, bytes));
   std::memcpy(h, grids.data(), bG);
   std::memcpy(h + oB, base.data(), bB);
   std::memcpy(h + oF, first.data(), bF);
-  SG_CHECK_HIP(hipMemcpyAsync(d, h, oF + bF, hipMemcpyHostToDevice, st));
-  if (!s.pinnedInDone) SG_CHECK_HIP(hipEventCreateWithFlags(&s.pinnedInDone, hipEventDisableTiming));
-  SG_CHECK_HIP(hipEventRecord(s.pinnedInDone, st));
+  z.from = reinterpret_cast<const uint32_t*>(h);
+  z.to = reinterpret_cast<uint32_t*>(d);
+  z.words = int64_t(bytes / 4);
+  s.pinnedInBusy = true;
   return base.back();
 }
 
@@ -1377,6 +1382,7 @@ void buildNeighborsD(Sim& s, double ext) {
   SG_CHECK_HIP(hipEventRecord(s.ev[0], st));
   // rows: those the caller set, or a ghost generation's whose count is still
   // on the device (read back with the bounds)
+  ZeroSet z{};
   const bool pending = s.genPending;
   s.genPending = false;
   const int64_t rows = pending ? s.genCap : s.nTot;
@@ -1443,7 +1449,7 @@ void buildNeighborsD(Sim& s, double ext) {
     s.rMax = ext / hb[6];
     s.posAbsMax = absMax;
     G = Grid{};
-    G.ncells = uploadGrids(s, grids, cells, first);
+    G.ncells = uploadGrids(s, grids, cells, first, z);
     sgr = SegGrids{s.seg.as<double>(), static_cast<const DGrid*>(s.gridList), s.gridCellBase, s.gridFirst, ext};
   } else {
     const int nbB = int(std::min<int64_t>(1024, nblocks(rows)));
@@ -1481,7 +1487,7 @@ void buildNeighborsD(Sim& s, double ext) {
       // smoothing scales spanning more than a factor 2: levels
       std::vector<int32_t> first = {0, int32_t(grids.size())};
       G = Grid{};
-      G.ncells = uploadGrids(s, grids, cells, first);
+      G.ncells = uploadGrids(s, grids, cells, first, z);
       sgr = SegGrids{nullptr, static_cast<const DGrid*>(s.gridList), s.gridCellBase, s.gridFirst, ext};
     }
   }
@@ -1500,13 +1506,10 @@ void buildNeighborsD(Sim& s, double ext) {
   const bool markUse = s.markGhostUse && s.nTot > s.nInt;
   if (markUse) s.slotKeep.ensure(sizeof(int32_t) * size_t(n + 1));
   s.flags.ensure(sizeof(int32_t) * kSearchFlags);
-  {
-    ZeroSet z{};
-    z.add(s.cellCount.as<int32_t>(), G.ncells + 1);
-    z.add(s.flags.as<int32_t>(), kSearchFlags);
-    if (markUse) z.add(s.slotKeep.as<int32_t>(), n);
-    zeroMany(z, s.stream);
-  }
+  z.add(s.cellCount.as<int32_t>(), G.ncells + 1);
+  z.add(s.flags.as<int32_t>(), kSearchFlags);
+  if (markUse) z.add(s.slotKeep.as<int32_t>(), n);
+  zeroMany(z, s.stream);
   hipLaunchKernelGGL((k_cell_count<D>), dim3(nblocks(n)), dim3(kBlock), 0, st, s.pos.as<double>(), s.H.as<double>(),
                      n, dg, sgr, s.cellOf.as<int32_t>(), s.cellCount.as<int32_t>(), s.cellRank.as<int32_t>());
   scanItems(CellScan{s.cellCount.as<int32_t>(), s.cellStart.as<int32_t>(), G.ncells}, G.ncells, s.scanTmp, st);
@@ -1555,9 +1558,9 @@ void buildNeighborsD(Sim& s, double ext) {
     if (attempt > 0) {
       // the first attempt's flags were zeroed with the cell counters; ghost
       // marks of the first attempt are a subset of the second's
-      ZeroSet z{};
-      z.add(s.flags.as<int32_t>(), kSearchFlags);
-      zeroMany(z, s.stream);
+      ZeroSet again{};
+      again.add(s.flags.as<int32_t>(), kSearchFlags);
+      zeroMany(again, s.stream);
     }
     if (stagedPath) {
       auto staged = [&](auto kern, int bs) {
@@ -1593,6 +1596,7 @@ void buildNeighborsD(Sim& s, double ext) {
     if (markUse) cullLaunch(s, reinterpret_cast<SearchFlags*>(hp), hcull);
     else SG_CHECK_HIP(hipMemcpyAsync(hp, s.flags.p, raw, hipMemcpyDeviceToHost, st));
     SG_CHECK_HIP(hipStreamSynchronize(st));
+    s.pinnedInBusy = false;
     const SearchFlags hf = markUse ? *reinterpret_cast<const SearchFlags*>(hp)
                                    : foldFlags(reinterpret_cast<const int32_t*>(hp));
     if (markUse) {
@@ -1623,22 +1627,27 @@ void buildNeighborsD(Sim& s, double ext) {
 void* hostStaging(Sim& s, int which, size_t bytes) {
   void*& p = which ? s.pinnedIn : s.pinnedOut;
   size_t& cap = which ? s.pinnedInBytes : s.pinnedOutBytes;
-  // uploads: the copies of the previous use must have read the buffer
-  if (which && s.pinnedInDone) SG_CHECK_HIP(hipEventSynchronize(s.pinnedInDone));
+  // uploads: the kernel of the previous use must have read the buffer (a build that
+  // ended early leaves it unknown)
+  if (which && s.pinnedInBusy) {
+    SG_CHECK_HIP(hipStreamSynchronize(s.stream));
+    s.pinnedInBusy = false;
+  }
   if (bytes > cap) {
     SG_CHECK_HIP(hipStreamSynchronize(s.stream));   // no copy still uses the old buffer
     if (p) SG_CHECK_HIP(hipHostFree(p));
     p = nullptr;
     cap = 0;
     const size_t want = std::max<size_t>(4096, ((bytes + 4095) / 4096) * 4096);
-    SG_CHECK_HIP(hipHostMalloc(&p, want, hipHostMallocDefault));
+    // uploads are read by a kernel: coherent, so none of it stays in a cache
+    SG_CHECK_HIP(hipHostMalloc(&p, want, which ? hipHostMallocCoherent : hipHostMallocDefault));
     cap = want;
   }
   return p;
 }
 
 void zeroMany(const ZeroSet& z, hipStream_t st) {
-  int64_t most = 0;
+  int64_t most = z.words;
   for (int q = 0; q < z.m; ++q) most = std::max(most, z.n[q]);
   if (most == 0) return;
   hipLaunchKernelGGL(k_zero_many, dim3(std::min(nblocks(most), 1024)), dim3(kBlock), 0, st, z);
