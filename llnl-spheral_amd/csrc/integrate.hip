@@ -121,12 +121,16 @@ __device__ __forceinline__ void rowMultEos(const SegArgs& sa, int64_t i, double&
 // One lane per caller row: its eleven state arrays are then read and written
 // contiguously, and only the five derivatives are gathered from its slot (an
 // internal row's slot is iperm[i]).  By slot it was the other way round.
+// In 2-D the lines of the slots that a row touches are touched again a few hundred
+// rows on: each XCD takes a run of workgroups, so they meet in one L2 (500^2: 33.5 ->
+// 27.1 us and 30.9 -> 24.7 us).  In 3-D they come again planes later, and the runs
+// cost 4 % at 128^3.
 template <int D, int REC, bool TRIAL>
 __global__ void __launch_bounds__(kBlock) k_update(const int32_t* __restrict__ iperm, int64_t nInt, Fields f, Base b,
                                                    DerivIn d, Bounds bd, Eos e, SegArgs sa, PackIn pin, PackOut pout,
                                                    double* __restrict__ dtIn) {
   constexpr int NS = NSym<D>::value;
-  const int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
+  const int64_t i = (D == 2 ? xcdBlock((nInt + kBlock - 1) / kBlock) : blockIdx.x) * int64_t(kBlock) + threadIdx.x;
   if (i >= nInt) return;
   const int64_t k = iperm[i];
   double mult;
@@ -525,8 +529,8 @@ template <int D, bool TRIAL> void updateD(Sim& s, const Base& b, const Bounds& b
   const PackIn pin = rec >= 0 ? packInputs(s) : PackIn{};
   const PackOut pout = rec >= 0 ? packOutputs(s, rec) : PackOut{};
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(nblocks(s.nInt)), dim3(kBlock), 0, s.stream, s.iperm.as<int32_t>(), s.nInt, f, b, d,
-                       bd, e, sa, pin, pout, s.dtIn.as<double>());
+    hipLaunchKernelGGL(kern, dim3(D == 2 ? xcdGrid(nblocks(s.nInt)) : nblocks(s.nInt)), dim3(kBlock), 0, s.stream,
+                       s.iperm.as<int32_t>(), s.nInt, f, b, d, bd, e, sa, pin, pout, s.dtIn.as<double>());
   };
   // the trial update writes the pair kernel's records, the final one the density sum's
   if constexpr (TRIAL) {
