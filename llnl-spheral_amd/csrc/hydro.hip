@@ -1527,22 +1527,6 @@ TabArgs tabArgs(const Sim& s) {
 
 }  // namespace
 
-double quantInv(const Sim& s) {
-  // only the 3-D mixed record holds quantised positions; with no finite search
-  // radius there is no pair to difference and any unit serves
-  if (s.dim != 3 || !(s.rMax > 0.0) || !std::isfinite(s.rMax)) return 1.0;
-  const int e = std::ilogb(s.rMax) + 1 - 30;     // rMax < 2^30 u
-  SG_REQUIRE(e > -120 && e < 120, SPHGPU_ERR_UNSUPPORTED,
-             "mixed precision: the search radius is outside the FP32 exponent range");
-  const double q = std::ldexp(1.0, -e);
-  // round(x / u) must fit a 64-bit integer; 2^61 leaves room for the motion
-  // of one step beyond the positions the neighbour build saw
-  SG_REQUIRE(s.posAbsMax * q < std::ldexp(1.0, 61), SPHGPU_ERR_UNSUPPORTED,
-             "mixed precision: positions too far from the origin for the 3-D fixed-point record (|x| >= 2^61 u, "
-             "u = largest search radius / 2^30)");
-  return q;
-}
-
 PackIn packInputs(Sim& s) {
   return PackIn{s.perm.as<int32_t>(), s.pos.as<double>(), s.vel.as<double>(), s.mass.as<double>(),
                 s.rho.as<double>(), s.P.as<double>(), s.cs.as<double>(), s.H.as<double>(), s.omega.as<double>(),

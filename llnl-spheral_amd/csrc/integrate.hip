@@ -719,7 +719,8 @@ __global__ void k_plain_seg_init(SegState* __restrict__ g, double t, double last
 // dt selection, both passes, updates, ghost refreshes, finalize, boundary
 // enforcement, clock advance) is launched without a host round trip.  Its
 // launches depend on the node and slot counts, the device buffers, the
-// parameters and the host-side record flags at its start: that is the key.
+// parameters and the host-side record flags at its start: that is the key
+// (stepkey.cpp).
 // The first step with a new key runs eagerly (sizing every buffer), the next
 // step with the same key is captured and instantiated, and later steps with
 // that key replay the graph; the host flags the step leaves are saved at the
@@ -727,46 +728,6 @@ __global__ void k_plain_seg_init(SegState* __restrict__ g, double t, double last
 // ghost counts hold still (most steps of a tube ensemble) replays one graph
 // per step.  Graphs hold no memset node (the pair count is cleared by a
 // kernel) and no stage-timing events.
-void keyBuf(std::vector<uint64_t>& k, const DBuf& b) {
-  k.push_back(reinterpret_cast<uint64_t>(b.p));
-  k.push_back(uint64_t(b.bytes));
-}
-template <class T> void keyBytes(std::vector<uint64_t>& k, const T& v) {
-  const unsigned char* c = reinterpret_cast<const unsigned char*>(&v);
-  for (size_t i = 0; i < sizeof(T); i += 8) {
-    uint64_t w = 0;
-    std::memcpy(&w, c + i, std::min<size_t>(8, sizeof(T) - i));
-    k.push_back(w);
-  }
-}
-std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip) {
-  std::vector<uint64_t> k;
-  k.reserve(256);
-  for (int64_t v : {int64_t(s.dim), s.nInt, s.nTot, s.nSlots, int64_t(s.ellCap), int64_t(s.nSeg), s.tableVersion,
-                    int64_t(s.isotropic), int64_t(s.rowOrder), int64_t(s.precision), int64_t(s.deviceGhosts),
-                    int64_t(s.hasMultipliers), int64_t(s.recValid), int64_t(s.recSValid), int64_t(s.recSMValid),
-                    int64_t(s.pairRec), int64_t(s.haveDtIn), int64_t(s.derivsValid), int64_t(s.subs.size()),
-                    int64_t(s.nLists), int64_t(s.sumAllLists), int64_t(s.listGammaHost.size())})
-    k.push_back(uint64_t(v));
-  for (int64_t v : s.subStart) k.push_back(uint64_t(v));
-  for (const SubBoundary& b : s.subs) keyBytes(k, b);
-  keyBytes(k, hp);
-  keyBytes(k, ip);
-  keyBytes(k, s.dtThreshold);
-  k.push_back(reinterpret_cast<uint64_t>(s.pinnedOut));
-  for (const DBuf* b : {&s.pos, &s.vel, &s.mass, &s.rho, &s.eps, &s.P, &s.cs, &s.H, &s.omega, &s.fCl, &s.fCq,
-                        &s.fshear, &s.cellOf, &s.cellCount, &s.cellStart, &s.cellRank, &s.cellMembers, &s.perm, &s.iperm, &s.xs,
-                        &s.rowCount, &s.nbr, &s.scanTmp, &s.reduceTmp, &s.flags, &s.rec, &s.recM, &s.recD,
-                        &s.recS, &s.recSM, &s.pairDv, &s.compDe, &s.compAcc, &s.compDe0, &s.compRec, &s.out,
-                        &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
-                        &s.work, &s.ghostIsControl, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
-                        &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts, &s.velS, &s.relV,
-                        &s.voteLow})
-    keyBuf(k, *b);
-  for (const DBuf& b : s.state0) keyBuf(k, b);
-  return k;
-}
-
 Sim::StepFlags stepFlagsOf(const Sim& s) {
   return Sim::StepFlags{s.recValid, s.recSValid, s.recSMValid, s.derivsValid, s.pairsValid, s.haveDtIn,
                         s.pairRec, s.outStride, s.timingPending, s.pairWaves};

@@ -368,6 +368,11 @@ bool stateFieldUsed(const Sim& s, int which); // caller-order fields, in culling
 DBuf& stateField(Sim& s, int which);
 int stateFieldComps(const Sim& s, int which);
 constexpr int kStateFields = 13;
+// stepkey.cpp
+// 1/u for the 3-D mixed record's positions (a power of two; from the last
+// neighbour build's largest search radius)
+double quantInv(const Sim& s);
+std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip);
 // hydro.hip
 void omegaGradh(Sim& s);          // computeSPHOmegaGradhCorrection into the omega field
 // one iterateIdealH pass over the current rows; returns the largest change

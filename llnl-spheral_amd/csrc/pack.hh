@@ -218,8 +218,5 @@ struct Sim;
 PackIn packInputs(Sim& s);
 // allocates the records that sec asks for; sets recSValid and recSMValid from bits 4 and 8
 PackOut packOutputs(Sim& s, int sec);
-// 1/u for the 3-D mixed record's positions (a power of two; from the last
-// neighbour build's largest search radius)
-double quantInv(const Sim& s);
 
 }  // namespace sphgpu

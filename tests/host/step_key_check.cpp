@@ -1,0 +1,38 @@
+// The key of a captured step (csrc/stepkey.cpp) must change with everything that the
+// captured launches hold.  Host code only: no device is touched, the buffers are
+// made-up addresses.
+#include "../../llnl-spheral_amd/csrc/internal.hh"
+
+#include <cmath>
+#include <cstdio>
+
+using namespace sphgpu;
+
+static int failures = 0;
+static void check(bool ok, const char* what) {
+  std::printf("%s: %s\n", ok ? "ok" : "FAIL", what);
+  failures += ok ? 0 : 1;
+}
+
+int main() {
+  Sim s;
+  sphgpu_hydro_params fp64{}, mixed{};
+  sphgpu_integrator_params ip{};
+  mixed.precision = SPHGPU_PRECISION_MIXED;
+  s.nInt = s.nTot = s.nSlots = 1000;
+
+  // the unit of the 3-D mixed positions is a power of two above the search radius
+  s.dim = 3;
+  s.posAbsMax = 1.0;
+  auto withRadius = [&](double r, const sphgpu_hydro_params& hp) {
+    s.rMax = r;
+    return stepKey(s, hp, ip);
+  };
+  check(withRadius(0.49, mixed) != withRadius(0.51, mixed), "3-D mixed: search radius across a power of two");
+  check(withRadius(0.26, mixed) == withRadius(0.49, mixed), "3-D mixed: search radius within one power of two");
+  check(withRadius(0.49, fp64) == withRadius(0.51, fp64), "3-D FP64: no unit");
+  check(withRadius(std::ldexp(1.0, 400), fp64) == withRadius(0.51, fp64), "3-D FP64: any search radius");
+  s.dim = 2;
+  check(withRadius(0.49, mixed) == withRadius(0.51, mixed), "2-D mixed: FP64 positions");
+  return failures;
+}
