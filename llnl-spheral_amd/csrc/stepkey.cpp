@@ -62,7 +62,7 @@ std::vector<uint64_t> stepKey(const Sim& s, const sphgpu_hydro_params& hp, const
                         &s.ghostControl, &s.ghostSub, &s.keep, &s.keepScan, &s.slotKeep, &s.hmaxOf, &s.genDev,
                         &s.work, &s.ghostIsControl, &s.omega0, &s.dtIn, &s.seg, &s.segState, &s.plainSeg,
                         &s.dTable, &s.dTable32, &s.dNperh, &s.dWsum, &s.listGamma, &s.subDev, &s.pairCounts, &s.velS, &s.relV,
-                        &s.voteLow})
+                        &s.voteLow, &s.slotList})
     keyBuf(k, *b);
   for (const DBuf& b : s.state0) keyBuf(k, b);
   return k;

@@ -34,5 +34,12 @@ int main() {
   check(withRadius(std::ldexp(1.0, 400), fp64) == withRadius(0.51, fp64), "3-D FP64: any search radius");
   s.dim = 2;
   check(withRadius(0.49, mixed) == withRadius(0.51, mixed), "2-D mixed: FP64 positions");
+
+  // the NodeList of every slot: mixed passes over several NodeLists read it
+  s.nLists = 2;
+  const auto before = stepKey(s, mixed, ip);
+  s.slotList.p = reinterpret_cast<void*>(uintptr_t(4096));
+  check(stepKey(s, mixed, ip) != before, "another buffer of the slots' NodeLists");
+  s.slotList.p = nullptr;                          // not this program's to free
   return failures;
 }

@@ -46,3 +46,47 @@ def test_position_unit_changes_between_replays(sphgpu, n):
     captures, replays = b.graph_counts()
     print(f"[unit] {captures} captures, {replays} replays", flush=True)
     assert captures >= 2 and replays >= 4
+
+
+def test_slot_lists_grow_between_replays(sphgpu):
+    """2-D mixed precision, two NodeLists: a step with more ghosts, and so more slots,
+    than any before it with lists comes between replays with fewer.  The records were
+    sized by steps without lists before, so only the slots' NodeLists grow."""
+    print("[slot lists]", flush=True)
+    n = 24
+    st, _ = problems.random_state(2, n, seed=71, jitter=0.1, vel_scale=0.05)
+    N = st["pos"].shape[0]
+    state = {k: st[k] for k in ("pos", "vel", "mass", "rho", "eps", "H")}
+    hp = sphgpu.hydro_params(precision=sphgpu.PRECISION_MIXED)
+    ip = sphgpu.integrator_params(gamma=1.4, dtMax=1.0e-6)
+    sims = []
+    for graphs in (False, True):
+        s = sphgpu.Sim(2)
+        s.set_row_order(sphgpu.ROW_ORDER_SEARCH)
+        s.set_table_bspline(1000)
+        s.set_boundaries(sphgpu.box_boundaries(2))
+        s.set_precision(sphgpu.PRECISION_MIXED)
+        s.set_graphs(graphs)
+        s.set_nodes(N, N)
+        s.upload_state(dict(state, H=state["H"] / 2.0))
+        s.eos_gamma_law(1.4)
+        s.rk2_step(hp, ip)
+        s.set_nodes(N, N)
+        s.upload_state(state)
+        s.set_node_lists([N // 2, N - N // 2])
+        s.eos_gamma_law(1.4)
+        sims.append(s)
+    a, b = sims
+    counts = []
+    for k, wide in enumerate([0] * 6 + [1] * 6 + [0, 1] * 3):
+        for s in sims:
+            s.upload("position", state["pos"])
+            s.upload("H", state["H"] / (1.9 if wide else 1.0))
+        assert a.rk2_step(hp, ip) == b.rk2_step(hp, ip), k
+        counts.append(b.node_counts())
+        assert a.node_counts() == counts[-1], k
+        for f in FIELDS:
+            assert np.array_equal(a.download(f, rows=N), b.download(f, rows=N)), (k, f)
+    captures, replays = b.graph_counts()
+    print(f"[slot lists] {sorted(set(counts))}, {captures} captures, {replays} replays", flush=True)
+    assert captures >= 2 and replays >= 4
