@@ -559,7 +559,8 @@ template <int D> __device__ __forceinline__ Acc<D> accOf(const double* a) {
 
 // One pair in node i's frame, with the reference's operations: every term goes
 // to add(sum, term), sums in ascending number.  Returns 1 for a pair i owns.
-template <int D, bool ISO, bool TENSILE, class Add>
+// RELV: the row maximum of the vote, where the pass leaves one.
+template <int D, bool ISO, bool TENSILE, bool RELV, class Add>
 __device__ __forceinline__ unsigned pairTerms(const Nbr<D, ISO>& me, const Nbr<D, ISO>& nb, int w, int64_t n, int64_t k,
                                               const double* __restrict__ tab, const TabArgs& t, const PassArgs& p,
                                               const OutArgs& o, double& maxVP, double& relV, Add&& add) {
@@ -568,7 +569,9 @@ __device__ __forceinline__ unsigned pairTerms(const Nbr<D, ISO>& me, const Nbr<D
   const bool ownerI = nb.orig > me.orig;
   const V<D> rij = vsub(me.x, nb.x);
   const V<D> vij = vsub(me.v, nb.v);
-  if (o.relV) relV = dmax(relV, relSpeed<D>(vij.c));
+  if constexpr (RELV) {
+    if (o.relV) relV = dmax(relV, relSpeed<D>(vij.c));
+  }
   const S<D>& Hi = me.H;
   const S<D>& Hj = nb.H;
   const double Hdetj = nb.hdet, mj = nb.m, rhoj = nb.rho, cj = nb.cs, morj = nb.mor;
@@ -654,7 +657,7 @@ __device__ __forceinline__ Self<D> selfOf(const Nbr<D, ISO>& me) {
   return s;
 }
 
-template <int D, bool ISO, bool TENSILE, bool LDS>
+template <int D, bool ISO, bool TENSILE, bool LDS, bool RELV>
 __global__ void __launch_bounds__(kBlock) k_derivs_fp64(const double* __restrict__ rec, const int32_t* __restrict__ rowCount,
                                                         const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
                                                         const int32_t* __restrict__ work, TabArgs t, PassArgs p,
@@ -679,10 +682,10 @@ __global__ void __launch_bounds__(kBlock) k_derivs_fp64(const double* __restrict
     for (int w = 0; w < len; ++w) {
       const Nbr<D, ISO> nb = nx;
       if (w + 1 < len) nx = loadNbr<D, ISO, TENSILE>(rec, nextIndex(nb4, n, k, len, w + 1, cur, nxt));
-      pairs += pairTerms<D, ISO, TENSILE>(me, nb, w, n, k, tab, t, p, o, maxVP, relV,
-                                          [&](int q, double v) { sum[q] += v; });
+      pairs += pairTerms<D, ISO, TENSILE, RELV>(me, nb, w, n, k, tab, t, p, o, maxVP, relV,
+                                                [&](int q, double v) { sum[q] += v; });
     }
-    if (o.relV) o.relV[k] = len > 0 ? relV : -1.0;
+    if constexpr (RELV) o.relV[k] = len > 0 ? relV : -1.0;
     Acc<D> a = accOf<D>(sum);
     a.maxVP = maxVP;
     epilogue<D>(k, len, selfOf(me), a, t, p, o);
@@ -724,7 +727,7 @@ __global__ void __launch_bounds__(kBlock) k_derivs_rows(const double* __restrict
     OutArgs oo = o;
     if (!live) oo.pairDv = nullptr;
     double vp = maxVP, rv = relV;
-    const unsigned own = pairTerms<D, ISO, TENSILE>(
+    const unsigned own = pairTerms<D, ISO, TENSILE, true>(
         me, nb, w, n, k, t.g, t, p, oo, vp, rv, [&](int q, double v) {
           terms[wave][q % L][lane] = live ? v : -0.0;
           if (q % L == L - 1 || q == COUNT - 1) {
@@ -1217,12 +1220,14 @@ __device__ __forceinline__ IsoPair<Real, D> isoPair(const IsoNode<Real, D>& m, c
 // L > 1 (mixed, small node sets): L lanes to a node, each taking whole blocks of
 // kSumBlock entries, and the blocks' FP32 sums enter the FP64 sums in row order:
 // the bits are those of one lane.
-// The 3-D mixed kernel is held to 168 VGPRs, three wavefronts per SIMD: one register
-// more, for the vote's maximum, and it would run at two.
-template <typename Real, int D, int L>
-constexpr int kIsoBlocks = std::is_same<Real, float>::value && D == 3 && L == 1 ? 3 : 1;
-template <typename Real, int D, bool LDS, bool PREFETCH, int BS = kBlock, int L = 1>
-__global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, L>)) k_derivs_iso(const double* __restrict__ rec,
+// RELV: the pass leaves the row maxima of the dt vote.  An instance of its own, so that
+// the passes that leave none hold no register for them.  The 3-D mixed one is held to
+// 168 VGPRs, three wavefronts per SIMD: it needs one register more and would run at two.
+template <typename Real, int D, int L> constexpr bool kCanRelV = !std::is_same<Real, float>::value || (D == 3 && L == 1);
+template <typename Real, int D, bool RELV>
+constexpr int kIsoBlocks = RELV && std::is_same<Real, float>::value && D == 3 ? 3 : 1;
+template <typename Real, int D, bool LDS, bool PREFETCH, int BS = kBlock, int L = 1, bool RELV = false>
+__global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, RELV>)) k_derivs_iso(const double* __restrict__ rec,
                                                        const typename IsoTab<Real>::Rec* __restrict__ recN,
                                                        const int32_t* __restrict__ rowCount,
                                                        const int32_t* __restrict__ nbr, int64_t n, int64_t nInt,
@@ -1233,6 +1238,7 @@ __global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, L>)) k_derivs_iso(con
   using E = typename IsoTab<Real>::Elem;
   constexpr bool F32 = std::is_same<Real, float>::value;
   static_assert(L == 1 || (F32 && !LDS), "several lanes to a node: mixed, the table through L1");
+  static_assert(!RELV || kCanRelV<Real, D, L>, "no row maxima here");
   extern __shared__ double ldsIso[];
   const E* tab;
   if constexpr (LDS) {
@@ -1262,14 +1268,12 @@ __global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, L>)) k_derivs_iso(con
     auto pair = [&](const INbr<Real>& nb, int32_t j, int w) {
       pairs += (nb.ghost || j > int32_t(k)) ? 1u : 0u;
       const IsoPair<Real, D> q = isoPair<Real, D>(me, nb, tab, tt, p);
-      if constexpr (!F32) {
-        if (o.relV) relV = dmax(relV, relSpeed<D>(q.vij));
-      } else if constexpr (D == 3 && L == 1) {
-        if (o.relV) {
-          float v2 = q.vij[0] * q.vij[0];
-          for (int c = 1; c < D; ++c) v2 = fmaR(q.vij[c], q.vij[c], v2);
-          relV = maxR(relV, v2);
-        }
+      if constexpr (RELV && !F32) {
+        relV = dmax(relV, relSpeed<D>(q.vij));
+      } else if constexpr (RELV) {
+        float v2 = q.vij[0] * q.vij[0];
+        for (int c = 1; c < D; ++c) v2 = fmaR(q.vij[c], q.vij[c], v2);
+        relV = maxR(relV, v2);
       }
       maxVP = maxR(maxVP, q.Qi);
       if (o.pairDv)
@@ -1363,9 +1367,7 @@ __global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, L>)) k_derivs_iso(con
     if (L == 1 || threadIdx.x % L == 0) {
       for (int c = 0; c < D; ++c)
         for (int b = 0; b < c; ++b) a.M.c[c * D + b] = a.M.c[b * D + c];
-      if constexpr (!F32 || (D == 3 && L == 1)) {
-        if (o.relV) o.relV[k] = len > 0 ? double(relV) : -1.0;
-      }
+      if constexpr (RELV) o.relV[k] = len > 0 ? double(relV) : -1.0;
       isoEpilogue<D>(k, len, ri_, a, t, p, o);
     }
   }
@@ -1738,14 +1740,19 @@ void isoLaunch(Sim& s, bool inLds, hipStream_t st, int64_t n, const TabArgs& t, 
   const Rec* recN = reinterpret_cast<const Rec*>(std::is_same<Real, float>::value ? s.recM.p : s.recD.p);
   const size_t lb = inLds ? sizeof(typename IsoTab<Real>::Elem) * IsoTab<Real>::PER * size_t(s.table.n) : 0;
   const dim3 g(unsigned(xcdGrid(nblocks(s.nInt * L, BS)))), b(BS);
-  if (L == 1 && inLds)
-    hipLaunchKernelGGL((k_derivs_iso<Real, D, L == 1, PF, BS, L>), g, b, lb, st, s.rec.as<double>(), recN,
-                       s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
-                       isoTable<Real>(s), p, o, counts);
-  else
-    hipLaunchKernelGGL((k_derivs_iso<Real, D, false, PF, BS, L>), g, b, 0, st, s.rec.as<double>(), recN,
-                       s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
-                       isoTable<Real>(s), p, o, counts);
+  auto go = [&](auto kern, size_t ldsB) {
+    hipLaunchKernelGGL(kern, g, b, ldsB, st, s.rec.as<double>(), recN, s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n,
+                       s.nInt, s.work.as<int32_t>(), t, isoTable<Real>(s), p, o, counts);
+  };
+  auto tables = [&](auto relV) {
+    constexpr bool RELV = decltype(relV)::value;
+    if (L == 1 && inLds) go(k_derivs_iso<Real, D, L == 1, PF, BS, L, RELV>, lb);
+    else go(k_derivs_iso<Real, D, false, PF, BS, L, RELV>, 0);
+  };
+  if constexpr (kCanRelV<Real, D, L>) {
+    if (o.relV) return tables(std::true_type{});
+  }
+  tables(std::false_type{});
 }
 template <typename Real, int D, bool PF>
 void isoVariant(Sim& s, int v, bool fits, hipStream_t st, int64_t n, const TabArgs& t, const PassArgs& p,
@@ -1829,11 +1836,12 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
     s.pairDv.ensure(sizeof(double) * size_t(D) * size_t(std::max<int64_t>(o.plane, 1)));
     o.pairDv = s.pairDv.as<double>();
   }
-  // Mixed: one record in flight per lane keeps the kernel at 168 VGPRs, three
+  // Mixed: one record in flight per lane keeps the kernel at 167 VGPRs, three
   // wavefronts per SIMD (2.11 ms at 128^3 against 2.53 ms with the next
-  // record prefetched at 179 VGPRs, two wavefronts; 2.20 ms since it can leave the
-  // row maxima of the vote).  FP64: the prefetch wins
-  // (3.44 ms at 194 VGPRs against 3.51 ms at 168).
+  // record prefetched at 179 VGPRs, two wavefronts).  The pass that leaves the
+  // vote's row maxima spills two registers to stay at three: 2.05 ms where a pass
+  // without them takes 2.00.  FP64: the prefetch wins (3.44 ms at 194 VGPRs
+  // against 3.51 ms at 168).
   if (mixed && lanes > 1) {
     if constexpr (D > 1) isoLaunch<float, D, false, kBlock, D == 3 ? 8 : 2>(s, false, st, n, t, p, o, counts);
     SG_CHECK_HIP(hipGetLastError());
@@ -1884,12 +1892,20 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
           else { if (tensile) any(no, yes); else any(no, no); }
         }
       });
-    } else if (lds) {
-      if (s.isotropic) { if (tensile) launch(k_derivs_fp64<D, true, true, true>); else launch(k_derivs_fp64<D, true, false, true>); }
-      else { if (tensile) launch(k_derivs_fp64<D, false, true, true>); else launch(k_derivs_fp64<D, false, false, true>); }
     } else {
-      if (s.isotropic) { if (tensile) launch(k_derivs_fp64<D, true, true, false>); else launch(k_derivs_fp64<D, true, false, false>); }
-      else { if (tensile) launch(k_derivs_fp64<D, false, true, false>); else launch(k_derivs_fp64<D, false, false, false>); }
+      auto any = [&](auto iso, auto tens, auto relv) {
+        constexpr bool ISO = decltype(iso)::value, TENSILE = decltype(tens)::value, RELV = decltype(relv)::value;
+        if (lds) launch(k_derivs_fp64<D, ISO, TENSILE, true, RELV>);
+        else launch(k_derivs_fp64<D, ISO, TENSILE, false, RELV>);
+      };
+      auto votes = [&](auto iso, auto tens) {
+        if (relV) any(iso, tens, std::true_type{});
+        else any(iso, tens, std::false_type{});
+      };
+      const std::true_type yes{};
+      const std::false_type no{};
+      if (s.isotropic) { if (tensile) votes(yes, yes); else votes(yes, no); }
+      else { if (tensile) votes(no, yes); else votes(no, no); }
     }
   }
   SG_CHECK_HIP(hipGetLastError());
