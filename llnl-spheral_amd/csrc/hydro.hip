@@ -1718,7 +1718,7 @@ void sumDensityD(Sim& s) {
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        s.rho.as<double>(), nrec, listOf, s.sumAllLists ? 1 : 0);
   };
-  withLanes<D>(rowLanes(RowPass::kDensity, D, s.nInt), [&](auto lanes) {
+  withLanes<D>(rowLanes(s.isotropic ? RowPass::kDensity : RowPass::kDensityAnyH, D, s.nInt), [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     auto any = [&](auto iso) {
       constexpr bool ISO = decltype(iso)::value;
@@ -1797,7 +1797,10 @@ void evalDerivsD(Sim& s, const sphgpu_hydro_params& hp, bool updateOnly, bool re
   const bool fast64 = sec == 2;
   // lanes to a node: mixed blocks need rows of several blocks, so 1-D keeps one
   const int lanes = mixed ? mixedLanes(D, s.nInt)
-                          : rowLanes(fast64 ? RowPass::kIsoPairs : RowPass::kPairs, D, s.nInt);
+                          : rowLanes(fast64 ? RowPass::kIsoPairs
+                                            : !s.isotropic ? RowPass::kPairsAnyH
+                                                           : compat ? RowPass::kPairsStored : RowPass::kPairs,
+                                     D, s.nInt);
   s.pairWaves = (s.nInt * lanes + 63) / 64;
   s.pairCounts.ensure(sizeof(uint32_t) * size_t(std::max<int64_t>(s.pairWaves, 1)));
   uint32_t* counts = s.pairCounts.as<uint32_t>();
@@ -1932,7 +1935,7 @@ void omegaGradhD(Sim& s) {
                        s.rowCount.as<int32_t>(), s.nbr.as<int32_t>(), n, s.nInt, s.work.as<int32_t>(), t,
                        s.omega.as<double>());
   };
-  withLanes<D>(rowLanes(RowPass::kOmega, D, s.nInt), [&](auto lanes) {
+  withLanes<D>(rowLanes(s.isotropic ? RowPass::kOmega : RowPass::kOmegaAnyH, D, s.nInt), [&](auto lanes) {
     constexpr int L = decltype(lanes)::value;
     auto any = [&](auto iso) {
       constexpr bool ISO = decltype(iso)::value;
