@@ -207,10 +207,11 @@ inline double fromOrderedBits(unsigned long long o) {
 // members (39 k rows), 18 -> 8 us for 24 tubes.  `clear` is the next build's table.
 constexpr int kSegGroups = 16;
 template <int D>
-__global__ void k_seg_bounds(const double* __restrict__ pos, const double* __restrict__ H,
-                             const double* __restrict__ seg, int64_t n, const int64_t* __restrict__ nDev, int groups,
-                             unsigned long long* __restrict__ bits, unsigned long long* __restrict__ clear,
-                             int words) {
+__global__ void __launch_bounds__(kBlock) k_seg_bounds(const double* __restrict__ pos, const double* __restrict__ H,
+                                                       const double* __restrict__ seg, int64_t n,
+                                                       const int64_t* __restrict__ nDev, int groups,
+                                                       unsigned long long* __restrict__ bits,
+                                                       unsigned long long* __restrict__ clear, int words) {
   if (nDev) n = *nDev;
   const int64_t tid = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
   for (int64_t q = tid; q < words; q += int64_t(gridDim.x) * blockDim.x) clear[q] = 0ull;

@@ -48,7 +48,7 @@ def kernels(tmp_path):
 
 
 @pytest.mark.skipif(not os.path.exists(LIB), reason="the library is not built")
-@pytest.mark.parametrize("part", ["k_derivs"])
+@pytest.mark.parametrize("part", ["k_derivs", ""], ids=["pair kernels", "all"])
 def test_no_kernel_spills_registers(tmp_path, part):
     found = kernels(tmp_path)
     assert len(found) > 100
