@@ -15,7 +15,9 @@
 // a first launch writes the tiles' sums and the second adds up those before its
 // tile.  Measured: 4.5 us for one launch of 8 k items; at 30 k 8 us for the two,
 // where one launch took 14-28 us (its last tile counts 28 k items again) and a
-// scan in one workgroup 11 us without the producer and the consumer.
+// scan in one workgroup 11 us without the producer and the consumer.  What the
+// second launch adds up grows with the square of the tiles, so from kScanPrefix
+// tiles on (the cells of a sparse grid) one workgroup sums them up between the two.
 #pragma once
 #include <cstdint>
 #include <type_traits>
@@ -32,6 +34,10 @@ constexpr int64_t kScanOnce = 8192;
 // sums before it costs more than that gives (2.4 M rows: 31 us at four, 38 at two,
 // 63 at one).
 constexpr int64_t kScanOnePer = 524288;
+// Tiles up to which each workgroup adds up the sums before its own.  A whole neighbour
+// build of 90 k nodes in two clumps, without and with the launch between: 37 M cells
+// (18 k tiles) 0.29 and 0.26 ms, 100 M 0.88 and 0.56, 0.9 G 23.2 and 3.9.
+constexpr int64_t kScanPrefix = 16384;
 
 // The workgroup's tile, given each thread's part of the sum before the tile.
 template <int PER, class F>
@@ -116,10 +122,52 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_sums(F f, int64_t n, int32_
   }
 }
 
-template <int PER, class F>
+// The tiles' sums become the sums before each tile (one workgroup).
+constexpr int kPrefixBlock = 1024, kPrefixPer = 4;
+static __global__ void __launch_bounds__(kPrefixBlock) k_scan_prefix(int32_t* __restrict__ tileSums, int64_t tiles) {
+  __shared__ int32_t waveSum[kPrefixBlock / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int32_t carry = 0;
+  for (int64_t t0 = 0; t0 < tiles; t0 += kPrefixBlock * kPrefixPer) {
+    const int64_t base = t0 + int64_t(threadIdx.x) * kPrefixPer;
+    int32_t v[kPrefixPer], local = 0;
+#pragma unroll
+    for (int q = 0; q < kPrefixPer; ++q) {
+      v[q] = base + q < tiles ? tileSums[base + q] : 0;
+      local += v[q];
+    }
+    int32_t incl = local;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+      const int32_t t = __shfl_up(incl, s);
+      if (lane >= s) incl += t;
+    }
+    if (lane == 63) waveSum[wave] = incl;
+    __syncthreads();
+    int32_t run = carry + incl - local;
+#pragma unroll
+    for (int w = 0; w < kPrefixBlock / 64; ++w) {
+      run += w < wave ? waveSum[w] : 0;
+      carry += waveSum[w];
+    }
+#pragma unroll
+    for (int q = 0; q < kPrefixPer; ++q) {
+      if (base + q < tiles) tileSums[base + q] = run;
+      run += v[q];
+    }
+    __syncthreads();                               // waveSum is written again
+  }
+}
+
+// PREFIX: tileSums holds the sums before each tile.
+template <int PER, bool PREFIX, class F>
 __global__ void __launch_bounds__(kScanBlock) k_scan_emit(F f, int64_t n, const int32_t* __restrict__ tileSums) {
   int32_t before = 0;
-  for (int64_t t = threadIdx.x; t < blockIdx.x; t += kScanBlock) before += tileSums[t];
+  if constexpr (PREFIX) {
+    if (threadIdx.x == 0) before = tileSums[blockIdx.x];
+  } else {
+    for (int64_t t = threadIdx.x; t < blockIdx.x; t += kScanBlock) before += tileSums[t];
+  }
   scanTile<PER>(f, n, before);
 }
 
@@ -131,7 +179,16 @@ template <class F> void scanItems(const F& f, int64_t n, DBuf& tmp, hipStream_t 
     const int64_t tiles = tilesOf(PER);
     tmp.ensure(sizeof(int32_t) * size_t(tiles));
     hipLaunchKernelGGL((k_scan_sums<PER, F>), dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n, tmp.as<int32_t>());
-    hipLaunchKernelGGL((k_scan_emit<PER, F>), dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n, tmp.as<int32_t>());
+    if constexpr (PER > 1) {
+      if (tiles > kScanPrefix) {
+        hipLaunchKernelGGL(k_scan_prefix, dim3(1), dim3(kPrefixBlock), 0, st, tmp.as<int32_t>(), tiles);
+        hipLaunchKernelGGL((k_scan_emit<PER, true, F>), dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n,
+                           tmp.as<int32_t>());
+        return;
+      }
+    }
+    hipLaunchKernelGGL((k_scan_emit<PER, false, F>), dim3(unsigned(tiles)), dim3(kScanBlock), 0, st, f, n,
+                       tmp.as<int32_t>());
   };
   if (n <= kScanOnce) hipLaunchKernelGGL(k_scan_once<F>, dim3(unsigned(tilesOf(4))), dim3(kScanBlock), 0, st, f, n);
   else if (n <= kScanOnePer) two(std::integral_constant<int, 1>{});
