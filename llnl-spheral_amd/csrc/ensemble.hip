@@ -239,16 +239,22 @@ int ensembleStep(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_
   return done;
 }
 
+// Device memory of one row, buffer by buffer (rows of ghosts count like nodes; slots of
+// culled ghosts, 2 % in a 3-D box, and row capacities beyond the default do not).
 int64_t ensembleBytesPerNode(int dim) {
   const int D = dim, NS = nsymOf(D);
-  const int64_t state = 8 * (2 * D + NS + 8);          // pos vel H m rho eps P cs omega seg hmax
-  const int64_t spare = state;                          // compaction spares
-  const int64_t rec = 128 + 64 + 128;                   // FP64, mixed and collapsed records
+  const int64_t fields = 8 * (2 * D + NS + 7);          // pos vel H m rho eps P cs omega seg
+  const int64_t state = 2 * (fields + fields / 4) + 8;  // grown a quarter at a time, the spares of a removal; hmaxOf
+  // FP64: rec, recD, recS, relV; mixed: rec, recM, recSM, velS, and in 3-D relV and voteLow
+  const int64_t velocities = 8 * (D == 3 ? 4 : D) + (D == 3 ? 16 : 0);
+  const int64_t rec = 128 + std::max<int64_t>(96 + 48 + 8, 64 + 32 + velocities);
   const int64_t out = 8 * int64_t(derivTotalDoubles(D));
   const int64_t ell = 4 * (D == 3 ? 160 : (D == 2 ? 48 : 16)) + 4;
-  const int64_t sortMaps = 4 * 8;                      // cellOf, perm, iperm, work, flags, scans
-  const int64_t step = 8 * (2 * D + 2 + NS) + 8 * (2 + D) + 8;   // state0, dt inputs, grad-h omega0
-  return state + spare + rec + out + ell + sortMaps + step;
+  // cellOf cellRank cellMembers perm iperm(2) work keep keepScan slotKeep, control sub
+  // (2 each) isControl, and the cells' counts and starts
+  const int64_t sortMaps = 4 * 10 + 4 * 5 + 4 * 2;
+  const int64_t step = 8 * (2 * D + 2) + 8 * (2 + D) + 8;   // state0, dt inputs, grad-h omega0
+  return state + rec + out + ell + sortMaps + step;
 }
 
 }  // namespace sphgpu
