@@ -94,6 +94,7 @@ struct ClearedTable {
   int half = 0;
   unsigned long long* take(size_t n, hipStream_t st, unsigned long long*& next) {
     if (n != words) {
+      words = 0;                   // until the new table is there: an allocation may fail
       buf.ensure(2 * n * sizeof(unsigned long long));
       ZeroSet z{};
       z.add(buf.as<int32_t>(), int64_t(4 * n));
