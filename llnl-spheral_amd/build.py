@@ -17,7 +17,7 @@ LIBDIR = os.path.join(PKG, "lib")
 LIB = os.path.join(LIBDIR, "libsphgpu.so")
 
 SOURCES = ["abi.cpp", "table.cpp", "neighbors.hip", "hydro.hip", "ghosts.hip", "integrate.hip", "stepkey.cpp", "ensemble.hip",
-           "serve.cpp", "probe.hip", "transfer.hip", "tune.cpp"]
+           "serve.cpp", "probe.hip", "transfer.hip", "download.cpp", "tune.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("SPHGPU_ARCH", "gfx950")

@@ -431,6 +431,7 @@ __host__ __device__ inline SearchFlags foldFlags(const int32_t* f) {
   }
   return o;
 }
+// download.cpp
 // Device memory to the caller's, complete on return.
 void copyToHost(Sim& s, void* host, const void* dev, size_t bytes);
 // First half of the ghost cull: keep flags and scan, the planes' new first

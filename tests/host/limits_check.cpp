@@ -5,12 +5,19 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <vector>
 
-static bool failDevice = false;
+static bool failDevice = false, failPinned = false;
+static hipError_t lastError = hipSuccess;
+static int copies = 0, failCopy = -1;              // copies so far; the one that fails
+static hipError_t set(hipError_t e) {
+  if (e != hipSuccess) lastError = e;
+  return e;
+}
 
 extern "C" {
 hipError_t hipMalloc(void** p, size_t n) {
-  if (failDevice) return hipErrorOutOfMemory;
+  if (failDevice) return set(hipErrorOutOfMemory);
   *p = std::malloc(n);
   return hipSuccess;
 }
@@ -19,6 +26,28 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t) { return "stand-in"; }
+hipError_t hipGetLastError() {
+  const hipError_t e = lastError;
+  lastError = hipSuccess;
+  return e;
+}
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (failPinned) return set(hipErrorOutOfMemory);
+  *p = std::malloc(n);
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  *e = nullptr;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void* to, const void* from, size_t n, hipMemcpyKind, hipStream_t) {
+  if (copies++ == failCopy) return set(hipErrorUnknown);
+  std::memcpy(to, from, n);
+  return hipSuccess;
+}
 }
 
 namespace sphgpu {
@@ -59,7 +88,46 @@ static void clearedTable() {
   }
 }
 
+// A large download without pinned memory, through it, and after a failed transfer.
+static void largeDownloads() {
+  const size_t mb = size_t(1) << 20;
+  std::vector<char> from(40 * mb);
+  for (size_t q = 0; q < from.size(); ++q) from[q] = char(q * 2654435761u >> 13);
+  auto copied = [&](Sim& s, size_t bytes) {
+    std::vector<char> to(bytes + 1, 77);
+    copyToHost(s, to.data(), from.data(), bytes);
+    return std::memcmp(to.data(), from.data(), bytes) == 0 && to[bytes] == 77;
+  };
+  Sim s;
+  failPinned = true;
+  bool ok = false;
+  try {
+    ok = copied(s, 9 * mb);
+  } catch (const Error&) {
+  }
+  check(ok, "9 MB without pinned memory");
+  check(hipGetLastError() == hipSuccess, "no error left for the next call");
+  failPinned = false;
+  for (size_t bytes : {size_t(0), size_t(8), 4 * mb - 8, 4 * mb, 4 * mb + 8, 8 * mb, 9 * mb + 16, 40 * mb - 24, 40 * mb})
+    check(copied(s, bytes), "through the slots, or straight below 4 MB");
+  check(s.ring != nullptr, "the slots are there");
+  copies = 0;
+  failCopy = 13;
+  bool threw = false;
+  try {
+    (void)copied(s, 40 * mb);
+  } catch (const Error&) {
+    threw = true;
+  }
+  failCopy = -1;
+  (void)hipGetLastError();
+  check(threw, "a failed transfer");
+  check(copied(s, 40 * mb), "and the next download");
+  std::free(s.ring);
+}
+
 int main() {
   clearedTable();
+  largeDownloads();
   return failures;
 }

@@ -9,8 +9,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 def test_limits(tmp_path):
     exe = str(tmp_path / "limits_check")
     cmd = ["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include",
-           "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "host", "limits_check.cpp"), "-o", exe,
-           "-pthread"]
+           "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "host", "limits_check.cpp"),
+           os.path.join(ROOT, "llnl-spheral_amd", "csrc", "download.cpp"), "-o", exe, "-pthread"]
     r = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
