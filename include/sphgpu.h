@@ -362,8 +362,9 @@ int sphgpu_graph_counts(sphgpu_sim* sim, int64_t* captures, int64_t* replays);
  * arithmetic, log2 buckets of row length and node count) times every launch
  * variant on the live inputs and keeps the fastest; variants compute the same
  * values in the same order, so results do not change.  Tuned now: the 1-D
- * and 2-D isotropic pair kernel (workgroups of 64-512 threads, table in LDS
- * or read through L1).  Decisions export as text lines and import again, so
+ * and 2-D isotropic pair kernel with one lane to a node (workgroups of 64-512
+ * threads, table in LDS or read through L1; smaller node sets take several lanes
+ * to a node in one launch shape).  Decisions export as text lines and import again, so
  * that measured choices are reused without timing. */
 int sphgpu_autotune(int on);
 /* Copy the decision table into buf (NUL-terminated, at most cap bytes);
