@@ -80,7 +80,7 @@ def test_options_at_every_lane_count(sphgpu, oracle, dim, n, option):
     assert np.array_equal(s.download("grad h corrections", rows=N), om)
 
 
-@pytest.mark.parametrize("dim,n", [(2, 128), (2, 129), (2, 250), (2, 287), (3, 25), (3, 26), (3, 50)])
+@pytest.mark.parametrize("dim,n", [(2, 128), (2, 129), (2, 250), (2, 287), (3, 25), (3, 26), (3, 50), (3, 55)])
 def test_nodelists_at_every_lane_count(sphgpu, oracle, dim, n):
     nodelists.test_pass_with_nodelists(sphgpu, oracle, (dim, n, "reflecting"), 0, False)
 
@@ -90,3 +90,10 @@ def test_stored_pair_terms_at_the_lines(sphgpu, oracle, n):
     """Compatible energy in 3-D: 97336 | 103823 nodes and 157464, 8 lanes to the pair
     pass, one, 8."""
     dispatch.test_compatible_energy_across_lanes(sphgpu, oracle, 3, n)
+
+
+@pytest.mark.parametrize("n", [32768, 32769])
+def test_ideal_h_and_compatible_energy_on_a_line(sphgpu, oracle, n):
+    """1-D: 8 lanes to a node and one."""
+    dispatch.test_ideal_h_across_lanes(sphgpu, oracle, 1, n)
+    dispatch.test_compatible_energy_across_lanes(sphgpu, oracle, 1, n)
