@@ -553,6 +553,56 @@ def periodic_bench(sphgpu, problems, n, steps):
     return res
 
 
+# The stdout line stays below this many characters, so that a log's tail holds it whole.
+LINE_LIMIT = 4000
+# What only the full report holds: explanations, and lists that grow with the sizes.
+REPORT_ONLY = ("note", "method", "oracle", "sample_points", "per_member", "per_request", "sample", "drift", "decisions",
+               "variants", "fields_rel_linf_l2", "flops_per_entry", "flops_per_launch", "flop_rate_tflops",
+               "flop_peaks_tflops", "fp64_row_order_control", "momentum_scale", "loads_per_launch", "dt", "step")
+# Dropped in this order from a line that is still too long; the contract's keys never are.
+OPTIONAL = ("autotune", "copy_probe", "density_gather", "periodic", "parity_vs_oracle", "mixed_pass", "rk2",
+            "cpu_baseline", "roofline", "serving", "ensemble")
+
+
+def stdout_line(report):
+    """The report's one JSON line: the measurement itself as it is, the rest in short."""
+    def short(v):
+        if isinstance(v, dict):
+            return {k: short(x) for k, x in v.items()
+                    if k not in REPORT_ONLY and not (isinstance(x, list) and len(x) > 4)}
+        if isinstance(v, float):
+            return float(f"{v:.6g}")
+        if isinstance(v, str) and len(v) > 160:
+            return v[:157] + "..."
+        return v
+
+    line = {k: short(v) if isinstance(v, dict) else v for k, v in report.items()}
+    for k in ("ensemble", "serving", "periodic"):
+        if k in line:
+            line[k].pop("workload", None)
+    if "mixed_pass" in line:
+        m = line["mixed_pass"]
+        line["mixed_pass"] = {k: m[k] for k in ("value", "unit", "ms_per_step", "speedup_vs_fp64", "dtype",
+                                                "parity_vs_oracle") if k in m}
+        line["mixed_pass"]["roofline_frac"] = m.get("roofline", {}).get("frac")
+    if "density_gather" in line:
+        line["density_gather"] = {"frac": line["density_gather"].get("frac")}
+    if isinstance(report.get("cpu_baseline"), dict):
+        line["cpu_baseline"] = dict(line["cpu_baseline"], sample=short(report["cpu_baseline"].get("sample")))
+    for k in OPTIONAL:
+        if len(json.dumps(line)) <= LINE_LIMIT:
+            break
+        line.pop(k, None)
+    return json.dumps(line)
+
+
+def emit(report, path):
+    if path:
+        with open(path, "w") as f:
+            json.dump(report, f, indent=1)
+    print(stdout_line(report), flush=True)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -593,6 +643,9 @@ def main():
     ap.add_argument("--periodic", type=int, default=256,
                     help="periodic mixed-vs-FP64 comparison at this lattice size (256 = the configuration; 0 = off)")
     ap.add_argument("--periodic-steps", type=int, default=200)
+    ap.add_argument("--report", default=None,
+                    help="file for the full report (every request, field and tuning decision; about 30 KB), of which "
+                         "the line on stdout is the short form")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py measures one GPU; --gpus {args.gpus} is not supported in this build "
@@ -632,7 +685,7 @@ def main():
             line["serving"] = serve_bench(sphgpu, problems, args.serve, args.serve_rate, args.batch_precision,
                                           args.serve_check, graphs=args.graphs)
         line["autotune"] = tuning_report()
-        print(json.dumps(line), flush=True)
+        emit(line, args.report)
         return
 
     t_setup = time.perf_counter()
@@ -802,7 +855,7 @@ def main():
             line["cpu_baseline"] = cpu_baseline(args.cpu_budget, boundaries=args.boundaries)
         except Exception as e:  # the baseline is reported, never required
             line["cpu_baseline"] = {"value": None, "error": str(e)}
-    print(json.dumps(line), flush=True)
+    emit(line, args.report)
 
 
 if __name__ == "__main__":
