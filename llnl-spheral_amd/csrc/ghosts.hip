@@ -14,16 +14,20 @@
 // control no other ghost are culled, the rest keep their order
 // (src/Integrator/Integrator.cc:491-570, src/Boundary/Boundary.cc:182-233).
 //
-// Device form: per sub-boundary one pass over the current nodes computes hmax
-// (wavefront max + one 64-bit atomic max per wavefront on the bit pattern of a
-// non-negative double), a second flags the controls, an exclusive scan places
-// the ghosts, and a third writes them after the current rows.  Ghost fields
-// are filled boundary by boundary (a ghost's control always precedes it).
-// Culling: the row search marks every ghost slot it puts in a row; a scan of
-// the keep flags in caller order gives the old -> new index map; the state is
-// compacted and the slot permutation renumbered.  Slots themselves stay where
-// they are (culled ghosts become dead slots that no row holds), so the rows,
-// their entries and their order are untouched and no second build is needed.
+// Device form: one launch over the internal rows enters h into the hmax of every plane
+// they are near (wavefront maximum, one 64-bit atomic max on the bit pattern of a
+// non-negative double); then per plane one launch (two for large node sets) flags the
+// controls, scans and appends their ghosts, which enter themselves for the planes
+// after their own (scan.hh).  The row counts stay on the device and the launches cover
+// a capacity; the neighbour build reads the counts back with its bounds.  Ghost fields
+// are filled by one launch, each ghost from its internal node through the maps of the
+// planes between.
+// Culling: the row search marks every ghost slot it puts in a row; a scan of the keep
+// flags over the ghosts gives the old -> new index map; the controls, the planes and the
+// caller <-> slot maps are renumbered and the kept ghosts' rows filled again at their
+// new place.  Slots themselves stay where they are (culled ghosts become dead slots that
+// no row holds), so the rows, their entries and their order are untouched and no second
+// build is needed.
 //
 // Floating-point order follows the reference exactly: plane distances
 // n.(x - p), closest points x + ((p - x).n) n (3-D), the 2-D and 1-D special

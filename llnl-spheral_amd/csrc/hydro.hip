@@ -807,7 +807,7 @@ template <typename Real> struct INbr {
   bool ghost;
 };
 template <int D>
-__device__ __forceinline__ void loadIso(const float4* __restrict__ recM, int64_t, int32_t j, INbr<float>& o) {
+__device__ __forceinline__ void loadIso(const float4* __restrict__ recM, int32_t j, INbr<float>& o) {
   const float4* p = recM + int64_t(j) * MixedRec<D>::F4;
   auto dbl = [](float lo, float hi) { return __hiloint2double(__float_as_int(hi), __float_as_int(lo)); };
   float h;
@@ -837,10 +837,9 @@ __device__ __forceinline__ void loadIso(const float4* __restrict__ recM, int64_t
 // (the off-diagonal products are exact zeros), so the value is bitwise the
 // packed one; m/rho is m * (1/rho), within an ulp.
 template <int D>
-__device__ __forceinline__ void loadIso(const double2* __restrict__ recD, int64_t, int32_t j, INbr<double>& o) {
-  const double2* a = recD + int64_t(j) * 6;
-  const double2* b = a + 4;
-  const double2 d0 = a[0], d1 = a[1], d2 = a[2], d3 = a[3], e0 = b[0], e1 = b[1];
+__device__ __forceinline__ void loadIso(const double2* __restrict__ recD, int32_t j, INbr<double>& o) {
+  const double2* p = recD + int64_t(j) * 6;
+  const double2 d0 = p[0], d1 = p[1], d2 = p[2], d3 = p[3], e0 = p[4], e1 = p[5];
   o.x[0] = d0.x; o.x[1] = d0.y; o.x[2] = d1.x;
   o.ghost = d1.y < 0.0;
   const double hinv = fabs(d1.y);
@@ -861,7 +860,7 @@ __global__ void k_pack_mixed(const double* __restrict__ rec, int64_t n, int64_t 
 template <int D>
 __global__ void k_pack_fast64(const double* __restrict__ rec, int64_t n, int64_t nInt, double2* __restrict__ recD) {
   const int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x;
-  if (k < n) writeFast64Rec<D>(rec + k * RL<true>::STRIDE, nInt, recD + k * 6, recD + k * 6 + 4);
+  if (k < n) writeFast64Rec<D>(rec + k * RL<true>::STRIDE, nInt, recD + k * 6);
 }
 
 template <int D>
@@ -1333,7 +1332,7 @@ __global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, RELV>)) k_derivs_iso(
         for (int w = wb; w < we; ++w) {
           const int32_t j = nbr[ellIndex(w, n, k)];
           INbr<Real> nb;
-          loadIso<D>(recN, n, j, nb);
+          loadIso<D>(recN, j, nb);
           pair(nb, j, w);
         }
         af.flushInto(a, [&](double s, double v) { return addInOrder<L>(s, v, wbuf); });
@@ -1346,7 +1345,7 @@ __global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, RELV>)) k_derivs_iso(
       int4 nxt = len > 4 ? nb4[ellChunk(1, n, k)] : make_int4(0, 0, 0, 0);
       INbr<Real> nx;
       int32_t jn = cur.x;
-      if (PREFETCH && len > 0) loadIso<D>(recN, n, jn, nx);
+      if (PREFETCH && len > 0) loadIso<D>(recN, jn, nx);
       for (int w = 0; w < len; ++w) {
         INbr<Real> nb;
         int32_t j;
@@ -1356,12 +1355,12 @@ __global__ void __launch_bounds__(BS, (kIsoBlocks<Real, D, RELV>)) k_derivs_iso(
           j = jn;
           if (w + 1 < len) {
             jn = nextIndex(nb4, n, k, len, w + 1, cur, nxt);
-            loadIso<D>(recN, n, jn, nx);
+            loadIso<D>(recN, jn, nx);
           }
         } else {
           // one record in flight per lane (fewer registers, more waves)
           j = w == 0 ? cur.x : nextIndex(nb4, n, k, len, w, cur, nxt);
-          loadIso<D>(recN, n, j, nb);
+          loadIso<D>(recN, j, nb);
         }
         pair(nb, j, w);
         if constexpr (F32) {
@@ -1470,7 +1469,7 @@ __global__ void __launch_bounds__(kBlock) k_derivs_iso_rows(const double* __rest
     const bool live = w < len;
     const int32_t j = live ? nbr[ellIndex(w, n, k)] : int32_t(k);
     INbr<double> nb;
-    loadIso<D>(recN, n, j, nb);
+    loadIso<D>(recN, j, nb);
     const IsoPair<double, D> q = isoPair<double, D>(me, nb, t.g, tt, p);
     if (live) {
       pairs += (nb.ghost || j > int32_t(k)) ? 1u : 0u;

@@ -570,7 +570,7 @@ template <int D> double hydroDtD(Sim& s, double nPerh, double cfl, int useVelMag
   return cfl * minDt;
 }
 
-// Per-member dt selection, the same expressions as rk2D's host selection.
+// Every member's vote and failure flags before a step.
 __global__ void k_seg_vote_init(SegState* __restrict__ st, int n, unsigned long long v) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
@@ -645,8 +645,10 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
     voteD<D, decltype(from)::value>(s, hp.nPerh, ip.useVelocityMagnitudeForDt, vote.seg, vote.bits, vote.stride);
   };
   // In 2-D a row has 28 neighbours and the gather is no slower than the two launches
-  // (250 k nodes: 20 and 18 + 5 us); a small 3-D set has several lanes to a node in
-  // the pair pass, which keep no maxima.
+  // (250 k nodes: 20 and 18 + 5 us).  In 3-D the pair pass keeps maxima with one lane to
+  // a node, from 49153 nodes; the bounds gain there already, a little (a whole step with
+  // the gather and with them: 51 k nodes 660 and 649 us, 104 k 839 and 817, 141 k 1053
+  // and 1027, 262 k 1612 and 1584), and are taken from 131073, where they were first measured.
   const bool bounds = mixed && D == 3 && s.nInt > 131072;
   if (mixed && !bounds) cast(std::integral_constant<int, kVoteSlots>{});
   if (ip.gradhCorrection) omegaGradh(s);
@@ -698,9 +700,8 @@ template <int D> void stepBody(Sim& s, const sphgpu_hydro_params& hp, const sphg
   enforceBoundaries(s);
 }
 
-// The clock of a plain simulation as one SegState, so that selectDt runs on
-// the device (k_seg_select_dt) and the step needs no host round trip before
-// its end.
+// The clock of a plain simulation as one SegState, so that the kernels of the step
+// select its dt (selectDt) and the step needs no host round trip before its end.
 __global__ void k_plain_seg_init(SegState* __restrict__ g, double t, double lastDt, double tEnd, double gamma,
                                  unsigned long long vote) {
   g->t = t;
@@ -726,8 +727,7 @@ __global__ void k_plain_seg_init(SegState* __restrict__ g, double t, double last
 // that key replay the graph; the host flags the step leaves are saved at the
 // capture and restored after each replay.  An ensemble whose membership and
 // ghost counts hold still (most steps of a tube ensemble) replays one graph
-// per step.  Graphs hold no memset node (the pair count is cleared by a
-// kernel) and no stage-timing events.
+// per step.  Graphs hold no memset node and no stage-timing events.
 Sim::StepFlags stepFlagsOf(const Sim& s) {
   return Sim::StepFlags{s.recValid, s.recSValid, s.recSMValid, s.derivsValid, s.pairsValid, s.haveDtIn,
                         s.pairRec, s.outStride, s.timingPending, s.pairWaves};
@@ -745,8 +745,9 @@ void restoreStepFlags(Sim& s, const Sim::StepFlags& f) {
   s.pairWaves = f.pairWaves;
 }
 
-// A few graphs and recent keys are kept: culling swaps the state fields with
-// their spares, so a step's buffers alternate between two sets.
+// A few graphs and recent keys are kept: culling swaps the ghosts' controls and planes
+// and the caller -> slot map with their spares, so a step's buffers alternate between
+// two sets.
 constexpr size_t kStepGraphs = 4;
 
 template <class F> void runStep(Sim& s, const sphgpu_hydro_params& hp, const sphgpu_integrator_params& ip, F&& launches) {

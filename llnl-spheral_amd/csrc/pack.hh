@@ -56,23 +56,22 @@ __device__ __forceinline__ void writeMixedRec(const double* r, int64_t nInt, dou
   }
 }
 // The FP64 isotropic pair kernel's record, 96 B per slot: x y z, 1/h (negative for
-// ghosts), m, 1/rho, c, P/rho^2/omega (a), v, 0 (b).  det H and m/rho are
-// recomputed by the loader.  230 MB at 2.4 M slots fit the 256 MB Infinity Cache,
+// ghosts), m, 1/rho, c, P/rho^2/omega, v, 0.  det H and m/rho are recomputed by
+// the loader.  230 MB at 2.4 M slots fit the 256 MB Infinity Cache,
 // and one plane beats two: the gather brings in 1.5 lines a record instead of 2
-// (loads of all records of the rows at 128^3: 2.15 ms, as 64 + 32 B 2.38 ms, one
-// to a 128-B line 2.55 ms).
+// (loads of all records of the rows at 128^3, in one run: 2.15 ms, as 64 + 32 B
+// 2.38 ms, one to a 128-B line 2.55 ms).
 template <int D>
-__device__ __forceinline__ void writeFast64Rec(const double* r, int64_t nInt, double2* __restrict__ a,
-                                               double2* __restrict__ b) {
+__device__ __forceinline__ void writeFast64Rec(const double* r, int64_t nInt, double2* __restrict__ p) {
   using R = RL<true>;
   const bool ghost = r[R::ORIG] >= double(nInt);
   const double rho = r[R::RHO];
-  a[0] = make_double2(r[R::X], D > 1 ? r[R::X + 1] : 0.0);
-  a[1] = make_double2(D > 2 ? r[R::X + 2] : 0.0, ghost ? -r[R::HINV] : r[R::HINV]);
-  a[2] = make_double2(r[R::M], rho != 0.0 ? 1.0 / rho : 0.0);
-  a[3] = make_double2(r[R::CS], r[R::PRHO]);
-  b[0] = make_double2(r[R::V], D > 1 ? r[R::V + 1] : 0.0);
-  b[1] = make_double2(D > 2 ? r[R::V + 2] : 0.0, 0.0);
+  p[0] = make_double2(r[R::X], D > 1 ? r[R::X + 1] : 0.0);
+  p[1] = make_double2(D > 2 ? r[R::X + 2] : 0.0, ghost ? -r[R::HINV] : r[R::HINV]);
+  p[2] = make_double2(r[R::M], rho != 0.0 ? 1.0 / rho : 0.0);
+  p[3] = make_double2(r[R::CS], r[R::PRHO]);
+  p[4] = make_double2(r[R::V], D > 1 ? r[R::V + 1] : 0.0);
+  p[5] = make_double2(D > 2 ? r[R::V + 2] : 0.0, 0.0);
 }
 
 // The density sum's neighbour record (DensRec).
@@ -150,7 +149,7 @@ __device__ __forceinline__ void storeRecords(int64_t k, const double* r, const P
   for (int c = 0; c < R::STRIDE / 2; ++c) dst[c] = make_double2(r[2 * c], r[2 * c + 1]);
   if constexpr ((SEC & 1) != 0) writeMixedRec<D>(r, o.nInt, o.qInv, static_cast<float4*>(o.sec) + k * MixedRec<D>::F4);
   if constexpr ((SEC & 2) != 0)
-    writeFast64Rec<D>(r, o.nInt, static_cast<double2*>(o.sec) + k * 6, static_cast<double2*>(o.sec) + k * 6 + 4);
+    writeFast64Rec<D>(r, o.nInt, static_cast<double2*>(o.sec) + k * 6);
   if constexpr ((SEC & 4) != 0) writeDensRec<D>(r, static_cast<double2*>(o.sec2) + k * 3);
   if constexpr ((SEC & 8) != 0) writeDensRecMixed<D>(r, static_cast<float4*>(o.sec3) + k * DensMixedRec<D>::F4);
 }
