@@ -61,9 +61,10 @@ template <int L> __device__ __forceinline__ int firstLane(bool c) {
 //     3-D 27 k 265 / 147, 51 k 280 / 249, 64 k 280 / 285; 69 k 528 / 317, 104 k 521 / 449,
 //         118 k 546 / 515, 125 k 528 / 546; 133 k 771 / 570, 166 k 772 / 707
 //     2-D 48 k 67 / 56, 58 k 67 / 69, 66 k 68 / 71; 66 k 95 / 76, 82 k 95 / 86, 102 k 99 / 111
-//   pairs, pair accelerations stored
-//     3-D 51 k 215 / 186, 64 k 224 / 217; 69 k 310 / 230, 91 k 327 / 308, 104 k 340 / 341,
-//         118 k 360 / 396; 133 k 523 / 431, 149 k 544 / 483, 166 k 560 / 539
+//   pairs, pair accelerations stored (five whole steps with the grad-h correction, ms)
+//     3-D 59 k 8.67 / 8.63; 80 k 9.79 / 9.17, 104 k 11.55 / 11.24, 118 k 12.26 / 12.17,
+//         125 k 12.66 / 12.74; 133 k 15.4 / 14.2, 149 k 16.3 / 15.5, 166 k 16.95 / 16.60
+//     2-D (one pass) 58 k 59 / 56, 66 k 60 / 58; 66 k 80 / 63, 82 k 81 / 69, 102 k 83 / 85
 //   pairs (search order, FP64)
 //     3-D 27 k 133 / 97, 39 k 139 / 133, 47 k 140 / 152
 //     2-D (tuned) 17 k 37 / 21, 48 k 43 / 40, 58 k 46 / 52
@@ -95,7 +96,7 @@ inline int rowLanes(RowPass pass, int dim, int64_t nodes) {
   constexpr int kMost[][2][kSteps] = {
       {{56, 80, 0, 0}, {56, 92, 136, 0}},         // kPairs
       {{56, 80, 0, 0}, {56, 116, 160, 0}},        // kPairsAnyH
-      {{56, 80, 0, 0}, {60, 100, 160, 0}},        // kPairsStored
+      {{64, 80, 0, 0}, {64, 116, 160, 0}},        // kPairsStored
       {{48, 0, 0, 0}, {40, 0, 0, 0}},             // kIsoPairs
       {{64, 128, 192, 256}, {64, 128, 0, 0}},     // kDensity
       {{64, 112, 192, 256}, {64, 112, 0, 0}},     // kDensityAnyH
