@@ -795,7 +795,12 @@ void setGhostNodes(Sim& s, double ext, bool doCull) {
   s.neighborsValid = false;
   s.recValid = false;
   s.derivsValid = false;
+  struct Pending {                       // neither outlives this call, however it ends
+    Sim& s;
+    ~Pending() { s.markGhostUse = s.genPending = false; }
+  };
   for (int64_t est = ghostGuess(s);; est *= 4) {
+    Pending pending{s};
     s.nTot = s.nInt;                     // drop the previous ghosts
     s.subStart.assign(s.subs.size() + 1, 0);
     if (!s.subs.empty()) {
@@ -809,15 +814,9 @@ void setGhostNodes(Sim& s, double ext, bool doCull) {
     try {
       buildNeighbors(s, ext);
       break;
-    } catch (const GhostCapacity&) {
-      s.markGhostUse = false;
-    } catch (...) {
-      s.markGhostUse = false;
-      s.genPending = false;
-      throw;
+    } catch (const GhostCapacity&) {     // again with room for four times as many
     }
   }
-  s.markGhostUse = false;
   SG_CHECK_HIP(hipEventRecord(s.ev[10], st));
   if (doCull) cull(s);
   SG_CHECK_HIP(hipEventRecord(s.ev[11], st));

@@ -439,7 +439,9 @@ void copyToHost(Sim& s, void* host, const void* dev, size_t bytes);
 void cullLaunch(Sim& s, SearchFlags* flagsOut, int32_t* starts);
 // Counts of a ghost generation, read back with the neighbour build's bounds;
 // throws GhostCapacity when its capacity was short.
-struct GhostCapacity {};
+struct GhostCapacity : Error {
+  GhostCapacity() : Error(SPHGPU_ERR_CAPACITY, "ghost capacity of a generation") {}
+};
 void finishGeneration(Sim& s, const int64_t* gen);
 
 // tune.cpp: launch-shape autotuner.  A workload class of one kernel family;

@@ -5,6 +5,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 static bool failDevice = false, failPinned = false;
@@ -57,6 +58,9 @@ void zeroMany(const ZeroSet& z, hipStream_t) {
 }  // namespace sphgpu
 
 using namespace sphgpu;
+
+// what the C entry points catch
+static_assert(std::is_base_of<Error, GhostCapacity>::value, "a generation's short capacity is an error like others");
 
 static int failures = 0;
 static void check(bool ok, const char* what) {
